@@ -72,6 +72,7 @@ def load_library() -> ctypes.CDLL:
     lib.cybq_destroy.argtypes = [vp]
     lib.cybq_destroy.restype = None
     lib.cybq_weight_upload.argtypes = [vp, ci, ci, i64, i64, vp, vp, ctypes.POINTER(vp)]
+    lib.cybq_weight_upload_many.argtypes = [vp, i64, vp, vp, vp, vp, vp, vp, vp]
     lib.cybq_weight_from_device.argtypes = [vp, ci, i64, i64, vp, vp, vp, ctypes.POINTER(vp)]
     lib.cybq_weight_clone.argtypes = [vp, vp, ctypes.POINTER(vp)]
     lib.cybq_weight_free.argtypes = [vp, vp]
@@ -249,12 +250,10 @@ class Backend:
         return self._lib.cybq_version().decode()
 
     # ---- weights
-    def upload(self, quant: int, layout: int, N: int, K: int, q: np.ndarray,
-               scales: Optional[np.ndarray] = None, name: Optional[str] = None) -> QWeight:
-        """Host interchange buffers -> device-native weight (repacked once, here)."""
+    @staticmethod
+    def _host_buffers(quant: int, layout: int, N: int, K: int, q, scales):
+        """(q, scales) contiguous and at least as large as the tensor: the library only sees addresses."""
         q = np.ascontiguousarray(q)
-        qp = q.ctypes.data_as(ctypes.c_void_p)
-        sp = None
         if N >= 1 and K >= 32 and K % 32 == 0 and quant in (formats.Q4, formats.Q8):
             groups = N * (K // 32)
             if layout == formats.PLANAR:
@@ -263,15 +262,38 @@ class Backend:
                 need_q, need_s = groups * (18 if quant == formats.Q4 else 34), 0
             if q.nbytes < need_q or (need_s and scales is not None and np.asarray(scales).nbytes < need_s):
                 raise CybqError(-2, "bad shape", f"host buffers are smaller than a [{N},{K}] Q{quant} tensor in this layout")
-        if scales is not None:
-            scales = np.ascontiguousarray(scales)
-            sp = scales.ctypes.data_as(ctypes.c_void_p)
+        return q, None if scales is None else np.ascontiguousarray(scales)
+
+    def upload(self, quant: int, layout: int, N: int, K: int, q: np.ndarray,
+               scales: Optional[np.ndarray] = None, name: Optional[str] = None) -> QWeight:
+        """Host interchange buffers -> device-native weight (repacked once, here)."""
+        q, scales = self._host_buffers(quant, layout, N, K, q, scales)
+        qp = q.ctypes.data_as(ctypes.c_void_p)
+        sp = None if scales is None else scales.ctypes.data_as(ctypes.c_void_p)
         out = ctypes.c_void_p()
         self._check(self._lib.cybq_weight_upload(self._ctx, quant, layout, N, K, qp, sp, ctypes.byref(out)))
         w = QWeight(self, out.value)
         if name is not None:
             self.weights[name] = w
         return w
+
+    def upload_many(self, tensors) -> list:
+        """cybq_weight_upload_many: a list of (quant, layout, N, K, q, scales or None, name or None), all or nothing.
+        A model switch in one call: copying, the bus and the repack overlap across the tensors."""
+        tensors = list(tensors)
+        keep = [self._host_buffers(*t[:6]) for t in tensors]
+        n = len(tensors)
+        ints, longs, ptrs = ctypes.c_int * n, ctypes.c_int64 * n, ctypes.c_void_p * n
+        out = ptrs()
+        self._check(self._lib.cybq_weight_upload_many(
+            self._ctx, n, ints(*[t[0] for t in tensors]), ints(*[t[1] for t in tensors]), longs(*[t[2] for t in tensors]),
+            longs(*[t[3] for t in tensors]), ptrs(*[q.ctypes.data for q, _ in keep]),
+            ptrs(*[None if s is None else s.ctypes.data for _, s in keep]), out))
+        ws = [QWeight(self, h) for h in out]
+        for t, w in zip(tensors, ws):
+            if t[6] is not None:
+                self.weights[t[6]] = w
+        return ws
 
     def upload_quantized(self, q: np.ndarray, scales: np.ndarray, quant: int, layout: int = formats.PLANAR,
                          name: Optional[str] = None) -> QWeight:

@@ -34,6 +34,7 @@ except ModuleNotFoundError:          # pragma: no cover
     import tomli as _toml
 
 DELIM = b"~~~"
+LOAD_BATCH_BYTES = 512 << 20
 
 
 class ContainerError(ValueError):
@@ -249,9 +250,16 @@ def load_into(backend, path: str) -> List[TensorRecord]:
     c = Container(path)
     try:
         recs = c.tensors()
+        # a few hundred MB per call: enough to keep the bus busy across tensors, and a model that replaces one of the
+        # same tensor names needs that much device memory on top, not twice its size
+        batch, held = [], 0
         for r in recs:
-            q, s = c.payload(r)
-            backend.upload(r.bits, r.layout_code, r.shape[0], r.shape[1], q, s, name=r.name)
+            batch.append((r.bits, r.layout_code, r.shape[0], r.shape[1], *c.payload(r), r.name))
+            held += r.nbytes + r.scales_nbytes
+            if held >= LOAD_BATCH_BYTES:
+                backend.upload_many(batch)
+                batch, held = [], 0
+        backend.upload_many(batch)
         return recs
     finally:
         c.close()

@@ -3,7 +3,7 @@
 // this boundary.
 #include <hip/hip_runtime.h>
 
-#include <cmath>
+#include <atomic>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -14,6 +14,8 @@
 #include "../../include/cybq.h"
 #include "cybq_debug.h"
 #include "cybq_internal.h"
+#include "pool.h"
+#include "upload.h"
 
 struct cybq_ctx {
     int device = 0;
@@ -23,6 +25,7 @@ struct cybq_ctx {
     void* workspace = nullptr;          // scratch for the prefill path, allocated once at init
     size_t workspace_bytes = 0;
     std::string last_error;
+    cybq::Uploader uploader;            // host memory -> native tiles; idle until the first upload
 };
 
 struct cybq_weight {
@@ -31,16 +34,15 @@ struct cybq_weight {
     int64_t N = 0, K = 0;
     int NT = 0, KT = 0;
     uint8_t* data = nullptr;            // native tiles (q words + scales per tile), strip-major
-    size_t bytes = 0;
+    size_t bytes = 0, block = 0;        // of the tiles; of the pool's block behind them
+    std::atomic<int> used_on{cybq::kUnused};        // streams that may still be reading `data` (pool.h)
     bool paired = false;                // made by cybq_weight_fuse_pairs: strips alternate gate / up
     // some |scale| * qmax exceeds what f16 holds: the prefill kernels, which form scale * q in
     // f16, would overflow; such a tensor takes the decode kernels (scale applied in fp32) for any M
     bool wide_scales = false;
-    // cybq_weight_from_device: the repack kernel ORs "some scale is wide" into a word behind the tiles and a
-    // copy of it to `scan_host` (pinned) is queued behind the kernel; the first call that needs the answer
-    // waits for `scan_done` (long since complete in practice) and moves it into wide_scales
-    hipEvent_t scan_done = nullptr;
-    uint32_t* scan_host = nullptr;
+    // cybq_weight_from_device: the repack kernel stores "some scale is wide" into a pinned word; the first call that
+    // needs the answer waits for the kernel (long since complete in practice) and moves it into wide_scales
+    cybq::ScanSlot scan;
     std::once_flag scan_once;
 };
 
@@ -126,38 +128,22 @@ cybq::WeightView view_of(const cybq_weight* w)
     return v;
 }
 
-// largest finite f16 magnitude a scale may have for scale * q to stay inside f16: 65504 / qmax
-bool scale_is_wide(uint16_t bits, int quant)
-{
-    const int e = (bits >> 10) & 31, m = bits & 1023;
-    if (e == 31) return true;                                  // Inf / NaN
-    const float v = e == 0 ? (float)m * (1.0f / 16777216.0f) : std::ldexp((float)(m + 1024), e - 25);
-    return v * (quant == CYBQ_Q4 ? 8.0f : 128.0f) > 65504.0f;
-}
-
-bool any_wide_scale(int quant, int layout, int64_t groups, const void* q, const void* scales)
-{
-    if (layout == CYBQ_LAYOUT_PLANAR) {
-        const uint16_t* s = static_cast<const uint16_t*>(scales);
-        for (int64_t g = 0; g < groups; g++)
-            if (scale_is_wide(s[g], quant)) return true;
-        return false;
-    }
-    const size_t bs = quant == CYBQ_Q4 ? 18 : 34;
-    const uint8_t* b = static_cast<const uint8_t*>(q);
-    for (int64_t g = 0; g < groups; g++)
-        if (scale_is_wide((uint16_t)(b[g * bs] | (b[g * bs + 1] << 8)), quant)) return true;
-    return false;
-}
-
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 size_t dtype_size(int dt) { return dt == CYBQ_F32 ? 4 : 2; }
 bool dtype_ok(int dt) { return dt == CYBQ_F32 || dt == CYBQ_F16 || dt == CYBQ_BF16; }
 
-constexpr size_t kWeightTailBytes = 256;
+// work that reads the weight has been queued on `stream`
+void mark_use(const cybq_weight* cw, const void* stream)
+{
+    cybq_weight* w = const_cast<cybq_weight*>(cw);
+    const int where = stream ? cybq::kElsewhere : cybq::kDefaultStream;
+    int seen = w->used_on.load(std::memory_order_relaxed);
+    while (seen < where && !w->used_on.compare_exchange_weak(seen, where, std::memory_order_relaxed)) {
+    }
+}
 
-int alloc_weight(cybq_ctx* ctx, int bits, int64_t N, int64_t K, cybq_weight** out)
+int alloc_weight(cybq_ctx* ctx, int bits, int64_t N, int64_t K, cybq::UsedOn first_use, cybq_weight** out)
 {
     cybq_weight* w = new (std::nothrow) cybq_weight();
     if (!w) return fail(ctx, CYBQ_ERR_NOMEM, "host allocation failed");
@@ -168,7 +154,7 @@ int alloc_weight(cybq_ctx* ctx, int bits, int64_t N, int64_t K, cybq_weight** ou
     w->NT = (int)((N + cybq::kTileN - 1) / cybq::kTileN);
     w->KT = (int)((K + cybq::kTileK - 1) / cybq::kTileK);
     w->bytes = (size_t)w->NT * w->KT * cybq::tile_bytes(bits);
-    hipError_t e = hipMalloc(reinterpret_cast<void**>(&w->data), w->bytes + kWeightTailBytes);      // (tail: the scan's flag word)
+    hipError_t e = cybq::pool_alloc(ctx->device, w->bytes, first_use, reinterpret_cast<void**>(&w->data), &w->block);
     if (e != hipSuccess) {
         delete w;
         return fail_hip(ctx, e, "hipMalloc(weight)");
@@ -179,9 +165,8 @@ int alloc_weight(cybq_ctx* ctx, int bits, int64_t N, int64_t K, cybq_weight** ou
 
 void release_weight(cybq_weight* w)
 {
-    if (w->scan_done) (void)hipEventDestroy(w->scan_done);
-    if (w->scan_host) (void)hipHostFree(w->scan_host);
-    (void)hipFree(w->data);
+    cybq::scan_release(w->device, w->scan);
+    cybq::pool_free(w->device, w->data, w->block, static_cast<cybq::UsedOn>(w->used_on.load(std::memory_order_relaxed)));
     delete w;
 }
 
@@ -189,10 +174,10 @@ void release_weight(cybq_weight* w)
 bool weight_is_wide(const cybq_weight* cw)
 {
     cybq_weight* w = const_cast<cybq_weight*>(cw);
-    if (w->scan_host) {
+    if (w->scan.word) {
         std::call_once(w->scan_once, [w]() {
-            if (w->scan_done) (void)hipEventSynchronize(w->scan_done);
-            w->wide_scales = w->wide_scales || *w->scan_host != 0u;
+            (void)hipEventSynchronize(w->scan.done);
+            w->wide_scales = w->wide_scales || *w->scan.word != 0u;
         });
     }
     return w->wide_scales;
@@ -277,6 +262,7 @@ int cybq_init(int device, cybq_ctx** out)
         delete ctx;
         return CYBQ_ERR_HIP;
     }
+    cybq::pool_retain(device);
     *out = ctx;
     return CYBQ_OK;
 }
@@ -284,8 +270,62 @@ int cybq_init(int device, cybq_ctx** out)
 void cybq_destroy(cybq_ctx* ctx)
 {
     if (!ctx) return;
-    if (ctx->workspace && hipSetDevice(ctx->device) == hipSuccess) (void)hipFree(ctx->workspace);
+    const int device = ctx->device;
+    if (hipSetDevice(device) == hipSuccess && ctx->workspace) (void)hipFree(ctx->workspace);
     delete ctx;
+    cybq::pool_release(device);
+}
+
+int cybq_weight_upload_many(cybq_ctx* ctx, int64_t count, const int* quant, const int* layout, const int64_t* N, const int64_t* K,
+                            const void* const* q, const void* const* scales, cybq_weight** out)
+{
+    if (!ctx) return CYBQ_ERR_INVALID;
+    if (count < 0 || (count > 0 && (!quant || !layout || !N || !K || !q || !out))) return fail(ctx, CYBQ_ERR_INVALID, "bad tensor list");
+    for (int64_t i = 0; i < count; i++) out[i] = nullptr;
+    for (int64_t i = 0; i < count; i++) {
+        const void* s = scales ? scales[i] : nullptr;
+        if (!q[i]) return fail(ctx, CYBQ_ERR_INVALID, "q is NULL");
+        if (layout[i] != CYBQ_LAYOUT_PLANAR && layout[i] != CYBQ_LAYOUT_BLOCK_AOS)
+            return fail(ctx, CYBQ_ERR_INVALID, "unknown layout");
+        if (layout[i] == CYBQ_LAYOUT_PLANAR && !s) return fail(ctx, CYBQ_ERR_INVALID, "PLANAR needs a scale plane");
+        if (layout[i] == CYBQ_LAYOUT_BLOCK_AOS && s) return fail(ctx, CYBQ_ERR_INVALID, "BLOCK_AOS carries its scales; pass NULL");
+        int rc = check_weight_shape(ctx, quant[i], N[i], K[i]);
+        if (rc) return rc;
+    }
+    DeviceGuard guard(ctx->device);
+    if (guard.err != hipSuccess) return fail_hip(ctx, guard.err, "hipSetDevice");
+    int rc = CYBQ_OK;
+    try {
+        std::vector<cybq::UploadItem> items((size_t)count);
+        for (int64_t i = 0; i < count && rc == CYBQ_OK; i++) {
+            rc = alloc_weight(ctx, quant[i], N[i], K[i], cybq::kElsewhere, &out[i]);
+            if (rc) break;
+            cybq::UploadItem& it = items[(size_t)i];
+            it.quant = quant[i];
+            it.layout = layout[i];
+            it.N = N[i];
+            it.K = K[i];
+            it.q = q[i];
+            it.scales = scales ? scales[i] : nullptr;
+            it.dst = out[i]->data;
+            it.NT = out[i]->NT;
+            it.KT = out[i]->KT;
+        }
+        if (rc == CYBQ_OK && count) {
+            const hipError_t e = ctx->uploader.run(items.data(), count);
+            if (e != hipSuccess) rc = fail_hip(ctx, e, "weight upload");
+            for (int64_t i = 0; i < count; i++) out[i]->wide_scales = items[(size_t)i].wide;
+        }
+    } catch (const std::bad_alloc&) {
+        rc = fail(ctx, CYBQ_ERR_NOMEM, "host allocation failed");
+    }
+    if (rc)
+        for (int64_t i = 0; i < count; i++)
+            if (out[i]) {
+                release_weight(out[i]);
+                out[i] = nullptr;
+            }
+    return rc;
 }
 
 int cybq_weight_upload(cybq_ctx* ctx, cybq_quant quant, cybq_layout layout, int64_t N, int64_t K,
@@ -293,52 +333,8 @@ int cybq_weight_upload(cybq_ctx* ctx, cybq_quant quant, cybq_layout layout, int6
 {
     if (!ctx) return CYBQ_ERR_INVALID;
     if (!out) return fail(ctx, CYBQ_ERR_INVALID, "out is NULL");
-    *out = nullptr;
-    if (!q) return fail(ctx, CYBQ_ERR_INVALID, "q is NULL");
-    if (layout != CYBQ_LAYOUT_PLANAR && layout != CYBQ_LAYOUT_BLOCK_AOS)
-        return fail(ctx, CYBQ_ERR_INVALID, "unknown layout");
-    if (layout == CYBQ_LAYOUT_PLANAR && !scales) return fail(ctx, CYBQ_ERR_INVALID, "PLANAR needs a scale plane");
-    if (layout == CYBQ_LAYOUT_BLOCK_AOS && scales) return fail(ctx, CYBQ_ERR_INVALID, "BLOCK_AOS carries its scales; pass NULL");
-    int rc = check_weight_shape(ctx, quant, N, K);
-    if (rc) return rc;
-    DeviceGuard guard(ctx->device);
-    if (guard.err != hipSuccess) return fail_hip(ctx, guard.err, "hipSetDevice");
-
-    const int64_t groups = N * (K / CYBQ_GROUP);
-    size_t q_src_bytes, s_src_bytes = 0;
-    if (layout == CYBQ_LAYOUT_PLANAR) {
-        q_src_bytes = (size_t)(quant == CYBQ_Q4 ? N * K / 2 : N * K);
-        s_src_bytes = (size_t)groups * 2;
-    } else {
-        q_src_bytes = (size_t)groups * (quant == CYBQ_Q4 ? 18 : 34);
-    }
-    void *q_tmp = nullptr, *s_tmp = nullptr;
-    hipError_t e = hipMalloc(&q_tmp, q_src_bytes);
-    if (e == hipSuccess && s_src_bytes) e = hipMalloc(&s_tmp, s_src_bytes);
-    if (e != hipSuccess) {
-        if (q_tmp) (void)hipFree(q_tmp);
-        return fail_hip(ctx, e, "hipMalloc(staging)");
-    }
-    cybq_weight* w = nullptr;
-    rc = alloc_weight(ctx, quant, N, K, &w);
-    if (rc == CYBQ_OK) {
-        e = hipMemcpy(q_tmp, q, q_src_bytes, hipMemcpyHostToDevice);
-        if (e == hipSuccess && s_src_bytes) e = hipMemcpy(s_tmp, scales, s_src_bytes, hipMemcpyHostToDevice);
-        if (e == hipSuccess)
-            e = cybq::launch_repack(quant, layout, q_tmp, s_tmp, w->data, (int)N, (int)K, w->NT, w->KT, nullptr, nullptr);
-        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
-        if (e != hipSuccess) {
-            rc = fail_hip(ctx, e, "weight upload");
-            release_weight(w);
-            w = nullptr;
-        }
-    }
-    (void)hipFree(q_tmp);
-    if (s_tmp) (void)hipFree(s_tmp);
-    if (rc) return rc;
-    w->wide_scales = any_wide_scale(quant, layout, groups, q, scales);
-    *out = w;
-    return CYBQ_OK;
+    const int quant_code = quant, layout_code = layout;
+    return cybq_weight_upload_many(ctx, 1, &quant_code, &layout_code, &N, &K, &q, &scales, out);
 }
 
 int cybq_weight_from_device(cybq_ctx* ctx, cybq_quant quant, int64_t N, int64_t K, const void* q_dev,
@@ -355,22 +351,18 @@ int cybq_weight_from_device(cybq_ctx* ctx, cybq_quant quant, int64_t N, int64_t 
     DeviceGuard guard(ctx->device);
     if (guard.err != hipSuccess) return fail_hip(ctx, guard.err, "hipSetDevice");
     cybq_weight* w = nullptr;
-    rc = alloc_weight(ctx, quant, N, K, &w);
+    rc = alloc_weight(ctx, quant, N, K, stream ? cybq::kElsewhere : cybq::kDefaultStream, &w);
     if (rc) return rc;
-    // the scales are scanned by the repack kernel itself: a word behind the tiles collects "some |scale| * qmax leaves
-    // f16", its copy to pinned host memory is queued behind the kernel and read by the first call that needs it
+    // the scales are scanned by the repack kernel itself: it stores 1 into a pinned word where "some |scale| * qmax leaves
+    // f16", and the first call that needs the word waits for the event behind the kernel
     hipStream_t st = static_cast<hipStream_t>(stream);
-    uint32_t* flag = reinterpret_cast<uint32_t*>(w->data + w->bytes);
-    hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&w->scan_host), sizeof(uint32_t), hipHostMallocDefault);
+    hipError_t e = cybq::scan_acquire(ctx->device, &w->scan);
     if (e == hipSuccess) {
-        *w->scan_host = 0u;
-        e = hipEventCreateWithFlags(&w->scan_done, hipEventDisableTiming);
+        *w->scan.word = 0u;
+        e = cybq::launch_repack(quant, CYBQ_LAYOUT_PLANAR, false, q_dev, scales_dev, w->data, (int)N, (int)K, w->NT, w->KT, w->scan.word, st);
     }
-    if (e == hipSuccess) e = hipMemsetAsync(flag, 0, sizeof(uint32_t), st);
-    if (e == hipSuccess)
-        e = cybq::launch_repack(quant, CYBQ_LAYOUT_PLANAR, q_dev, scales_dev, w->data, (int)N, (int)K, w->NT, w->KT, flag, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(w->scan_host, flag, sizeof(uint32_t), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipEventRecord(w->scan_done, st);
+    if (e == hipSuccess) e = hipEventRecord(w->scan.done, st);
+    mark_use(w, stream);
     if (e != hipSuccess) {
         (void)hipStreamSynchronize(st);          // nothing may still write the pinned word
         release_weight(w);
@@ -389,7 +381,11 @@ int cybq_weight_clone(cybq_ctx* ctx, const cybq_weight* src, cybq_weight** out)
     DeviceGuard guard(ctx->device);
     if (guard.err != hipSuccess) return fail_hip(ctx, guard.err, "hipSetDevice");
     cybq_weight* w = nullptr;
-    int rc = alloc_weight(ctx, src->bits, src->N, src->K, &w);
+    int rc = alloc_weight(ctx, src->bits, src->N, src->K, cybq::kDefaultStream, &w);
+    if (rc == CYBQ_OK) {
+        mark_use(w, nullptr);
+        mark_use(src, nullptr);
+    }
     if (rc) return rc;
     hipError_t e = hipMemcpy(w->data, src->data, src->bytes, hipMemcpyDeviceToDevice);
     if (e != hipSuccess) {
@@ -405,14 +401,12 @@ int cybq_weight_clone(cybq_ctx* ctx, const cybq_weight* src, cybq_weight** out)
 int cybq_weight_free(cybq_ctx* ctx, cybq_weight* w)
 {
     if (!w) return CYBQ_OK;
-    hipError_t e = hipSetDevice(w->device);
-    if (e == hipSuccess) {
-        if (w->scan_done) (void)hipEventDestroy(w->scan_done);
-        if (w->scan_host) (void)hipHostFree(w->scan_host);
-        e = hipFree(w->data);
+    const hipError_t e = hipSetDevice(w->device);
+    if (e != hipSuccess) {
+        delete w;
+        return fail_hip(ctx, e, "hipSetDevice");
     }
-    delete w;
-    if (e != hipSuccess) return fail_hip(ctx, e, "hipFree(weight)");
+    release_weight(w);
     return CYBQ_OK;
 }
 
@@ -462,6 +456,7 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
     if (guard.err != hipSuccess) return fail_hip(ctx, guard.err, "hipSetDevice");
     hipStream_t st = static_cast<hipStream_t>(stream);
     cybq::WeightView v = view_of(w);
+    mark_use(w, stream);
     hipError_t e;
     // the tail of the scratch belongs to the decode kernels (tickets and slabs of a K split), the rest to prefill
     void* dscr = nullptr;
@@ -571,7 +566,7 @@ int cybq_weight_fuse_pairs(cybq_ctx* ctx, const cybq_weight* gate, const cybq_we
     DeviceGuard guard(ctx->device);
     if (guard.err != hipSuccess) return fail_hip(ctx, guard.err, "hipSetDevice");
     cybq_weight* w = nullptr;
-    int rc = alloc_weight(ctx, gate->bits, 2 * gate->N, gate->K, &w);
+    int rc = alloc_weight(ctx, gate->bits, 2 * gate->N, gate->K, cybq::kDefaultStream, &w);
     if (rc) return rc;
     // the native layout is strip-major: output strip 2i is gate strip i, 2i+1 is up strip i
     const size_t sb = (size_t)gate->KT * cybq::tile_bytes(gate->bits);          // bytes of one strip
@@ -653,6 +648,7 @@ int cybq_dequant(cybq_ctx* ctx, const cybq_weight* w, float* out, void* stream)
     if (!aligned16(out)) return fail(ctx, CYBQ_ERR_ALIGN, "out must be 16-byte aligned");
     DeviceGuard guard(ctx->device);
     if (guard.err != hipSuccess) return fail_hip(ctx, guard.err, "hipSetDevice");
+    mark_use(w, stream);
     hipError_t e = cybq::launch_dequant(view_of(w), out, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail_hip(ctx, e, "dequant launch");
     return CYBQ_OK;
@@ -698,6 +694,7 @@ int cybq_debug_read_weight(cybq_ctx* ctx, int64_t count, const cybq_weight* cons
     if (guard.err != hipSuccess) return fail_hip(ctx, guard.err, "hipSetDevice");
     for (int64_t i = 0; i < count; i++) {
         if (!w[i]) return fail(ctx, CYBQ_ERR_INVALID, "w[i] is NULL");
+        mark_use(w[i], stream);
         hipError_t e = cybq::launch_read_probe(view_of(w[i]), with_io != 0, x, y, static_cast<hipStream_t>(stream));
         if (e == hipErrorInvalidValue) {
             (void)hipGetLastError();
@@ -716,6 +713,7 @@ int cybq_debug_read_pattern(cybq_ctx* ctx, int64_t count, const cybq_weight* con
     if (guard.err != hipSuccess) return fail_hip(ctx, guard.err, "hipSetDevice");
     for (int64_t i = 0; i < count; i++) {
         if (!w[i]) return fail(ctx, CYBQ_ERR_INVALID, "w[i] is NULL");
+        mark_use(w[i], stream);
         hipError_t e = cybq::launch_read_pattern(view_of(w[i]), pattern, ctx->num_cus, static_cast<hipStream_t>(stream));
         if (e == hipErrorInvalidValue) {
             (void)hipGetLastError();

@@ -13,9 +13,10 @@ namespace cybq {
 // dtype codes mirror enum cybq_dtype
 constexpr int kF32 = 0, kF16 = 1, kBF16 = 2;
 
-// q: PLANAR q plane (4-byte aligned) with `scales`, or BLOCK_AOS blocks (2-byte aligned, scales unused)
-// wide_flag: device word that receives 1 when some scale times the largest q leaves f16 (nullptr: no scan)
-hipError_t launch_repack(int bits, int layout, const void* q, const void* scales, uint8_t* dst, int N, int K, int NT, int KT,
+// q: PLANAR q plane (4-byte aligned) with `scales`, or BLOCK_AOS blocks (16-byte aligned with 15 readable bytes behind
+// them, scales unused); device memory, or pinned host memory that the kernel reads across the bus (from_host)
+// wide_flag: word (device or pinned host memory) that receives 1 when some scale times the largest q leaves f16 (nullptr: no scan)
+hipError_t launch_repack(int bits, int layout, bool from_host, const void* q, const void* scales, uint8_t* dst, int N, int K, int NT, int KT,
                          uint32_t* wide_flag, hipStream_t st);
 hipError_t launch_dequant(const WeightView& w, float* out, hipStream_t st);
 

@@ -51,24 +51,29 @@ __device__ __forceinline__ void staged_q4_octet(const uint8_t* row, int gl, int 
     }
 }
 
-// One workgroup repacks CT consecutive K tiles of one 16-row strip.  The source rows of
+// One workgroup (CT = kRepackTiles or kRepackTilesHost) repacks CT consecutive K tiles of one 16-row strip.  The source rows of
 // that piece are first copied into LDS with coalesced loads (a row's piece is one
 // contiguous run in either interchange layout), then every thread assembles one lane's
 // share of a native tile from LDS - a few aligned words and a handful of bit operations -
 // and stores it with 128-bit stores: global memory only sees whole runs, the gathering
 // stays inside the CU.
+// Sources in device memory: four tiles, one per wave.  Sources in pinned host memory, read across the bus: runs of
+// 2 KiB per row (a whole strip of a 4096-wide tensor), because every run that does not end on a 64-byte line fetches
+// that line twice (4 MiB pieces of Q4 blocks: 36 GB/s with four tiles, 52 with 32).
 constexpr int kRepackTiles = 4;
+template <int BITS> constexpr int kRepackTilesHost = BITS == 4 ? 32 : 16;
 
-template <int BITS, int LAYOUT>
+template <int BITS, int LAYOUT, int CT>
 __global__ __launch_bounds__(256) void repack_kernel(const uint8_t* __restrict__ q, const uint16_t* __restrict__ scales,
                                                       uint8_t* __restrict__ dst, int N, int K, int KT, uint32_t* __restrict__ wide_flag)
 {
-    constexpr int CT = kRepackTiles;
     constexpr int GB = kSrcGroupBytes<BITS, LAYOUT>;
     constexpr int ROWB = CT * kGroupsPerTile * GB;                  // bytes of one row's piece
-    constexpr int UNIT = LAYOUT == 0 ? 16 : 2;                      // load width the source alignment allows
-    constexpr int UPR = ROWB / UNIT;                                // units per row
-    constexpr int PITCH = ROWB + (LAYOUT == 0 ? 16 : 4);            // (rows land in different LDS banks)
+    // A row's piece is read as the 16-byte units that cover it: PLANAR pieces start on one, a BLOCK_AOS piece (18- or
+    // 34-byte blocks) up to 15 bytes into its first one (`head`); what a unit holds beyond the piece is the neighbouring
+    // groups, or up to 15 bytes behind the buffer (its owner leaves room), and is not used.
+    constexpr int UPR = (ROWB + (LAYOUT == 0 ? 0 : 30)) / 16;       // units per row
+    constexpr int PITCH = UPR * 16 + 16;                             // (rows land in different LDS banks)
     __shared__ __attribute__((aligned(16))) uint8_t rows[kTileN][PITCH];
 
     const int t = threadIdx.x;
@@ -77,67 +82,70 @@ __global__ __launch_bounds__(256) void repack_kernel(const uint8_t* __restrict__
     const int G = K / kGroup;
     const int g0 = kt0 * kGroupsPerTile;
     const int ng = min(CT * kGroupsPerTile, G - g0);                // groups of this piece that exist
+    auto head = [&](int r) -> int { return LAYOUT == 0 ? 0 : (int)((((int64_t)nt * kTileN + r) * G + g0) * GB & 15); };
     for (int i = t; i < kTileN * UPR; i += 256) {
         const int r = i / UPR, u = i - r * UPR;
         const int64_t n = (int64_t)nt * kTileN + r;
-        if (n < N && u * UNIT < ng * GB) {
-            const uint8_t* src = q + (n * G + g0) * GB + u * UNIT;
-            if (UNIT == 16) *reinterpret_cast<u32x4_t*>(&rows[r][u * 16]) = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(src));
-            else *reinterpret_cast<uint16_t*>(&rows[r][u * 2]) = *reinterpret_cast<const uint16_t*>(src);
+        if (n < N && u * 16 < head(r) + ng * GB) {
+            const uint8_t* src = q + (n * G + g0) * GB - head(r) + u * 16;
+            *reinterpret_cast<u32x4_t*>(&rows[r][u * 16]) = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(src));
         }
     }
     __syncthreads();
 
-    const int b = t >> 6, lane = t & 63;
-    const int kt = kt0 + b;
-    if (kt >= KT) return;
+    const int lane = t & 63;
     const int row = lane & 15, oct = lane >> 4;
     const bool row_ok = (int64_t)nt * kTileN + row < N;
-    uint8_t* tile = dst + ((int64_t)nt * KT + kt) * kTileBytes<BITS>;
-    if (BITS == 4) {
-        uint32_t w[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int gl = b * 4 + j;
-            uint32_t lo = 0x08080808u, hi = 0x08080808u;             // q = 0 where the source has nothing
-            if (row_ok && gl < ng) staged_q4_octet<LAYOUT>(rows[row], gl, oct, lo, hi);
-            w[2 * (j >> 1)] |= lo << (4 * (j & 1));
-            w[2 * (j >> 1) + 1] |= hi << (4 * (j & 1));
-        }
-        reinterpret_cast<u32x4_t*>(tile)[lane] = (u32x4_t){w[0], w[1], w[2], w[3]};
-    } else {
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
+    const uint8_t* const my_row = rows[row] + head(row);
+    for (int b = t >> 6; b < CT; b += 4) {
+        const int kt = kt0 + b;
+        if (kt >= KT) return;
+        uint8_t* tile = dst + ((int64_t)nt * KT + kt) * kTileBytes<BITS>;
+        if (BITS == 4) {
             uint32_t w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-            for (int wd = 0; wd < 4; wd++) {
-                const int gl = b * 4 + 2 * h + (wd >> 1);
-                const bool ok = row_ok && gl < ng;
-#pragma unroll
-                for (int s = 0; s < 4; s++) {
-                    const int v = ok ? staged_weight<8, LAYOUT>(rows[row], gl, oct * 8 + (wd & 1) * 4 + s) : 0;
-                    w[wd] |= (uint32_t)((v + 128) & 255) << (8 * s);
-                }
+            for (int j = 0; j < 4; j++) {
+                const int gl = b * 4 + j;
+                uint32_t lo = 0x08080808u, hi = 0x08080808u;             // q = 0 where the source has nothing
+                if (row_ok && gl < ng) staged_q4_octet<LAYOUT>(my_row, gl, oct, lo, hi);
+                w[2 * (j >> 1)] |= lo << (4 * (j & 1));
+                w[2 * (j >> 1) + 1] |= hi << (4 * (j & 1));
             }
-            reinterpret_cast<u32x4_t*>(tile)[h * 64 + lane] = (u32x4_t){w[0], w[1], w[2], w[3]};
+            reinterpret_cast<u32x4_t*>(tile)[lane] = (u32x4_t){w[0], w[1], w[2], w[3]};
+        } else {
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+                for (int wd = 0; wd < 4; wd++) {
+                    const int gl = b * 4 + 2 * h + (wd >> 1);
+                    const bool ok = row_ok && gl < ng;
+#pragma unroll
+                    for (int s = 0; s < 4; s++) {
+                        const int v = ok ? staged_weight<8, LAYOUT>(my_row, gl, oct * 8 + (wd & 1) * 4 + s) : 0;
+                        w[wd] |= (uint32_t)((v + 128) & 255) << (8 * s);
+                    }
+                }
+                reinterpret_cast<u32x4_t*>(tile)[h * 64 + lane] = (u32x4_t){w[0], w[1], w[2], w[3]};
+            }
         }
-    }
-    // the tile's 64 scales: [row][group]
-    {
-        const int r = lane >> 2, j = lane & 3;
-        const int gl = b * 4 + j;
-        const int64_t n = (int64_t)nt * kTileN + r;
-        uint16_t v = 0;
-        if (n < N && gl < ng) {
-            if (LAYOUT == 0) v = scales[n * G + g0 + gl];
-            else v = (uint16_t)(rows[r][gl * GB] | (rows[r][gl * GB + 1] << 8));
-        }
-        reinterpret_cast<uint16_t*>(tile + kTileQBytes<BITS>)[lane] = v;
-        // a scale whose product with the largest q leaves f16 (or that is not finite): the prefill kernels, which
-        // form scale * q in f16, cannot serve this tensor; every thread that sees one stores the same 1
-        if (wide_flag) {
-            const bool wide = ((v >> 10) & 31u) == 31u || f16_bits_to_f32(v & 0x7fffu) * (BITS == 4 ? 8.0f : 128.0f) > 65504.0f;
-            if (wide) *wide_flag = 1u;
+        // the tile's 64 scales: [row][group]
+        {
+            const int r = lane >> 2, j = lane & 3;
+            const int gl = b * 4 + j;
+            const int64_t n = (int64_t)nt * kTileN + r;
+            uint16_t v = 0;
+            if (n < N && gl < ng) {
+                if (LAYOUT == 0) v = scales[n * G + g0 + gl];
+                else v = (uint16_t)(rows[r][head(r) + gl * GB] | (rows[r][head(r) + gl * GB + 1] << 8));
+            }
+            reinterpret_cast<uint16_t*>(tile + kTileQBytes<BITS>)[lane] = v;
+            // a scale whose product with the largest q leaves f16 (or that is not finite): the prefill kernels, which
+            // form scale * q in f16, cannot serve this tensor; every thread that sees one stores the same 1
+            if (wide_flag) {
+                const bool wide = ((v >> 10) & 31u) == 31u || f16_bits_to_f32(v & 0x7fffu) * (BITS == 4 ? 8.0f : 128.0f) > 65504.0f;
+                if (wide) *wide_flag = 1u;
+            }
         }
     }
 }
@@ -174,26 +182,34 @@ __global__ void dequant_kernel(WeightView w, float* __restrict__ out)
     o[1] = make_float4(v[4], v[5], v[6], v[7]);
 }
 
-template <int BITS, int LAYOUT>
-hipError_t launch_repack_t(const void* q, const void* scales, uint8_t* dst, int N, int K, int NT, int KT, uint32_t* wide_flag,
+template <int BITS, int LAYOUT, int CT>
+hipError_t launch_repack_c(const void* q, const void* scales, uint8_t* dst, int N, int K, int NT, int KT, uint32_t* wide_flag,
                            hipStream_t st)
 {
-    const int64_t groups = (int64_t)((KT + kRepackTiles - 1) / kRepackTiles) * NT;
+    const int64_t groups = (int64_t)((KT + CT - 1) / CT) * NT;
     if (groups > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((repack_kernel<BITS, LAYOUT>), dim3((unsigned)groups), dim3(256), 0, st, (const uint8_t*)q, (const uint16_t*)scales, dst, N, K,
+    hipLaunchKernelGGL((repack_kernel<BITS, LAYOUT, CT>), dim3((unsigned)groups), dim3(256), 0, st, (const uint8_t*)q, (const uint16_t*)scales, dst, N, K,
                        KT, wide_flag);
     return hipGetLastError();
 }
 
+template <int BITS, int LAYOUT>
+hipError_t launch_repack_t(bool from_host, const void* q, const void* scales, uint8_t* dst, int N, int K, int NT, int KT, uint32_t* wide_flag,
+                           hipStream_t st)
+{
+    if (from_host) return launch_repack_c<BITS, LAYOUT, kRepackTilesHost<BITS>>(q, scales, dst, N, K, NT, KT, wide_flag, st);
+    return launch_repack_c<BITS, LAYOUT, kRepackTiles>(q, scales, dst, N, K, NT, KT, wide_flag, st);
+}
+
 }  // namespace
 
-hipError_t launch_repack(int bits, int layout, const void* q, const void* scales, uint8_t* dst, int N, int K, int NT, int KT,
+hipError_t launch_repack(int bits, int layout, bool from_host, const void* q, const void* scales, uint8_t* dst, int N, int K, int NT, int KT,
                          uint32_t* wide_flag, hipStream_t st)
 {
-    if (bits == 4 && layout == 0) return launch_repack_t<4, 0>(q, scales, dst, N, K, NT, KT, wide_flag, st);
-    if (bits == 4 && layout == 1) return launch_repack_t<4, 1>(q, scales, dst, N, K, NT, KT, wide_flag, st);
-    if (bits == 8 && layout == 0) return launch_repack_t<8, 0>(q, scales, dst, N, K, NT, KT, wide_flag, st);
-    if (bits == 8 && layout == 1) return launch_repack_t<8, 1>(q, scales, dst, N, K, NT, KT, wide_flag, st);
+    if (bits == 4 && layout == 0) return launch_repack_t<4, 0>(from_host, q, scales, dst, N, K, NT, KT, wide_flag, st);
+    if (bits == 4 && layout == 1) return launch_repack_t<4, 1>(from_host, q, scales, dst, N, K, NT, KT, wide_flag, st);
+    if (bits == 8 && layout == 0) return launch_repack_t<8, 0>(from_host, q, scales, dst, N, K, NT, KT, wide_flag, st);
+    if (bits == 8 && layout == 1) return launch_repack_t<8, 1>(from_host, q, scales, dst, N, K, NT, KT, wide_flag, st);
     return hipErrorInvalidValue;
 }
 

@@ -1,0 +1,142 @@
+// pool.hip - see pool.h.  Host code only.  Callers have made `device` current.
+#include "pool.h"
+
+#include <deque>
+#include <list>
+#include <map>
+#include <mutex>
+#include <vector>
+
+namespace cybq {
+
+namespace {
+
+constexpr size_t kGrain = (size_t)64 << 10;             // blocks are multiples of it
+constexpr size_t kScanWords = 1024;                     // pinned words per slab
+constexpr size_t kScanPitch = 16;                       // (words of different tensors on different host cache lines)
+
+struct Block {
+    void* p;
+    size_t bytes;
+    UsedOn used_on;
+};
+
+struct DevicePool {
+    std::mutex m;
+    int contexts = 0;
+    std::list<Block> blocks;                            // oldest first
+    size_t held = 0;
+    std::deque<ScanSlot> scans;                         // free slots, the longest free first
+    std::vector<void*> slabs;                           // pinned memory behind the words; kept for the process
+};
+
+DevicePool& pool_of(int device)
+{
+    static std::mutex m;
+    static std::map<int, DevicePool>* pools = new std::map<int, DevicePool>();      // (never destroyed: handles may be freed at exit)
+    std::lock_guard<std::mutex> lock(m);
+    return (*pools)[device];
+}
+
+void empty(DevicePool& pool)                            // pool.m held
+{
+    for (const Block& b : pool.blocks) (void)hipFree(b.p);
+    pool.blocks.clear();
+    pool.held = 0;
+}
+
+}  // namespace
+
+void pool_retain(int device)
+{
+    DevicePool& pool = pool_of(device);
+    std::lock_guard<std::mutex> lock(pool.m);
+    pool.contexts++;
+}
+
+void pool_release(int device)
+{
+    DevicePool& pool = pool_of(device);
+    std::lock_guard<std::mutex> lock(pool.m);
+    if (--pool.contexts == 0) empty(pool);
+}
+
+hipError_t pool_alloc(int device, size_t bytes, UsedOn first_use, void** p, size_t* block)
+{
+    bytes = (bytes + kGrain - 1) / kGrain * kGrain;
+    DevicePool& pool = pool_of(device);
+    std::lock_guard<std::mutex> lock(pool.m);
+    // the smallest block that holds it, if that wastes no more than a quarter
+    auto best = pool.blocks.end();
+    for (auto it = pool.blocks.begin(); it != pool.blocks.end(); ++it)
+        if (it->bytes >= bytes && it->bytes - bytes <= bytes / 4 && (best == pool.blocks.end() || it->bytes < best->bytes)) best = it;
+    if (best != pool.blocks.end()) {
+        const bool ordered = best->used_on == kUnused || (best->used_on == kDefaultStream && first_use == kDefaultStream);
+        if (!ordered) {
+            const hipError_t e = hipDeviceSynchronize();
+            if (e != hipSuccess) return e;
+            for (Block& b : pool.blocks) b.used_on = kUnused;
+        }
+        *p = best->p;
+        *block = best->bytes;
+        pool.held -= best->bytes;
+        pool.blocks.erase(best);
+        return hipSuccess;
+    }
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && !pool.blocks.empty()) {
+        (void)hipGetLastError();
+        empty(pool);
+        e = hipMalloc(p, bytes);
+    }
+    *block = bytes;
+    return e;
+}
+
+void pool_free(int device, void* p, size_t block, UsedOn used_on)
+{
+    if (!p) return;
+    DevicePool& pool = pool_of(device);
+    std::lock_guard<std::mutex> lock(pool.m);
+    if (pool.contexts == 0 || block > kPoolBytes) {
+        (void)hipFree(p);
+        return;
+    }
+    pool.blocks.push_back({p, block, used_on});
+    pool.held += block;
+    while (pool.held > kPoolBytes) {
+        (void)hipFree(pool.blocks.front().p);
+        pool.held -= pool.blocks.front().bytes;
+        pool.blocks.pop_front();
+    }
+}
+
+hipError_t scan_acquire(int device, ScanSlot* s)
+{
+    DevicePool& pool = pool_of(device);
+    std::lock_guard<std::mutex> lock(pool.m);
+    if (pool.scans.empty()) {
+        void* slab = nullptr;
+        hipError_t e = hipHostMalloc(&slab, kScanWords * kScanPitch * sizeof(uint32_t), hipHostMallocDefault);
+        if (e != hipSuccess) return e;
+        pool.slabs.push_back(slab);
+        for (size_t i = 0; i < kScanWords; i++) pool.scans.push_back({static_cast<uint32_t*>(slab) + i * kScanPitch, nullptr});
+    }
+    ScanSlot got = pool.scans.front();
+    // (events are made as slots are first used, and stay with them; a slot given back ahead of its kernel is waited for)
+    const hipError_t e = got.done ? hipEventSynchronize(got.done) : hipEventCreateWithFlags(&got.done, hipEventDisableTiming);
+    if (e != hipSuccess) return e;
+    pool.scans.pop_front();
+    *s = got;
+    return hipSuccess;
+}
+
+void scan_release(int device, ScanSlot s)
+{
+    if (!s.word) return;
+    DevicePool& pool = pool_of(device);
+    std::lock_guard<std::mutex> lock(pool.m);
+    pool.scans.push_back(s);
+}
+
+}  // namespace cybq

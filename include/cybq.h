@@ -136,6 +136,13 @@ const char* cybq_version(void);
 int cybq_weight_upload(cybq_ctx* ctx, cybq_quant quant, cybq_layout layout,
                        int64_t N, int64_t K, const void* q, const void* scales,
                        cybq_weight** out);
+/* The same for a whole list of tensors - what a model switch hands over: tensor i is quant[i] (cybq_quant),
+ * layout[i] (cybq_layout), [N[i], K[i]], q[i], scales[i] as in cybq_weight_upload (`scales` itself may be NULL when
+ * every tensor is BLOCK_AOS).  One call keeps the copy out of host memory, the bus and the repack going
+ * across the tensors.  All or nothing: on failure every out[i] is NULL.  The source buffers are not needed
+ * any more when either call returns, and the weights may be used on any stream. */
+int cybq_weight_upload_many(cybq_ctx* ctx, int64_t count, const int* quant, const int* layout, const int64_t* N,
+                            const int64_t* K, const void* const* q, const void* const* scales, cybq_weight** out);
 /* A second device copy of the same tensor at a different address (used by
  * benchmarks to stream more bytes than the last-level cache holds). */
 int cybq_weight_clone(cybq_ctx* ctx, const cybq_weight* src, cybq_weight** out);

@@ -59,6 +59,9 @@ extern "C" {
 
     pub fn cybq_weight_upload(ctx: *mut cybq_ctx, quant: c_int, layout: c_int, N: i64, K: i64, q: *const c_void,
                               scales: *const c_void, out: *mut *mut cybq_weight) -> c_int;
+    pub fn cybq_weight_upload_many(ctx: *mut cybq_ctx, count: i64, quant: *const c_int, layout: *const c_int,
+                                   N: *const i64, K: *const i64, q: *const *const c_void,
+                                   scales: *const *const c_void, out: *mut *mut cybq_weight) -> c_int;
     pub fn cybq_weight_clone(ctx: *mut cybq_ctx, src: *const cybq_weight, out: *mut *mut cybq_weight) -> c_int;
     pub fn cybq_weight_free(ctx: *mut cybq_ctx, w: *mut cybq_weight) -> c_int;
     pub fn cybq_weight_info(w: *const cybq_weight, quant: *mut c_int, N: *mut i64, K: *mut i64,

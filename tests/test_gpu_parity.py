@@ -65,6 +65,33 @@ def test_dequant_bit_exact(backend, oracle, bits, layout, shape):
     qw.free()
 
 
+# (a slot of the upload ring holds whole 16-row strips, 4 MiB: one short piece, several pieces with a ragged last strip,
+# pieces of exactly one strip, and a strip that does not fit a slot at all)
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("layout", [formats.PLANAR, formats.BLOCK_AOS])
+def test_upload_many_is_bit_exact_across_pieces(backend, bits, layout):
+    rng = np.random.default_rng(5)
+    tensors, want = [], []
+    for N, K in [(1, 32), (17, 160), (4111, 4096), (2050, 2080), (33, 262144), (19, 524288 + 32)]:
+        q = rng.integers(-8 if bits == 4 else -128, 8 if bits == 4 else 128, size=(N, K), dtype=np.int8)
+        s = (rng.random((N, K // 32), dtype=np.float32) * 0.01).astype(np.float16).view(np.uint16)
+        planar = layout == formats.PLANAR
+        tensors.append((bits, layout, N, K, formats.pack_planar(q, bits) if planar else formats.pack_blocks(q, s, bits), s if planar else None, None))
+        want.append(formats.dequantize(q, s))
+    for ws in (backend.upload_many(tensors), backend.upload_many(tensors[::-1])[::-1]):
+        for w, ref in zip(ws, want):
+            out = torch.empty(ref.shape, dtype=torch.float32, device="cuda")
+            backend.dequant(w, out)
+            torch.cuda.synchronize()
+            assert np.array_equal(out.cpu().numpy().view(np.uint32), ref.view(np.uint32)), ref.shape
+            w.free()
+    bad = list(tensors[0])
+    bad[3] = 48                                                # K % 32: nothing of the list is made
+    with pytest.raises(CybqError):
+        backend.upload_many([tensors[1], tuple(bad)])
+    assert backend.upload_many([]) == []
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 def test_dequant_exhaustive_scales_and_values(backend, oracle, bits):
     # every finite f16 scale against every representable q (extremes included)
