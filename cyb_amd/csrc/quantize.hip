@@ -1,6 +1,6 @@
 // quantize.hip - import-stage quantiser on the device: f32 [N,K] -> PLANAR
-// interchange layout (q plane + f16 scale plane).  HBM-bound, one pass:
-// 8 lanes share a 32-weight group, each lane owns 4 consecutive weights.
+// interchange layout (q plane + f16 scale plane).  One pass, bound by the 4 bytes per weight it reads:
+// 4 lanes share a 32-weight group, each lane owns 8 consecutive weights.
 //   d = f16(absmax / qmax), q = clamp(round_half_away(w / f32(d))), d == 0 -> q = 0
 #include "cybq_device.h"
 #include "cybq_internal.h"
@@ -9,59 +9,81 @@ namespace cybq {
 
 namespace {
 
+// round_half_away(w / d) for the correctly rounded quotient, without dividing in the common case.
+// r = w * rcp(d) is within 3 units in the last place of the quotient (v_rcp_f32: 1, the product: half, the quotient's own
+// rounding: half).  What is wanted is how |w / d| lies to the half-integers; where r is further than 2^-20 of
+// its size (8 units, and at least 2^-20) from one, both agree, and adding 1/2 and dropping the fraction gives the
+// answer.  Otherwise - two elements in a hundred thousand - the lane divides.  (An IEEE division and a roundf per
+// weight, some 25 instructions, bounded the kernel: 14336 x 4096 to Q4 62 us, now 46.6, 5.8 TB/s.)
+__device__ __forceinline__ float quotient_rounded(float w, float d, float rd)
+{
+    const float r = w * rd;
+    const float h = fabsf(r) + 0.5f;
+    const float f = truncf(h);
+    const float away = fminf(h - f, f + 1.0f - h);             // distance to the next integer of h
+    float res = f;
+    if (!(away > h * (1.0f / 1048576.0f))) res = truncf(fabsf(roundf(w / d)));
+    return copysignf(res, w);
+}
+
 template <int BITS>
-__global__ void quantize_kernel(const float* __restrict__ src, int64_t ngroups, uint8_t* __restrict__ q_out,
-                                uint16_t* __restrict__ s_out)
+__global__ __launch_bounds__(256) void quantize_kernel(const float4_t* __restrict__ src, int64_t ngroups, uint32_t* __restrict__ q_out,
+                                                        uint16_t* __restrict__ s_out)
 {
     const float qmax = BITS == 4 ? 7.0f : 127.0f;
     const float lo = BITS == 4 ? -8.0f : -127.0f;
-    int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t g = t >> 3;
-    const bool live = g < ngroups;
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (live) v = reinterpret_cast<const float4*>(src)[t];
-    float amax = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t g = t >> 2;
+    if (g >= ngroups) return;                                  // (the four lanes of a group leave together)
+    const float4_t v0 = __builtin_nontemporal_load(src + 2 * t), v1 = __builtin_nontemporal_load(src + 2 * t + 1);
+    const float w[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+    float amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(w[i]));
     amax = fmaxf(amax, __shfl_xor(amax, 1));
     amax = fmaxf(amax, __shfl_xor(amax, 2));
-    amax = fmaxf(amax, __shfl_xor(amax, 4));
     _Float16 dh = (_Float16)(amax / qmax);
     uint16_t dbits = __builtin_bit_cast(uint16_t, dh);
     if ((dbits & 0x7fffu) >= 0x7c00u) { dbits = 0x7bffu; dh = __builtin_bit_cast(_Float16, dbits); }
     const float d = (float)dh;
-    float w4[4] = {v.x, v.y, v.z, v.w};
-    int qi[4];
+    const float rd = __builtin_amdgcn_rcpf(d);
+    int qi[8];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        float r = 0.f;
-        if (d != 0.f) r = fminf(fmaxf(roundf(w4[i] / d), lo), qmax);
-        qi[i] = (int)r;
+    for (int i = 0; i < 8; i++) {
+        const float r = d != 0.f ? quotient_rounded(w[i], d, rd) : 0.f;
+        qi[i] = (int)fminf(fmaxf(r, lo), qmax);
     }
-    if (!live) return;
     if (BITS == 4) {
-        uint16_t packed = (uint16_t)((qi[0] & 15) | ((qi[1] & 15) << 4) | ((qi[2] & 15) << 8) | ((qi[3] & 15) << 12));
-        reinterpret_cast<uint16_t*>(q_out)[t] = packed;
+        uint32_t p = 0;
+#pragma unroll
+        for (int i = 0; i < 8; i++) p |= (uint32_t)(qi[i] & 15) << (4 * i);
+        q_out[t] = p;
     } else {
-        uint32_t packed = (uint32_t)(qi[0] & 255) | ((uint32_t)(qi[1] & 255) << 8) |
-                          ((uint32_t)(qi[2] & 255) << 16) | ((uint32_t)(qi[3] & 255) << 24);
-        reinterpret_cast<uint32_t*>(q_out)[t] = packed;
+        uint32_t p0 = 0, p1 = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            p0 |= (uint32_t)(qi[i] & 255) << (8 * i);
+            p1 |= (uint32_t)(qi[4 + i] & 255) << (8 * i);
+        }
+        q_out[2 * t] = p0;
+        q_out[2 * t + 1] = p1;
     }
-    if ((t & 7) == 0) s_out[g] = dbits;
+    if ((t & 3) == 0) s_out[g] = dbits;
 }
 
 }  // namespace
 
 hipError_t launch_quantize(int bits, const float* src, int N, int K, void* q_out, void* s_out, hipStream_t st)
 {
-    int64_t ngroups = (int64_t)N * (K / kGroup);
-    int64_t threads_total = ngroups * 8;
-    const int threads = 256;
-    unsigned blocks = (unsigned)((threads_total + threads - 1) / threads);
+    const int64_t ngroups = (int64_t)N * (K / kGroup);
+    const int64_t blocks = (ngroups * 4 + 255) / 256;
+    if (blocks > 0x7fffffff) return hipErrorInvalidValue;
     if (bits == 4)
-        hipLaunchKernelGGL(quantize_kernel<4>, dim3(blocks), dim3(threads), 0, st, src, ngroups,
-                           (uint8_t*)q_out, (uint16_t*)s_out);
+        hipLaunchKernelGGL(quantize_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, st, (const float4_t*)src, ngroups,
+                           (uint32_t*)q_out, (uint16_t*)s_out);
     else
-        hipLaunchKernelGGL(quantize_kernel<8>, dim3(blocks), dim3(threads), 0, st, src, ngroups,
-                           (uint8_t*)q_out, (uint16_t*)s_out);
+        hipLaunchKernelGGL(quantize_kernel<8>, dim3((unsigned)blocks), dim3(256), 0, st, (const float4_t*)src, ngroups,
+                           (uint32_t*)q_out, (uint16_t*)s_out);
     return hipGetLastError();
 }
 

@@ -1393,6 +1393,29 @@ def test_device_quantizer_bit_exact(backend, oracle, bits):
     assert np.array_equal(out.cpu().numpy().view(np.uint32), oracle.dequant(q, s).view(np.uint32))
 
 
+# quotients at and next to the half-integers (the ties the quantiser rounds away from zero, and the values whose correctly
+# rounded quotient is a tie although they are not), scales from subnormal f16 to the largest; a last workgroup of one group
+@pytest.mark.parametrize("bits", [4, 8])
+def test_device_quantizer_at_the_ties(backend, oracle, bits):
+    qmax = 7 if bits == 4 else 127
+    K, rows = 32 * 65, []
+    for d in np.array([1, 3, 1023, 1024, 5000, 15360, 15361, 20001, 31743], dtype=np.uint16).view(np.float16).astype(np.float32):
+        half = (np.arange(qmax, dtype=np.float32) + np.float32(0.5)) * d
+        below, above = np.nextafter(half, np.float32(0)), np.nextafter(half, np.float32(np.inf))
+        v = np.concatenate([half, below, above, np.nextafter(below, np.float32(0)), half * np.float32(1 + 2e-6), half * np.float32(1 - 2e-6)])
+        v = np.resize(np.concatenate([v, -v]), (K // 32, 31))
+        rows.append(np.concatenate([np.full((K // 32, 1), np.float32(qmax) * d, dtype=np.float32), v], axis=1).reshape(-1))
+    w = np.stack(rows).astype(np.float32)
+    N = w.shape[0]
+    qd = torch.empty(N * K * bits // 8, dtype=torch.uint8, device="cuda")
+    sd = torch.empty(N * K // 32, dtype=torch.int16, device="cuda")
+    backend.quantize(bits, torch.from_numpy(w).cuda(), N, K, qd, sd)
+    torch.cuda.synchronize()
+    q, s = oracle.quantize(w, bits)
+    assert np.array_equal(sd.cpu().numpy().view(np.uint16).reshape(N, -1), s)
+    assert np.array_equal(qd.cpu().numpy(), oracle.pack_planar(q, bits))
+
+
 # ------------------------------------------------------------ interface / errors
 
 def test_graph_node_execution(backend, oracle):
