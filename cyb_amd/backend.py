@@ -20,7 +20,10 @@ use cyb_amd.formats), but constructing a Backend raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
+import sys
 from dataclasses import dataclass, field
 from typing import Dict, Optional
 
@@ -30,6 +33,7 @@ from . import formats
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_PATH = os.path.join(_HERE, "lib", "libcybq.so")
+_CALLS_PATH = os.path.join(_HERE, "lib", "_torch_calls.so")
 
 F32, F16, BF16 = 0, 1, 2
 EPILOGUES = {"none": 0, "add": 1, "swiglu": 2}      # enum cybq_epilogue
@@ -101,6 +105,22 @@ def load_library() -> ctypes.CDLL:
     return lib
 
 
+_calls = None
+
+
+def _load_calls():
+    """The native call path for torch tensors (csrc/torch_calls.cpp), once the program has torch."""
+    global _calls
+    if _calls is None and "torch" in sys.modules:
+        if not os.path.exists(_CALLS_PATH):
+            raise CybqError(-4, "library missing", f"{_CALLS_PATH} not built; run __graft_entry__.build()")
+        loader = importlib.machinery.ExtensionFileLoader("_torch_calls", _CALLS_PATH)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_torch_calls", _CALLS_PATH, loader=loader))
+        loader.exec_module(mod)
+        _calls = mod
+    return _calls
+
+
 def _ptr(t) -> int:
     if t is None:
         return 0
@@ -142,6 +162,7 @@ class QWeight:
     def __init__(self, backend: "Backend", handle: int):
         self._backend = backend
         self._h = ctypes.c_void_p(handle)
+        self._addr = handle or 0                        # the same for the native call path; 0 once freed
         q, n, k, b = ctypes.c_int(), ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int64()
         backend._check(backend._lib.cybq_weight_info(self._h, q, n, k, b))
         self.quant, self.N, self.K, self.device_bytes = q.value, n.value, k.value, b.value
@@ -166,6 +187,7 @@ class QWeight:
         if self._h and self._backend._ctx:
             self._backend._lib.cybq_weight_free(self._backend._ctx, self._h)
         self._h = ctypes.c_void_p()
+        self._addr = 0
 
     def __del__(self):
         try:
@@ -222,6 +244,7 @@ class Backend:
         if rc != 0:
             self._ctx = ctypes.c_void_p()
             raise CybqError(rc, self._lib.cybq_strerror(rc).decode())
+        self._addr = self._ctx.value
         self.device = device
         self.weights: Dict[str, QWeight] = {}
 
@@ -238,6 +261,7 @@ class Backend:
         if self._ctx:
             self._lib.cybq_destroy(self._ctx)
             self._ctx = ctypes.c_void_p()
+            self._addr = 0
 
     def __del__(self):
         try:
@@ -335,6 +359,11 @@ class Backend:
 
     def matmul(self, w: QWeight, x, y, M: Optional[int] = None, xdt: Optional[int] = None,
                ydt: Optional[int] = None, stream: int = 0) -> None:
+        calls = _calls or _load_calls()
+        if calls is not None:                           # (positive: not a plain call on tensors, looked at below)
+            rc = calls.matmul(self._addr, self.device, w._addr, x, y, M, xdt, ydt, stream)
+            if rc <= 0:
+                return self._check(rc)
         if M is None:
             M = int(x.shape[0]) if x.dim() == 2 else 1
         self._check_call(w, x, y, M)
@@ -343,6 +372,11 @@ class Backend:
 
     def matmul_static(self, w: QWeight, x, y, M: Optional[int] = None, stream: int = 0) -> None:
         """cybq_matmul_static: the same op with its scratch in a static device array (allocates nothing)."""
+        calls = _calls or _load_calls()
+        if calls is not None:
+            rc = calls.matmul_static(self._addr, self.device, w._addr, x, y, M, stream)
+            if rc <= 0:
+                return self._check(rc)
         if M is None:
             M = int(x.shape[0]) if x.dim() == 2 else 1
         self._check_call(w, x, y, M)
@@ -355,6 +389,11 @@ class Backend:
         fuse_pairs; y has half as many columns as w has rows)."""
         if epilogue not in EPILOGUES:
             raise CybqError(-1, "invalid argument", f"unknown epilogue {epilogue!r}")
+        calls = _calls or _load_calls()
+        if calls is not None:
+            rc = calls.matmul_fused(self._addr, self.device, w._addr, x, None, 0.0, y, EPILOGUES[epilogue], residual, M, stream)
+            if rc <= 0:
+                return self._check(rc)
         if M is None:
             M = int(x.shape[0]) if x.dim() == 2 else 1
         self._check_call(w, x, y, M, epilogue, residual)
@@ -366,6 +405,11 @@ class Backend:
         """cybq_matmul_norm: RMSNorm (gamma [K], eps) folded into the activation load, then the epilogue."""
         if epilogue not in EPILOGUES:
             raise CybqError(-1, "invalid argument", f"unknown epilogue {epilogue!r}")
+        calls = _calls or _load_calls()
+        if calls is not None and gamma is not None:
+            rc = calls.matmul_fused(self._addr, self.device, w._addr, x, gamma, float(eps), y, EPILOGUES[epilogue], residual, M, stream)
+            if rc <= 0:
+                return self._check(rc)
         if M is None:
             M = int(x.shape[0]) if x.dim() == 2 else 1
         self._check_call(w, x, y, M, epilogue, residual, gamma)
