@@ -466,9 +466,9 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
         dscr = static_cast<char*>(workspace) + workspace_bytes;
         dscr_bytes = cybq::kDecodeScratchBytes;
     }
-    if (M <= 16 || (M <= 32 && cybq::gemv_serves_32((int)xdt, (int)M, epi))) {
+    if (M <= 16 || (M <= 32 && cybq::gemv_serves_32(v, (int)xdt, (int)M, ctx->num_cus, epi))) {
         e = cybq::launch_gemv(v, x, xdt, (int)M, y, ydt, ctx->num_cus, ctx->decode_exact, epi, dscr, dscr_bytes, st);
-    } else if (M <= 64 && (int64_t)w->N * w->K <= (int64_t)6144 * 4096 && cybq::gemv_serves_32((int)xdt, 32, epi) &&
+    } else if (M <= 64 && (int64_t)w->N * w->K <= (int64_t)6144 * 4096 && cybq::gemv_serves_32(v, (int)xdt, 32, ctx->num_cus, epi) &&
                (ctx->prefill_exact || weight_is_wide(w) || !cybq::gemm_rows_takes(v, (int)M, ctx->num_cus, epi))) {
         // 33..64 rows on a small weight (up to 4096 -> 6144) that the few-rows MFMA kernel does not take (exact
         // mode, wide scales, K outside 2048 .. 8192, a folded SwiGLU): the tiled MFMA
@@ -501,7 +501,7 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
         // time where the batched-rows kernel takes them in one pass: the weights stream once per 32 rows.
         e = hipSuccess;
         const int64_t n_out = epi.kind == cybq::kEpiSwiglu ? w->N / 2 : w->N;
-        const int64_t step = cybq::gemv_serves_32((int)xdt, 32, epi) ? 32 : 16;
+        const int64_t step = cybq::gemv_serves_32(v, (int)xdt, 32, ctx->num_cus, epi) ? 32 : 16;
         for (int64_t m0 = 0; m0 < M && e == hipSuccess; m0 += step) {
             int mm = (int)((M - m0) < step ? (M - m0) : step);
             const char* xp = static_cast<const char*>(x) + (size_t)m0 * w->K * dtype_size(xdt);

@@ -22,7 +22,8 @@ hipError_t launch_dequant(const WeightView& w, float* out, hipStream_t st);
 
 // decode path, 1 <= M <= 16 per call, and 17 .. 32 rows where gemv_serves_32 says so (api.hip
 // walks the other 17..32-row calls 16 rows at a time)
-bool gemv_serves_32(int xdt, int M, const Epilogue& epi);
+bool gemv_serves_32(const WeightView& w, int xdt, int M, int num_cus, const Epilogue& epi);
+bool gemv_is_automatic();            // no tuning override is set
 // exact_operands: keep the weight operands exact integers for one and two f16 rows too (the LDS
 // kernel) instead of the subnormal-operand kernel of gemv1.hip
 // scratch: device memory the batched-rows kernel may use when it splits K over workgroups (few strips, a
@@ -31,6 +32,9 @@ bool gemv_serves_32(int xdt, int M, const Epilogue& epi);
 constexpr size_t kDecodeScratchBytes = (size_t)8 << 20;
 hipError_t launch_gemv(const WeightView& w, const void* x, int xdt, int M, void* y, int ydt,
                        int num_cus, bool exact_operands, const Epilogue& epi, void* scratch, size_t scratch_bytes, hipStream_t st);
+// 3 .. 32 rows on outputs with several pairs of strips per CU (gemv_stream.hip)
+bool gemv_stream_serves(const WeightView& w, int xdt, int M, int num_cus, const Epilogue& epi);
+hipError_t launch_gemv_stream(const WeightView& w, const void* x, int xdt, int M, void* y, int ydt, int num_cus, const Epilogue& epi, hipStream_t st);
 // decode kernel for one and two rows (f16 / bf16 activations, no folded norm): weight operands are f16 subnormals
 // (bf16: 128 + u),
 // the +8 / +128 bias comes off inside the MFMA accumulation (gemv1.hip)

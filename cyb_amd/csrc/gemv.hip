@@ -16,48 +16,11 @@
 #include <type_traits>
 #include "cybq_device.h"
 #include "cybq_internal.h"
+#include "gemv_parts.h"
 
 namespace cybq {
 
 namespace {
-
-constexpr int XF16 = 0, XBF16 = 1, XF32 = 2;
-
-template <int BITS>
-struct TileRegs {
-    u32x4_t q[BITS == 4 ? 1 : 2];
-    u32x2_t s;
-};
-
-template <int BITS>
-__device__ __forceinline__ void load_tile(TileRegs<BITS>& t, const WeightView& w, int64_t tile, int lane)
-{
-    const u32x4_t* qp = tile_q<BITS>(w, tile);
-    t.q[0] = __builtin_nontemporal_load(qp + lane);
-    if (BITS == 8) t.q[BITS == 8 ? 1 : 0] = __builtin_nontemporal_load(qp + 64 + lane);
-    t.s = __builtin_nontemporal_load(tile_s<BITS>(w, tile) + (lane & 15));
-}
-
-__device__ __forceinline__ void store_out(void* y, int ydt, int64_t idx, float v)
-{
-    if (ydt == kF32) reinterpret_cast<float*>(y)[idx] = v;
-    else if (ydt == kF16) reinterpret_cast<_Float16*>(y)[idx] = (_Float16)v;
-    else reinterpret_cast<uint16_t*>(y)[idx] = f32_to_bf16_bits(v);
-}
-
-__device__ __forceinline__ float load_out(const void* p, int dt, int64_t idx)
-{
-    if (dt == kF32) return reinterpret_cast<const float*>(p)[idx];
-    if (dt == kF16) return (float)reinterpret_cast<const _Float16*>(p)[idx];
-    return __builtin_bit_cast(float, (uint32_t)reinterpret_cast<const uint16_t*>(p)[idx] << 16);
-}
-
-// one finished output element: residual add (fp32, before the single rounding to ydt), store
-__device__ __forceinline__ void emit(void* y, int ydt, const Epilogue& epi, int64_t idx, float v)
-{
-    if (epi.kind == kEpiAdd) v += load_out(epi.residual, ydt, idx);
-    store_out(y, ydt, idx, v);
-}
 
 // x rows of one K slab -> LDS (row stride ldx 16-bit elements; XF32: a second
 // plane of low halves follows the first at plane_elems).  Split in two so that
@@ -188,18 +151,6 @@ __device__ __forceinline__ void tile_issue(const TileRegs<BITS>& t, const uint16
     }
 }
 
-template <int RMAX>
-__device__ __forceinline__ void tile_accum(u32x2_t s, const float4_t d[4], float acc[RMAX])
-{
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        uint32_t sb = (j & 1) ? (s[j >> 1] >> 16) : (s[j >> 1] & 0xffffu);
-        float sc = f16_bits_to_f32(sb);
-#pragma unroll
-        for (int r = 0; r < RMAX; r++) acc[r] = __builtin_fmaf(sc, d[j][r], acc[r]);
-    }
-}
-
 // The hot region is kept free of branches on purpose: vmcnt retires in order
 // and the compiler can only count outstanding loads along straight-line code;
 // a conditional load forces it to wait for everything (vmcnt(0)) and nothing
@@ -238,23 +189,6 @@ __device__ __forceinline__ void compute_batch(const TileRegs<BITS> (&buf)[U], in
         sprev = sc;
     }
     tile_accum<RMAX>(sprev, dprev, acc);
-}
-
-// Sum of the waves' partial sums red[k * stride], k = 0 .. nwaves-1, added in wave
-// order.  The reads go out eight at a time: one LDS round trip per eight waves
-// instead of one per wave.  (Slots past nwaves add +0, which changes nothing: a sum
-// that starts from +0 is never -0.)
-__device__ __forceinline__ float sum_partials(const float* red, int nwaves, int stride)
-{
-    float v = 0.f;
-    for (int k0 = 0; k0 < nwaves; k0 += 8) {
-        float t[8];
-#pragma unroll
-        for (int i = 0; i < 8; i++) t[i] = red[min(k0 + i, nwaves - 1) * stride];
-#pragma unroll
-        for (int i = 0; i < 8; i++) v += (k0 + i < nwaves) ? t[i] : 0.f;
-    }
-    return v;
 }
 
 // ---- RMSNorm folded into the staged x (LDS kernel) ------------------------------
@@ -534,49 +468,6 @@ __global__ __launch_bounds__(1024) void gemv_kernel(const uint8_t* __restrict__ 
 // partials are summed in wave order: deterministic, and a row's bits do not depend
 // on the batch it is part of (within this kernel; the LDS kernel may split K over
 // a different number of waves).
-template <int BITS, int XMODE>
-__device__ __forceinline__ void tile_operands(const TileRegs<BITS>& t, uint32_t magic, Frag16 (&b)[4])
-{
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        uint32_t bw[4];
-        if (BITS == 4 && XMODE == XBF16) {
-            unpack_q4_bf16_biased(t.q[0][2 * (j >> 1)], t.q[0][2 * (j >> 1) + 1], j & 1, magic, bw);
-        } else if (XMODE == XBF16) {
-            unpack_q8_bf16_biased(t.q[j >> 1][(j & 1) * 2], t.q[j >> 1][(j & 1) * 2 + 1], bw);
-        } else {
-            if (BITS == 4) unpack_q4_f16(t.q[0][2 * (j >> 1)], t.q[0][2 * (j >> 1) + 1], j & 1, magic, bw);
-            else unpack_q8_f16(t.q[j >> 1][(j & 1) * 2], t.q[j >> 1][(j & 1) * 2 + 1], bw);
-        }
-        b[j].u = (u32x4_t){bw[0], bw[1], bw[2], bw[3]};
-    }
-}
-
-template <int BITS, int XMODE>
-__device__ __forceinline__ void tile_multiply(const Frag16 (&a)[4], const Frag16 (&b)[4], float4_t d[4])
-{
-    const float4_t zero = {0.f, 0.f, 0.f, 0.f};
-    Frag16 off;
-    const uint32_t offw = BITS == 4 ? kBf16Neg136x2 : kBf16Neg128x2;
-    off.u = (u32x4_t){offw, offw, offw, offw};
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        if (XMODE == XBF16) {
-            d[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j].b, b[j].b, zero, 0, 0, 0);
-            d[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j].b, off.b, d[j], 0, 0, 0);
-        } else d[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j].h, b[j].h, zero, 0, 0, 0);
-    }
-}
-
-template <int BITS, int XMODE>
-__device__ __forceinline__ void tile_issue_regs(const TileRegs<BITS>& t, const Frag16 (&a)[4], uint32_t magic,
-                                                float4_t d[4])
-{
-    Frag16 b[4];
-    tile_operands<BITS, XMODE>(t, magic, b);
-    tile_multiply<BITS, XMODE>(a, b, d);
-}
-
 // NORM: RMSNorm folded into the activation load (epi.gamma / epi.eps).  A lane multiplies the 16 B
 // piece of x it loaded (eight neighbouring k of one row) by gamma and adds up its squares while the
 // piece is still as loaded: every element of the batch is touched once per workgroup, where the
@@ -585,65 +476,6 @@ __device__ __forceinline__ void tile_issue_regs(const TileRegs<BITS>& t, const F
 // GH: x and gamma are both f16 - gamma sits in LDS as loaded and the product is one packed f16
 // multiply per pair (the product of two f16 is exact in fp32, so its single rounding to f16 is the
 // rounding the fp32 form makes); otherwise gamma is fp32 in LDS and the pair goes through fp32.
-// v as the lanes named by a DPP control see it (quad permutations, mirrors within a row of 16)
-template <int CTRL>
-__device__ __forceinline__ float lane_cross(float v)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
-}
-
-// (the LDS reads of a tile's pieces are issued together, ahead of the arithmetic)
-struct GammaPiece {
-    u32x4_t lo, hi;           // 8 x fp32, or (GH) 8 x f16 in lo
-};
-
-template <bool GH>
-__device__ __forceinline__ GammaPiece gamma_piece(const void* gamma_lds, int k)
-{
-    GammaPiece g;
-    if constexpr (GH) {
-        g.lo = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint16_t*>(gamma_lds) + k);
-        g.hi = g.lo;
-    } else {
-        g.lo = reinterpret_cast<const u32x4_t*>(reinterpret_cast<const float*>(gamma_lds) + k)[0];
-        g.hi = reinterpret_cast<const u32x4_t*>(reinterpret_cast<const float*>(gamma_lds) + k)[1];
-    }
-    return g;
-}
-
-template <int XMODE, bool GH>
-__device__ __forceinline__ void norm_piece(u32x4_t& v, const GammaPiece& gp, bool counts, float& ssq)
-{
-    float sq = ssq;
-    if constexpr (GH) {
-        const u32x4_t g = gp.lo;
-#pragma unroll
-        for (int p = 0; p < 4; p++) {
-            const half2_t h = as_h2(v[p]);
-            sq = __builtin_amdgcn_fdot2(h, h, sq, false);
-            v[p] = as_u32(h * as_h2(g[p]));
-        }
-    } else {
-#pragma unroll
-        for (int p = 0; p < 4; p++) {
-            const uint32_t ua = p < 2 ? gp.lo[2 * p] : gp.hi[2 * p - 4], ub = p < 2 ? gp.lo[2 * p + 1] : gp.hi[2 * p - 3];
-            const float ga = __builtin_bit_cast(float, ua), gb = __builtin_bit_cast(float, ub);
-            if (XMODE == XBF16) {
-                const float v0 = __builtin_bit_cast(float, v[p] << 16);
-                const float v1 = __builtin_bit_cast(float, v[p] & 0xffff0000u);
-                sq = fmaf(v1, v1, fmaf(v0, v0, sq));
-                v[p] = pack_bf16x2(v0 * ga, v1 * gb);
-            } else {
-                const half2_t h = as_h2(v[p]);
-                sq = __builtin_amdgcn_fdot2(h, h, sq, false);
-                const half2_t o = {(_Float16)((float)h.x * ga), (_Float16)((float)h.y * gb)};
-                v[p] = as_u32(o);
-            }
-        }
-    }
-    ssq = counts ? sq : ssq;
-}
-
 // MB: blocks of 16 batch rows (2 = 17..32 rows: every unpacked weight operand is multiplied with
 // two activation operands, the weights still stream once).
 // gamma / gamma_dt (NORM) sit ahead of y in the argument list: everything the first loads need is
@@ -1302,10 +1134,13 @@ void set_gemv_tuning(int waves_per_group, int rows_kernel, int unroll)
     g_tune_unroll = unroll;
 }
 
-// 17 .. 32 rows in one pass (weights streamed once): 16-bit activations, no folded norm
-bool gemv_serves_32(int xdt, int M, const Epilogue& epi)
+bool gemv_is_automatic() { return g_tune_waves == 0 && g_tune_rows == 0 && g_tune_unroll == 0; }
+
+// 17 .. 32 rows in one pass (weights streamed once): 16-bit activations, with a folded norm only the kernel of gemv_stream.hip
+bool gemv_serves_32(const WeightView& w, int xdt, int M, int num_cus, const Epilogue& epi)
 {
-    return M > 16 && M <= 32 && xdt != kF32 && !epi.gamma && g_tune_rows != 2;
+    if (M <= 16 || M > 32 || xdt == kF32 || g_tune_rows == 2) return false;
+    return !epi.gamma || (gemv_is_automatic() && gemv_stream_serves(w, xdt, M, num_cus, epi));
 }
 
 hipError_t launch_gemv(const WeightView& w, const void* x, int xdt, int M, void* y, int ydt,
@@ -1345,10 +1180,13 @@ hipError_t launch_gemv(const WeightView& w, const void* x, int xdt, int M, void*
     // (Q8 on wide outputs: up to four rows the LDS kernel is still the quicker one, 24.0 against
     // 27.6 us at 4096 -> 28672)
     const bool wide_q8 = w.bits == 8 && (w.NT + num_cus / 2) / num_cus >= 3;
-    const bool rows_kernel = g_tune_rows == 1 || g_tune_rows >= 3 || (g_tune_rows == 0 && M >= (wide_q8 ? 5 : 3));
-    if (M > 16 && !gemv_serves_32(xdt, M, epi)) return hipErrorInvalidValue;
+    const bool rows_kernel = (g_tune_rows == 1 || g_tune_rows == 3 || g_tune_rows == 4) || ((g_tune_rows == 0 || g_tune_rows == 5) && M >= (wide_q8 ? 5 : 3));
+    if (M > 16 && !gemv_serves_32(w, xdt, M, num_cus, epi)) return hipErrorInvalidValue;
+    // outputs with several pairs of strips per CU: workgroups that stay (tuning 5: never)
+    if (gemv_is_automatic() && gemv_stream_serves(w, xdt, M, num_cus, epi))
+        return launch_gemv_stream(w, x, xdt, M, y, ydt, num_cus, epi, st);
     // few strips, a long K, twelve rows or more: K split over workgroups (tuning 3: never, 4: from three rows on)
-    if (rows_kernel && xdt != kF32 && scratch && g_tune_rows != 3 && g_tune_waves == 0 && (M >= kSplitMinRows || g_tune_rows == 4)) {
+    if (rows_kernel && xdt != kF32 && scratch && g_tune_rows != 3 && g_tune_rows != 5 && g_tune_waves == 0 && (M >= kSplitMinRows || g_tune_rows == 4)) {
         SplitPlan sp;
         if (rows_split_plan(w, xdt, M, num_cus, epi, scratch_bytes, sp)) {
             if (xdt == kF16) return launch_rows_split<XF16>(w, x, M, y, ydt, epi, !exact_operands, sp, scratch, st);

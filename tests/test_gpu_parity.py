@@ -242,6 +242,50 @@ def test_decode_17_to_32_rows_in_one_pass(backend, oracle, bits, xdt, shape):
         assert ((y3.double() - ref).norm() / ref.norm()).item() < TIGHT
 
 
+# the kernel whose workgroups stay: four or eight waves of two to four K tiles, the last one missing for some waves or ragged;
+# an odd number of strips, the last one ragged; one, two and three rounds of pairs; both row blocks
+@pytest.mark.parametrize("bits,xdt", [(4, "f16"), (4, "bf16"), (8, "f16"), (8, "bf16")])
+@pytest.mark.parametrize("shape", [(6144, 1024), (6149, 1056), (10241, 1888), (6160, 2048), (6149, 2080), (17000, 2592), (10241, 3104), (6144, 4096)])
+def test_decode_rows_streamed_by_staying_workgroups(backend, bits, xdt, shape):
+    N, K = shape
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    w = torch.empty((N, K), device="cuda").normal_(0.0, 0.02, generator=g)
+    qd = torch.empty(N * K * bits // 8, dtype=torch.uint8, device="cuda")
+    sd = torch.empty(N * (K // 32), dtype=torch.int16, device="cuda")
+    backend.quantize(bits, w, N, K, qd, sd)
+    qw = backend.weight_from_device(bits, N, K, qd, sd)
+    backend.dequant(qw, w)
+    wd = w.double()
+    x = torch.empty((32, K), device="cuda").normal_(generator=g).to(TDT[xdt])
+    r = torch.empty((32, N), device="cuda").normal_(generator=g)
+    gamma = (1.0 + 0.25 * torch.empty(K, device="cuda").normal_(generator=g)).to(torch.float16)
+    plain = x.double() @ wd.t()
+    rstd = 1.0 / torch.sqrt((x.double() ** 2).mean(dim=1, keepdim=True) + 1e-5)
+    normed = ((x.float() * gamma.float()).to(TDT[xdt]).double() @ wd.t()) * rstd
+    rel = lambda a, b: ((a.double() - b).norm() / b.norm()).item()
+    full = torch.empty((32, N), device="cuda")
+    backend.matmul(qw, x, full)
+    for M in (3, 8, 9, 16, 17, 32):
+        y = torch.full((M, N), float("nan"), device="cuda")
+        backend.matmul(qw, x[:M].contiguous(), y)
+        assert rel(y, plain[:M]) < TIGHT, M
+        backend.matmul_ex(qw, x[:M].contiguous(), y, "add", r[:M].contiguous())
+        assert rel(y, plain[:M] + r[:M].double()) < TIGHT, M
+        if M <= 16 or xdt == "f16":           # (17 bf16 rows or more with a norm are not this kernel's)
+            backend.matmul_norm(qw, x[:M].contiguous(), gamma, 1e-5, y)
+            # (K of four tiles per wave: registers for x or for gamma, not both; those calls are FAST ones)
+            four = -(-K // 128) > (12 if K <= 1920 else 24)
+            assert rel(y, normed[:M]) < (FAST if M > 16 and four else TIGHT), M
+    half = N // 32 * 16
+    qb, sb = half * K * bits // 8, half * (K // 32)
+    pair = backend.fuse_pairs(backend.weight_from_device(bits, half, K, qd[:qb], sd[:sb]),
+                              backend.weight_from_device(bits, half, K, qd[qb:2 * qb], sd[sb:2 * sb]))
+    for M in (5, 16, 30):
+        y = torch.full((M, half), float("nan"), device="cuda")
+        backend.matmul_ex(pair, x[:M].contiguous(), y, "swiglu")
+        assert rel(y, torch.nn.functional.silu(plain[:M, :half]) * plain[:M, half:2 * half]) < TIGHT, M
+
+
 @pytest.mark.parametrize("N", [8192, 12288])
 def test_decode_modes_in_the_batched_rows_kernel(backend, oracle, N):
     """3 .. 32 f16 rows on outputs wide enough for two / four strips per workgroup: STREAM feeds the Q4
