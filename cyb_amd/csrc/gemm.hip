@@ -547,6 +547,8 @@ hipError_t launch_roles(const WeightView& w, const void* x, int M, void* y, int 
     return hipGetLastError();
 }
 
+constexpr int kMaxSplits = 8;
+
 // y = epilogue(out_scale * (part[0] + part[1] + ... + part[splits-1])), slabs added in that order.
 // One thread per output element; N = columns of a slab (for SwiGLU y has N / 2).
 __global__ void splitk_reduce_kernel(const float* __restrict__ part, int splits, int M, int N, void* __restrict__ y, int ydt,
@@ -577,29 +579,107 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ part, int splits,
     store_out_g(y, ydt, i, v);
 }
 
-// The same sum, four neighbouring elements per thread with 128-bit slab reads (slab a multiple of
-// four elements, no SwiGLU): the pass is pure memory traffic, splits + 1 times the output.
-__global__ void splitk_reduce4_kernel(const float* __restrict__ part, int splits, int M, int N, void* __restrict__ y, int ydt,
-                                      float out_scale, Epilogue epi, NormStats ns, int K)
+// The same sum for N a multiple of four, four neighbouring elements of a row per thread.  The pass is latency: everything a
+// thread needs - its pieces of all the slabs, its residual, its row's factors - is requested before anything is used, and
+// the row is the workgroup's (blockIdx.y), not a division per element.  (Before: slab after slab, then four 64-bit
+// divisions, each in front of its own loads of the row's factor and the residual.)
+// RESULT
+template <int SPLITS, bool SWIGLU>
+__global__ __launch_bounds__(256) void splitk_reduce4_kernel(const float* __restrict__ part, int M, int N, void* __restrict__ y, int ydt,
+                                                             float out_scale, Epilogue epi, NormStats ns, int K)
 {
-    const int64_t slab = (int64_t)M * N;
-    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-    if (i >= slab) return;
-    float4_t v = *reinterpret_cast<const float4_t*>(part + i);
-    for (int s = 1; s < splits; s++) v += *reinterpret_cast<const float4_t*>(part + s * slab + i);
+    const int n_out = SWIGLU ? N >> 1 : N;
+    const int n = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4, m = blockIdx.y;
+    if (n >= n_out) return;
+    const int64_t slab = (int64_t)M * N, at = (int64_t)m * n_out + n;
+    // (a pair's 16 gate columns sit in front of its 16 up columns)
+    const float* const p0 = part + (int64_t)m * N + (SWIGLU ? (n >> 4) * 32 + (n & 15) : n);
+    float4_t g[SPLITS], u[SWIGLU ? SPLITS : 1];
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-        float t = v[e] * out_scale;
-        if (epi.gamma || ns.unscale) t *= row_factor(ns, epi.gamma != nullptr, (int)((i + e) / N), K, epi.eps);
-        if (epi.kind == kEpiAdd) t += load_out_g(epi.residual, ydt, i + e);
-        v[e] = t;
+    for (int s = 0; s < SPLITS; s++) {
+        g[s] = *reinterpret_cast<const float4_t*>(p0 + s * slab);
+        if (SWIGLU) u[SWIGLU ? s : 0] = *reinterpret_cast<const float4_t*>(p0 + s * slab + 16);
     }
-    if (ydt == kF32) {
-        *reinterpret_cast<float4_t*>(reinterpret_cast<float*>(y) + i) = v;
+    const uintptr_t mask = ydt == kF32 ? 15u : 7u;
+    const bool aligned = ((reinterpret_cast<uintptr_t>(y) | (epi.kind == kEpiAdd ? reinterpret_cast<uintptr_t>(epi.residual) : 0u)) & mask) == 0;
+    float4_t res = {0.f, 0.f, 0.f, 0.f};
+    if (epi.kind == kEpiAdd) {
+        if (!aligned) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) res[e] = load_out_g(epi.residual, ydt, at + e);
+        } else if (ydt == kF32) {
+            res = *reinterpret_cast<const float4_t*>(static_cast<const float*>(epi.residual) + at);
+        } else {
+            const u32x2_t r = *reinterpret_cast<const u32x2_t*>(static_cast<const uint16_t*>(epi.residual) + at);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t h = (e & 1) ? r[e >> 1] >> 16 : r[e >> 1] & 0xffffu;
+                res[e] = ydt == kF16 ? f16_bits_to_f32(h) : __builtin_bit_cast(float, h << 16);
+            }
+        }
+    }
+    const float f = out_scale * (epi.gamma || ns.unscale ? row_factor(ns, epi.gamma != nullptr, m, K, epi.eps) : 1.0f);
+    float4_t v = g[0];
+#pragma unroll
+    for (int s = 1; s < SPLITS; s++) v += g[s];
+    if (SWIGLU) {
+        float4_t w = u[0];
+#pragma unroll
+        for (int s = 1; s < SPLITS; s++) w += u[SWIGLU ? s : 0];
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = silu_mul(v[e] * f, w[e] * f);
     } else {
 #pragma unroll
-        for (int e = 0; e < 4; e++) store_out_g(y, ydt, i + e, v[e]);
+        for (int e = 0; e < 4; e++) v[e] = v[e] * f + res[e];
     }
+    if (!aligned) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) store_out_g(y, ydt, at + e, v[e]);
+    } else if (ydt == kF32) {
+        *reinterpret_cast<float4_t*>(static_cast<float*>(y) + at) = v;
+    } else {
+        u32x2_t o;
+        if (ydt == kF16) {
+            const half2_t a = {(_Float16)v[0], (_Float16)v[1]}, b = {(_Float16)v[2], (_Float16)v[3]};
+            o = (u32x2_t){as_u32(a), as_u32(b)};
+        } else {
+            o = (u32x2_t){pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+        }
+        *reinterpret_cast<u32x2_t*>(static_cast<uint16_t*>(y) + at) = o;
+    }
+}
+
+template <bool SWIGLU>
+hipError_t launch_reduce4(const float* part, int splits, int M, int N, void* y, int ydt, float out_scale, const Epilogue& epi, const NormStats& ns,
+                          int K, hipStream_t st)
+{
+    const dim3 grid((unsigned)(((SWIGLU ? N / 2 : N) / 4 + 255) / 256), (unsigned)M);
+    auto go = [&](auto count) {
+        hipLaunchKernelGGL((splitk_reduce4_kernel<decltype(count)::value, SWIGLU>), grid, dim3(256), 0, st, part, M, N, y, ydt, out_scale, epi, ns, K);
+        return hipGetLastError();
+    };
+    switch (splits) {
+        case 2: return go(std::integral_constant<int, 2>{});
+        case 3: return go(std::integral_constant<int, 3>{});
+        case 4: return go(std::integral_constant<int, 4>{});
+        case 5: return go(std::integral_constant<int, 5>{});
+        case 6: return go(std::integral_constant<int, 6>{});
+        case 7: return go(std::integral_constant<int, 7>{});
+        case 8: return go(std::integral_constant<int, 8>{});
+    }
+    return hipErrorInvalidValue;               // kMaxSplits
+}
+
+// adds the slabs of a K split (2 .. kMaxSplits of them) and applies the epilogue
+hipError_t launch_reduce(const float* part, int splits, int M, int N, void* y, int ydt, float out_scale, const Epilogue& epi, const NormStats& ns,
+                         int K, hipStream_t st)
+{
+    const bool rows_fit = M <= 65535;          // the grid's second dimension
+    if (rows_fit && epi.kind == kEpiSwiglu) return launch_reduce4<true>(part, splits, M, N, y, ydt, out_scale, epi, ns, K, st);
+    if (rows_fit && N % 4 == 0) return launch_reduce4<false>(part, splits, M, N, y, ydt, out_scale, epi, ns, K, st);
+    const int64_t total = (int64_t)M * N;
+    hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, part, splits, M, N, y, ydt, out_scale, epi, ns, K);
+    return hipGetLastError();
 }
 
 template <int BITS, int XBF, int NF, bool EXACT, int MF, int WAVES>
@@ -615,7 +695,7 @@ hipError_t launch_m(const WeightView& w, const void* x, int M, void* y, int ydt,
     // K range in fp32 into its own slab of `part`; a second kernel adds the slabs in
     // a fixed order (no atomics: results are reproducible).
     const int64_t tiles = (int64_t)n_tiles * m_tiles;
-    int splits = (int)std::min<int64_t>(8, num_cus / tiles);
+    int splits = (int)std::min<int64_t>(kMaxSplits, num_cus / tiles);
     splits = std::min(splits, w.KT / 4);                         // at least 4 K tiles per split
     while (splits > 1 && (size_t)splits * M * w.N * 4 > part_bytes) splits--;
     if (splits < 1) splits = 1;
@@ -626,14 +706,7 @@ hipError_t launch_m(const WeightView& w, const void* x, int M, void* y, int ydt,
                        (M + 15) / 16, M, n_tiles, m_tiles, splits, kt_per_split, (int)groups, w.N, y, ydt, w.K, out_scale, part, epi, ns);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || splits == 1) return e;
-    const int64_t total = (int64_t)M * w.N;
-    if (total % 4 == 0 && epi.kind != kEpiSwiglu && (ydt != kF32 || (reinterpret_cast<uintptr_t>(y) & 15u) == 0))
-        hipLaunchKernelGGL(splitk_reduce4_kernel, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, st, part, splits, M, w.N, y,
-                           ydt, out_scale, epi, ns, w.K);
-    else
-        hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, part, splits, M, w.N, y, ydt,
-                           out_scale, epi, ns, w.K);
-    return hipGetLastError();
+    return launch_reduce(part, splits, M, w.N, y, ydt, out_scale, epi, ns, w.K, st);
 }
 
 // Workgroup shapes: every wave owns 2 row blocks.
