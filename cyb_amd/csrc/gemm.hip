@@ -583,7 +583,8 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ part, int splits,
 // thread needs - its pieces of all the slabs, its residual, its row's factors - is requested before anything is used, and
 // the row is the workgroup's (blockIdx.y), not a division per element.  (Before: slab after slab, then four 64-bit
 // divisions, each in front of its own loads of the row's factor and the residual.)
-// RESULT
+// 14336 -> 4096, bf16 rows with a residual, us per call with staging and multiply: 45 rows 36.5 -> 33.9, 128 rows 38.6 -> 36.9,
+// 512 rows 76.0 -> 74.1.
 template <int SPLITS, bool SWIGLU>
 __global__ __launch_bounds__(256) void splitk_reduce4_kernel(const float* __restrict__ part, int M, int N, void* __restrict__ y, int ydt,
                                                              float out_scale, Epilogue epi, NormStats ns, int K)
@@ -629,8 +630,15 @@ __global__ __launch_bounds__(256) void splitk_reduce4_kernel(const float* __rest
 #pragma unroll
         for (int e = 0; e < 4; e++) v[e] = silu_mul(v[e] * f, w[e] * f);
     } else {
+        {
+            // (scaled, rounded, then added: with and without the residual the scaled sum has the same bits)
+#pragma clang fp contract(off)
 #pragma unroll
-        for (int e = 0; e < 4; e++) v[e] = v[e] * f + res[e];
+            for (int e = 0; e < 4; e++) {
+                v[e] *= f;
+                if (epi.kind == kEpiAdd) v[e] += res[e];
+            }
+        }
     }
     if (!aligned) {
 #pragma unroll
