@@ -51,10 +51,13 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
 
 // few rows (17 .. 64 on an output wide enough, up to 512 on a narrow one), FAST mode, activations already staged as f16 operands
 // (gemm_rows.hip); ssq_part / ssq_blocks / unscale: the staging pass's per-row statistics
-int gemm_rows_blocks(const WeightView& w, int M, int num_cus, const Epilogue& epi);
-bool gemm_rows_serves(const WeightView& w, int M, int num_cus, const Epilogue& epi);
+struct RowsPlan {
+    int nf;                  // column blocks of 16 per workgroup (1, 2 or 4); 0: the kernel does not take the call
+    int splits;              // K is split over that many workgroups, whose sums go to slabs (fp32 [M][N] each, together 4 MB at most)
+};
+RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi);
 hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, void* y, int ydt, const Epilogue& epi,
-                            const float* ssq_part, int ssq_blocks, const float* unscale, int num_cus, hipStream_t st);
+                            const float* ssq_part, int ssq_blocks, const float* unscale, const RowsPlan& plan, float* slabs, hipStream_t st);
 // test/bench hook: 2 = never take the few-rows kernel, 1 = whatever the width, 0 = automatic
 void set_gemm_tuning(int rows_kernel);
 // whether launch_gemm hands a FAST-mode call of M rows with this epilogue to the few-rows kernel (the hook included)

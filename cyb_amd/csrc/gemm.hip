@@ -821,6 +821,7 @@ hipError_t launch_nf(const WeightView& w, const void* x, int M, void* y, int ydt
 struct Touch {
     const uint8_t* base;          // the weight tensor (first_group past the grid: nothing to do)
     int first_group, NT, KT, NF, tile_bytes, ahead;
+    int groups, kt_per_split;     // K split: workgroup b works on group b % groups, on the K tiles of split b / groups
     int per_xcd, tiles;           // the tiled kernels' order: workgroup b works on column tile (b % 8) * per_xcd + b / 8 of `tiles` (0: on b)
 };
 
@@ -831,14 +832,16 @@ __device__ __forceinline__ void touch_weights(const Touch& tc, int b, int tid, i
         b = (b & 7) * tc.per_xcd + (b >> 3);
         if (b >= tc.tiles) return;
     }
-    const int kt0 = b % tc.KT;                     // (the multiply's workgroups start their K walk there)
+    const int kt_lo = b / tc.groups * tc.kt_per_split, KT = min(tc.kt_per_split, tc.KT - kt_lo);
+    if (tc.kt_per_split < tc.KT) b %= tc.groups;
+    const int kt0 = b % KT;                        // (the multiply's workgroups start their K walk there)
     uint32_t acc = 0;
     for (int idx = tid; idx < tc.NF * tc.ahead * lines; idx += nthreads) {
         const int line = idx % lines, ft = idx / lines, t = ft % tc.ahead, f = ft / tc.ahead;
         const int nt = min(b * tc.NF + f, tc.NT - 1);
         int kt = kt0 + t;
-        if (kt >= tc.KT) kt -= tc.KT;
-        acc ^= *reinterpret_cast<const uint32_t*>(tc.base + ((int64_t)nt * tc.KT + kt) * tc.tile_bytes + min(line * 128, tc.tile_bytes - 4));
+        if (kt >= KT) kt -= KT;
+        acc ^= *reinterpret_cast<const uint32_t*>(tc.base + ((int64_t)nt * tc.KT + kt_lo + kt) * tc.tile_bytes + min(line * 128, tc.tile_bytes - 4));
     }
     asm volatile("" ::"v"(acc));                   // (the loads have to be issued and waited for; nothing is stored)
 }
@@ -1086,9 +1089,17 @@ int g_rows_kernel = 0;        // (set_gemm_tuning: 2 = experiments switch the fe
 int g_touch = 2;              // (5 = the staging launch asks for no weights ahead of the multiply, 6 = only ahead of the few-rows kernel)
 void set_gemm_tuning(int rows_kernel) { g_rows_kernel = rows_kernel >= 5 ? 0 : rows_kernel; g_touch = rows_kernel == 5 ? 0 : rows_kernel == 6 ? 1 : 2; }
 
+static RowsPlan rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi)
+{
+    if (g_rows_kernel == 2) return {0, 1};
+    return gemm_rows_plan(w, M, g_rows_kernel == 1 ? 1 : num_cus, epi);
+}
+
+// (the calls whose way here api.hip decides by this; a long K takes the kernel only where the tiled ones would have run)
 bool gemm_rows_takes(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
-    return g_rows_kernel != 2 && gemm_rows_serves(w, M, g_rows_kernel == 1 ? 1 : num_cus, epi);
+    const RowsPlan plan = rows_plan(w, M, num_cus, epi);
+    return plan.nf != 0 && plan.splits == 1;
 }
 
 // the extra workgroups of a staging launch (grid_x grows by them) for a call of 33 rows or more that goes through the
@@ -1108,13 +1119,19 @@ static bool few_rows_tiles64(const WeightView& w, int M, int num_cus, const Epil
 
 static Touch plan_touch(const WeightView& w, int mc, int num_cus, const Epilogue& ec, bool exact, unsigned& grid_x)
 {
-    Touch tc = {nullptr, 0x7fffffff, w.NT, w.KT, 1, tile_bytes(w.bits), 0, 0, 0};
+    Touch tc = {nullptr, 0x7fffffff, w.NT, w.KT, 1, tile_bytes(w.bits), 0, 0x7fffffff, w.KT, 0, 0};
     if (g_touch == 0 || exact || mc < 33 || w.KT < 32) return tc;
     const int64_t per_k_tile = (int64_t)w.NT * tile_bytes(w.bits);
     int nf = 0, groups = 0;
-    if (gemm_rows_takes(w, mc, num_cus, ec)) {
-        nf = gemm_rows_blocks(w, mc, g_rows_kernel == 1 ? 1 : num_cus, ec);
+    const RowsPlan plan = rows_plan(w, mc, num_cus, ec);
+    if (plan.nf) {
+        nf = plan.nf;
         groups = (w.NT + nf - 1) / nf;
+        if (plan.splits > 1) {                       // (the multiply's workgroups of a split follow those of the split before it)
+            tc.groups = groups;
+            tc.kt_per_split = (w.KT + plan.splits - 1) / plan.splits;
+            groups *= plan.splits;
+        }
     } else if (g_touch >= 2 && per_k_tile * w.KT <= ((int64_t)40 << 20) && few_rows_tiles64(w, mc, num_cus, ec)) {
         // the 128 x 64 / 64 x 64 tiles of the tiled kernels (65 .. 128 rows on wide outputs; 4096 -> 14336 at 128 rows:
         // 27.5 us, 24.3 with the same tensor every call): 4096 -> 14336 at 65 / 100 / 128 rows 25.3 / 27.1 / 28.1 ->
@@ -1129,6 +1146,7 @@ static Touch plan_touch(const WeightView& w, int mc, int num_cus, const Epilogue
     tc.base = w.base;
     tc.NF = nf;
     tc.ahead = (int)std::min<int64_t>(w.KT, std::max<int64_t>(4, ((int64_t)16 << 20) / per_k_tile));
+    if (tc.kt_per_split < w.KT) tc.ahead = std::min(w.KT % tc.kt_per_split ? w.KT % tc.kt_per_split : tc.kt_per_split, std::max(4, tc.ahead * tc.kt_per_split / w.KT));
     tc.first_group = (int)((grid_x + 7) / 8 * 8);
     grid_x = (unsigned)(tc.first_group + groups);
     return tc;
@@ -1203,8 +1221,10 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         // few rows on a wide output, FAST mode: the kernel of gemm_rows.hip (waves split K, no LDS on the way)
-        if (!exact && kdt == kF16 && gemm_rows_takes(w, mc, num_cus, ec)) {
-            e = launch_gemm_rows(w, workspace, mc, yc, ydt, ec, ns.part, ns.nblk, ns.unscale, g_rows_kernel == 1 ? 1 : num_cus, st);
+        const RowsPlan plan = !exact && kdt == kF16 ? rows_plan(w, mc, num_cus, ec) : RowsPlan{0, 1};
+        if (plan.nf) {
+            e = launch_gemm_rows(w, workspace, mc, yc, ydt, ec, ns.part, ns.nblk, ns.unscale, plan, part, st);
+            if (e == hipSuccess && plan.splits > 1) e = launch_reduce(part, plan.splits, mc, w.N, yc, ydt, out_scale, ec, ns, w.K, st);
             if (e != hipSuccess) return e;
             continue;
         }

@@ -88,10 +88,11 @@ __device__ __forceinline__ void dequant_group(const WRegs<BITS>& r, int j, uint3
 
 // MF row blocks of 16 per workgroup (blockIdx.y-th MF * 16 rows of the call), NF column blocks per workgroup, WAVES
 // waves that split K, DEPTH K tiles of packed weights and XD K tiles of X in flight per wave.
-template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD>
+// SPLIT: the blockIdx.z-th kt_per_split K tiles only, and the sums go to that split's slab of `slabs`, fp32 [M][N].
+template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD, bool SPLIT>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(WAVES / 4, WAVES / 4))) void gemm_rows_kernel(
     const uint8_t* __restrict__ wbase, const u32x4_t* __restrict__ x, int KT_, int NT_, int x_row_blocks, int M, int N_,
-    void* __restrict__ y, int ydt, int K_, Epilogue epi, NormStats ns)
+    void* __restrict__ y, int ydt, int K_, Epilogue epi, NormStats ns, int kt_per_split, float* __restrict__ slabs)
 {
     const WeightView w = {wbase, N_, K_, NT_, KT_, BITS};
     constexpr int FR = MF * NF;                        // accumulator blocks per wave
@@ -103,7 +104,9 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(WAVE
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nt0 = (int)blockIdx.x * NF;
-    const int KT = w.KT, K = w.K, G = K / kGroup;
+    const int K = w.K, G = K / kGroup;
+    const int kt_lo = SPLIT ? (int)blockIdx.z * kt_per_split : 0;
+    const int KT = SPLIT ? min(kt_per_split, w.KT - kt_lo) : w.KT;      // my workgroup's K tiles: kt_lo ..
     const uint32_t magic = q4_magic_vgpr();
     const int T = KT > wv ? (KT - wv + WAVES - 1) / WAVES : 0;        // my K tiles: number t is tile wv + WAVES * t
     // Workgroups that run side by side read the same rows of X: walking K in the same order they would all
@@ -113,7 +116,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(WAVE
     // (a tile number past my last one is clamped to the last K tile: loaded again, never used)
     auto tile_of = [&](int t) __attribute__((always_inline)) {
         const int kt = min(wv + WAVES * t, KT - 1) + kt0;
-        return kt >= KT ? kt - KT : kt;
+        return kt_lo + (kt >= KT ? kt - KT : kt);
     };
     // (row blocks and column blocks past the end are clamped to the last real one: computed again, never
     // stored; the offsets are wave-uniform, the lane's part of an address is one register)
@@ -192,6 +195,11 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(WAVE
         tot[0][f] = s;
     }
     const int m0 = (rb0 + wv) * 16;
+    if constexpr (SPLIT) {
+        const Epilogue plain = {kEpiNone, nullptr, nullptr, 0, 0.f};
+        write_rows<1, NF>(tot, stg + wv * (16 * NF * 16), m0, nt0, M, w.N, slabs + (int64_t)blockIdx.z * M * w.N, kF32, 1.0f, plain, lane);
+        return;
+    }
     if (epi.gamma || ns.unscale) {
 #pragma unroll
         for (int r4 = 0; r4 < 4; r4++) {
@@ -215,15 +223,16 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(WAVE
     write_rows<1, NF>(tot, stg + wv * (16 * NF * 16), m0, nt0, M, w.N, y, ydt, 1.0f, epi, lane);
 }
 
-template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD>
-hipError_t launch_rows_t(const WeightView& w, const void* x, int M, void* y, int ydt, const Epilogue& epi, const NormStats& ns,
-                         hipStream_t st)
+template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD, bool SPLIT>
+hipError_t launch_rows_t(const WeightView& w, const void* x, int M, void* y, int ydt, const Epilogue& epi, const NormStats& ns, int splits,
+                         float* slabs, hipStream_t st)
 {
     constexpr int lds = WAVES * MF * NF * 1024 + MF * 16 * NF * 16 * 4;
-    (void)LdsRequest<&gemm_rows_kernel<BITS, MF, NF, WAVES, DEPTH, XD>, lds>::registered;
+    (void)LdsRequest<&gemm_rows_kernel<BITS, MF, NF, WAVES, DEPTH, XD, SPLIT>, lds>::registered;
     const unsigned groups = (unsigned)((w.NT + NF - 1) / NF), row_parts = (unsigned)((M + 16 * MF - 1) / (16 * MF));
-    hipLaunchKernelGGL((gemm_rows_kernel<BITS, MF, NF, WAVES, DEPTH, XD>), dim3(groups, row_parts), dim3(WAVES * 64), lds, st, w.base,
-                       reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT, (M + 15) / 16, M, w.N, y, ydt, w.K, epi, ns);
+    hipLaunchKernelGGL((gemm_rows_kernel<BITS, MF, NF, WAVES, DEPTH, XD, SPLIT>), dim3(groups, row_parts, (unsigned)splits), dim3(WAVES * 64), lds, st,
+                       w.base, reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT, (M + 15) / 16, M, w.N, y, ydt, w.K, epi, ns,
+                       (w.KT + splits - 1) / splits, slabs);
     return hipGetLastError();
 }
 
@@ -234,33 +243,38 @@ hipError_t launch_rows_t(const WeightView& w, const void* x, int M, void* y, int
 // column blocks a wave carries, so: the fewest column blocks that still fit one round of workgroups
 // (4096 -> 4096 at 128 rows: 256 workgroups of two column blocks 14.3 us, 128 of four 17.0; 4096 -> 2048 at 24
 // rows: 128 of one 11.6, the tiled kernels 17.5), at least a quarter of a round (4096 -> 1024 at 24 rows, 64
-// workgroups: 11.4 against 17.4), K of 16 .. 64 tiles (beyond that the tiled kernels split K over workgroups:
-// 14336 -> 4096 33.6 against 43 us here).  More than 64 rows are one workgroup per 64 rows and column group:
-// narrow outputs only, where all of them fit one round.
-int rows_column_blocks(const WeightView& w, int M, int num_cus, const Epilogue& epi)
+// workgroups: 11.4 against 17.4), K of at least 16 tiles.  More than 64 rows are one workgroup per 64 rows and column
+// group: narrow outputs only, where all of them fit one round.
+// K of more than 64 tiles is shared out over workgroups of four column blocks, as many shares as fit one round (eight at
+// most, sixteen K tiles each at least): a CU then takes in its rows' share of K instead of all of it, four column blocks'
+// weights beside it, and the slab-adding pass joins them.  Without two shares the tiled kernels stay.
+// us per call with all passes, against the tiled kernels (which split K as well): 14336 -> 4096 bf16 at 45 / 64 / 96 rows
+// 26.5 / 28.5 / 33.9 against 33.9 / 34.4 / 35; f16 at 45 rows 21.5 against 28.2; 14336 -> 8192 at 45 rows 34.8 against
+// 48; 14336 -> 1024 at 100 / 256 rows 23.6 / 32.4 against 33 / 43; 12288 -> 512 at 400 rows 29.3 against 39.
+RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
-    if (M <= 16 || M > 512 || w.KT < 16 || w.KT > 64) return 0;
+    if (M <= 16 || M > 512 || w.KT < 16) return {0, 1};
     const int64_t parts = (M + 63) / 64;
+    if (w.KT > 64) {
+        const int64_t groups = (w.NT + 3) / 4 * parts;
+        int splits = (int)std::min<int64_t>(8, num_cus / std::max<int64_t>(groups, 1));
+        splits = std::min(splits, w.KT / 16);
+        if (splits < 2) return {0, 1};
+        const int per = (w.KT + splits - 1) / splits;
+        return {4, (w.KT + per - 1) / per};                     // (no empty split)
+    }
     for (int nf : {1, 2, 4}) {
         if (nf == 1 && epi.kind == kEpiSwiglu) continue;        // (a gate block and its up block sit in one workgroup)
         const int64_t groups = (w.NT + nf - 1) / nf * parts;
-        if (groups <= num_cus) return groups * 4 >= num_cus ? nf : 0;
+        if (groups <= num_cus) return {groups * 4 >= num_cus ? nf : 0, 1};
     }
-    return parts == 1 ? 4 : 0;       // (up to 64 rows a wide output may take more than one round)
-}
-
-int gemm_rows_blocks(const WeightView& w, int M, int num_cus, const Epilogue& epi) { return rows_column_blocks(w, M, num_cus, epi); }
-
-bool gemm_rows_serves(const WeightView& w, int M, int num_cus, const Epilogue& epi)
-{
-    return rows_column_blocks(w, M, num_cus, epi) != 0;
+    return {parts == 1 ? 4 : 0, 1};       // (up to 64 rows a wide output may take more than one round)
 }
 
 hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, void* y, int ydt, const Epilogue& epi,
-                            const float* ssq_part, int ssq_blocks, const float* unscale, int num_cus, hipStream_t st)
+                            const float* ssq_part, int ssq_blocks, const float* unscale, const RowsPlan& plan, float* slabs, hipStream_t st)
 {
     const NormStats ns = {ssq_part, ssq_blocks, unscale};
-    const int nf = rows_column_blocks(w, M, num_cus, epi);
     // four waves, one per SIMD with the whole register file: four K tiles of packed weights and one K tile of
     // X in flight per wave.  Measured against it on 4096 -> 14336 at 64 bf16 rows (19.1 us per call with the
     // staging pass; the tiled kernel 22.1): eight waves with two / three weight tiles in flight 22.8 / 20.2;
@@ -270,19 +284,21 @@ hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, vo
     // Up to 48 rows the workgroup carries two or three row blocks instead of four: the rows of X are most of what
     // a CU takes in, and its L1 delivers 64 bytes a cycle.
     const int mf = M > 48 ? 4 : M > 32 ? 3 : 2;
-    auto go = [&](auto bits, auto nfc) {
+    auto go = [&](auto bits, auto nfc, auto split) {
         constexpr int B = decltype(bits)::value, F = decltype(nfc)::value;
-        if (mf == 2) return launch_rows_t<B, 2, F, 4, 4, 1>(w, x_staged, M, y, ydt, epi, ns, st);
-        if (mf == 3) return launch_rows_t<B, 3, F, 4, 4, 1>(w, x_staged, M, y, ydt, epi, ns, st);
-        return launch_rows_t<B, 4, F, 4, 4, 1>(w, x_staged, M, y, ydt, epi, ns, st);
+        constexpr bool S = decltype(split)::value;
+        if (mf == 2) return launch_rows_t<B, 2, F, 4, 4, 1, S>(w, x_staged, M, y, ydt, epi, ns, plan.splits, slabs, st);
+        if (mf == 3) return launch_rows_t<B, 3, F, 4, 4, 1, S>(w, x_staged, M, y, ydt, epi, ns, plan.splits, slabs, st);
+        return launch_rows_t<B, 4, F, 4, 4, 1, S>(w, x_staged, M, y, ydt, epi, ns, plan.splits, slabs, st);
     };
-    auto with_bits = [&](auto nfc) {
-        if (w.bits == 8) return go(std::integral_constant<int, 8>{}, nfc);
-        return go(std::integral_constant<int, 4>{}, nfc);
+    auto with_bits = [&](auto nfc, auto split) {
+        if (w.bits == 8) return go(std::integral_constant<int, 8>{}, nfc, split);
+        return go(std::integral_constant<int, 4>{}, nfc, split);
     };
-    if (nf == 1) return with_bits(std::integral_constant<int, 1>{});
-    if (nf == 2) return with_bits(std::integral_constant<int, 2>{});
-    return with_bits(std::integral_constant<int, 4>{});
+    if (plan.splits > 1) return with_bits(std::integral_constant<int, 4>{}, std::true_type{});
+    if (plan.nf == 1) return with_bits(std::integral_constant<int, 1>{}, std::false_type{});
+    if (plan.nf == 2) return with_bits(std::integral_constant<int, 2>{}, std::false_type{});
+    return with_bits(std::integral_constant<int, 4>{}, std::false_type{});
 }
 
 }  // namespace cybq

@@ -925,6 +925,61 @@ def test_prefill_few_rows_waves_split_k(backend, oracle, bits, shape):
     qw.free()
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("shape", [(4096, 14336, 45), (992, 65 * 128, 64), (16, 16384 + 32, 512), (1030, 9216 + 64, 130),
+                                   (2048, 8192 + 32, 33), (4096, 65 * 128 - 32, 17)])
+def test_prefill_few_rows_long_k_split_over_workgroups(backend, oracle, bits, shape):
+    """FAST mode, K of more than 64 tiles: workgroups of the kernel whose waves split K take a share of K each and the
+    slab-adding pass joins them.  The fewest K tiles, shares of unequal size, one strip, N that ends inside a column block
+    and is no multiple of four (the pass's scalar form), y off its vector alignment, every epilogue; against float64 and
+    (33 rows and more) against the tiled kernels; 17 rows are fp32 (16-bit rows that few keep the decode kernels)."""
+    N, K, M = shape
+    q, s = _quant(oracle, bits, N, K, cfg=65)
+    qw = backend.upload_quantized(q, s, bits)
+    wd = torch.from_numpy(oracle.dequant(q, s)).cuda().double()
+    r = torch.from_numpy(synth.activations(66, M, N)).cuda()
+    try:
+        for xdt, ydt in (("bf16", "f32"), ("f16", "bf16"), ("f32", "f16")) if M > 32 else (("f32", "f32"), ("f32", "bf16")):
+            x = _x(M, K, xdt, cfg=67)
+            ref = x.double() @ wd.T
+            bar = FAST if ydt == "f32" else 4e-3            # (a 16-bit output rounds every element once more)
+            y = _run(backend, qw, x, ydt)
+            assert ((y.double() - ref).norm() / ref.norm()).item() < bar, (xdt, ydt)
+            assert torch.equal(_run(backend, qw, x, ydt), y)             # reproducible
+            backend.set_gemm_tuning(2)
+            y_tiled = _run(backend, qw, x, ydt)
+            backend.set_gemm_tuning(0)
+            assert ((y.double() - y_tiled.double()).norm() / ref.norm()).item() < 2 * bar, (xdt, ydt)
+            want = ref + r.to(TDT[ydt]).double()
+            for off in (0, 1):
+                y2 = torch.empty(M * N + 1, dtype=TDT[ydt], device="cuda")[off:off + M * N].view(M, N)
+                r2 = torch.empty_like(y2).copy_(r)
+                backend.matmul_ex(qw, x, y2, "add", r2)
+                torch.cuda.synchronize()
+                assert ((y2.double() - want).norm() / want.norm()).item() < bar, (xdt, ydt, off)
+        if M > 32:
+            x = _x(M, K, "f16", cfg=67)
+            gamma = (1.0 + 0.1 * torch.from_numpy(synth.activations(68, 1, K))[0]).cuda()
+            y3 = torch.empty((M, N), dtype=torch.float32, device="cuda")
+            backend.matmul_norm(qw, x, gamma, 1e-5, y3, "add", r)
+            torch.cuda.synchronize()
+            xd = x.double()
+            ref = (xd * torch.rsqrt((xd * xd).mean(dim=1, keepdim=True) + 1e-5) * gamma.double()) @ wd.T + r.double()
+            assert ((y3.double() - ref).norm() / ref.norm()).item() < 2 * FAST
+            if N % 16 == 0:
+                pair = backend.fuse_pairs(qw, qw)
+                y4 = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+                backend.matmul_ex(pair, x, y4, "swiglu")
+                torch.cuda.synchronize()
+                z = xd @ wd.T
+                ref = torch.nn.functional.silu(z) * z
+                assert ((y4.double() - ref).norm() / ref.norm()).item() < 4e-3
+                pair.free()
+    finally:
+        backend.set_gemm_tuning(0)
+    qw.free()
+
+
 @pytest.mark.parametrize("shape", [(14336, 4096, 17), (4096, 4096, 32), (8200, 2048 + 128, 24)])
 def test_prefill_fp32_rows_17_to_32_fast_mode(backend, oracle, shape):
     """fp32 activations leave the decode kernels at 17 rows; in FAST mode they are rounded to f16 by the staging
