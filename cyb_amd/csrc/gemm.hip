@@ -174,7 +174,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2
     // they would all ask the same few L2 channels for the same lines at the same
     // moment (a row of X is a multiple of the channel interleave long), so each
     // column tile starts its walk at a different K tile and wraps around.  The
-    // order depends on the column tile only: a row of Y does not depend on M.
+    // order depends on the column tile only: with one tile width a row of Y does not depend on M.
     const int kt0 = tile_n % KT;
     auto rot = [&](int kt) {
         const int r = min(kt, KT - 1) + kt0;
@@ -362,7 +362,7 @@ __device__ __forceinline__ void static_for(F&& f)
 template <int BITS, int NF, int MF, int MW, int XD>
 __global__ __launch_bounds__((MW + 4) * 64) __attribute__((amdgpu_waves_per_eu((MW + 7) / 4, (MW + 7) / 4))) void gemm_roles_kernel(
     const uint8_t* __restrict__ wbase, const u32x4_t* __restrict__ x, int KT_, int NT_, int x_row_blocks, int M, int n_tiles,
-    int m_tiles, int groups, int N_, void* __restrict__ y, int ydt, int K_, float out_scale, Epilogue epi, NormStats ns)
+    int m_tiles, int groups, int nt_first, int N_, void* __restrict__ y, int ydt, int K_, float out_scale, Epilogue epi, NormStats ns)
 {
     const WeightView w = {wbase, N_, K_, NT_, KT_, BITS};
     constexpr int SW = 4;                             // staging waves
@@ -381,7 +381,7 @@ __global__ __launch_bounds__((MW + 4) * 64) __attribute__((amdgpu_waves_per_eu((
     const int tile_m = item / n_tiles, tile_n = item - tile_m * n_tiles;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nt0 = tile_n * NF;
+    const int nt0 = nt_first + tile_n * NF;          // (the call's column tiles start at strip nt_first)
     const int KT = w.KT, K = w.K;
     const int kt0 = tile_n % KT;
     auto rot = [&](int kt) {
@@ -529,22 +529,89 @@ __global__ __launch_bounds__((MW + 4) * 64) __attribute__((amdgpu_waves_per_eu((
                 for (int f = 0; f < NF; f++) acc[i][f][r] *= rs;
             }
     }
+    if constexpr (NF % 2 == 0) {
+        if (epi.kind == kEpiSwiglu) {      // column blocks 2p / 2p+1 are gate / up of output block (nt0 >> 1) + p
+            float4_t act[MF][NF / 2];
+#pragma unroll
+            for (int i = 0; i < MF; i++)
+#pragma unroll
+                for (int p = 0; p < NF / 2; p++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) act[i][p][r] = silu_mul(acc[i][2 * p][r] * out_scale, acc[i][2 * p + 1][r] * out_scale);
+            const Epilogue plain = {kEpiNone, nullptr, nullptr, 0, 0.f};
+            write_rows<MF, NF / 2>(act, reinterpret_cast<float*>(smem) + wave * (16 * NF * 16), m0, nt0 >> 1, M, w.N >> 1, y, ydt, 1.0f, plain, lane);
+            return;
+        }
+    }
     write_rows<MF, NF>(acc, reinterpret_cast<float*>(smem) + wave * (16 * NF * 16), m0, nt0, M, w.N, y, ydt, out_scale, epi, lane);
 }
 
+// nt_first, strips: the part of the output's strips that the launch covers (all of them unless said otherwise)
 template <int BITS, int NF, int MF, int MW, int XD>
 hipError_t launch_roles(const WeightView& w, const void* x, int M, void* y, int ydt, float out_scale, const Epilogue& epi,
-                        const NormStats& ns, hipStream_t st)
+                        const NormStats& ns, hipStream_t st, int nt_first = 0, int strips = 0)
 {
     constexpr int lds = 2 * NF * (4 * 64) * 16;
     constexpr int BM = MW * MF * 16;
     (void)LdsRequest<&gemm_roles_kernel<BITS, NF, MF, MW, XD>, lds>::registered;
-    const int n_tiles = (w.NT + NF - 1) / NF, m_tiles = (M + BM - 1) / BM;
+    const int n_tiles = ((strips ? strips : w.NT) + NF - 1) / NF, m_tiles = (M + BM - 1) / BM;
     const unsigned groups = (unsigned)(((int64_t)n_tiles * m_tiles + 7) / 8 * 8);
     hipLaunchKernelGGL((gemm_roles_kernel<BITS, NF, MF, MW, XD>), dim3(groups), dim3((MW + 4) * 64), lds, st, w.base,
-                       reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT, (M + 15) / 16, M, n_tiles, m_tiles, (int)groups, w.N, y, ydt, w.K,
+                       reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT, (M + 15) / 16, M, n_tiles, m_tiles, (int)groups, nt_first, w.N, y, ydt, w.K,
                        out_scale, epi, ns);
     return hipGetLastError();
+}
+
+// Whole rounds of 256-row tiles.  A round of workgroups costs about as much whether it is full or not, so the columns are
+// cut into one or two launches of tiles as wide as makes the sum of the rounds' widths smallest (4096 -> 28672 in gate / up
+// pairs at 512 rows: 448 tiles of 128 columns are 1.75 rounds; 256 of them and 256 tiles of 96 columns are two).
+// us per call, bf16, against one width (and, for the pairs, the kernel without roles): 4096 -> 28672 norm + SwiGLU at 512 /
+// 1024 rows 130.8 / 257.5 -> 121.1 / 231.4, SwiGLU at 2048 (one width) 439.8 -> 412.6; 4096 -> 20000 at 512 rows 106.4 ->
+// 92.5, 4096 -> 25008 at 300 rows 106.9 -> 102.4.
+struct RoundPlan {
+    int nf1, strips1, nf2;          // strips1 columns blocks in tiles nf1 wide, the rest in tiles nf2 wide (0: nothing left)
+};
+RoundPlan plan_rounds(int NT, int M, int num_cus, int nf, bool pairs)
+{
+    const int64_t m = (M + 255) / 256;
+    auto cost = [&](int64_t strips, int width) {      // in column blocks of one row tile; + 1: start and end of a round
+        return ((strips + width - 1) / width * m + num_cus - 1) / num_cus * (width + 1);
+    };
+    RoundPlan best = {nf, NT, 0};
+    const int64_t one = cost(NT, nf);
+    int64_t least = one;
+    for (int a : {8, 7})
+        for (int b : {8, 7, 6, 4}) {
+            if (a == b || (pairs && (a % 2 || b % 2))) continue;
+            for (int64_t rounds = 1; rounds <= 8; rounds++) {
+                const int64_t strips1 = rounds * num_cus / m * a;
+                if (strips1 <= 0 || strips1 >= NT) continue;
+                const int64_t c = cost(strips1, a) + cost(NT - strips1, b);
+                if (c < least) {
+                    least = c;
+                    best = {a, (int)strips1, b};
+                }
+            }
+        }
+    return least * 20 <= one * 19 ? best : RoundPlan{nf, NT, 0};        // (5 % at least: the second launch costs about 2 us)
+}
+
+template <int BITS>
+hipError_t launch_rounds(const WeightView& w, const void* x, int M, void* y, int ydt, float out_scale, const Epilogue& epi, const NormStats& ns,
+                         int num_cus, int nf, hipStream_t st)
+{
+    // (a row's bits depend on the tile its column sits in, and with two widths that depends on the number of row tiles: outputs
+    // in multiples of 112 columns, whose rows have the same bits at every row count, keep their one width)
+    const RoundPlan plan = nf == 7 ? RoundPlan{7, w.NT, 0} : plan_rounds(w.NT, M, num_cus, nf, epi.kind == kEpiSwiglu);
+    auto go = [&](int width, int first, int strips) {
+        if (width == 8) return launch_roles<BITS, 8, 2, 8, 2>(w, x, M, y, ydt, out_scale, epi, ns, st, first, strips);
+        if (width == 7) return launch_roles<BITS, 7, 2, 8, 2>(w, x, M, y, ydt, out_scale, epi, ns, st, first, strips);
+        if (width == 6) return launch_roles<BITS, 6, 2, 8, 2>(w, x, M, y, ydt, out_scale, epi, ns, st, first, strips);
+        return launch_roles<BITS, 4, 2, 8, 2>(w, x, M, y, ydt, out_scale, epi, ns, st, first, strips);
+    };
+    const hipError_t e = go(plan.nf1, 0, plan.strips1);
+    if (e != hipSuccess || !plan.nf2) return e;
+    return go(plan.nf2, plan.strips1, w.NT - plan.strips1);
 }
 
 constexpr int kMaxSplits = 8;
@@ -737,10 +804,9 @@ hipError_t launch_t(const WeightView& w, const void* x, int M, void* y, int ydt,
         if (tiles512 >= num_cus && (rem == 0 || rem > 256))
             return launch_m<BITS, XBF, NF, EXACT, 4, 8>(w, x, M, y, ydt, out_scale, part, part_bytes, num_cus, epi, ns, st);
     }
-    // enough 256-row tiles to fill the chip without a K split: the role-split kernel (the SwiGLU
-    // epilogue is not among what it writes)
+    // enough 256-row tiles to fill the chip without a K split: the role-split kernel
     if constexpr (!EXACT) {
-        if (tiles256 >= num_cus && epi.kind != kEpiSwiglu) return launch_roles<BITS, NF, 2, 8, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
+        if (tiles256 >= num_cus) return launch_rounds<BITS>(w, x, M, y, ydt, out_scale, epi, ns, num_cus, NF, st);
     }
     if (tiles256 < num_cus && few_rows) return launch_m<BITS, XBF, NF, EXACT, 2, 4>(w, x, M, y, ydt, out_scale, part, part_bytes, num_cus, epi, ns, st);
     return launch_m<BITS, XBF, NF, EXACT, 2, 8>(w, x, M, y, ydt, out_scale, part, part_bytes, num_cus, epi, ns, st);

@@ -980,6 +980,50 @@ def test_prefill_few_rows_long_k_split_over_workgroups(backend, oracle, bits, sh
     qw.free()
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("N,M,pair", [(28672, 300, True), (28672, 257, True), (32 * 1083, 512, True), (20000, 300, False),
+                                      (24998, 700, False), (20016, 512, False)])
+def test_prefill_rounds_of_two_widths(backend, oracle, bits, N, M, pair):
+    """FAST mode, enough 256-row tiles to fill the chip: the columns are cut into launches of wide and of narrower tiles so
+    that whole rounds come out.  SwiGLU pairs (even widths only) and plain outputs, a second launch that ends inside a
+    tile, N that is no multiple of 16 or 4, ragged rows, residual add and folded norm; every column against float64."""
+    K = 288                                             # (a last K tile that is a quarter full)
+    half = N // 2 if pair else N
+    q, s = _quant(oracle, bits, half, K, cfg=71)
+    qw = backend.upload_quantized(q, s, bits)
+    wd = torch.from_numpy(oracle.dequant(q, s)).cuda().double()
+    x = _x(M, K, "bf16", cfg=72)
+    ref = x.double() @ wd.T
+    if pair:
+        q2, s2 = _quant(oracle, bits, half, K, cfg=73)
+        q2w = backend.upload_quantized(q2, s2, bits)
+        up = x.double() @ torch.from_numpy(oracle.dequant(q2, s2)).cuda().double().T
+        fused = backend.fuse_pairs(qw, q2w)
+        for ydt in ("f32", "bf16"):
+            y = torch.full((M, half), float("nan"), dtype=TDT[ydt], device="cuda")
+            backend.matmul_ex(fused, x, y, "swiglu")
+            torch.cuda.synchronize()
+            want = torch.nn.functional.silu(ref) * up
+            assert ((y.double() - want).norm(dim=0) / want.norm(dim=0)).max().item() < (3e-3 if ydt == "f32" else 6e-3)    # column by column
+            assert ((y.double() - want).norm() / want.norm()).item() < (2 * FAST if ydt == "f32" else 4e-3)
+        for w in (q2w, fused):
+            w.free()
+    else:
+        y = _run(backend, qw, x)
+        assert ((y.double() - ref).norm(dim=0) / ref.norm(dim=0)).max().item() < 3e-3
+        assert ((y.double() - ref).norm() / ref.norm()).item() < FAST
+        assert torch.equal(_run(backend, qw, x), y)
+        r = torch.from_numpy(synth.activations(74, M, N)).cuda()
+        gamma = (1.0 + 0.1 * torch.from_numpy(synth.activations(75, 1, K))[0]).cuda()
+        y2 = torch.empty_like(y)
+        backend.matmul_norm(qw, x, gamma, 1e-5, y2, "add", r)
+        torch.cuda.synchronize()
+        xd = x.double()
+        want = (xd * torch.rsqrt((xd * xd).mean(dim=1, keepdim=True) + 1e-5) * gamma.double()) @ wd.T + r.double()
+        assert ((y2.double() - want).norm() / want.norm()).item() < 2 * FAST
+    qw.free()
+
+
 @pytest.mark.parametrize("shape", [(14336, 4096, 17), (4096, 4096, 32), (8200, 2048 + 128, 24)])
 def test_prefill_fp32_rows_17_to_32_fast_mode(backend, oracle, shape):
     """fp32 activations leave the decode kernels at 17 rows; in FAST mode they are rounded to f16 by the staging
