@@ -54,6 +54,7 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
 struct RowsPlan {
     int nf;                  // column blocks of 16 per workgroup (1, 2 or 4); 0: the kernel does not take the call
     int splits;              // K is split over that many workgroups, whose sums go to slabs (fp32 [M][N] each, together 4 MB at most)
+    bool two_per_cu = false; // two workgroups share a CU (nf = 4, up to 48 rows)
 };
 RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi);
 hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, void* y, int ydt, const Epilogue& epi,

@@ -89,8 +89,9 @@ __device__ __forceinline__ void dequant_group(const WRegs<BITS>& r, int j, uint3
 // MF row blocks of 16 per workgroup (blockIdx.y-th MF * 16 rows of the call), NF column blocks per workgroup, WAVES
 // waves that split K, DEPTH K tiles of packed weights and XD K tiles of X in flight per wave.
 // SPLIT: the blockIdx.z-th kt_per_split K tiles only, and the sums go to that split's slab of `slabs`, fp32 [M][N].
-template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD, bool SPLIT>
-__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(WAVES / 4, WAVES / 4))) void gemm_rows_kernel(
+// OCC: workgroups per CU.
+template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD, bool SPLIT, int OCC = 1>
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC * WAVES / 4, OCC * WAVES / 4))) void gemm_rows_kernel(
     const uint8_t* __restrict__ wbase, const u32x4_t* __restrict__ x, int KT_, int NT_, int x_row_blocks, int M, int N_,
     void* __restrict__ y, int ydt, int K_, Epilogue epi, NormStats ns, int kt_per_split, float* __restrict__ slabs)
 {
@@ -223,14 +224,14 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(WAVE
     write_rows<1, NF>(tot, stg + wv * (16 * NF * 16), m0, nt0, M, w.N, y, ydt, 1.0f, epi, lane);
 }
 
-template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD, bool SPLIT>
+template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD, bool SPLIT, int OCC = 1>
 hipError_t launch_rows_t(const WeightView& w, const void* x, int M, void* y, int ydt, const Epilogue& epi, const NormStats& ns, int splits,
                          float* slabs, hipStream_t st)
 {
     constexpr int lds = WAVES * MF * NF * 1024 + MF * 16 * NF * 16 * 4;
-    (void)LdsRequest<&gemm_rows_kernel<BITS, MF, NF, WAVES, DEPTH, XD, SPLIT>, lds>::registered;
+    (void)LdsRequest<&gemm_rows_kernel<BITS, MF, NF, WAVES, DEPTH, XD, SPLIT, OCC>, lds>::registered;
     const unsigned groups = (unsigned)((w.NT + NF - 1) / NF), row_parts = (unsigned)((M + 16 * MF - 1) / (16 * MF));
-    hipLaunchKernelGGL((gemm_rows_kernel<BITS, MF, NF, WAVES, DEPTH, XD, SPLIT>), dim3(groups, row_parts, (unsigned)splits), dim3(WAVES * 64), lds, st,
+    hipLaunchKernelGGL((gemm_rows_kernel<BITS, MF, NF, WAVES, DEPTH, XD, SPLIT, OCC>), dim3(groups, row_parts, (unsigned)splits), dim3(WAVES * 64), lds, st,
                        w.base, reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT, (M + 15) / 16, M, w.N, y, ydt, w.K, epi, ns,
                        (w.KT + splits - 1) / splits, slabs);
     return hipGetLastError();
@@ -268,7 +269,12 @@ RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue&
         const int64_t groups = (w.NT + nf - 1) / nf * parts;
         if (groups <= num_cus) return {groups * 4 >= num_cus ? nf : 0, 1};
     }
-    return {parts == 1 ? 4 : 0, 1};       // (up to 64 rows a wide output may take more than one round)
+    // up to 64 rows a wide output may take more than one round.  Up to 48 rows two workgroups share a CU then (two or three
+    // packed weight tiles in flight per wave instead of four, 256 registers): one's start and end overlap the other's
+    // K loop (4096 -> 28672 bf16 norm + SwiGLU at 45 rows 35.0 -> 30.2 us, fp32 at 24 rows 28.3 -> 25.6, 2048 -> 20000 at 40
+    // rows 20.5 -> 17.6, 2048 -> 128256 at 40 rows 71.0 -> 51.1).  With four row blocks they do not fit 256 registers
+    // without giving up the lead of the weights: 38.3 against 38.1 us, 35.7 against 36.1.
+    return {parts == 1 ? 4 : 0, 1, M <= 48};
 }
 
 hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, void* y, int ydt, const Epilogue& epi,
@@ -295,6 +301,14 @@ hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, vo
         if (w.bits == 8) return go(std::integral_constant<int, 8>{}, nfc, split);
         return go(std::integral_constant<int, 4>{}, nfc, split);
     };
+    if (plan.two_per_cu) {
+        if (w.bits == 8) {
+            if (mf == 2) return launch_rows_t<8, 2, 4, 4, 2, 1, false, 2>(w, x_staged, M, y, ydt, epi, ns, 1, slabs, st);
+            return launch_rows_t<8, 3, 4, 4, 2, 1, false, 2>(w, x_staged, M, y, ydt, epi, ns, 1, slabs, st);
+        }
+        if (mf == 2) return launch_rows_t<4, 2, 4, 4, 3, 1, false, 2>(w, x_staged, M, y, ydt, epi, ns, 1, slabs, st);
+        return launch_rows_t<4, 3, 4, 4, 3, 1, false, 2>(w, x_staged, M, y, ydt, epi, ns, 1, slabs, st);
+    }
     if (plan.splits > 1) return with_bits(std::integral_constant<int, 4>{}, std::true_type{});
     if (plan.nf == 1) return with_bits(std::integral_constant<int, 1>{}, std::false_type{});
     if (plan.nf == 2) return with_bits(std::integral_constant<int, 2>{}, std::false_type{});

@@ -1024,6 +1024,49 @@ def test_prefill_rounds_of_two_widths(backend, oracle, bits, N, M, pair):
     qw.free()
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("N,K,M,xdt", [(16656, 2048, 24, "f32"), (16660, 2048 + 32, 48, "bf16"), (17024, 4096, 33, "f16"), (33000, 2048, 40, "bf16")])
+def test_prefill_few_rows_two_workgroups_per_cu(backend, oracle, bits, N, K, M, xdt):
+    """Up to 48 rows and more column groups than CUs: the few-row kernel with fewer weight tiles in flight, two workgroups
+    per CU.  Just past one round, several rounds, N inside a column block, K tiles that no wave count divides; and the
+    bits of the rows equal those of a call of 17 rows less (fp32: two rows less)."""
+    q, s = _quant(oracle, bits, N, K, cfg=81)
+    qw = backend.upload_quantized(q, s, bits)
+    wd = torch.from_numpy(oracle.dequant(q, s)).cuda().double()
+    x = _x(M, K, xdt, cfg=82)
+    y = _run(backend, qw, x)
+    ref = x.double() @ wd.T
+    assert ((y.double() - ref).norm(dim=0) / ref.norm(dim=0)).max().item() < 4e-3
+    assert ((y.double() - ref).norm() / ref.norm()).item() < FAST
+    fewer = 33 if M > 33 else M - 2 if xdt == "f32" else M
+    assert torch.equal(_run(backend, qw, x[:fewer].contiguous()), y[:fewer])
+    qw.free()
+
+
+@pytest.mark.parametrize("xdt", ["bf16", "f32"])
+@pytest.mark.parametrize("K", [512 - 32, 4096 + 32, 8192, 8192 + 32, 16384 + 64, 32768 + 512])
+def test_prefill_row_scaling_pass_rows_per_workgroup(backend, oracle, K, xdt):
+    """The row-scaling pass gives a workgroup one, two or four rows by K and the number of rows: last rows of a workgroup
+    missing, K that ends inside a piece, rows that stay in registers and rows that are read again, rows of very different
+    size, with a folded norm; and the same rows in calls of the sizes at which the rule changes."""
+    N = 48
+    q, s = _quant(oracle, 4, N, K, cfg=83)
+    qw = backend.upload_quantized(q, s, 4)
+    wd = torch.from_numpy(oracle.dequant(q, s)).cuda().double()
+    gamma = (1.0 + 0.1 * torch.from_numpy(synth.activations(84, 1, K))[0]).cuda()
+    for M in (33, 47, 49, 127, 130, 513):
+        x = (_x(M, K, "f32", cfg=85) * torch.logspace(-6, 6, M, device="cuda")[:, None]).to(TDT[xdt])
+        xd = x.double()
+        for y, ref in ((_run(backend, qw, x), xd @ wd.T), (torch.empty((M, N), device="cuda"), None)):
+            if ref is None:
+                backend.matmul_norm(qw, x, gamma, 1e-30, y)
+                torch.cuda.synchronize()
+                ref = (xd * torch.rsqrt((xd * xd).mean(dim=1, keepdim=True) + 1e-30) * gamma.double()) @ wd.T
+            # row by row: 48 sums of K products, weights (and fp32 rows, or x * gamma) rounded to f16 (2^-11 each)
+            assert ((y.double() - ref).norm(dim=1) / ref.norm(dim=1)).max().item() < 2e-3, M
+    qw.free()
+
+
 @pytest.mark.parametrize("shape", [(14336, 4096, 17), (4096, 4096, 32), (8200, 2048 + 128, 24)])
 def test_prefill_fp32_rows_17_to_32_fast_mode(backend, oracle, shape):
     """fp32 activations leave the decode kernels at 17 rows; in FAST mode they are rounded to f16 by the staging
