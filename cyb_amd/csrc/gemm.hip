@@ -988,8 +988,8 @@ __global__ __launch_bounds__(256) void stage_x_kernel(const u32x4_t* __restrict_
 // multiplied by its row's s on the way to f16, and leave as 64-byte runs (four neighbouring rows of
 // one k octet in operand order).
 // Whatever the magnitude of a row, its largest element lands in [2^13, 2^14) and elements down to
-// 2^-27 of it stay normal f16 numbers.  Rows of up to 4 * CH * 512 elements stay in registers
-// between the two steps (CH chunks of 8 values per lane in each of a row's four waves, all requested
+// 2^-27 of it stay normal f16 numbers.  Rows of up to PW * CH * 512 elements stay in registers
+// between the two steps (CH chunks of 8 values per lane in each of a row's PW waves, all requested
 // at once); longer rows are read again (the second read hits the L2).
 template <int XT>
 struct RowChunk {                 // 8 consecutive activations of a row as loaded
@@ -1025,12 +1025,11 @@ __device__ __forceinline__ void row_chunk_values(const RowChunk<XT>& c, float v[
     }
 }
 
-// A workgroup owns four rows and gives every row four waves: wave (r, p) takes the pieces of 512 k
-// numbered p, p + 4, ... of row r (CH of them at most stay in registers between the two steps), the
-// four parts of a row meet once through LDS for the row's largest magnitude (and sum of squares, added
-// in part order).  One wave per row took 5 - 7 us for 512 rows of 4096 and 10 - 12 us for rows of 14336,
-// most of it the latency of one wave walking its row.
-template <int XT, bool NORM, int CH>
+// A workgroup of sixteen waves owns ROWS rows (4, 2 or 1) and gives every row PW = 16 / ROWS waves: wave (r, p) takes the
+// pieces of 512 k numbered p, p + PW, ... of row r (CH of them at most stay in registers between the two steps), the parts
+// of a row meet once through LDS for the row's largest magnitude (and sum of squares).  One wave per row took 5 - 7 us for
+// 512 rows of 4096 and 10 - 12 us for rows of 14336, most of it the latency of one wave walking its row.
+template <int XT, bool NORM, int CH, int ROWS>
 __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict__ src, u32x4_t* __restrict__ dst, int M, int K,
                                                           Epilogue epi, float* __restrict__ ssq, float* __restrict__ unscale, Touch touch)
 {
@@ -1039,13 +1038,14 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
         touch_weights(touch, (int)blockIdx.x - touch.first_group, (int)threadIdx.x, 1024);
         return;
     }
-    if ((int)(blockIdx.x >> 2) * 16 >= M) return;              // (padding up to first_group)
-    constexpr int PW = 4;                                      // waves per row
-    __shared__ u32x4_t tile[PW][2][4 * kStagePitch];
-    __shared__ float amax_part[4][PW], sq_part[4][PW];
-    const int rb = blockIdx.x >> 2, r0 = (blockIdx.x & 3) * 4;          // row block, first of this workgroup's rows in it
+    if ((int)blockIdx.x * ROWS >= M) return;                   // (rows past M; padding up to first_group)
+    constexpr int PW = 16 / ROWS;                              // waves per row
+    __shared__ u32x4_t tile[PW][2][ROWS * kStagePitch];
+    __shared__ float amax_part[ROWS][PW];
+    __shared__ float sq_part[NORM ? ROWS : 1][16];
+    const int rb = (int)blockIdx.x * ROWS >> 4, r0 = (int)blockIdx.x * ROWS & 15;      // row block, first of this workgroup's rows in it
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    const int r = wv & 3, part = wv >> 2;                               // my row of the four, my part of the row
+    const int r = wv % ROWS, part = wv / ROWS;                           // my row of the workgroup's, my part of the row
     const int64_t row = min(rb * 16 + r0 + r, M - 1);      // (rows past M repeat the last one and are never read back)
     const int K8 = K >> 3, G = K8 >> 2;
     const int pieces = (K8 + 63) >> 6;                     // pieces of 64 chunks (512 k) in a row
@@ -1053,7 +1053,10 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
 
     // ---- the row's largest magnitude (and sum of squares)
     RowChunk<XT> keep[CH];
-    float amax = 0.f, sq = 0.f;
+    // (squares: piece number c of 512 k is summed with the pieces c + 16, c + 32, ..., and the sixteen sums are added in order,
+    // whatever the number of rows per workgroup: a row's sum does not depend on the rows it travels with)
+    // (rows that take more than one round have CH = 4 or 8, a multiple of ROWS)
+    float amax = 0.f, sq[ROWS] = {};
     for (int p0 = 0; p0 < pieces; p0 += PW * CH) {
 #pragma unroll
         for (int i = 0; i < CH; i++) {
@@ -1072,7 +1075,7 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
                     load_gamma8_g(epi.gamma, epi.gamma_dt, c * 8, g);
 #pragma unroll
                     for (int e = 0; e < 8; e++) {
-                        sq = fmaf(v[e], v[e], sq);
+                        sq[i % ROWS] = fmaf(v[e], v[e], sq[i % ROWS]);
                         v[e] *= g[e];
                     }
                 }
@@ -1084,15 +1087,27 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
         amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-        if (NORM) sq += __shfl_xor(sq, off, 64);
+        if (NORM) {
+#pragma unroll
+            for (int i = 0; i < ROWS; i++) sq[i] += __shfl_xor(sq[i], off, 64);
+        }
     }
     if (lane == 0) {
         amax_part[r][part] = amax;
-        if (NORM) sq_part[r][part] = sq;
+        if (NORM) {
+#pragma unroll
+            for (int i = 0; i < ROWS; i++) sq_part[NORM ? r : 0][i * PW + part] = sq[i];
+        }
     }
     __syncthreads();
-    amax = fmaxf(fmaxf(amax_part[r][0], amax_part[r][1]), fmaxf(amax_part[r][2], amax_part[r][3]));
-    if (NORM) sq = ((sq_part[r][0] + sq_part[r][1]) + sq_part[r][2]) + sq_part[r][3];
+    amax = amax_part[r][0];
+#pragma unroll
+    for (int p = 1; p < PW; p++) amax = fmaxf(amax, amax_part[r][p]);
+    float sum = 0.f;
+    if (NORM) {
+#pragma unroll
+        for (int c = 0; c < 16; c++) sum += sq_part[NORM ? r : 0][c];
+    }
     // amax = f * 2^e with f in [0.5, 1): s = 2^(14 - e) puts it in [2^13, 2^14); zero, Inf and NaN rows keep s = 1
     float s = 1.0f;
     if (amax > 0.f && amax < __builtin_inff()) {
@@ -1102,7 +1117,7 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
     }
     if (lane == 0 && part == 0 && rb * 16 + r0 + r < M) {
         unscale[row] = 1.0f / s;
-        if (NORM) ssq[row] = sq;
+        if (NORM) ssq[row] = sum;
     }
 
     // ---- scale, round to f16, through LDS into operand order (two tiles per part: one barrier per piece)
@@ -1123,8 +1138,8 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
         }
         return a.u;
     };
-    const int tp = r * 64 + lane;                           // my place among the 256 threads of my part
-    const int gl = tp >> 4, oct = (tp >> 2) & 3, rr = tp & 3;  // when writing out: group within the piece, k octet, row
+    const int tp = r * 64 + lane;                           // my place among the threads of my part
+    const int gl = tp / (4 * ROWS), oct = tp / ROWS & 3, rr = tp % ROWS;  // when writing out: group within the piece, k octet, row
     int round = 0;
     for (int p0 = 0; p0 < pieces; p0 += PW * CH) {
         if (!resident) {
@@ -1259,23 +1274,37 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
         if (widen) {
             // per-row scaled f16 operands; one sum of squares per row
             ns = NormStats{ssq_part, 1, unscale};
-            dim3 rgrid((unsigned)((mc + 15) / 16) * 4);
+            // Rows per workgroup of sixteen waves: with few of them one workgroup per four rows leaves the chip idle and a
+            // row's waves walk it piece after piece.  us per call, 4 / 2 / 1 rows (bf16): 14336 -> 4096 at 45 rows 26.4 /
+            // 24.8 / 24.0, 128 rows 37.2 / 34.3 / 33.7, 512 rows 73.4 / 72.8 / 78.0; 14336 -> 1024, fp32, 256 rows 33.3 /
+            // 30.0 / 33.2; 4096 -> 6144 with a norm at 45 rows 14.6 / 13.0 / 12.9, 4096 -> 4096 at 45 rows 12.1 / 11.3 /
+            // 11.3; 4096 -> 14336 at 64 / 128 rows 19.4 / 19.4 / 19.9, 27.5 / 28.4 / 28.5.  (The fewer rows, the shorter
+            // the runs in which the operands leave: 64, 32, 16 bytes.)
+            const int stage_rows = w.K > 8192 ? (mc <= 128 ? 1 : mc <= 512 ? 2 : 4) : (mc <= 48 ? 2 : 4);
+            dim3 rgrid((unsigned)((mc + 15) / 16) * (16 / stage_rows));
             const Touch touch = plan_touch(w, mc, num_cus, ec, exact, rgrid.x);
-            // pieces of 512 k a lane keeps in registers (a row is split over four waves): the whole row when it has
-            // at most 16384 (bf16) or 8192 (fp32) elements
-            const int batches = ((K8 + 63) / 64 + 3) / 4;
-#define CYBQ_STAGE_ROWS(XT, NORM, CH) \
-    hipLaunchKernelGGL((stage_rows_kernel<XT, NORM, CH>), rgrid, dim3(1024), 0, st, xs, xst, mc, w.K, epi, ssq_part, unscale, touch)
-#define CYBQ_STAGE_ROWS_CH(XT, NORM, C1, C2, C3)              \
-    do {                                                      \
-        if (batches <= C1) CYBQ_STAGE_ROWS(XT, NORM, C1);     \
-        else if (batches <= C2) CYBQ_STAGE_ROWS(XT, NORM, C2); \
-        else CYBQ_STAGE_ROWS(XT, NORM, C3);                   \
+            // pieces of 512 k a lane keeps in registers: the whole row when it has at most 16384 (bf16) or 8192 (fp32)
+            // elements, 16384 with two rows per workgroup, 32768 with one
+            const int per_row = 16 / stage_rows, batches = ((K8 + 63) / 64 + per_row - 1) / per_row;
+#define CYBQ_STAGE_ROWS(XT, NORM, CH, ROWS) \
+    hipLaunchKernelGGL((stage_rows_kernel<XT, NORM, CH, ROWS>), rgrid, dim3(1024), 0, st, xs, xst, mc, w.K, epi, ssq_part, unscale, touch)
+#define CYBQ_STAGE_ROWS_CH(XT, NORM, ROWS, C1, C2, C3)              \
+    do {                                                            \
+        if (batches <= C1) CYBQ_STAGE_ROWS(XT, NORM, C1, ROWS);     \
+        else if (batches <= C2) CYBQ_STAGE_ROWS(XT, NORM, C2, ROWS); \
+        else CYBQ_STAGE_ROWS(XT, NORM, C3, ROWS);                   \
     } while (0)
-            if (xdt == kF32 && epi.gamma) CYBQ_STAGE_ROWS_CH(2, true, 1, 2, 4);
-            else if (xdt == kF32) CYBQ_STAGE_ROWS_CH(2, false, 1, 2, 4);
-            else if (epi.gamma) CYBQ_STAGE_ROWS_CH(1, true, 2, 4, 8);
-            else CYBQ_STAGE_ROWS_CH(1, false, 2, 4, 8);
+#define CYBQ_STAGE_ROWS_N(XT, NORM)                                                        \
+    do {                                                                                   \
+        if (stage_rows == 1) CYBQ_STAGE_ROWS_CH(XT, NORM, 1, 1, 2, 4);                     \
+        else if (stage_rows == 2) CYBQ_STAGE_ROWS_CH(XT, NORM, 2, 1, 2, 4);                \
+        else CYBQ_STAGE_ROWS_CH(XT, NORM, 4, (XT == 2 ? 1 : 2), (XT == 2 ? 2 : 4), (XT == 2 ? 4 : 8)); \
+    } while (0)
+            if (xdt == kF32 && epi.gamma) CYBQ_STAGE_ROWS_N(2, true);
+            else if (xdt == kF32) CYBQ_STAGE_ROWS_N(2, false);
+            else if (epi.gamma) CYBQ_STAGE_ROWS_N(1, true);
+            else CYBQ_STAGE_ROWS_N(1, false);
+#undef CYBQ_STAGE_ROWS_N
 #undef CYBQ_STAGE_ROWS_CH
 #undef CYBQ_STAGE_ROWS
         } else if (epi.gamma) {
