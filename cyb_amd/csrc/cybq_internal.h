@@ -53,7 +53,7 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
 // (gemm_rows.hip); ssq_part / ssq_blocks / unscale: the staging pass's per-row statistics
 struct RowsPlan {
     int nf;                  // column blocks of 16 per workgroup (1, 2 or 4); 0: the kernel does not take the call
-    int splits;              // K is split over that many workgroups, whose sums go to slabs (fp32 [M][N] each, together 4 MB at most)
+    int shares;              // > 0: K is cut into that many shares, one per wave; more than four go to shares - 3 slabs, fp32 [M][N]
     bool two_per_cu = false; // two workgroups share a CU (nf = 4, up to 48 rows)
 };
 RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi);

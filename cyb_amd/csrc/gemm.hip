@@ -174,7 +174,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2
     // they would all ask the same few L2 channels for the same lines at the same
     // moment (a row of X is a multiple of the channel interleave long), so each
     // column tile starts its walk at a different K tile and wraps around.  The
-    // order depends on the column tile only: with one tile width a row of Y does not depend on M.
+    // order depends on the column tile only: a row of Y does not depend on M.
     const int kt0 = tile_n % KT;
     auto rot = [&](int kt) {
         const int r = min(kt, KT - 1) + kt0;
@@ -362,7 +362,7 @@ __device__ __forceinline__ void static_for(F&& f)
 template <int BITS, int NF, int MF, int MW, int XD>
 __global__ __launch_bounds__((MW + 4) * 64) __attribute__((amdgpu_waves_per_eu((MW + 7) / 4, (MW + 7) / 4))) void gemm_roles_kernel(
     const uint8_t* __restrict__ wbase, const u32x4_t* __restrict__ x, int KT_, int NT_, int x_row_blocks, int M, int n_tiles,
-    int m_tiles, int groups, int nt_first, int N_, void* __restrict__ y, int ydt, int K_, float out_scale, Epilogue epi, NormStats ns)
+    int m_tiles, int groups, int N_, void* __restrict__ y, int ydt, int K_, float out_scale, Epilogue epi, NormStats ns)
 {
     const WeightView w = {wbase, N_, K_, NT_, KT_, BITS};
     constexpr int SW = 4;                             // staging waves
@@ -381,7 +381,7 @@ __global__ __launch_bounds__((MW + 4) * 64) __attribute__((amdgpu_waves_per_eu((
     const int tile_m = item / n_tiles, tile_n = item - tile_m * n_tiles;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nt0 = nt_first + tile_n * NF;          // (the call's column tiles start at strip nt_first)
+    const int nt0 = tile_n * NF;
     const int KT = w.KT, K = w.K;
     const int kt0 = tile_n % KT;
     auto rot = [&](int kt) {
@@ -546,72 +546,19 @@ __global__ __launch_bounds__((MW + 4) * 64) __attribute__((amdgpu_waves_per_eu((
     write_rows<MF, NF>(acc, reinterpret_cast<float*>(smem) + wave * (16 * NF * 16), m0, nt0, M, w.N, y, ydt, out_scale, epi, lane);
 }
 
-// nt_first, strips: the part of the output's strips that the launch covers (all of them unless said otherwise)
 template <int BITS, int NF, int MF, int MW, int XD>
 hipError_t launch_roles(const WeightView& w, const void* x, int M, void* y, int ydt, float out_scale, const Epilogue& epi,
-                        const NormStats& ns, hipStream_t st, int nt_first = 0, int strips = 0)
+                        const NormStats& ns, hipStream_t st)
 {
     constexpr int lds = 2 * NF * (4 * 64) * 16;
     constexpr int BM = MW * MF * 16;
     (void)LdsRequest<&gemm_roles_kernel<BITS, NF, MF, MW, XD>, lds>::registered;
-    const int n_tiles = ((strips ? strips : w.NT) + NF - 1) / NF, m_tiles = (M + BM - 1) / BM;
+    const int n_tiles = (w.NT + NF - 1) / NF, m_tiles = (M + BM - 1) / BM;
     const unsigned groups = (unsigned)(((int64_t)n_tiles * m_tiles + 7) / 8 * 8);
     hipLaunchKernelGGL((gemm_roles_kernel<BITS, NF, MF, MW, XD>), dim3(groups), dim3((MW + 4) * 64), lds, st, w.base,
-                       reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT, (M + 15) / 16, M, n_tiles, m_tiles, (int)groups, nt_first, w.N, y, ydt, w.K,
+                       reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT, (M + 15) / 16, M, n_tiles, m_tiles, (int)groups, w.N, y, ydt, w.K,
                        out_scale, epi, ns);
     return hipGetLastError();
-}
-
-// Whole rounds of 256-row tiles.  A round of workgroups costs about as much whether it is full or not, so the columns are
-// cut into one or two launches of tiles as wide as makes the sum of the rounds' widths smallest (4096 -> 28672 in gate / up
-// pairs at 512 rows: 448 tiles of 128 columns are 1.75 rounds; 256 of them and 256 tiles of 96 columns are two).
-// us per call, bf16, against one width (and, for the pairs, the kernel without roles): 4096 -> 28672 norm + SwiGLU at 512 /
-// 1024 rows 130.8 / 257.5 -> 121.1 / 231.4, SwiGLU at 2048 (one width) 439.8 -> 412.6; 4096 -> 20000 at 512 rows 106.4 ->
-// 92.5, 4096 -> 25008 at 300 rows 106.9 -> 102.4.
-struct RoundPlan {
-    int nf1, strips1, nf2;          // strips1 columns blocks in tiles nf1 wide, the rest in tiles nf2 wide (0: nothing left)
-};
-RoundPlan plan_rounds(int NT, int M, int num_cus, int nf, bool pairs)
-{
-    const int64_t m = (M + 255) / 256;
-    auto cost = [&](int64_t strips, int width) {      // in column blocks of one row tile; + 1: start and end of a round
-        return ((strips + width - 1) / width * m + num_cus - 1) / num_cus * (width + 1);
-    };
-    RoundPlan best = {nf, NT, 0};
-    const int64_t one = cost(NT, nf);
-    int64_t least = one;
-    for (int a : {8, 7})
-        for (int b : {8, 7, 6, 4}) {
-            if (a == b || (pairs && (a % 2 || b % 2))) continue;
-            for (int64_t rounds = 1; rounds <= 8; rounds++) {
-                const int64_t strips1 = rounds * num_cus / m * a;
-                if (strips1 <= 0 || strips1 >= NT) continue;
-                const int64_t c = cost(strips1, a) + cost(NT - strips1, b);
-                if (c < least) {
-                    least = c;
-                    best = {a, (int)strips1, b};
-                }
-            }
-        }
-    return least * 20 <= one * 19 ? best : RoundPlan{nf, NT, 0};        // (5 % at least: the second launch costs about 2 us)
-}
-
-template <int BITS>
-hipError_t launch_rounds(const WeightView& w, const void* x, int M, void* y, int ydt, float out_scale, const Epilogue& epi, const NormStats& ns,
-                         int num_cus, int nf, hipStream_t st)
-{
-    // (a row's bits depend on the tile its column sits in, and with two widths that depends on the number of row tiles: outputs
-    // in multiples of 112 columns, whose rows have the same bits at every row count, keep their one width)
-    const RoundPlan plan = nf == 7 ? RoundPlan{7, w.NT, 0} : plan_rounds(w.NT, M, num_cus, nf, epi.kind == kEpiSwiglu);
-    auto go = [&](int width, int first, int strips) {
-        if (width == 8) return launch_roles<BITS, 8, 2, 8, 2>(w, x, M, y, ydt, out_scale, epi, ns, st, first, strips);
-        if (width == 7) return launch_roles<BITS, 7, 2, 8, 2>(w, x, M, y, ydt, out_scale, epi, ns, st, first, strips);
-        if (width == 6) return launch_roles<BITS, 6, 2, 8, 2>(w, x, M, y, ydt, out_scale, epi, ns, st, first, strips);
-        return launch_roles<BITS, 4, 2, 8, 2>(w, x, M, y, ydt, out_scale, epi, ns, st, first, strips);
-    };
-    const hipError_t e = go(plan.nf1, 0, plan.strips1);
-    if (e != hipSuccess || !plan.nf2) return e;
-    return go(plan.nf2, plan.strips1, w.NT - plan.strips1);
 }
 
 constexpr int kMaxSplits = 8;
@@ -806,7 +753,7 @@ hipError_t launch_t(const WeightView& w, const void* x, int M, void* y, int ydt,
     }
     // enough 256-row tiles to fill the chip without a K split: the role-split kernel
     if constexpr (!EXACT) {
-        if (tiles256 >= num_cus) return launch_rounds<BITS>(w, x, M, y, ydt, out_scale, epi, ns, num_cus, NF, st);
+        if (tiles256 >= num_cus) return launch_roles<BITS, NF, 2, 8, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
     }
     if (tiles256 < num_cus && few_rows) return launch_m<BITS, XBF, NF, EXACT, 2, 4>(w, x, M, y, ydt, out_scale, part, part_bytes, num_cus, epi, ns, st);
     return launch_m<BITS, XBF, NF, EXACT, 2, 8>(w, x, M, y, ydt, out_scale, part, part_bytes, num_cus, epi, ns, st);
@@ -887,7 +834,6 @@ hipError_t launch_nf(const WeightView& w, const void* x, int M, void* y, int ydt
 struct Touch {
     const uint8_t* base;          // the weight tensor (first_group past the grid: nothing to do)
     int first_group, NT, KT, NF, tile_bytes, ahead;
-    int groups, kt_per_split;     // K split: workgroup b works on group b % groups, on the K tiles of split b / groups
     int per_xcd, tiles;           // the tiled kernels' order: workgroup b works on column tile (b % 8) * per_xcd + b / 8 of `tiles` (0: on b)
 };
 
@@ -898,16 +844,14 @@ __device__ __forceinline__ void touch_weights(const Touch& tc, int b, int tid, i
         b = (b & 7) * tc.per_xcd + (b >> 3);
         if (b >= tc.tiles) return;
     }
-    const int kt_lo = b / tc.groups * tc.kt_per_split, KT = min(tc.kt_per_split, tc.KT - kt_lo);
-    if (tc.kt_per_split < tc.KT) b %= tc.groups;
-    const int kt0 = b % KT;                        // (the multiply's workgroups start their K walk there)
+    const int kt0 = b % tc.KT;                     // (the multiply's workgroups start their K walk there)
     uint32_t acc = 0;
     for (int idx = tid; idx < tc.NF * tc.ahead * lines; idx += nthreads) {
         const int line = idx % lines, ft = idx / lines, t = ft % tc.ahead, f = ft / tc.ahead;
         const int nt = min(b * tc.NF + f, tc.NT - 1);
         int kt = kt0 + t;
-        if (kt >= KT) kt -= KT;
-        acc ^= *reinterpret_cast<const uint32_t*>(tc.base + ((int64_t)nt * tc.KT + kt_lo + kt) * tc.tile_bytes + min(line * 128, tc.tile_bytes - 4));
+        if (kt >= tc.KT) kt -= tc.KT;
+        acc ^= *reinterpret_cast<const uint32_t*>(tc.base + ((int64_t)nt * tc.KT + kt) * tc.tile_bytes + min(line * 128, tc.tile_bytes - 4));
     }
     asm volatile("" ::"v"(acc));                   // (the loads have to be issued and waited for; nothing is stored)
 }
@@ -1042,7 +986,7 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
     constexpr int PW = 16 / ROWS;                              // waves per row
     __shared__ u32x4_t tile[PW][2][ROWS * kStagePitch];
     __shared__ float amax_part[ROWS][PW];
-    __shared__ float sq_part[NORM ? ROWS : 1][16];
+    __shared__ float sq_part[ROWS][PW];
     const int rb = (int)blockIdx.x * ROWS >> 4, r0 = (int)blockIdx.x * ROWS & 15;      // row block, first of this workgroup's rows in it
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     const int r = wv % ROWS, part = wv / ROWS;                           // my row of the workgroup's, my part of the row
@@ -1053,10 +997,9 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
 
     // ---- the row's largest magnitude (and sum of squares)
     RowChunk<XT> keep[CH];
-    // (squares: piece number c of 512 k is summed with the pieces c + 16, c + 32, ..., and the sixteen sums are added in order,
-    // whatever the number of rows per workgroup: a row's sum does not depend on the rows it travels with)
-    // (rows that take more than one round have CH = 4 or 8, a multiple of ROWS)
-    float amax = 0.f, sq[ROWS] = {};
+    // (a folded norm's sum of squares is formed in an order that goes with PW = 4: the launcher keeps to it)
+    static_assert(!NORM || ROWS == 4, "one order for the sums of squares");
+    float amax = 0.f, sq = 0.f;
     for (int p0 = 0; p0 < pieces; p0 += PW * CH) {
 #pragma unroll
         for (int i = 0; i < CH; i++) {
@@ -1075,7 +1018,7 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
                     load_gamma8_g(epi.gamma, epi.gamma_dt, c * 8, g);
 #pragma unroll
                     for (int e = 0; e < 8; e++) {
-                        sq[i % ROWS] = fmaf(v[e], v[e], sq[i % ROWS]);
+                        sq = fmaf(v[e], v[e], sq);
                         v[e] *= g[e];
                     }
                 }
@@ -1087,27 +1030,17 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
         amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-        if (NORM) {
-#pragma unroll
-            for (int i = 0; i < ROWS; i++) sq[i] += __shfl_xor(sq[i], off, 64);
-        }
+        if (NORM) sq += __shfl_xor(sq, off, 64);
     }
     if (lane == 0) {
         amax_part[r][part] = amax;
-        if (NORM) {
-#pragma unroll
-            for (int i = 0; i < ROWS; i++) sq_part[NORM ? r : 0][i * PW + part] = sq[i];
-        }
+        if (NORM) sq_part[r][part] = sq;
     }
     __syncthreads();
     amax = amax_part[r][0];
 #pragma unroll
     for (int p = 1; p < PW; p++) amax = fmaxf(amax, amax_part[r][p]);
-    float sum = 0.f;
-    if (NORM) {
-#pragma unroll
-        for (int c = 0; c < 16; c++) sum += sq_part[NORM ? r : 0][c];
-    }
+    if constexpr (NORM) sq = ((sq_part[r][0] + sq_part[r][1]) + sq_part[r][2]) + sq_part[r][3];
     // amax = f * 2^e with f in [0.5, 1): s = 2^(14 - e) puts it in [2^13, 2^14); zero, Inf and NaN rows keep s = 1
     float s = 1.0f;
     if (amax > 0.f && amax < __builtin_inff()) {
@@ -1117,7 +1050,7 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
     }
     if (lane == 0 && part == 0 && rb * 16 + r0 + r < M) {
         unscale[row] = 1.0f / s;
-        if (NORM) ssq[row] = sum;
+        if (NORM) ssq[row] = sq;
     }
 
     // ---- scale, round to f16, through LDS into operand order (two tiles per part: one barrier per piece)
@@ -1172,7 +1105,7 @@ void set_gemm_tuning(int rows_kernel) { g_rows_kernel = rows_kernel >= 5 ? 0 : r
 
 static RowsPlan rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
-    if (g_rows_kernel == 2) return {0, 1};
+    if (g_rows_kernel == 2) return {0, 0};
     return gemm_rows_plan(w, M, g_rows_kernel == 1 ? 1 : num_cus, epi);
 }
 
@@ -1180,7 +1113,7 @@ static RowsPlan rows_plan(const WeightView& w, int M, int num_cus, const Epilogu
 bool gemm_rows_takes(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
     const RowsPlan plan = rows_plan(w, M, num_cus, epi);
-    return plan.nf != 0 && plan.splits == 1;
+    return plan.nf != 0 && plan.shares == 0;
 }
 
 // the extra workgroups of a staging launch (grid_x grows by them) for a call of 33 rows or more that goes through the
@@ -1200,7 +1133,7 @@ static bool few_rows_tiles64(const WeightView& w, int M, int num_cus, const Epil
 
 static Touch plan_touch(const WeightView& w, int mc, int num_cus, const Epilogue& ec, bool exact, unsigned& grid_x)
 {
-    Touch tc = {nullptr, 0x7fffffff, w.NT, w.KT, 1, tile_bytes(w.bits), 0, 0x7fffffff, w.KT, 0, 0};
+    Touch tc = {nullptr, 0x7fffffff, w.NT, w.KT, 1, tile_bytes(w.bits), 0, 0, 0};
     if (g_touch == 0 || exact || mc < 33 || w.KT < 32) return tc;
     const int64_t per_k_tile = (int64_t)w.NT * tile_bytes(w.bits);
     int nf = 0, groups = 0;
@@ -1208,11 +1141,7 @@ static Touch plan_touch(const WeightView& w, int mc, int num_cus, const Epilogue
     if (plan.nf) {
         nf = plan.nf;
         groups = (w.NT + nf - 1) / nf;
-        if (plan.splits > 1) {                       // (the multiply's workgroups of a split follow those of the split before it)
-            tc.groups = groups;
-            tc.kt_per_split = (w.KT + plan.splits - 1) / plan.splits;
-            groups *= plan.splits;
-        }
+        if (plan.shares) return tc;
     } else if (g_touch >= 2 && per_k_tile * w.KT <= ((int64_t)40 << 20) && few_rows_tiles64(w, mc, num_cus, ec)) {
         // the 128 x 64 / 64 x 64 tiles of the tiled kernels (65 .. 128 rows on wide outputs; 4096 -> 14336 at 128 rows:
         // 27.5 us, 24.3 with the same tensor every call): 4096 -> 14336 at 65 / 100 / 128 rows 25.3 / 27.1 / 28.1 ->
@@ -1227,7 +1156,6 @@ static Touch plan_touch(const WeightView& w, int mc, int num_cus, const Epilogue
     tc.base = w.base;
     tc.NF = nf;
     tc.ahead = (int)std::min<int64_t>(w.KT, std::max<int64_t>(4, ((int64_t)16 << 20) / per_k_tile));
-    if (tc.kt_per_split < w.KT) tc.ahead = std::min(w.KT % tc.kt_per_split ? w.KT % tc.kt_per_split : tc.kt_per_split, std::max(4, tc.ahead * tc.kt_per_split / w.KT));
     tc.first_group = (int)((grid_x + 7) / 8 * 8);
     grid_x = (unsigned)(tc.first_group + groups);
     return tc;
@@ -1280,7 +1208,8 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
             // 30.0 / 33.2; 4096 -> 6144 with a norm at 45 rows 14.6 / 13.0 / 12.9, 4096 -> 4096 at 45 rows 12.1 / 11.3 /
             // 11.3; 4096 -> 14336 at 64 / 128 rows 19.4 / 19.4 / 19.9, 27.5 / 28.4 / 28.5.  (The fewer rows, the shorter
             // the runs in which the operands leave: 64, 32, 16 bytes.)
-            const int stage_rows = w.K > 8192 ? (mc <= 128 ? 1 : mc <= 512 ? 2 : 4) : (mc <= 48 ? 2 : 4);
+            // (4096 -> 6144 with a norm: four rows, one order of its sums.)
+            const int stage_rows = epi.gamma ? 4 : w.K > 8192 ? (mc <= 128 ? 1 : mc <= 512 ? 2 : 4) : (mc <= 48 ? 2 : 4);
             dim3 rgrid((unsigned)((mc + 15) / 16) * (16 / stage_rows));
             const Touch touch = plan_touch(w, mc, num_cus, ec, exact, rgrid.x);
             // pieces of 512 k a lane keeps in registers: the whole row when it has at most 16384 (bf16) or 8192 (fp32)
@@ -1296,8 +1225,8 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
     } while (0)
 #define CYBQ_STAGE_ROWS_N(XT, NORM)                                                        \
     do {                                                                                   \
-        if (stage_rows == 1) CYBQ_STAGE_ROWS_CH(XT, NORM, 1, 1, 2, 4);                     \
-        else if (stage_rows == 2) CYBQ_STAGE_ROWS_CH(XT, NORM, 2, 1, 2, 4);                \
+        if (stage_rows == 1) CYBQ_STAGE_ROWS_CH(XT, false, 1, 1, 2, 4);                    \
+        else if (stage_rows == 2) CYBQ_STAGE_ROWS_CH(XT, false, 2, 1, 2, 4);               \
         else CYBQ_STAGE_ROWS_CH(XT, NORM, 4, (XT == 2 ? 1 : 2), (XT == 2 ? 2 : 4), (XT == 2 ? 4 : 8)); \
     } while (0)
             if (xdt == kF32 && epi.gamma) CYBQ_STAGE_ROWS_N(2, true);
@@ -1316,10 +1245,10 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         // few rows on a wide output, FAST mode: the kernel of gemm_rows.hip (waves split K, no LDS on the way)
-        const RowsPlan plan = !exact && kdt == kF16 ? rows_plan(w, mc, num_cus, ec) : RowsPlan{0, 1};
+        const RowsPlan plan = !exact && kdt == kF16 ? rows_plan(w, mc, num_cus, ec) : RowsPlan{0, 0};
         if (plan.nf) {
             e = launch_gemm_rows(w, workspace, mc, yc, ydt, ec, ns.part, ns.nblk, ns.unscale, plan, part, st);
-            if (e == hipSuccess && plan.splits > 1) e = launch_reduce(part, plan.splits, mc, w.N, yc, ydt, out_scale, ec, ns, w.K, st);
+            if (e == hipSuccess && plan.shares > 4) e = launch_reduce(part, plan.shares - 3, mc, w.N, yc, ydt, out_scale, ec, ns, w.K, st);
             if (e != hipSuccess) return e;
             continue;
         }
