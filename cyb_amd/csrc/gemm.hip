@@ -1205,11 +1205,11 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
             // Rows per workgroup of sixteen waves: with few of them one workgroup per four rows leaves the chip idle and a
             // row's waves walk it piece after piece.  us per call, 4 / 2 / 1 rows (bf16): 14336 -> 4096 at 45 rows 26.4 /
             // 24.8 / 24.0, 128 rows 37.2 / 34.3 / 33.7, 512 rows 73.4 / 72.8 / 78.0; 14336 -> 1024, fp32, 256 rows 33.3 /
-            // 30.0 / 33.2; 4096 -> 6144 with a norm at 45 rows 14.6 / 13.0 / 12.9, 4096 -> 4096 at 45 rows 12.1 / 11.3 /
+            // 30.0 / 33.2 (10240 -> 3507, fp32, 444 rows: 64.3 / 64.9 with four / two); 4096 -> 6144 with a norm at 45 rows 14.6 / 13.0 / 12.9, 4096 -> 4096 at 45 rows 12.1 / 11.3 /
             // 11.3; 4096 -> 14336 at 64 / 128 rows 19.4 / 19.4 / 19.9, 27.5 / 28.4 / 28.5.  (The fewer rows, the shorter
             // the runs in which the operands leave: 64, 32, 16 bytes.)
             // (4096 -> 6144 with a norm: four rows, one order of its sums.)
-            const int stage_rows = epi.gamma ? 4 : w.K > 8192 ? (mc <= 128 ? 1 : mc <= 512 ? 2 : 4) : (mc <= 48 ? 2 : 4);
+            const int stage_rows = epi.gamma ? 4 : w.K > 8192 ? (mc <= 128 ? 1 : mc <= 256 || (mc <= 512 && w.K > 12288) ? 2 : 4) : (mc <= 48 ? 2 : 4);
             dim3 rgrid((unsigned)((mc + 15) / 16) * (16 / stage_rows));
             const Touch touch = plan_touch(w, mc, num_cus, ec, exact, rgrid.x);
             // pieces of 512 k a lane keeps in registers: the whole row when it has at most 16384 (bf16) or 8192 (fp32)
