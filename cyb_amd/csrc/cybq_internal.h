@@ -34,7 +34,8 @@ hipError_t launch_gemv(const WeightView& w, const void* x, int xdt, int M, void*
                        int num_cus, bool exact_operands, const Epilogue& epi, void* scratch, size_t scratch_bytes, hipStream_t st);
 // 3 .. 32 rows on outputs with several pairs of strips per CU (gemv_stream.hip)
 bool gemv_stream_serves(const WeightView& w, int xdt, int M, int num_cus, const Epilogue& epi);
-hipError_t launch_gemv_stream(const WeightView& w, const void* x, int xdt, int M, void* y, int ydt, int num_cus, const Epilogue& epi, hipStream_t st);
+hipError_t launch_gemv_stream(const WeightView& w, const void* x, int xdt, int M, void* y, int ydt, int num_cus, bool exact_operands,
+                              const Epilogue& epi, hipStream_t st);
 // decode kernel for one and two rows (f16 / bf16 activations, no folded norm): weight operands are f16 subnormals
 // (bf16: 128 + u),
 // the +8 / +128 bias comes off inside the MFMA accumulation (gemv1.hip)

@@ -672,12 +672,6 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
                             (uint32_t)__builtin_amdgcn_ds_bpermute(from_lane + (j % GPL) * 16, (int)raw[j / GPL][p]);
             }
         if constexpr (BY_TILE) {
-            const float4_t zero = {0.f, 0.f, 0.f, 0.f};
-            Frag16 off, off_odd;            // the constant operand(s) that take the bias off
-            const uint32_t offw = SUB ? kSubBiasL : (BITS == 4 ? kBf16Neg136x2 : kBf16Neg128x2);
-            const uint32_t offw_odd = SUB ? kSubBiasH : offw;
-            off.u = (u32x4_t){offw, offw, offw, offw};
-            off_odd.u = (u32x4_t){offw_odd, offw_odd, offw_odd, offw_odd};
 #pragma unroll
             for (int u = 0; u < TS; u++) {
                 if (NS > 2) __builtin_amdgcn_sched_barrier(0);
@@ -688,44 +682,21 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
                 if (NS > 2) __builtin_amdgcn_sched_barrier(0);
                 float4_t bias[MB][4];
 #pragma unroll
-                for (int b = 0; b < MB; b++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        if constexpr (SUB)
-                            bias[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[b][u][j].h, ((j & 1) ? off_odd : off).h, zero, 0, 0, 0);
-                        else bias[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[b][u][j].b, off.b, zero, 0, 0, 0);
-                    }
+                for (int b = 0; b < MB; b++) tile_bias<XMODE>(a[b][u], bias[b]);
 #pragma unroll
                 for (int s = 0; s < NS; s++) {
                     Frag16 bop[4];
-                    if constexpr (SUB) {
-#pragma unroll
-                        for (int j = 0; j < 4; j++) {
-                            uint32_t bw[4];
-                            unpack_q4_sub(buf[s][u].q[0][2 * (j >> 1)], buf[s][u].q[0][2 * (j >> 1) + 1], j & 1, bw);
-                            bop[j].u = (u32x4_t){bw[0], bw[1], bw[2], bw[3]};
-                        }
-                    } else tile_operands<BITS, XMODE>(buf[s][u], magic, bop);
+                    if constexpr (SUB) tile_operands_sub(buf[s][u], bop);
+                    else tile_operands<BITS, XMODE>(buf[s][u], magic, bop);
                     u32x2_t sc = buf[s][u].s;
                     sc[0] = valid[u] ? sc[0] : 0u;
                     sc[1] = valid[u] ? sc[1] : 0u;
 #pragma unroll
                     for (int b = 0; b < MB; b++) {
                         float4_t d[4];
-#pragma unroll
-                        for (int j = 0; j < 4; j++) {
-                            if constexpr (SUB) d[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[b][u][j].h, bop[j].h, bias[b][j], 0, 0, 0);
-                            else d[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[b][u][j].b, bop[j].b, bias[b][j], 0, 0, 0);
-                        }
-                        if constexpr (SUB) {
-#pragma unroll
-                            for (int j = 0; j < 4; j++) {
-                                const uint32_t sb = (j & 1) ? (sc[j >> 1] >> 16) : (sc[j >> 1] & 0xffffu);
-                                const float sf = (j & 1) ? f16_bits_to_f32(sb) * 0.0625f : f16_bits_to_f32(sb);
-#pragma unroll
-                                for (int r = 0; r < 4; r++) acc[s][b][r] = __builtin_fmaf(sf, d[j][r], acc[s][b][r]);
-                            }
-                        } else tile_accum<4>(sc, d, acc[s][b]);
+                        tile_multiply_from<XMODE>(a[b][u], bop, bias[b], d);
+                        if constexpr (SUB) tile_accum_sub(sc, d, acc[s][b]);
+                        else tile_accum<4>(sc, d, acc[s][b]);
                     }
                 }
             }
@@ -890,7 +861,8 @@ hipError_t launch_rows_x(const WeightView& w, const void* x, int M, void* y, int
     }
     // decode mode STREAM, Q4 and f16 activations, two to four strips: subnormal operands
     // (with two row blocks, 17..32 rows, it measures 0.3 us slower than the integer operands, but a row keeps
-    // the bits it has in a batch of up to 16)
+    // the bits it has in a batch of up to 16.  Not so gate / up pairs of seven strips per CU and of eight or more: up to 16 rows
+    // those go strip by strip, with integer operands)
     if constexpr (BITS == 4 && XMODE == XF16 && NS >= 2 && NS <= 4 && (TS == 4 || MB == 2)) {
         if (sub && !epi.gamma) {
             if constexpr (NS * MB * 8 * 1024 + 512 > 64 * 1024)
@@ -1184,7 +1156,7 @@ hipError_t launch_gemv(const WeightView& w, const void* x, int xdt, int M, void*
     if (M > 16 && !gemv_serves_32(w, xdt, M, num_cus, epi)) return hipErrorInvalidValue;
     // outputs with several pairs of strips per CU: workgroups that stay (tuning 5: never)
     if (gemv_is_automatic() && gemv_stream_serves(w, xdt, M, num_cus, epi))
-        return launch_gemv_stream(w, x, xdt, M, y, ydt, num_cus, epi, st);
+        return launch_gemv_stream(w, x, xdt, M, y, ydt, num_cus, exact_operands, epi, st);
     // few strips, a long K, twelve rows or more: K split over workgroups (tuning 3: never, 4: from three rows on)
     if (rows_kernel && xdt != kF32 && scratch && g_tune_rows != 3 && g_tune_rows != 5 && g_tune_waves == 0 && (M >= kSplitMinRows || g_tune_rows == 4)) {
         SplitPlan sp;

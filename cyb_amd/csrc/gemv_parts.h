@@ -111,6 +111,55 @@ __device__ __forceinline__ void tile_multiply(const Frag16 (&a)[4], const Frag16
     }
 }
 
+// ---- the walk by tile (Q4): one product of the activations with the constant(s) that take the bias off, the C operand of
+// every strip's MFMAs.  f16 activations: subnormal weights, 1/16 for the odd groups on their scale, 2^22 on the final sums;
+// bf16: the numbers 128 + u (tile_operands).
+template <int XMODE>
+__device__ __forceinline__ void tile_bias(const Frag16 (&a)[4], float4_t bias[4])
+{
+    const float4_t zero = {0.f, 0.f, 0.f, 0.f};
+    Frag16 off, off_odd;
+    const uint32_t offw = XMODE == XF16 ? kSubBiasL : kBf16Neg136x2, offw_odd = XMODE == XF16 ? kSubBiasH : offw;
+    off.u = (u32x4_t){offw, offw, offw, offw};
+    off_odd.u = (u32x4_t){offw_odd, offw_odd, offw_odd, offw_odd};
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        if constexpr (XMODE == XF16) bias[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j].h, ((j & 1) ? off_odd : off).h, zero, 0, 0, 0);
+        else bias[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j].b, off.b, zero, 0, 0, 0);
+    }
+}
+
+__device__ __forceinline__ void tile_operands_sub(const TileRegs<4>& t, Frag16 (&b)[4])
+{
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        uint32_t bw[4];
+        unpack_q4_sub(t.q[0][2 * (j >> 1)], t.q[0][2 * (j >> 1) + 1], j & 1, bw);
+        b[j].u = (u32x4_t){bw[0], bw[1], bw[2], bw[3]};
+    }
+}
+
+template <int XMODE>
+__device__ __forceinline__ void tile_multiply_from(const Frag16 (&a)[4], const Frag16 (&b)[4], const float4_t bias[4], float4_t d[4])
+{
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        if constexpr (XMODE == XF16) d[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j].h, b[j].h, bias[j], 0, 0, 0);
+        else d[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j].b, b[j].b, bias[j], 0, 0, 0);
+    }
+}
+
+__device__ __forceinline__ void tile_accum_sub(u32x2_t s, const float4_t d[4], float acc[4])
+{
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint32_t sb = (j & 1) ? (s[j >> 1] >> 16) : (s[j >> 1] & 0xffffu);
+        const float sf = (j & 1) ? f16_bits_to_f32(sb) * 0.0625f : f16_bits_to_f32(sb);
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[r] = __builtin_fmaf(sf, d[j][r], acc[r]);
+    }
+}
+
 // v as the lanes named by a DPP control see it (quad permutations, mirrors within a row of 16)
 template <int CTRL>
 __device__ __forceinline__ float lane_cross(float v)

@@ -9,8 +9,10 @@
 // way.  The waves' partial sums of a pair meet in one of two LDS areas - one barrier per pair - and the waves that
 // add them up do so while the others are already multiplying.
 //
-// Which wave owns which K tile, and the order of every sum, is that of gemv.hip's kernel with eight waves and
-// integer operands: a row's bits do not depend on the batch it travels in.
+// Which wave owns which K tile, and the order of every sum, is that of gemv.hip's kernel with the same waves, with its plain
+// operands (f16 rows: exact integers) or, where that kernel shares a shape by row count and walks it by tile, with those of that
+// walk (TILE): a row's bits do not depend on the batch of 3 .. 32 rows it travels in.  (With a folded norm the squares are summed as
+// loaded, so they do: 3 .. 8, 9 .. 32 rows here, up to 4, 8, 16 in gemv.hip.)
 // (f16 rows, us per call before -> after: Q8 2560 -> 32003 at 8 / 27 rows 20.1 -> 16.1, 36.4 -> 17.9 (12.4 at 7 TB/s); Q4 2048 ->
 // 20000 with a norm 17.6 -> 8.2, 22.0 -> 10.6; Q4 4096 -> 128256 at 27 rows 92.6 -> 66.2.  Two or three pairs ahead
 // instead of one changed nothing on long outputs and cost 2 us on short ones.)
@@ -22,12 +24,16 @@ namespace {
 
 // TS: K tiles a wave owns at most (kt = wave, wave + 8, ...).  MB: blocks of 16 rows.
 // S: strips of a step, 2 or (where the registers do not hold two) 1.
-template <int BITS, int XMODE, int W, int TS, int MB, int XR, bool NORM, int S>
+// TILE (Q4): the operands and the order of sums of the batched-rows kernel's walk by tile - the product of the activations
+// with the constant that takes the bias off comes first, one for all strips of a step, and f16 activations meet subnormal
+// weights (gemv_rows_kernel, SUB).  For shapes where that kernel has the calls with fewer, or more, rows: a row keeps its bits.
+template <int BITS, int XMODE, int W, int TS, int MB, int XR, bool NORM, int S, bool TILE>
 __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemv_stream_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restrict__ x, const void* __restrict__ gamma, int KT, int K, int NT,
                         int M, int gamma_dt, int steps, int N, void* __restrict__ y, int ydt, Epilogue epi)
 {
     static_assert(W == 4 || W == 8, "a wave finishes output registers of one row in four");
+    static_assert(!TILE || (BITS == 4 && !NORM), "by tile: Q4, no folded norm");
     const WeightView w = {wbase, N, K, NT, KT, BITS};
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const uint32_t magic = (BITS == 4 && XMODE == XBF16) ? q4_magic_vgpr_bf16() : q4_magic_vgpr();
@@ -148,7 +154,7 @@ void gemv_stream_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __res
 
         float scale[MB];                                        // 1 / rms of the rows whose outputs this wave finishes
 #pragma unroll
-        for (int b = 0; b < MB; b++) scale[b] = 1.f;
+        for (int b = 0; b < MB; b++) scale[b] = TILE && XMODE == XF16 ? kSubUnscale : 1.f;
         if constexpr (NORM) {
             // P lanes hold a row's pieces
 #pragma unroll
@@ -183,20 +189,33 @@ void gemv_stream_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __res
 #pragma unroll
                     for (int r = 0; r < 4; r++) acc[s][b][r] = 0.f;
 #pragma unroll
-            for (int u = 0; u < TV; u++)
+            for (int u = 0; u < TV; u++) {
+                float4_t bias[TILE ? MB : 1][4];
+                if constexpr (TILE) {
+#pragma unroll
+                    for (int b = 0; b < MB; b++) tile_bias<XMODE>(a[b][u], bias[b]);
+                }
 #pragma unroll
                 for (int s = 0; s < S; s++) {
                     Frag16 bop[4];
-                    tile_operands<BITS, XMODE>(buf[s][u], magic, bop);
+                    if constexpr (TILE && XMODE == XF16) tile_operands_sub(buf[s][u], bop);
+                    else tile_operands<BITS, XMODE>(buf[s][u], magic, bop);
                     const u32x2_t sc = buf[s][u].s;
                     if constexpr (decltype(more)::value) request(buf[s][u], i + stride, s, u);
                     float4_t d[MB][4];
 #pragma unroll
-                    for (int b = 0; b < MB; b++) tile_multiply<BITS, XMODE>(a[b][u], bop, d[b]);
+                    for (int b = 0; b < MB; b++) {
+                        if constexpr (TILE) tile_multiply_from<XMODE>(a[b][u], bop, bias[b], d[b]);
+                        else tile_multiply<BITS, XMODE>(a[b][u], bop, d[b]);
+                    }
 #pragma unroll
-                    for (int b = 0; b < MB; b++) tile_accum<4>(sc, d[b], acc[s][b]);
+                    for (int b = 0; b < MB; b++) {
+                        if constexpr (TILE && XMODE == XF16) tile_accum_sub(sc, d[b], acc[s][b]);
+                        else tile_accum<4>(sc, d[b], acc[s][b]);
+                    }
                     if (MB == 2) __builtin_amdgcn_sched_barrier(0);          // (unpacking ahead would spill)
                 }
+            }
 #pragma unroll
             for (int s = 0; s < S; s++)
 #pragma unroll
@@ -236,57 +255,91 @@ void gemv_stream_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __res
     else run(std::integral_constant<int, TS - 1>{});
 }
 
-template <int BITS, int XMODE, int W, int TS, int MB, int XR, bool NORM>
+template <int BITS, int XMODE, int W, int TS, int MB, int XR, bool NORM, bool TILE = false>
 hipError_t launch_k(const WeightView& w, const void* x, int M, void* y, int ydt, int num_cus, const Epilogue& epi, hipStream_t st)
 {
     constexpr int S = (TS == 4 && MB == 2) ? 1 : 2;
     const int steps = (w.NT + S - 1) / S;
     // two exchange areas, the waves' sums of squares, each wave's tiles of gamma as fp32
     constexpr int lds = (2 * S * MB * W * 4 * 64 + MB * W * 16 + (NORM ? W * TS * kTileK : 0)) * (int)sizeof(float);
-    auto kern = gemv_stream_kernel<BITS, XMODE, W, TS, MB, XR, NORM, S>;
-    if constexpr (lds > 64 * 1024) (void)LdsRequest<&gemv_stream_kernel<BITS, XMODE, W, TS, MB, XR, NORM, S>, lds>::registered;
+    auto kern = gemv_stream_kernel<BITS, XMODE, W, TS, MB, XR, NORM, S, TILE>;
+    if constexpr (lds > 64 * 1024) (void)LdsRequest<&gemv_stream_kernel<BITS, XMODE, W, TS, MB, XR, NORM, S, TILE>, lds>::registered;
     hipLaunchKernelGGL(kern, dim3((unsigned)min(steps, num_cus * (8 / W))), dim3(W * 64), lds, st, w.base, static_cast<const uint16_t*>(x), epi.gamma,
                        w.KT, w.K, w.NT, M, epi.gamma_dt, steps, w.N, y, ydt, epi);
     return hipGetLastError();
 }
 
-template <int BITS, int XMODE, int W, int TS>
+template <int BITS, int XMODE, int W, int TS, bool TILE>
 hipError_t launch_m(const WeightView& w, const void* x, int M, void* y, int ydt, int num_cus, const Epilogue& epi, hipStream_t st)
 {
     if (M > 16) {
         if constexpr (TS < 4 && XMODE == XF16) {
             if (epi.gamma) return launch_k<BITS, XMODE, W, TS, 2, 16, true>(w, x, M, y, ydt, num_cus, epi, st);
         }
-        return launch_k<BITS, XMODE, W, TS, 2, 16, false>(w, x, M, y, ydt, num_cus, epi, st);
+        return launch_k<BITS, XMODE, W, TS, 2, 16, false, TILE && W == 8>(w, x, M, y, ydt, num_cus, epi, st);     // (four waves: only pairs go by tile, not here)
     }
     if constexpr (W == 8) {
         if (M <= 8) {
-            if (epi.gamma) return launch_k<BITS, XMODE, W, TS, 1, 8, true>(w, x, M, y, ydt, num_cus, epi, st);
-            return launch_k<BITS, XMODE, W, TS, 1, 8, false>(w, x, M, y, ydt, num_cus, epi, st);
+            if (!TILE && epi.gamma) return launch_k<BITS, XMODE, W, TS, 1, 8, true>(w, x, M, y, ydt, num_cus, epi, st);
+            return launch_k<BITS, XMODE, W, TS, 1, 8, false, TILE>(w, x, M, y, ydt, num_cus, epi, st);
         }
     }
-    if (epi.gamma) return launch_k<BITS, XMODE, W, TS, 1, 16, true>(w, x, M, y, ydt, num_cus, epi, st);
-    return launch_k<BITS, XMODE, W, TS, 1, 16, false>(w, x, M, y, ydt, num_cus, epi, st);
-}
-
-template <int BITS, int XMODE, int W>
-hipError_t launch_w(const WeightView& w, const void* x, int M, void* y, int ydt, int num_cus, const Epilogue& epi, hipStream_t st)
-{
-    const int ts = (w.KT + W - 1) / W;
-    if (ts == 2) return launch_m<BITS, XMODE, W, 2>(w, x, M, y, ydt, num_cus, epi, st);
-    if (ts == 3) return launch_m<BITS, XMODE, W, 3>(w, x, M, y, ydt, num_cus, epi, st);
-    if (ts == 4) return launch_m<BITS, XMODE, W, 4>(w, x, M, y, ydt, num_cus, epi, st);
-    return hipErrorInvalidValue;         // gemv_stream_serves() said no
+    if (!TILE && epi.gamma) return launch_k<BITS, XMODE, W, TS, 1, 16, true>(w, x, M, y, ydt, num_cus, epi, st);
+    return launch_k<BITS, XMODE, W, TS, 1, 16, false, TILE>(w, x, M, y, ydt, num_cus, epi, st);
 }
 
 // the wave count the batched-rows kernel gives these K
 int waves_of(const WeightView& w) { return w.KT < 16 ? 4 : 8; }
+int tiles_per_wave(const WeightView& w) { return (w.KT + waves_of(w) - 1) / waves_of(w); }
+
+// Four K tiles per wave, one row block, Q4: the batched-rows kernel is as quick, or quicker, where its workgroups (four strips,
+// or two; seven or eight where that is one per CU) come in nearly full rounds, and on the widest outputs, where two
+// of its workgroups share a CU; else the partly empty last round is what it loses.  us per call, this kernel / that one, f16 rows
+// (bf16): K = 4096, 4 rows, N = 20000 12.3 / 15 - 16.6; 14336 (0.88 of a round) at 8 / 16 rows 8.7 / 8.4, 10.1 / 9.1; 28672, exactly seven
+// strips per CU, at 4 / 16 rows 15.5 / 14.0, 16.3 / 14.6 (14.0 / 13.7, 15.4 / 14.6), with its neighbours 28160 and 29184 at
+// 15.5 / 15.3 - 15.4, 16.3 / 17.0 (14.0 / 15.7, 15.4 / 17.3); 128256 at 4 / 16 rows 57.8 / 49.3, 56.7 / 60.4; 6144, rounds three quarters
+// full, at 8 rows 5.3 / 5.7, with a norm 6.8 both.
+bool leaves_few_rows(const WeightView& w, int num_cus, const Epilogue& epi)
+{
+    if (waves_of(w) != 8 || tiles_per_wave(w) != 4 || w.bits != 4) return false;
+    if (w.NT >= 8 * num_cus || w.NT == 7 * num_cus) return true;
+    const int ns = (w.NT + num_cus / 2) / num_cus >= 3 ? 4 : 2;
+    const int groups = (w.NT + ns - 1) / ns, rounds = (groups + num_cus - 1) / num_cus;
+    return epi.gamma ? groups * 4 >= rounds * num_cus * 3 : groups * 5 >= rounds * num_cus * 4;
+}
+
+// Whether the batched-rows kernel has other row counts of this shape and walks them by tile (gemv_rows_kernel, BY_TILE): 17 .. 32
+// rows of pairs, 3 .. 16 where leaves_few_rows says so (there not with seven strips, nor on the widest outputs: those go
+// strip by strip, with the sums of this kernel's plain form).  f16 rows only in decode mode STREAM.
+// us per call, by tile / the plain form / the batched-rows kernel.  K = 4096, f16 rows: 14336 at 17 / 24 / 32 rows 12.5 / 11.3 / 12.6,
+// 12.7 / 11.8 / 13.3, 13.5 / 12.7 / 14.3; 8192 at 17 / 32 rows 8.6 / 8.2 / 8.5, 9.9 / 9.6 / 10.3; 32000 at 32 rows 22.9 / 21.2 / 27.9; pairs: 20000 at
+// 4 / 8 / 16 rows 11.3 / 11.9 / 14.9, 11.4 / 11.9 / 15.7, 12.3 / 13.0 / 16.2.  bf16 rows: 14336 at 32 rows 13.7 / 13.6 / 14.3, pairs of 20000 at 8 rows
+// 11.3 / 11.8 / 16.1.
+bool by_tile(const WeightView& w, int xdt, int num_cus, bool exact_operands, const Epilogue& epi)
+{
+    if (w.bits != 4 || tiles_per_wave(w) != 4 || epi.gamma || (xdt == kF16 && exact_operands)) return false;
+    if (epi.kind == kEpiSwiglu) return true;
+    return leaves_few_rows(w, num_cus, epi) && w.NT < 8 * num_cus && w.NT != 7 * num_cus;
+}
+
+template <int BITS, int XMODE, int W>
+hipError_t launch_w(const WeightView& w, const void* x, int M, void* y, int ydt, int num_cus, bool tile, const Epilogue& epi, hipStream_t st)
+{
+    const int ts = tiles_per_wave(w);
+    if (ts == 2) return launch_m<BITS, XMODE, W, 2, false>(w, x, M, y, ydt, num_cus, epi, st);
+    if (ts == 3) return launch_m<BITS, XMODE, W, 3, false>(w, x, M, y, ydt, num_cus, epi, st);
+    if constexpr (BITS == 4) {
+        if (ts == 4 && tile) return launch_m<BITS, XMODE, W, 4, true>(w, x, M, y, ydt, num_cus, epi, st);
+    }
+    if (ts == 4) return launch_m<BITS, XMODE, W, 4, false>(w, x, M, y, ydt, num_cus, epi, st);
+    return hipErrorInvalidValue;         // gemv_stream_serves() said no
+}
 
 template <int BITS, int XMODE>
-hipError_t launch_x(const WeightView& w, const void* x, int M, void* y, int ydt, int num_cus, const Epilogue& epi, hipStream_t st)
+hipError_t launch_x(const WeightView& w, const void* x, int M, void* y, int ydt, int num_cus, bool tile, const Epilogue& epi, hipStream_t st)
 {
-    if (waves_of(w) == 4) return launch_w<BITS, XMODE, 4>(w, x, M, y, ydt, num_cus, epi, st);
-    return launch_w<BITS, XMODE, 8>(w, x, M, y, ydt, num_cus, epi, st);
+    if (waves_of(w) == 4) return launch_w<BITS, XMODE, 4>(w, x, M, y, ydt, num_cus, tile, epi, st);
+    return launch_w<BITS, XMODE, 8>(w, x, M, y, ydt, num_cus, tile, epi, st);
 }
 
 }  // namespace
@@ -296,31 +349,22 @@ bool gemv_stream_serves(const WeightView& w, int xdt, int M, int num_cus, const 
     if (M < 3 || M > 32 || xdt == kF32) return false;
     // two to four K tiles per wave: operands that fit the registers
     if (w.KT < 8 || w.KT > 32 || (int64_t)w.NT * 2 < (int64_t)num_cus * 3) return false;
-    const int waves = waves_of(w), ts = (w.KT + waves - 1) / waves;
-    if (ts == 4 && M > 16 && (epi.kind == kEpiSwiglu || epi.gamma)) return false;          // (pairs, or gamma, do not fit them)
+    if (tiles_per_wave(w) == 4 && M > 16 && (epi.kind == kEpiSwiglu || epi.gamma)) return false;          // (pairs, or gamma, do not fit them)
     // (x * gamma is rounded to the operand type: the prefill kernels, which take these calls otherwise, round it to f16)
     if (M > 16 && epi.gamma && xdt == kBF16) return false;
-    if (waves == 8 && ts == 4 && M <= 16 && w.bits == 4) {
-        // four K tiles per wave, one row block, Q4: the batched-rows kernel is as quick where its workgroups (four strips, or
-        // two; seven or eight where that is one per CU) come in nearly full rounds, and on the widest outputs, where two
-        // of its workgroups share a CU; else the partly empty last round is what it loses (4096 -> 20000 at 4 rows 15.0
-        // against 11.6 us; 4096 -> 6144, rounds three quarters full, at 8 rows 5.7 against 5.3, with a norm 6.8 both)
-        if (w.NT >= 8 * num_cus || w.NT == 7 * num_cus) return false;
-        const int ns = (w.NT + num_cus / 2) / num_cus >= 3 ? 4 : 2;
-        const int groups = (w.NT + ns - 1) / ns, rounds = (groups + num_cus - 1) / num_cus;
-        if (epi.gamma ? groups * 4 >= rounds * num_cus * 3 : groups * 5 >= rounds * num_cus * 4) return false;
-    }
-    return true;
+    return M > 16 || !leaves_few_rows(w, num_cus, epi);
 }
 
-hipError_t launch_gemv_stream(const WeightView& w, const void* x, int xdt, int M, void* y, int ydt, int num_cus, const Epilogue& epi, hipStream_t st)
+hipError_t launch_gemv_stream(const WeightView& w, const void* x, int xdt, int M, void* y, int ydt, int num_cus, bool exact_operands,
+                              const Epilogue& epi, hipStream_t st)
 {
+    const bool tile = by_tile(w, xdt, num_cus, exact_operands, epi);
     if (w.bits == 4) {
-        if (xdt == kF16) return launch_x<4, XF16>(w, x, M, y, ydt, num_cus, epi, st);
-        return launch_x<4, XBF16>(w, x, M, y, ydt, num_cus, epi, st);
+        if (xdt == kF16) return launch_x<4, XF16>(w, x, M, y, ydt, num_cus, tile, epi, st);
+        return launch_x<4, XBF16>(w, x, M, y, ydt, num_cus, tile, epi, st);
     }
-    if (xdt == kF16) return launch_x<8, XF16>(w, x, M, y, ydt, num_cus, epi, st);
-    return launch_x<8, XBF16>(w, x, M, y, ydt, num_cus, epi, st);
+    if (xdt == kF16) return launch_x<8, XF16>(w, x, M, y, ydt, num_cus, tile, epi, st);
+    return launch_x<8, XBF16>(w, x, M, y, ydt, num_cus, tile, epi, st);
 }
 
 }  // namespace cybq

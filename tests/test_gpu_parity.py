@@ -286,6 +286,44 @@ def test_decode_rows_streamed_by_staying_workgroups(backend, bits, xdt, shape):
         assert rel(y, torch.nn.functional.silu(plain[:M, :half]) * plain[:M, half:2 * half]) < TIGHT, M
 
 
+# two kernels share these shapes by row count: full rounds of four and two strips up to 16 rows and staying workgroups beyond (an odd
+# last strip, a ragged K tile, waves with three and four K tiles), the reverse for gate / up pairs (four waves too),
+# seven strips per CU, several rounds per CU, and shapes that one kernel has for itself
+@pytest.mark.parametrize("bits,N,K,pair", [(4, 14336, 4096, False), (4, 14341, 4064, False), (4, 8180, 3104, False), (4, 32000, 3200, False),
+                                           (4, 28672, 4096, False), (4, 32784, 3200, False), (4, 10241, 3104, False), (4, 20480, 4096, True),
+                                           (4, 6176, 3104, True), (4, 20480, 1792, True), (4, 6176, 1664, True), (8, 14336, 4096, False),
+                                           (8, 8224, 3104, True)])
+@pytest.mark.parametrize("xdt", ["f16", "bf16"])
+def test_a_row_keeps_its_bits_from_3_to_32_rows(backend, bits, N, K, pair, xdt):
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    rows, parts, wd = N // 2 if pair else N, [], []
+    for _ in range(2 if pair else 1):
+        w = torch.empty((rows, K), device="cuda").normal_(0.0, 0.02, generator=g)
+        qd = torch.empty(rows * K * bits // 8, dtype=torch.uint8, device="cuda")
+        sd = torch.empty(rows * (K // 32), dtype=torch.int16, device="cuda")
+        backend.quantize(bits, w, rows, K, qd, sd)
+        parts.append(backend.weight_from_device(bits, rows, K, qd, sd))
+        backend.dequant(parts[-1], w)
+        wd.append(w.double())
+    qw = backend.fuse_pairs(*parts) if pair else parts[0]
+    x = torch.empty((32, K), device="cuda").normal_(generator=g).to(TDT[xdt])
+    ref = x.double() @ wd[0].t()
+    if pair:
+        ref = torch.nn.functional.silu(ref) * (x.double() @ wd[1].t())
+    try:
+        for mode in ("stream", "exact"):
+            backend.set_decode_mode(mode)
+            full = torch.full((32, rows), float("nan"), device="cuda")
+            backend.matmul_ex(qw, x, full, "swiglu" if pair else "none")
+            assert ((full.double() - ref).norm() / ref.norm()).item() < TIGHT, mode
+            for M in (3, 4, 8, 9, 16, 17, 24):
+                y = torch.full((M, rows), float("nan"), device="cuda")
+                backend.matmul_ex(qw, x[:M].contiguous(), y, "swiglu" if pair else "none")
+                assert torch.equal(y, full[:M]), (mode, M)
+    finally:
+        backend.set_decode_mode("stream")
+
+
 @pytest.mark.parametrize("N", [8192, 12288])
 def test_decode_modes_in_the_batched_rows_kernel(backend, oracle, N):
     """3 .. 32 f16 rows on outputs wide enough for two / four strips per workgroup: STREAM feeds the Q4
