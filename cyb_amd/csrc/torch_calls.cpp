@@ -2,8 +2,11 @@
 //
 // A small linear is bound by the host: the launch itself takes 2.9 us of host time, the kernel behind it less.  Looking
 // the tensors over in Python (shape, device, contiguity, type, address: a dozen attribute calls) and going through
-// ctypes added 2.5 us to that; here both cost 0.5 us (one row, 4096 -> 1024, call to call: 5.8 -> 3.7 us).  Nothing is decided here: a call whose arguments are not exactly
-// what the checks in backend.py accept is handed back (kSlow), and the Python code answers it, errors included.
+// ctypes added 2.5 us to that; here both cost 0.5 us (one row, 4096 -> 1024, call to call: 5.8 -> 3.7 us).  Nothing is decided here: a call whose
+// arguments are not exactly what the checks in backend.py accept is handed back (kSlow), and the Python code answers it, errors
+// included.  That goes for tensors that cannot be looked over from here too: subclasses, which may answer in Python, and
+// tensors of a transform (torch.vmap, torch.func.grad), which have no address - asking them throws, and nothing that is thrown
+// leaves an entry.
 #include <Python.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -24,7 +27,7 @@ struct Args {
 // number of elements `t` has to hold -> its address, or nullptr where the Python checks have to look at it
 void* address(PyObject* o, int device, int64_t elems, int* dtype)
 {
-    if (!THPVariable_Check(o)) return nullptr;
+    if (!THPVariable_CheckExact(o)) return nullptr;
     const at::Tensor& t = THPVariable_Unpack(o);
     if (!t.is_cuda() || t.get_device() != device || !t.is_contiguous() || t.numel() < elems) return nullptr;
     if (dtype) {
@@ -57,7 +60,7 @@ bool common(PyObject* const* a, PyObject* x, PyObject* m, PyObject* stream, Args
     r->device = (int)device;
     r->stream = reinterpret_cast<void*>(static_cast<uintptr_t>(st));
     if (m == Py_None) {
-        if (!THPVariable_Check(x)) return false;
+        if (!THPVariable_CheckExact(x)) return false;
         const at::Tensor& t = THPVariable_Unpack(x);
         r->M = t.dim() == 2 ? t.size(0) : 1;
     } else if (!as_int(m, &r->M)) {
@@ -68,8 +71,27 @@ bool common(PyObject* const* a, PyObject* x, PyObject* m, PyObject* stream, Args
 
 PyObject* answer(int rc) { return PyLong_FromLong(rc); }
 
+// the library runs without the interpreter's lock, as under ctypes
+struct Unlocked {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
+using Call = PyObject*(PyObject* const*, Py_ssize_t);
+
+template <Call* F>
+PyObject* entry(PyObject*, PyObject* const* a, Py_ssize_t n)
+{
+    try {
+        return F(a, n);
+    } catch (...) {
+        PyErr_Clear();                  // (a subclass's own exception; the Python checks meet it again)
+        return answer(kSlow);
+    }
+}
+
 // matmul(ctx, device, w, x, y, M, xdt, ydt, stream)
-PyObject* matmul(PyObject*, PyObject* const* a, Py_ssize_t n)
+PyObject* matmul(PyObject* const* a, Py_ssize_t n)
 {
     Args r;
     if (n != 9 || !common(a, a[3], a[5], a[8], &r)) return answer(kSlow);
@@ -87,14 +109,15 @@ PyObject* matmul(PyObject*, PyObject* const* a, Py_ssize_t n)
         ydt = (int)code;
     }
     int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = cybq_matmul(r.ctx, r.w, x, (cybq_dtype)xdt, r.M, y, (cybq_dtype)ydt, r.stream);
-    Py_END_ALLOW_THREADS
+    {
+        Unlocked u;
+        rc = cybq_matmul(r.ctx, r.w, x, (cybq_dtype)xdt, r.M, y, (cybq_dtype)ydt, r.stream);
+    }
     return answer(rc);
 }
 
 // matmul_static(ctx, device, w, x, y, M, stream)
-PyObject* matmul_static(PyObject*, PyObject* const* a, Py_ssize_t n)
+PyObject* matmul_static(PyObject* const* a, Py_ssize_t n)
 {
     Args r;
     if (n != 7 || !common(a, a[3], a[5], a[6], &r)) return answer(kSlow);
@@ -103,14 +126,15 @@ PyObject* matmul_static(PyObject*, PyObject* const* a, Py_ssize_t n)
     void* y = address(a[4], r.device, r.M * r.N, &ydt);
     if (!x || !y) return answer(kSlow);
     int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = cybq_matmul_static(r.ctx, r.w, x, (cybq_dtype)xdt, r.M, y, (cybq_dtype)ydt, r.stream);
-    Py_END_ALLOW_THREADS
+    {
+        Unlocked u;
+        rc = cybq_matmul_static(r.ctx, r.w, x, (cybq_dtype)xdt, r.M, y, (cybq_dtype)ydt, r.stream);
+    }
     return answer(rc);
 }
 
 // matmul_fused(ctx, device, w, x, gamma or None, eps, y, epilogue, residual or None, M, stream)
-PyObject* matmul_fused(PyObject*, PyObject* const* a, Py_ssize_t n)
+PyObject* matmul_fused(PyObject* const* a, Py_ssize_t n)
 {
     Args r;
     int64_t epi;
@@ -129,20 +153,21 @@ PyObject* matmul_fused(PyObject*, PyObject* const* a, Py_ssize_t n)
         eps = PyFloat_AS_DOUBLE(a[5]);
     }
     int rc;
-    Py_BEGIN_ALLOW_THREADS
-    if (gamma)
-        rc = cybq_matmul_norm(r.ctx, r.w, x, (cybq_dtype)xdt, r.M, gamma, (cybq_dtype)gdt, (float)eps, y, (cybq_dtype)ydt,
-                              (cybq_epilogue)epi, residual, r.stream);
-    else
-        rc = cybq_matmul_ex(r.ctx, r.w, x, (cybq_dtype)xdt, r.M, y, (cybq_dtype)ydt, (cybq_epilogue)epi, residual, r.stream);
-    Py_END_ALLOW_THREADS
+    {
+        Unlocked u;
+        if (gamma)
+            rc = cybq_matmul_norm(r.ctx, r.w, x, (cybq_dtype)xdt, r.M, gamma, (cybq_dtype)gdt, (float)eps, y, (cybq_dtype)ydt,
+                                  (cybq_epilogue)epi, residual, r.stream);
+        else
+            rc = cybq_matmul_ex(r.ctx, r.w, x, (cybq_dtype)xdt, r.M, y, (cybq_dtype)ydt, (cybq_epilogue)epi, residual, r.stream);
+    }
     return answer(rc);
 }
 
 PyMethodDef kMethods[] = {
-    {"matmul", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(matmul)), METH_FASTCALL, nullptr},
-    {"matmul_static", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(matmul_static)), METH_FASTCALL, nullptr},
-    {"matmul_fused", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(matmul_fused)), METH_FASTCALL, nullptr},
+    {"matmul", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(entry<matmul>)), METH_FASTCALL, nullptr},
+    {"matmul_static", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(entry<matmul_static>)), METH_FASTCALL, nullptr},
+    {"matmul_fused", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(entry<matmul_fused>)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_torch_calls", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};

@@ -1,0 +1,74 @@
+"""The native call path of Backend.matmul and its like (cyb_amd/csrc/torch_calls.cpp), without a GPU: what it cannot look over it
+hands back to the Python checks, which answer as they did when they were the only path.
+
+The tensors here claim to be on cuda:0 and have no memory; the handle and the context are blank memory that no call gets as far
+as reading into.  Each case runs in a process of its own: a C++ exception that leaves an entry ends the process."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+torch = pytest.importorskip("torch")
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+_PROLOGUE = """
+import ctypes, torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+from cyb_amd import backend as B
+blank = ctypes.create_string_buffer(4096)
+addr = ctypes.addressof(blank)
+calls = B._load_calls()
+assert calls is not None
+
+class NoAnswers(torch.Tensor):
+    @staticmethod
+    def __new__(cls):
+        return torch.Tensor._make_wrapper_subclass(cls, (1, 4), dtype=torch.float16, device="cuda:0")
+    @classmethod
+    def __torch_dispatch__(cls, f, types, args=(), kwargs=None):
+        raise RuntimeError("not answered")
+
+def hand_backs(t):
+    return [calls.matmul(addr, 0, addr, t, t, None, None, None, 0), calls.matmul(addr, 0, addr, t, t, 1, None, None, 0),
+            calls.matmul_static(addr, 0, addr, t, t, None, 0), calls.matmul_fused(addr, 0, addr, t, t, 1e-5, t, 0, t, None, 0)]
+
+be = B.Backend.__new__(B.Backend)            # the Python checks alone: no context, no device
+be.device, be._addr, be._ctx = 0, addr, ctypes.c_void_p()
+be.weights, be._lib = {}, B.load_library()
+w = B.QWeight.__new__(B.QWeight)
+w._h, w._addr, w._backend, w.N, w.K = ctypes.c_void_p(addr), addr, be, 1, 4
+
+def through_backend(t):
+    assert hand_backs(t) == [1, 1, 1, 1]
+    try:
+        be.matmul(w, t, t)
+    except RuntimeError as e:
+        print("raised", type(e).__name__, flush=True)
+        raise SystemExit(0)                  # (there is nothing to return to a transform)
+"""
+
+_CASES = {
+    "subclass that raises": "through_backend(NoAnswers())",
+    "vmap": "with FakeTensorMode():\n    torch.vmap(through_backend)(torch.empty((2, 1, 4), device='cuda', dtype=torch.float16))",
+    "grad": "with FakeTensorMode():\n    torch.func.grad(through_backend)(torch.empty((1, 4), device='cuda'))",
+    "fake": "with FakeTensorMode():\n    through_backend(torch.empty((1, 4), device='cuda', dtype=torch.float16))",
+    "cpu": "through_backend(torch.empty((1, 4), dtype=torch.float16))",
+}
+
+
+@pytest.mark.parametrize("case", _CASES)
+def test_tensors_without_an_address_are_handed_back_and_raise(case):
+    p = subprocess.run([sys.executable, "-c", _PROLOGUE + _CASES[case]], cwd=ROOT, capture_output=True, text=True, timeout=110)
+    assert p.returncode == 0, p.stderr[-2000:]
+    assert "raised" in p.stdout, p.stdout + p.stderr[-2000:]
+
+
+@pytest.mark.parametrize("args", ["(addr, 0, addr, x, x, True, None, None, 0)", "(addr, 0, addr, x, x, 1 << 70, None, None, 0)",
+                                  "(0, 0, addr, x, x, None, None, None, 0)", "(addr, 0, 0, x, x, None, None, None, 0)",
+                                  "(addr, 0, addr, None, x, None, None, None, 0)", "(addr, 0, addr, 4096, x, 1, None, None, 0)",
+                                  "(addr, 0, addr, x, x, None, None, None, None)", "(addr, 0, addr, x, x)", "()"])
+def test_arguments_that_are_not_a_plain_call_are_handed_back(args):
+    code = _PROLOGUE + f"x = torch.empty((1, 4), dtype=torch.float16)\nassert calls.matmul{args} == 1"
+    p = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=110)
+    assert p.returncode == 0, p.stderr[-2000:]
