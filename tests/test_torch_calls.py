@@ -24,7 +24,7 @@ assert calls is not None
 class NoAnswers(torch.Tensor):
     @staticmethod
     def __new__(cls):
-        return torch.Tensor._make_wrapper_subclass(cls, (1, 4), dtype=torch.float16, device="cuda:0")
+        return torch.Tensor._make_wrapper_subclass(cls, (1, 4), dtype=torch.float16, device="cuda:0", dispatch_sizes_strides_policy="strides")
     @classmethod
     def __torch_dispatch__(cls, f, types, args=(), kwargs=None):
         raise RuntimeError("not answered")
