@@ -24,6 +24,7 @@ import importlib.machinery
 import importlib.util
 import os
 import sys
+import warnings
 from dataclasses import dataclass, field
 from typing import Dict, Optional
 
@@ -105,19 +106,26 @@ def load_library() -> ctypes.CDLL:
     return lib
 
 
-_calls = None
+_calls = None          # the module; False once it turned out not to be there, or not to be this torch's
 
 
 def _load_calls():
-    """The native call path for torch tensors (csrc/torch_calls.cpp), once the program has torch."""
+    """The native call path for torch tensors (csrc/torch_calls.cpp), once the program has torch.  It saves host time and does
+    nothing that the ctypes calls below do not do: without it, or built for another torch or Python, those serve."""
     global _calls
     if _calls is None and "torch" in sys.modules:
-        if not os.path.exists(_CALLS_PATH):
-            raise CybqError(-4, "library missing", f"{_CALLS_PATH} not built; run __graft_entry__.build()")
-        loader = importlib.machinery.ExtensionFileLoader("_torch_calls", _CALLS_PATH)
-        mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_torch_calls", _CALLS_PATH, loader=loader))
-        loader.exec_module(mod)
-        _calls = mod
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("_torch_calls", _CALLS_PATH)
+            mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_torch_calls", _CALLS_PATH, loader=loader))
+            loader.exec_module(mod)
+            here = sys.modules["torch"].__version__.split("+")[0]
+            if mod.TORCH_VERSION != here:
+                raise ImportError(f"built for torch {mod.TORCH_VERSION}, not {here}")
+            _calls = mod
+        except (ImportError, OSError) as e:
+            _calls = False
+            warnings.warn(f"small calls take 2 us more of host time without {_CALLS_PATH} ({e}); make -C cyb_amd/csrc python builds it",
+                          RuntimeWarning, stacklevel=3)
     return _calls
 
 
@@ -360,7 +368,7 @@ class Backend:
     def matmul(self, w: QWeight, x, y, M: Optional[int] = None, xdt: Optional[int] = None,
                ydt: Optional[int] = None, stream: int = 0) -> None:
         calls = _calls or _load_calls()
-        if calls is not None:                           # (positive: not a plain call on tensors, looked at below)
+        if calls:                                       # (positive: not a plain call on tensors, looked at below)
             rc = calls.matmul(self._addr, self.device, w._addr, x, y, M, xdt, ydt, stream)
             if rc <= 0:
                 return self._check(rc)
@@ -373,7 +381,7 @@ class Backend:
     def matmul_static(self, w: QWeight, x, y, M: Optional[int] = None, stream: int = 0) -> None:
         """cybq_matmul_static: the same op with its scratch in a static device array (allocates nothing)."""
         calls = _calls or _load_calls()
-        if calls is not None:
+        if calls:
             rc = calls.matmul_static(self._addr, self.device, w._addr, x, y, M, stream)
             if rc <= 0:
                 return self._check(rc)
@@ -390,7 +398,7 @@ class Backend:
         if epilogue not in EPILOGUES:
             raise CybqError(-1, "invalid argument", f"unknown epilogue {epilogue!r}")
         calls = _calls or _load_calls()
-        if calls is not None:
+        if calls:
             rc = calls.matmul_fused(self._addr, self.device, w._addr, x, None, 0.0, y, EPILOGUES[epilogue], residual, M, stream)
             if rc <= 0:
                 return self._check(rc)
@@ -406,7 +414,7 @@ class Backend:
         if epilogue not in EPILOGUES:
             raise CybqError(-1, "invalid argument", f"unknown epilogue {epilogue!r}")
         calls = _calls or _load_calls()
-        if calls is not None and gamma is not None:
+        if calls and gamma is not None:
             rc = calls.matmul_fused(self._addr, self.device, w._addr, x, gamma, float(eps), y, EPILOGUES[epilogue], residual, M, stream)
             if rc <= 0:
                 return self._check(rc)

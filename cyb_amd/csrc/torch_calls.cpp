@@ -9,6 +9,7 @@
 // leaves an entry.
 #include <Python.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include "../../include/cybq.h"
 
@@ -177,6 +178,6 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_torch_calls", nullptr, -1, kMeth
 PyMODINIT_FUNC PyInit__torch_calls(void)
 {
     PyObject* m = PyModule_Create(&kModule);
-    if (m) PyModule_AddIntConstant(m, "SLOW", kSlow);
+    if (m && PyModule_AddStringConstant(m, "TORCH_VERSION", TORCH_VERSION) != 0) Py_CLEAR(m);
     return m;
 }

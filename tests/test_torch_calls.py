@@ -72,3 +72,36 @@ def test_arguments_that_are_not_a_plain_call_are_handed_back(args):
     code = _PROLOGUE + f"x = torch.empty((1, 4), dtype=torch.float16)\nassert calls.matmul{args} == 1"
     p = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=110)
     assert p.returncode == 0, p.stderr[-2000:]
+
+
+@pytest.mark.parametrize("what", ["missing", "not a library", "another torch"])
+def test_without_the_native_path_the_ctypes_calls_serve(what, tmp_path, monkeypatch):
+    import ctypes
+
+    from cyb_amd import backend as B
+    monkeypatch.setattr(B, "_calls", None)
+    if what == "another torch":
+        monkeypatch.setattr(torch, "__version__", "1.0.0")
+    else:
+        path = tmp_path / "_torch_calls.so"
+        if what == "not a library":
+            path.write_bytes(b"not a library")
+        monkeypatch.setattr(B, "_CALLS_PATH", str(path))
+    be = B.Backend.__new__(B.Backend)
+    be._lib, be._ctx, be._addr, be.device, be.weights = B.load_library(), ctypes.c_void_p(), 0, 0, {}
+    w = B.QWeight.__new__(B.QWeight)
+    w._h, w._addr, w._backend, w.N, w.K = ctypes.c_void_p(), 0, be, 4, 4
+    x = torch.empty((1, 4), dtype=torch.float16)
+    with pytest.warns(RuntimeWarning, match="_torch_calls.so"):
+        with pytest.raises(B.CybqError, match="must live on cuda:0"):           # (the Python checks have the call)
+            be.matmul(w, x, x)
+    for call in (lambda: be.matmul_static(w, x, x), lambda: be.matmul_ex(w, x, x), lambda: be.matmul_norm(w, x, x, 1e-5, x)):
+        with pytest.raises(B.CybqError, match="must live on cuda:0"):
+            call()
+
+
+def test_the_library_builds_without_torch():
+    """`make` is also what the C++ and Rust users run."""
+    p = subprocess.run(["make", "-n", "-B", "PYTHON=/bin/false"], cwd=os.path.join(ROOT, "cyb_amd", "csrc"), capture_output=True, text=True)
+    assert p.returncode == 0 and "libcybq.so" in p.stdout, p.stderr
+    assert "torch" not in p.stdout
