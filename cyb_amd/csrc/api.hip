@@ -43,7 +43,8 @@ struct cybq_weight {
     // cybq_weight_from_device: the repack kernel stores "some scale is wide" into a pinned word; the first call that
     // needs the answer waits for the kernel (long since complete in practice) and moves it into wide_scales
     cybq::ScanSlot scan;
-    std::once_flag scan_once;
+    std::mutex scan_mutex;
+    std::atomic<bool> scan_read{false};
 };
 
 namespace cybq {
@@ -170,17 +171,22 @@ void release_weight(cybq_weight* w)
     delete w;
 }
 
-// wide_scales of a weight whose scales were scanned on the device: the answer is taken the first time it is needed
-bool weight_is_wide(const cybq_weight* cw)
+// wide_scales of a weight whose scales were scanned on the device: the answer is taken the first time it is needed.  A wait that
+// fails leaves the question open: no kernel is chosen by an answer that never came.
+hipError_t weight_is_wide(const cybq_weight* cw, bool* wide)
 {
     cybq_weight* w = const_cast<cybq_weight*>(cw);
-    if (w->scan.word) {
-        std::call_once(w->scan_once, [w]() {
-            (void)hipEventSynchronize(w->scan.done);
-            w->wide_scales = w->wide_scales || *w->scan.word != 0u;
-        });
+    if (w->scan.word && !w->scan_read.load(std::memory_order_acquire)) {
+        std::lock_guard<std::mutex> lock(w->scan_mutex);
+        if (!w->scan_read.load(std::memory_order_relaxed)) {
+            const hipError_t e = hipEventSynchronize(w->scan.done);
+            if (e != hipSuccess) return e;
+            w->wide_scales = *w->scan.word != 0u;
+            w->scan_read.store(true, std::memory_order_release);
+        }
     }
-    return w->wide_scales;
+    *wide = w->wide_scales;
+    return hipSuccess;
 }
 
 int check_weight_shape(cybq_ctx* ctx, int quant, int64_t N, int64_t K)
@@ -350,13 +356,19 @@ int cybq_weight_from_device(cybq_ctx* ctx, cybq_quant quant, int64_t N, int64_t 
     if (rc) return rc;
     DeviceGuard guard(ctx->device);
     if (guard.err != hipSuccess) return fail_hip(ctx, guard.err, "hipSetDevice");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    // A recorded repack has not run when the call returns and would run again with every replay, into memory that a free hands
+    // on; with a pooled block nothing below would refuse it.
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    hipError_t e = hipStreamIsCapturing(st, &capture);
+    if (e != hipSuccess) return fail_hip(ctx, e, "hipStreamIsCapturing");
+    if (capture != hipStreamCaptureStatusNone) return fail(ctx, CYBQ_ERR_UNSUPPORTED, "cybq_weight_from_device: the stream is being captured");
     cybq_weight* w = nullptr;
     rc = alloc_weight(ctx, quant, N, K, stream ? cybq::kElsewhere : cybq::kDefaultStream, &w);
     if (rc) return rc;
     // the scales are scanned by the repack kernel itself: it stores 1 into a pinned word where "some |scale| * qmax leaves
     // f16", and the first call that needs the word waits for the event behind the kernel
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    hipError_t e = cybq::scan_acquire(ctx->device, &w->scan);
+    e = cybq::scan_acquire(ctx->device, &w->scan);
     if (e == hipSuccess) {
         *w->scan.word = 0u;
         e = cybq::launch_repack(quant, CYBQ_LAYOUT_PLANAR, false, q_dev, scales_dev, w->data, (int)N, (int)K, w->NT, w->KT, w->scan.word, st);
@@ -388,12 +400,12 @@ int cybq_weight_clone(cybq_ctx* ctx, const cybq_weight* src, cybq_weight** out)
     }
     if (rc) return rc;
     hipError_t e = hipMemcpy(w->data, src->data, src->bytes, hipMemcpyDeviceToDevice);
+    if (e == hipSuccess) e = weight_is_wide(src, &w->wide_scales);
     if (e != hipSuccess) {
         release_weight(w);
         return fail_hip(ctx, e, "weight clone");
     }
     w->paired = src->paired;
-    w->wide_scales = weight_is_wide(src);
     *out = w;
     return CYBQ_OK;
 }
@@ -456,8 +468,25 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
     if (guard.err != hipSuccess) return fail_hip(ctx, guard.err, "hipSetDevice");
     hipStream_t st = static_cast<hipStream_t>(stream);
     cybq::WeightView v = view_of(w);
+    hipError_t e = hipSuccess;
+    // (asked only where the way of the call hangs on it: the first time it is a wait)
+    auto wide = [&]() {
+        bool is = false;
+        if (e == hipSuccess) e = weight_is_wide(w, &is);
+        return is;
+    };
+    enum { kDecode, kTwoPasses, kPrefill, kWalk } way;
+    if (M <= 16 || (M <= 32 && cybq::gemv_serves_32(v, (int)xdt, (int)M, ctx->num_cus, epi)))
+        way = kDecode;
+    else if (M <= 64 && (int64_t)w->N * w->K <= (int64_t)6144 * 4096 && cybq::gemv_serves_32(v, (int)xdt, 32, ctx->num_cus, epi) &&
+             (ctx->prefill_exact || wide() || !cybq::gemm_rows_takes(v, (int)M, ctx->num_cus, epi)))
+        way = kTwoPasses;
+    else if (!wide() && (xdt == CYBQ_F32 ? !ctx->prefill_exact : (M > 32 || (!ctx->prefill_exact && cybq::gemm_rows_takes(v, (int)M, ctx->num_cus, epi)))))
+        way = kPrefill;
+    else
+        way = kWalk;
+    if (e != hipSuccess) return fail_hip(ctx, e, "scale scan");
     mark_use(w, stream);
-    hipError_t e;
     // the tail of the scratch belongs to the decode kernels (tickets and slabs of a K split), the rest to prefill
     void* dscr = nullptr;
     size_t dscr_bytes = 0;
@@ -466,10 +495,9 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
         dscr = static_cast<char*>(workspace) + workspace_bytes;
         dscr_bytes = cybq::kDecodeScratchBytes;
     }
-    if (M <= 16 || (M <= 32 && cybq::gemv_serves_32(v, (int)xdt, (int)M, ctx->num_cus, epi))) {
+    if (way == kDecode) {
         e = cybq::launch_gemv(v, x, xdt, (int)M, y, ydt, ctx->num_cus, ctx->decode_exact, epi, dscr, dscr_bytes, st);
-    } else if (M <= 64 && (int64_t)w->N * w->K <= (int64_t)6144 * 4096 && cybq::gemv_serves_32(v, (int)xdt, 32, ctx->num_cus, epi) &&
-               (ctx->prefill_exact || weight_is_wide(w) || !cybq::gemm_rows_takes(v, (int)M, ctx->num_cus, epi))) {
+    } else if (way == kTwoPasses) {
         // 33..64 rows on a small weight (up to 4096 -> 6144) that the few-rows MFMA kernel does not take (exact
         // mode, wide scales, K outside 2048 .. 8192, a folded SwiGLU): the tiled MFMA
         // kernel would split K over workgroups and add the slabs in a second pass; two passes of the
@@ -485,7 +513,7 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
         if (e == hipSuccess)
             e = cybq::launch_gemv(v, static_cast<const char*>(x) + (size_t)32 * w->K * dtype_size(xdt), xdt, (int)M - 32,
                                   static_cast<char*>(y) + yoff, ydt, ctx->num_cus, exact_ops, ec, dscr, dscr_bytes, st);
-    } else if (!weight_is_wide(w) && (xdt == CYBQ_F32 ? !ctx->prefill_exact : (M > 32 || (!ctx->prefill_exact && cybq::gemm_rows_takes(v, (int)M, ctx->num_cus, epi))))) {
+    } else if (way == kPrefill) {
         e = cybq::launch_gemm(v, x, xdt, (int)M, y, ydt, ctx->num_cus, ctx->prefill_exact, workspace, workspace_bytes,
                               epi, st);
     } else {
@@ -499,7 +527,6 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
         // tile mostly empty (without the norm they are one pass, two row blocks per weight operand).
         // A tensor with wide scales (scale * q leaves f16) is walked the same way for any M, 32 rows at a
         // time where the batched-rows kernel takes them in one pass: the weights stream once per 32 rows.
-        e = hipSuccess;
         const int64_t n_out = epi.kind == cybq::kEpiSwiglu ? w->N / 2 : w->N;
         const int64_t step = cybq::gemv_serves_32(v, (int)xdt, 32, ctx->num_cus, epi) ? 32 : 16;
         for (int64_t m0 = 0; m0 < M && e == hipSuccess; m0 += step) {
@@ -573,12 +600,15 @@ int cybq_weight_fuse_pairs(cybq_ctx* ctx, const cybq_weight* gate, const cybq_we
     hipError_t e = hipMemcpy2D(w->data, 2 * sb, gate->data, sb, sb, gate->NT, hipMemcpyDeviceToDevice);
     if (e == hipSuccess) e = hipMemcpy2D(w->data + sb, 2 * sb, up->data, sb, sb, up->NT, hipMemcpyDeviceToDevice);
     if (e == hipSuccess) e = hipDeviceSynchronize();
+    bool wide_gate = false, wide_up = false;
+    if (e == hipSuccess) e = weight_is_wide(gate, &wide_gate);
+    if (e == hipSuccess) e = weight_is_wide(up, &wide_up);
     if (e != hipSuccess) {
         release_weight(w);
         return fail_hip(ctx, e, "weight fuse");
     }
     w->paired = true;
-    w->wide_scales = weight_is_wide(gate) || weight_is_wide(up);
+    w->wide_scales = wide_gate || wide_up;
     *out = w;
     return CYBQ_OK;
 }

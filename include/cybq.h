@@ -273,7 +273,8 @@ int cybq_quantize(cybq_ctx* ctx, cybq_quant quant, const float* src, int64_t N, 
  * (cybq_weight_clone, cybq_weight_fuse_pairs, a matmul on another stream) must be ordered after it
  * by the caller.  The scales are scanned on the device by the same kernel (a tensor whose
  * |scale| * 8 (Q4) or |scale| * 128 (Q8) leaves f16's range is served by the decode kernels for
- * every M, as after cybq_weight_upload); the first call that needs the answer waits for that kernel. */
+ * every M, as after cybq_weight_upload); the first call that needs the answer waits for that kernel.
+ * A stream that is being captured is refused (CYBQ_ERR_UNSUPPORTED). */
 int cybq_weight_from_device(cybq_ctx* ctx, cybq_quant quant, int64_t N, int64_t K,
                             const void* q_dev, const void* scales_dev, void* stream,
                             cybq_weight** out);

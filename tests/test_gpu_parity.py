@@ -2066,6 +2066,42 @@ def test_first_call_of_a_kernel_may_sit_inside_a_capture(oracle):
         be.close()
 
 
+def test_a_weight_is_not_made_on_a_capturing_stream(backend):
+    """Also where nothing has to be allocated for it (the memory and the scan word of a weight freed before): the recorded repack
+    would not have run when the call returns.  The capture goes on, and the first prefill call of a weight made outside of it may
+    sit inside."""
+    N, K, M = 1024, 2048, 100
+    w = torch.empty((N, K), device="cuda").normal_(0.0, 0.02)
+    qd = torch.empty(N * K // 2, dtype=torch.uint8, device="cuda")
+    sd = torch.empty(N * (K // 32), dtype=torch.int16, device="cuda")
+    backend.quantize(4, w, N, K, qd, sd)
+    qw = backend.weight_from_device(4, N, K, qd, sd)
+    backend.weight_from_device(4, N, K, qd, sd).free()
+    x = torch.empty((M, K), device="cuda").normal_().to(torch.bfloat16)
+    y, want = torch.zeros((M, N), device="cuda"), torch.zeros((M, N), device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        st = torch.cuda.current_stream().cuda_stream
+        with pytest.raises(CybqError) as err:
+            backend.weight_from_device(4, N, K, qd, sd, stream=st)
+        assert err.value.status == -7
+        backend.matmul(qw, x, y, stream=st)
+    backend.matmul(qw, x, want)
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+    again = backend.weight_from_device(4, N, K, qd, sd)          # (and nothing was left behind by the refusal)
+    backend.matmul(again, x, y)
+    torch.cuda.synchronize()
+    assert torch.equal(y, want)
+    again.free()
+    qw.free()
+
+
 def test_read_pattern_probes_run(backend, oracle):
     """The pure-read probes the benchmark records as ceilings: every pattern runs on the headline tensor's
     K and on a ragged tensor (flat patterns), and the strip patterns refuse shapes they do not cover."""
