@@ -88,16 +88,23 @@ static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 void* g_scratch_ptr[kMaxDevices] = {};
 std::mutex g_scratch_mutex;              // contexts may be created from several threads
 
+// (no memory for the text: the code alone)
 int fail(cybq_ctx* ctx, int code, const char* what)
 {
-    if (ctx) ctx->last_error = what ? what : "";
+    try {
+        if (ctx) ctx->last_error = what ? what : "";
+    } catch (const std::bad_alloc&) {
+        ctx->last_error.clear();
+    }
     return code;
 }
 
 int fail_hip(cybq_ctx* ctx, hipError_t e, const char* where)
 {
-    if (ctx) {
-        ctx->last_error = std::string(where) + ": " + hipGetErrorString(e);
+    try {
+        if (ctx) ctx->last_error = std::string(where) + ": " + hipGetErrorString(e);
+    } catch (const std::bad_alloc&) {
+        ctx->last_error.clear();
     }
     (void)hipGetLastError();   // clear the sticky error so the next call starts clean
     return e == hipErrorOutOfMemory ? CYBQ_ERR_NOMEM : CYBQ_ERR_HIP;
@@ -268,7 +275,11 @@ int cybq_init(int device, cybq_ctx** out)
         delete ctx;
         return CYBQ_ERR_HIP;
     }
-    cybq::pool_retain(device);
+    if (cybq::pool_retain(device) != hipSuccess) {
+        (void)hipFree(ctx->workspace);
+        delete ctx;
+        return CYBQ_ERR_NOMEM;
+    }
     *out = ctx;
     return CYBQ_OK;
 }

@@ -21,7 +21,7 @@ enum UsedOn : int { kUnused = 0, kDefaultStream = 1, kElsewhere = 2 };
 
 constexpr size_t kPoolBytes = (size_t)512 << 20;
 
-void pool_retain(int device);           // a context lives on `device`
+hipError_t pool_retain(int device);     // a context lives on `device`
 void pool_release(int device);          // ... and is gone
 
 // `block` receives the size to hand back with the pointer.  `first_use`: where the caller writes it first.

@@ -1,11 +1,12 @@
-// pool.hip - see pool.h.  Host code only.  Callers have made `device` current.
+// pool.hip - see pool.h.  Host code only.  Callers have made `device` current.  The containers allocate, and these functions are
+// called from C entries: what they throw ends here, as hipErrorOutOfMemory or as a block or slot that is not kept.
 #include "pool.h"
 
 #include <deque>
 #include <list>
 #include <map>
 #include <mutex>
-#include <vector>
+#include <new>
 
 namespace cybq {
 
@@ -26,8 +27,7 @@ struct DevicePool {
     int contexts = 0;
     std::list<Block> blocks;                            // oldest first
     size_t held = 0;
-    std::deque<ScanSlot> scans;                         // free slots, the longest free first
-    std::vector<void*> slabs;                           // pinned memory behind the words; kept for the process
+    std::deque<ScanSlot> scans;                         // free slots, the longest free first (their pinned memory is kept for the process)
 };
 
 DevicePool& pool_of(int device)
@@ -47,11 +47,14 @@ void empty(DevicePool& pool)                            // pool.m held
 
 }  // namespace
 
-void pool_retain(int device)
-{
+hipError_t pool_retain(int device)
+try {
     DevicePool& pool = pool_of(device);
     std::lock_guard<std::mutex> lock(pool.m);
     pool.contexts++;
+    return hipSuccess;
+} catch (const std::bad_alloc&) {
+    return hipErrorOutOfMemory;
 }
 
 void pool_release(int device)
@@ -102,7 +105,12 @@ void pool_free(int device, void* p, size_t block, UsedOn used_on)
         (void)hipFree(p);
         return;
     }
-    pool.blocks.push_back({p, block, used_on});
+    try {
+        pool.blocks.push_back({p, block, used_on});
+    } catch (const std::bad_alloc&) {
+        (void)hipFree(p);
+        return;
+    }
     pool.held += block;
     while (pool.held > kPoolBytes) {
         (void)hipFree(pool.blocks.front().p);
@@ -112,23 +120,26 @@ void pool_free(int device, void* p, size_t block, UsedOn used_on)
 }
 
 hipError_t scan_acquire(int device, ScanSlot* s)
-{
+try {
     DevicePool& pool = pool_of(device);
     std::lock_guard<std::mutex> lock(pool.m);
     if (pool.scans.empty()) {
         void* slab = nullptr;
+        std::deque<ScanSlot> fresh(kScanWords);
         hipError_t e = hipHostMalloc(&slab, kScanWords * kScanPitch * sizeof(uint32_t), hipHostMallocDefault);
         if (e != hipSuccess) return e;
-        pool.slabs.push_back(slab);
-        for (size_t i = 0; i < kScanWords; i++) pool.scans.push_back({static_cast<uint32_t*>(slab) + i * kScanPitch, nullptr});
+        for (size_t i = 0; i < kScanWords; i++) fresh[i].word = static_cast<uint32_t*>(slab) + i * kScanPitch;
+        pool.scans.swap(fresh);
     }
-    ScanSlot got = pool.scans.front();
+    ScanSlot& got = pool.scans.front();
     // (events are made as slots are first used, and stay with them; a slot given back ahead of its kernel is waited for)
     const hipError_t e = got.done ? hipEventSynchronize(got.done) : hipEventCreateWithFlags(&got.done, hipEventDisableTiming);
     if (e != hipSuccess) return e;
-    pool.scans.pop_front();
     *s = got;
+    pool.scans.pop_front();
     return hipSuccess;
+} catch (const std::bad_alloc&) {
+    return hipErrorOutOfMemory;
 }
 
 void scan_release(int device, ScanSlot s)
@@ -136,7 +147,10 @@ void scan_release(int device, ScanSlot s)
     if (!s.word) return;
     DevicePool& pool = pool_of(device);
     std::lock_guard<std::mutex> lock(pool.m);
-    pool.scans.push_back(s);
+    try {
+        pool.scans.push_back(s);
+    } catch (const std::bad_alloc&) {
+    }
 }
 
 }  // namespace cybq
