@@ -81,6 +81,7 @@ def load_library() -> ctypes.CDLL:
     lib.cybq_weight_from_device.argtypes = [vp, ci, i64, i64, vp, vp, vp, ctypes.POINTER(vp)]
     lib.cybq_weight_clone.argtypes = [vp, vp, ctypes.POINTER(vp)]
     lib.cybq_weight_free.argtypes = [vp, vp]
+    lib.cybq_trim.argtypes = [vp]
     lib.cybq_weight_info.argtypes = [vp, ctypes.POINTER(ci), ctypes.POINTER(i64), ctypes.POINTER(i64),
                                      ctypes.POINTER(i64)]
     lib.cybq_matmul.argtypes = [vp, vp, vp, ci, i64, vp, ci, vp]
@@ -344,6 +345,10 @@ class Backend:
         if name is not None:
             self.weights[name] = w
         return w
+
+    def trim(self) -> None:
+        """cybq_trim: the device memory of freed weights (up to 512 MiB are kept for the next ones) back to the device."""
+        self._check(self._lib.cybq_trim(self._ctx))
 
     # ---- ops (x / y / out: torch tensors on this device, or raw device addresses)
     def _check_tensor(self, t, what: str, elems: int) -> None:

@@ -433,6 +433,16 @@ int cybq_weight_free(cybq_ctx* ctx, cybq_weight* w)
     return CYBQ_OK;
 }
 
+int cybq_trim(cybq_ctx* ctx)
+{
+    if (!ctx) return CYBQ_ERR_INVALID;
+    DeviceGuard guard(ctx->device);
+    if (guard.err != hipSuccess) return fail_hip(ctx, guard.err, "hipSetDevice");
+    const hipError_t e = cybq::pool_trim(ctx->device);
+    if (e != hipSuccess) return fail_hip(ctx, e, "hipFree");
+    return CYBQ_OK;
+}
+
 int cybq_weight_info(const cybq_weight* w, int* quant, int64_t* N, int64_t* K, int64_t* device_bytes)
 {
     if (!w) return CYBQ_ERR_INVALID;

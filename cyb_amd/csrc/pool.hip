@@ -38,11 +38,16 @@ DevicePool& pool_of(int device)
     return (*pools)[device];
 }
 
-void empty(DevicePool& pool)                            // pool.m held
+hipError_t empty(DevicePool& pool)                      // pool.m held
 {
-    for (const Block& b : pool.blocks) (void)hipFree(b.p);
+    hipError_t first = hipSuccess;
+    for (const Block& b : pool.blocks) {
+        const hipError_t e = hipFree(b.p);
+        if (first == hipSuccess) first = e;
+    }
     pool.blocks.clear();
     pool.held = 0;
+    return first;
 }
 
 }  // namespace
@@ -61,7 +66,7 @@ void pool_release(int device)
 {
     DevicePool& pool = pool_of(device);
     std::lock_guard<std::mutex> lock(pool.m);
-    if (--pool.contexts == 0) empty(pool);
+    if (--pool.contexts == 0) (void)empty(pool);
 }
 
 hipError_t pool_alloc(int device, size_t bytes, UsedOn first_use, void** p, size_t* block)
@@ -89,7 +94,7 @@ hipError_t pool_alloc(int device, size_t bytes, UsedOn first_use, void** p, size
     hipError_t e = hipMalloc(p, bytes);
     if (e == hipErrorOutOfMemory && !pool.blocks.empty()) {
         (void)hipGetLastError();
-        empty(pool);
+        (void)empty(pool);
         e = hipMalloc(p, bytes);
     }
     *block = bytes;
@@ -117,6 +122,13 @@ void pool_free(int device, void* p, size_t block, UsedOn used_on)
         pool.held -= pool.blocks.front().bytes;
         pool.blocks.pop_front();
     }
+}
+
+hipError_t pool_trim(int device)
+{
+    DevicePool& pool = pool_of(device);
+    std::lock_guard<std::mutex> lock(pool.m);
+    return empty(pool);
 }
 
 hipError_t scan_acquire(int device, ScanSlot* s)

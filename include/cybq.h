@@ -146,9 +146,16 @@ int cybq_weight_upload_many(cybq_ctx* ctx, int64_t count, const int* quant, cons
 /* A second device copy of the same tensor at a different address (used by
  * benchmarks to stream more bytes than the last-level cache holds). */
 int cybq_weight_clone(cybq_ctx* ctx, const cybq_weight* src, cybq_weight** out);
+/* Takes the handle back.  Does not wait: calls that were queued before it may still be reading the weight.  The device memory
+ * stays with the library for the next tensors of that device (model switches and imports would otherwise wait for the device
+ * once per tensor): at most 512 MiB of it, until the device's last context is destroyed, until an allocation of the
+ * library's own fails, or until cybq_trim.  A caller that wants the memory for itself after unloading a model calls that. */
 int cybq_weight_free(cybq_ctx* ctx, cybq_weight* w);
+/* Gives the memory of freed weights that the library keeps on the context's device back to the device.  Waits for the device. */
+int cybq_trim(cybq_ctx* ctx);
 /* any of the out pointers may be NULL.  device_bytes = bytes the tensor
- * occupies in HBM (with padding of N to 16 and K to 128). */
+ * occupies in HBM (with padding of N to 16 and K to 128); memory taken over from a freed weight may be up to a
+ * quarter larger, until that weight is freed in turn. */
 int cybq_weight_info(const cybq_weight* w, int* quant, int64_t* N, int64_t* K,
                      int64_t* device_bytes);
 

@@ -116,7 +116,9 @@ public:
         if (s) weights_[name] = std::move(w);
         return s;
     }
+    // (the memory stays with the library for the next tensors; trim() gives it back to the device)
     void unload(const std::string& name) { weights_.erase(name); }
+    Status trim() { return wrap(cybq_trim(ctx_)); }
     const Weight* find(const std::string& name) const
     {
         auto it = weights_.find(name);

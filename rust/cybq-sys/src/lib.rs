@@ -64,6 +64,7 @@ extern "C" {
                                    scales: *const *const c_void, out: *mut *mut cybq_weight) -> c_int;
     pub fn cybq_weight_clone(ctx: *mut cybq_ctx, src: *const cybq_weight, out: *mut *mut cybq_weight) -> c_int;
     pub fn cybq_weight_free(ctx: *mut cybq_ctx, w: *mut cybq_weight) -> c_int;
+    pub fn cybq_trim(ctx: *mut cybq_ctx) -> c_int;
     pub fn cybq_weight_info(w: *const cybq_weight, quant: *mut c_int, N: *mut i64, K: *mut i64,
                             device_bytes: *mut i64) -> c_int;
 

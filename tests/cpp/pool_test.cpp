@@ -125,6 +125,13 @@ int main()
     CHECK(in_use == before - na);
     CHECK(scan_acquire(0, &s[2]) == hipSuccess);
 
+    // everything kept goes back when asked
+    CHECK(pool_alloc(0, 4 * MB, kDefaultStream, &a, &na) == hipSuccess && pool_alloc(0, 5 * MB, kDefaultStream, &b, &nb) == hipSuccess);
+    pool_free(0, a, na, kElsewhere);
+    CHECK(pool_trim(0) == hipSuccess && in_use == nb);
+    pool_free(0, b, nb, kUnused);
+    CHECK(pool_trim(0) == hipSuccess && pool_trim(0) == hipSuccess && in_use == 0);
+
     // the last context takes everything with it; what is freed later goes back at once
     CHECK(pool_alloc(0, 4 * MB, kDefaultStream, &a, &na) == hipSuccess && pool_alloc(0, 4 * MB, kDefaultStream, &b, &nb) == hipSuccess);
     pool_free(0, a, na, kElsewhere);

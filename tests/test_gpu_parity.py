@@ -2066,6 +2066,30 @@ def test_first_call_of_a_kernel_may_sit_inside_a_capture(oracle):
         be.close()
 
 
+def test_trim_gives_the_memory_of_freed_weights_back(backend):
+    """A program that unloads a model and wants the memory for something else gets it: what the library keeps for the
+    next tensors is bounded, and cybq_trim hands it to the device."""
+    N, K = 16384, 8192                                           # 75.5 MB packed
+    qd = torch.zeros(N * K // 2, dtype=torch.uint8, device="cuda")
+    sd = torch.zeros(N * (K // 32), dtype=torch.int16, device="cuda")
+    torch.cuda.synchronize()
+    backend.trim()
+    free0 = torch.cuda.mem_get_info()[0]
+    ws = [backend.weight_from_device(4, N, K, qd, sd) for _ in range(9)]
+    assert torch.cuda.mem_get_info()[0] <= free0 - 9 * ws[0].device_bytes
+    for w in ws:
+        w.free()
+    assert torch.cuda.mem_get_info()[0] >= free0 - (512 << 20) - (16 << 20)
+    backend.trim()
+    assert torch.cuda.mem_get_info()[0] >= free0 - (16 << 20)    # (the runtime's own bookkeeping may move)
+    w = backend.weight_from_device(4, N, K, qd, sd)              # and the next tensor is made as ever
+    out = torch.full((N, K), 1.0, device="cuda")
+    backend.dequant(w, out)
+    torch.cuda.synchronize()
+    assert not out.any()
+    w.free()
+
+
 def test_a_weight_is_not_made_on_a_capturing_stream(backend):
     """Also where nothing has to be allocated for it (the memory and the scan word of a weight freed before): the recorded repack
     would not have run when the call returns.  The capture goes on, and the first prefill call of a weight made outside of it may
