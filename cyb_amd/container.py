@@ -27,6 +27,7 @@ from typing import Dict, List, Optional, Tuple
 import numpy as np
 
 from . import formats
+from .backend import CybqError
 
 try:
     import tomllib as _toml          # Python >= 3.11
@@ -245,21 +246,31 @@ class Container:
         return q, None
 
 
+def _upload_batch(backend, batch) -> None:
+    """All tensors in one call; where that fails (it is all or nothing, and a model that replaces another needs the batch's memory
+    on top of it) one by one: what comes before a bad tensor is loaded, and a replaced tensor's memory serves the next."""
+    try:
+        backend.upload_many(batch)
+    except CybqError:
+        for tensor in batch:
+            backend.upload(*tensor)
+
+
 def load_into(backend, path: str) -> List[TensorRecord]:
-    """Uploads every quantised tensor of a container into `backend.weights` by name."""
+    """Uploads every quantised tensor of a container into `backend.weights` by name, in the container's order."""
     c = Container(path)
     try:
         recs = c.tensors()
-        # a few hundred MB per call: enough to keep the bus busy across tensors, and a model that replaces one of the
-        # same tensor names needs that much device memory on top, not twice its size
+        # a few hundred MB per call: enough to keep the bus busy across tensors, and not twice the model's memory where it
+        # replaces one of the same tensor names
         batch, held = [], 0
         for r in recs:
             batch.append((r.bits, r.layout_code, r.shape[0], r.shape[1], *c.payload(r), r.name))
             held += r.nbytes + r.scales_nbytes
             if held >= LOAD_BATCH_BYTES:
-                backend.upload_many(batch)
+                _upload_batch(backend, batch)
                 batch, held = [], 0
-        backend.upload_many(batch)
+        _upload_batch(backend, batch)
         return recs
     finally:
         c.close()

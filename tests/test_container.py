@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from cyb_amd import container, formats, synth
+from cyb_amd.backend import CybqError
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HOST_TEST = os.path.join(ROOT, "tests", "cpp", "_build", "host_test")
@@ -20,6 +21,45 @@ def _entries():
             [container.tensor_entry("model.layers.0.mlp.up_proj.weight", q4, s4, 4, formats.BLOCK_AOS),
              container.tensor_entry("model.layers.0.mlp.down_proj.weight", q8, s8, 8, formats.PLANAR),
              container.tensor_entry("model.layers.0.self_attn.q_proj.weight", q4, s4, 4, formats.PLANAR)])
+
+
+class _Library:
+    """The loading side of a Backend: refuses tensors named `bad`, and lists with one among them or of more than `room`."""
+
+    def __init__(self, bad=(), room=99):
+        self.bad, self.room, self.weights, self.calls = bad, room, {}, []
+
+    def upload(self, quant, layout, N, K, q, scales=None, name=None):
+        if name in self.bad:
+            raise CybqError(-6, "out of memory")
+        self.weights[name] = (quant, layout, N, K, bytes(q), None if scales is None else bytes(scales))
+
+    def upload_many(self, tensors):
+        self.calls.append(len(tensors))
+        if len(tensors) > self.room or any(t[6] in self.bad for t in tensors):
+            raise CybqError(-6, "out of memory")
+        for t in tensors:
+            self.upload(*t)
+
+
+@pytest.mark.parametrize("batch_bytes", [1, 5000, 512 << 20])
+def test_a_load_that_fails_leaves_the_tensors_before_the_bad_one(tmp_path, monkeypatch, batch_bytes):
+    ents = _entries()[4]
+    path = str(tmp_path / "tiny.model")
+    container.write_container(path, "tiny", "", ents)
+    names = [e["name"] for e in ents]
+    monkeypatch.setattr(container, "LOAD_BATCH_BYTES", batch_bytes)
+    whole = _Library()
+    assert [r.name for r in container.load_into(whole, path)] == names == list(whole.weights)
+    for i, bad in enumerate(names):
+        lib = _Library(bad=(bad,))
+        with pytest.raises(CybqError):
+            container.load_into(lib, path)
+        assert list(lib.weights) == names[:i]
+    # no room for a list: its tensors are loaded one by one
+    lib = _Library(room=1)
+    container.load_into(lib, path)
+    assert lib.weights == whole.weights and max(whole.calls) == max(lib.calls)
 
 
 def test_round_trip(tmp_path):

@@ -2090,6 +2090,29 @@ def test_trim_gives_the_memory_of_freed_weights_back(backend):
     w.free()
 
 
+def test_upload_of_a_list_that_fails_half_way_leaves_nothing(backend):
+    """The second tensor of the list asks for more memory than any device has (its source is never read): the first one's memory
+    comes back, no handle is left, and the library goes on."""
+    import ctypes
+    N, K = 1024, 4096
+    blocks = np.zeros(N * (K // 32) * 18, np.uint8)
+    backend.trim()
+    free0 = torch.cuda.mem_get_info()[0]
+    two = lambda t, *v: (t * 2)(*v)
+    out = two(ctypes.c_void_p, 1, 1)
+    rc = backend._lib.cybq_weight_upload_many(backend._ctx, 2, two(ctypes.c_int, 4, 4), two(ctypes.c_int, 1, 1), two(ctypes.c_int64, N, 1 << 20),
+                                              two(ctypes.c_int64, K, 1 << 20), two(ctypes.c_void_p, blocks.ctypes.data, blocks.ctypes.data), None, out)
+    assert rc == -6 and not out[0] and not out[1]
+    backend.trim()
+    assert torch.cuda.mem_get_info()[0] >= free0 - (1 << 20)
+    w = backend.upload(4, formats.BLOCK_AOS, N, K, blocks)
+    y = torch.ones((N, K), device="cuda")
+    backend.dequant(w, y)
+    torch.cuda.synchronize()
+    assert not y.any()
+    w.free()
+
+
 def test_a_weight_is_not_made_on_a_capturing_stream(backend):
     """Also where nothing has to be allocated for it (the memory and the scan word of a weight freed before): the recorded repack
     would not have run when the call returns.  The capture goes on, and the first prefill call of a weight made outside of it may
