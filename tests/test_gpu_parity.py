@@ -2090,6 +2090,53 @@ def test_trim_gives_the_memory_of_freed_weights_back(backend):
     w.free()
 
 
+@pytest.mark.parametrize("first", ["default", "side"])
+@pytest.mark.parametrize("then", ["default", "side", "host"])
+def test_a_freed_weight_s_memory_waits_for_the_work_that_reads_it(backend, first, then):
+    """A weight is freed while milliseconds of calls that read it are queued, and the next one (made on the same stream, on
+    another, or from host memory) gets its memory: the queued calls still see the old tensor, later ones the new one."""
+    N, K, calls = 28672, 4096, 300
+    packed = []
+    for seed in (1, 2):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        w = torch.empty((N, K), device="cuda").normal_(0.0, 0.02, generator=g)
+        qd = torch.empty(N * K // 2, dtype=torch.uint8, device="cuda")
+        sd = torch.empty(N * (K // 32), dtype=torch.int16, device="cuda")
+        backend.quantize(4, w, N, K, qd, sd)
+        packed.append((qd, sd))
+    host = [t.cpu().numpy() for t in packed[1]]
+    x = torch.empty((1, K), device="cuda").normal_().to(torch.float16)
+    want = []
+    for qd, sd in packed:                                        # each tensor alone, nothing shared
+        w = backend.weight_from_device(4, N, K, qd, sd)
+        want.append(torch.empty((1, N), device="cuda"))
+        backend.matmul(w, x, want[-1])
+        torch.cuda.synchronize()
+        w.free()
+        backend.trim()
+    y = torch.zeros((calls, N), device="cuda")
+    late = torch.zeros((1, N), device="cuda")
+    rows = [y[i:i + 1] for i in range(calls)]
+    side = [torch.cuda.Stream(), torch.cuda.Stream()]
+    st = [0 if s == "default" else side[i].cuda_stream for i, s in enumerate((first, then))]
+    torch.cuda.synchronize()
+    old = backend.weight_from_device(4, N, K, *packed[0], stream=st[0])
+    free1 = torch.cuda.mem_get_info()[0]
+    for r in rows:
+        backend.matmul(old, x, r, stream=st[0])
+    old.free()
+    if then == "host":
+        new = backend.upload(4, formats.PLANAR, N, K, host[0], host[1].view(np.uint16))
+    else:
+        new = backend.weight_from_device(4, N, K, *packed[1], stream=st[1])
+    backend.matmul(new, x, late, stream=0 if then == "host" else st[1])
+    torch.cuda.synchronize()
+    assert torch.cuda.mem_get_info()[0] >= free1 - (32 << 20)    # (no second tensor's worth was allocated)
+    assert torch.equal(y, want[0].expand(calls, N))
+    assert torch.equal(late, want[1])
+    new.free()
+
+
 def test_upload_of_a_list_that_fails_half_way_leaves_nothing(backend):
     """The second tensor of the list asks for more memory than any device has (its source is never read): the first one's memory
     comes back, no handle is left, and the library goes on."""
