@@ -593,30 +593,38 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ part, int splits,
     store_out_g(y, ydt, i, v);
 }
 
-// The same sum for N a multiple of four, four neighbouring elements of a row per thread.  The pass is latency: everything a
+// The same sum for N of four or more, four neighbouring elements of a row per thread.  The pass is latency: everything a
 // thread needs - its pieces of all the slabs, its residual, its row's factors - is requested before anything is used, and
 // the row is the workgroup's (blockIdx.y), not a division per element.  (Before: slab after slab, then four 64-bit
 // divisions, each in front of its own loads of the row's factor and the residual.)
 // 14336 -> 4096, bf16 rows with a residual, us per call with staging and multiply: 45 rows 36.5 -> 33.9, 128 rows 38.6 -> 36.9,
 // 512 rows 76.0 -> 74.1.
-template <int SPLITS, bool SWIGLU>
+// RAGGED: N is no multiple of four.  Rows start at any multiple of four bytes (which 128-bit loads and stores of floats take), and
+// the last thread of a row steps back to its last four elements and stores those that are its own.  us per call, against one
+// thread per element (with a 64-bit division each): 14336 -> 4090 at 512 rows 77.5 -> 74.9, -> 2050 at 256 rows 43.4 -> 40.7, with a norm
+// -> 4094 at 512 rows 81.9 -> 78.1, fp32 10240 -> 3507 at 444 rows 57.4 -> 54.8.
+typedef float4_t float4_any __attribute__((aligned(4)));
+
+template <int SPLITS, bool SWIGLU, bool RAGGED>
 __global__ __launch_bounds__(256) void splitk_reduce4_kernel(const float* __restrict__ part, int M, int N, void* __restrict__ y, int ydt,
                                                              float out_scale, Epilogue epi, NormStats ns, int K)
 {
     const int n_out = SWIGLU ? N >> 1 : N;
-    const int n = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4, m = blockIdx.y;
-    if (n >= n_out) return;
+    const int first = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4, m = blockIdx.y;
+    if (first >= n_out) return;
+    const int n = RAGGED ? min(first, n_out - 4) : first;
     const int64_t slab = (int64_t)M * N, at = (int64_t)m * n_out + n;
     // (a pair's 16 gate columns sit in front of its 16 up columns)
     const float* const p0 = part + (int64_t)m * N + (SWIGLU ? (n >> 4) * 32 + (n & 15) : n);
     float4_t g[SPLITS], u[SWIGLU ? SPLITS : 1];
 #pragma unroll
     for (int s = 0; s < SPLITS; s++) {
-        g[s] = *reinterpret_cast<const float4_t*>(p0 + s * slab);
+        if constexpr (RAGGED) g[s] = *reinterpret_cast<const float4_any*>(p0 + s * slab);
+        else g[s] = *reinterpret_cast<const float4_t*>(p0 + s * slab);
         if (SWIGLU) u[SWIGLU ? s : 0] = *reinterpret_cast<const float4_t*>(p0 + s * slab + 16);
     }
     const uintptr_t mask = ydt == kF32 ? 15u : 7u;
-    const bool aligned = ((reinterpret_cast<uintptr_t>(y) | (epi.kind == kEpiAdd ? reinterpret_cast<uintptr_t>(epi.residual) : 0u)) & mask) == 0;
+    const bool aligned = !RAGGED && ((reinterpret_cast<uintptr_t>(y) | (epi.kind == kEpiAdd ? reinterpret_cast<uintptr_t>(epi.residual) : 0u)) & mask) == 0;
     float4_t res = {0.f, 0.f, 0.f, 0.f};
     if (epi.kind == kEpiAdd) {
         if (!aligned) {
@@ -654,9 +662,12 @@ __global__ __launch_bounds__(256) void splitk_reduce4_kernel(const float* __rest
             }
         }
     }
-    if (!aligned) {
+    if (RAGGED && ydt == kF32 && n == first) {
+        *reinterpret_cast<float4_any*>(static_cast<float*>(y) + at) = v;
+    } else if (!aligned) {
 #pragma unroll
-        for (int e = 0; e < 4; e++) store_out_g(y, ydt, at + e, v[e]);
+        for (int e = 0; e < 4; e++)
+            if (!RAGGED || n + e >= first) store_out_g(y, ydt, at + e, v[e]);
     } else if (ydt == kF32) {
         *reinterpret_cast<float4_t*>(static_cast<float*>(y) + at) = v;
     } else {
@@ -671,13 +682,13 @@ __global__ __launch_bounds__(256) void splitk_reduce4_kernel(const float* __rest
     }
 }
 
-template <bool SWIGLU>
+template <bool SWIGLU, bool RAGGED>
 hipError_t launch_reduce4(const float* part, int splits, int M, int N, void* y, int ydt, float out_scale, const Epilogue& epi, const NormStats& ns,
                           int K, hipStream_t st)
 {
-    const dim3 grid((unsigned)(((SWIGLU ? N / 2 : N) / 4 + 255) / 256), (unsigned)M);
+    const dim3 grid((unsigned)(((SWIGLU ? N / 2 : N) + 1023) / 1024), (unsigned)M);
     auto go = [&](auto count) {
-        hipLaunchKernelGGL((splitk_reduce4_kernel<decltype(count)::value, SWIGLU>), grid, dim3(256), 0, st, part, M, N, y, ydt, out_scale, epi, ns, K);
+        hipLaunchKernelGGL((splitk_reduce4_kernel<decltype(count)::value, SWIGLU, RAGGED>), grid, dim3(256), 0, st, part, M, N, y, ydt, out_scale, epi, ns, K);
         return hipGetLastError();
     };
     switch (splits) {
@@ -697,8 +708,9 @@ hipError_t launch_reduce(const float* part, int splits, int M, int N, void* y, i
                          int K, hipStream_t st)
 {
     const bool rows_fit = M <= 65535;          // the grid's second dimension
-    if (rows_fit && epi.kind == kEpiSwiglu) return launch_reduce4<true>(part, splits, M, N, y, ydt, out_scale, epi, ns, K, st);
-    if (rows_fit && N % 4 == 0) return launch_reduce4<false>(part, splits, M, N, y, ydt, out_scale, epi, ns, K, st);
+    if (rows_fit && epi.kind == kEpiSwiglu) return launch_reduce4<true, false>(part, splits, M, N, y, ydt, out_scale, epi, ns, K, st);
+    if (rows_fit && N % 4 == 0) return launch_reduce4<false, false>(part, splits, M, N, y, ydt, out_scale, epi, ns, K, st);
+    if (rows_fit && N > 4) return launch_reduce4<false, true>(part, splits, M, N, y, ydt, out_scale, epi, ns, K, st);
     const int64_t total = (int64_t)M * N;
     hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, part, splits, M, N, y, ydt, out_scale, epi, ns, K);
     return hipGetLastError();

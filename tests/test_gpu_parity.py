@@ -785,6 +785,38 @@ def test_prefill_few_tiles_split_k(backend, oracle, prefill_mode, bits, shape):
             assert torch.equal(_run(backend, qw, x, ydt), y.to(TDT[ydt]))   # rounded once
 
 
+# rows that are no multiple of four elements: the slab-adding pass steps back at the end of a row (its smallest row, one thread, several
+# workgroups); outputs at any element, in place, and with a factor per row
+@pytest.mark.parametrize("N", [3, 5, 1001, 4090])
+@pytest.mark.parametrize("ydt", ["f32", "f16", "bf16"])
+def test_prefill_split_k_on_ragged_rows(backend, oracle, N, ydt):
+    M, K, dt = 257, 8320, TDT[ydt]
+    q, s = _quant(oracle, 4, N, K, cfg=53)
+    qw = backend.upload_quantized(q, s, 4)
+    wd = torch.from_numpy(oracle.dequant(q, s)).cuda().double()
+    x = _x(M, K, "bf16", cfg=54)
+    gamma = torch.linspace(0.5, 1.5, K, device="cuda")
+    ref = x.double() @ wd.T
+    rstd = 1.0 / torch.sqrt((x.double() ** 2).mean(dim=1, keepdim=True) + 1e-5)
+    normed = ((x.double() * gamma.double()) @ wd.T) * rstd
+    bar = FAST + {"f32": 0.0, "f16": 5e-4, "bf16": 4e-3}[ydt]          # (one rounding of the result)
+    for off in (0, 1):                                                  # y and the residual at an odd element of their buffers
+        room = torch.full((M * N + 9,), 7.0, dtype=dt, device="cuda")
+        y = room[off:off + M * N].view(M, N)
+        backend.matmul(qw, x, y)
+        assert ((y.double() - ref).norm() / ref.norm()).item() < bar
+        r = y.clone()
+        backend.matmul_ex(qw, x, y, "add", y)                           # in place: r + x W^T
+        want = r.double() + ref
+        assert ((y.double() - want).norm() / want.norm()).item() < bar
+        if ydt == "f32":
+            assert torch.equal(y, r + r)
+        backend.matmul_norm(qw, x, gamma, 1e-5, y)
+        assert ((y.double() - normed).norm() / normed.norm()).item() < bar + 2e-4      # (x * gamma rounded to f16)
+        assert (room[:off] == 7.0).all() and (room[off + M * N:] == 7.0).all()
+    qw.free()
+
+
 def test_prefill_more_rows_than_the_stage_holds(backend, oracle, prefill_mode):
     # 4200 x 16384 activations are 131 MiB: they pass through the 128 MiB staging area
     # in two row chunks
