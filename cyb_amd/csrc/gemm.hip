@@ -1215,13 +1215,16 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
             // per-row scaled f16 operands; one sum of squares per row
             ns = NormStats{ssq_part, 1, unscale};
             // Rows per workgroup of sixteen waves: with few of them one workgroup per four rows leaves the chip idle and a
-            // row's waves walk it piece after piece.  us per call, 4 / 2 / 1 rows (bf16): 14336 -> 4096 at 45 rows 26.4 /
-            // 24.8 / 24.0, 128 rows 37.2 / 34.3 / 33.7, 512 rows 73.4 / 72.8 / 78.0; 14336 -> 1024, fp32, 256 rows 33.3 /
-            // 30.0 / 33.2 (10240 -> 3507, fp32, 444 rows: 64.3 / 64.9 with four / two); 4096 -> 6144 with a norm at 45 rows 14.6 / 13.0 / 12.9, 4096 -> 4096 at 45 rows 12.1 / 11.3 /
-            // 11.3; 4096 -> 14336 at 64 / 128 rows 19.4 / 19.4 / 19.9, 27.5 / 28.4 / 28.5.  (The fewer rows, the shorter
-            // the runs in which the operands leave: 64, 32, 16 bytes.)
-            // (4096 -> 6144 with a norm: four rows, one order of its sums.)
-            const int stage_rows = epi.gamma ? 4 : w.K > 8192 ? (mc <= 128 ? 1 : mc <= 256 || (mc <= 512 && w.K > 12288) ? 2 : 4) : (mc <= 48 ? 2 : 4);
+            // row's waves walk it piece after piece; with many, the shorter runs in which the operands leave cost more (64, 32, 16
+            // bytes).  us per call, 4 / 2 / 1 rows, bf16 unless noted.  K over 8192: 14336 -> 4096 at 45 rows 28.0 / 26.5 / 25.8, 128 rows
+            // 39.6 / 37.1 / 35.8, 160 rows 49.3 / 47.9 / 47.4, 256 rows 47.3 / 45.9 / 47.5, 300 rows 66.5 / 64.7 / 67.3, 384 rows 68.3 / 67.8 /
+            // 70.9, 448 rows 69.5 / 69.6 / 73.9, 512 rows 72.6 / 73.4 / 78.6; 9216 -> 4096 at 300 / 384 rows 48.9 / 47.5 / 48.8, 49.9 / 49.4 / 51.2;
+            // 10240 -> 4096 at 384 rows 53.4 / 52.9 / 54.9; 14336 -> 1024 at 384 / 512 rows 39.6 / 40.4 / 42.0, 38.0 / 39.5 / 44.6; fp32 (twice the bytes to a row), 4 / 2 rows, 14336 -> 4096 at
+            // 512 / 640 rows 76.0 / 74.4, 106.9 / 107.4, 10240 -> 14336 and 9216 -> 4096 at 512 rows 134.0 / 132.8, 54.6 / 54.3.  Shorter K:
+            // 8192 -> 4096 at 45 rows 18.7 / 17.2 / 17.1, at 64 rows 21.4 / 20.0 / 19.8, at 100 rows 21.8 / 21.6 / 21.6; 4096 -> 4096 at 45 rows
+            // 11.2 / 10.9 / 11.3, fp32 at 24 rows 10.5 / 10.1 / 10.4; 4096 -> 14336 at 45 / 64 rows 17.2 / 17.2 / 17.6, 18.8 / 19.0 / 19.4.
+            // (A folded norm: always four, one order of its sums.)
+            const int stage_rows = epi.gamma ? 4 : w.K > 8192 ? (mc <= 128 ? 1 : mc <= (xdt == kF32 ? 512 : 384) ? 2 : 4) : (mc <= 48 ? 2 : 4);
             dim3 rgrid((unsigned)((mc + 15) / 16) * (16 / stage_rows));
             const Touch touch = plan_touch(w, mc, num_cus, ec, exact, rgrid.x);
             // pieces of 512 k a lane keeps in registers: the whole row when it has at most 16384 (bf16) or 8192 (fp32)

@@ -268,7 +268,9 @@ hipError_t launch_rows_t(const WeightView& w, const void* x, int M, void* y, int
 // wider output are not K-split there.  us per call with all passes, against the tiled kernels (their adding pass included
 // before it was made quicker): 14336 -> 4096 bf16 at 45 / 64 / 96 / 128 rows 26.6 / 30.1 / 33.1 / 36.8 against 36.5 / 37.7 /
 // 39.0 / 39.8, fp32 at 24 rows 21.9 against 36.2, f16 at 45 rows 24.3 against 30.2; 14336 -> 8192 at 45 rows 36.2 against
-// 50.2; 14336 -> 1024 at 100 rows 24.1 against 34.5; 12288 -> 512, f16, 40 rows 26.2 both.
+// 50.2; 14336 -> 1024 at 100 rows 24.1 against 34.5 (23.4 against 27.6 with that pass as it is now), 12288 -> 512 at 100 / 128 rows
+// 17.3 / 21.6 against 22.0 / 24.7, 9216 -> 512 at 128 rows 15.1 against 18.6.  (Up to 64 rows of 16-bit activations on weights of up to
+// 6144 x 4096 are two decode passes and never get here.)
 RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
     if (M <= 16 || M > 512 || w.KT < 16) return {0, 0};

@@ -1136,6 +1136,19 @@ def test_prefill_row_scaling_pass_rows_per_workgroup(backend, oracle, K, xdt):
     qw.free()
 
 
+@pytest.mark.parametrize("xdt,M", [("bf16", 384), ("bf16", 385), ("f32", 512), ("f32", 513)])
+@pytest.mark.parametrize("K", [8192 + 32, 16384 + 64])
+def test_prefill_row_scaling_pass_where_two_rows_become_four(backend, oracle, K, xdt, M):
+    N = 48
+    q, s = _quant(oracle, 4, N, K, cfg=86)
+    qw = backend.upload_quantized(q, s, 4)
+    x = (_x(M, K, "f32", cfg=87) * torch.logspace(-6, 6, M, device="cuda")[:, None]).to(TDT[xdt])
+    ref = x.double() @ torch.from_numpy(oracle.dequant(q, s)).cuda().double().T
+    # (row by row; the bar of the test above)
+    assert ((_run(backend, qw, x).double() - ref).norm(dim=1) / ref.norm(dim=1)).max().item() < 2e-3
+    qw.free()
+
+
 @pytest.mark.parametrize("shape", [(14336, 4096, 17), (4096, 4096, 32), (8200, 2048 + 128, 24)])
 def test_prefill_fp32_rows_17_to_32_fast_mode(backend, oracle, shape):
     """fp32 activations leave the decode kernels at 17 rows; in FAST mode they are rounded to f16 by the staging
