@@ -529,5 +529,6 @@ class Backend:
 
     def set_gemv_tuning(self, waves: int = 0, rows_kernel: int = 0, unroll: int = 0) -> None:
         """Diagnostics: waves per workgroup; decode kernel choice (0 auto, 1 always the
-        x-in-registers kernel, 2 never); streaming batch size.  0 = automatic."""
+        x-in-registers kernel, 2 never, 3 / 4 always, its K split never / from three rows on, 5 automatic without
+        the workgroups that stay); streaming batch size.  0 = automatic."""
         self._lib.cybq_debug_set_gemv_tuning(waves, rows_kernel, unroll)

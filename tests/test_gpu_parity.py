@@ -324,6 +324,43 @@ def test_a_row_keeps_its_bits_from_3_to_32_rows(backend, bits, N, K, pair, xdt):
         backend.set_decode_mode("stream")
 
 
+# with the same operands (f16 rows and exact integers; Q8) the staying workgroups and the batched-rows kernel (decode tuning 5: the
+# former never) give the same bits: every epilogue and output type, a folded norm where both load the rows alike
+# (Q4 bf16 rows: another order of sums; the test above has the shapes that the kernels share)
+@pytest.mark.parametrize("xdt,bits,N,K", [("f16", 4, 6144, 4096), ("f16", 4, 10241, 3104), ("f16", 4, 8192, 2560), ("f16", 4, 6160, 2048),
+                                          ("f16", 4, 6149, 1056)] + [(t, 8, n, k) for t in ("f16", "bf16")
+                                                                     for n, k in ((14336, 4096), (6149, 2080), (20480, 1792))])
+def test_staying_workgroups_against_the_batched_rows_kernel(backend, bits, N, K, xdt):
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    w = torch.empty((N, K), device="cuda").normal_(0.0, 0.02, generator=g)
+    qd = torch.empty(N * K * bits // 8, dtype=torch.uint8, device="cuda")
+    sd = torch.empty(N * (K // 32), dtype=torch.int16, device="cuda")
+    backend.quantize(bits, w, N, K, qd, sd)
+    qw = backend.weight_from_device(bits, N, K, qd, sd)
+    gamma = (1.0 + 0.25 * torch.empty(K, device="cuda").normal_(generator=g)).to(torch.float16)
+    try:
+        backend.set_decode_mode("exact")
+        for M in (5, 8, 9, 16, 17, 32):
+            x = torch.empty((M, K), device="cuda").normal_(generator=g).to(TDT[xdt])
+            for ydt in ("f32", "f16", "bf16"):
+                r = torch.empty((M, N), device="cuda").normal_(generator=g).to(TDT[ydt])
+                outs = []
+                for tuning in (0, 5):
+                    backend.set_gemv_tuning(0, tuning, 0)
+                    ys = [torch.full((M, N), float("nan"), dtype=TDT[ydt], device="cuda") for _ in range(3)]
+                    backend.matmul(qw, x, ys[0])
+                    backend.matmul_ex(qw, x, ys[1], "add", r)
+                    if M <= 16 and K > 1920:             # (four waves load up to 16 rows in one form)
+                        backend.matmul_norm(qw, x, gamma, 1e-5, ys[2])
+                    torch.cuda.synchronize()
+                    outs.append(ys)
+                for a, b in zip(*outs):
+                    assert torch.equal(a, b) or a.isnan().all() and b.isnan().all(), (M, ydt)
+    finally:
+        backend.set_gemv_tuning(0, 0, 0)
+        backend.set_decode_mode("stream")
+
+
 @pytest.mark.parametrize("N", [8192, 12288])
 def test_decode_modes_in_the_batched_rows_kernel(backend, oracle, N):
     """3 .. 32 f16 rows on outputs wide enough for two / four strips per workgroup: STREAM feeds the Q4
