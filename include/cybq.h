@@ -75,11 +75,11 @@ typedef enum cybq_layout { CYBQ_LAYOUT_PLANAR = 0, CYBQ_LAYOUT_BLOCK_AOS = 1 } c
 typedef enum cybq_dtype { CYBQ_F32 = 0, CYBQ_F16 = 1, CYBQ_BF16 = 2 } cybq_dtype;
 
 /* How the prefill kernels (M > 32; in FAST mode also 17 .. 32 rows of fp32 activations, or of 16-bit
- * activations with a folded RMSNorm, on weights with K of 2048 .. 8192) feed the matrix cores.  Both stay
- * inside the operator's 1e-3 relative-L2 tolerance.  (Calls of up to 16 rows, other calls of up to 32 rows,
- * and 33 .. 64 rows on weights of up to 6144 x 4096 that the FAST kernels do not take - always so with
- * CYBQ_PREFILL_EXACT, which gives them the decode kernels' EXACT operands - take the decode kernels, whose
- * operand form cybq_decode_mode describes.)
+ * activations with a folded RMSNorm on weights with K of 2048 .. 8192, unless the decode kernels have them in
+ * one pass, see cybq_matmul) feed the matrix cores.  Both stay inside the operator's 1e-3 relative-L2
+ * tolerance.  (Calls of up to 16 rows, other calls of up to 32 rows, and 33 .. 64 rows on weights of up to
+ * 6144 x 4096 that the FAST kernels do not take - always so with CYBQ_PREFILL_EXACT, which gives them the
+ * decode kernels' EXACT operands - take the decode kernels, whose operand form cybq_decode_mode describes.)
  *   FAST   (default) one f16 MFMA per 32-group; the weight operand is
  *          round_f16(scale * q), relative error <= 2^-11 per weight (about 2e-4
  *          relative L2 on y).  bf16 and fp32 activations become f16 operands behind a
@@ -94,18 +94,22 @@ typedef enum cybq_prefill_mode { CYBQ_PREFILL_FAST = 0, CYBQ_PREFILL_EXACT = 1 }
 /* How the decode kernels form their weight operands.  Every form accumulates in fp32, applies the
  * f16 group scale in fp32 and stays far inside the 1e-3 tolerance.  Which form runs:
  *   f16 activations   1 - 2 rows: STREAM -> subnormal operands, EXACT -> exact integers.
- *                     3 - 32 rows (and the 33 - 64-row walk): STREAM -> subnormal operands for Q4 on
- *                     outputs wide enough for two to four 16-row strips per workgroup, exact integers
- *                     otherwise; EXACT -> exact integers.
+ *                     3 - 32 rows (and the 33 - 64-row walk): EXACT -> exact integers.  STREAM -> subnormal
+ *                     operands for Q4 without a folded norm where the kernel that has the shape takes a
+ *                     weight tile's two to four 16-row strips together, exact integers otherwise (both well
+ *                     inside the tolerance; the kernel goes with N, K and the epilogue).
  *   bf16 activations  any row count, either mode: the bf16 numbers 128 + (q + bias) with the bias
  *                     removed inside the accumulation (bf16 has no packed add to take it off
  *                     beforehand); the mode only chooses the kernel for 1 - 2 rows.
  *   fp32 activations  exact integers in either mode (activations split into two f16 halves).
+ * A 16-bit row keeps its bits in any batch of 3 .. 32 rows on weights of N = 6144 .. 28656 and K = 928 .. 4096
+ * without a folded norm; elsewhere the kernel, and with it the last bits of a row, may change with the batch.
  *   STREAM (default) the packed nibbles / bytes are used straight from memory - as f16 subnormals
  *          (q + bias) * 2^-22 with f16 activations - and the bias is removed inside the same fp32
  *          accumulation; about 4e-7 (bf16: 1e-6) relative L2.  The sums carry the bias until it
  *          cancels: a tensor of zeros gives values around 1e-7 of the activations' scale, not exact
- *          zeros (the same holds for bf16 activations in either mode).  The quickest form.
+ *          zeros (the same holds for bf16 activations in either mode; where 3 - 32 f16 rows take
+ *          integers, see above, zeros are exact).  The quickest form.
  *   EXACT  the weight operand is the exact integer q (more unpack arithmetic per byte);
  *          about 3e-7 relative L2, and a tensor of zeros gives exact zeros. */
 typedef enum cybq_decode_mode { CYBQ_DECODE_STREAM = 0, CYBQ_DECODE_EXACT = 1 } cybq_decode_mode;
@@ -167,8 +171,9 @@ int cybq_weight_info(const cybq_weight* w, int* quant, int64_t* N, int64_t* K,
  *   x  [M,K] row-major, xdt in {F16,BF16,F32}, 16-byte aligned
  *   y  [M,N] row-major, ydt in {F32,F16,BF16} (fp32 accumulator rounded once)
  *   M >= 1.  M <= 32 runs the HBM-streaming decode kernels (17..32 rows of 16-bit
- *   activations: one pass with two row blocks; with a folded norm two passes of 16
- *   rows; 33..64 rows of 16-bit activations on a weight of up to 6144 x 4096
+ *   activations: one pass with two row blocks; with a folded norm that holds for f16
+ *   on outputs of 6144 or more with K of 928..1536 and 1952..3072, elsewhere it is two
+ *   passes of 16 rows or, in FAST mode, a prefill kernel; 33..64 rows of 16-bit activations on a weight of up to 6144 x 4096
  *   elements: two passes, 32 rows and the rest), larger M the LDS-tiled MFMA prefill kernel (fp32
  *   activations in CYBQ_PREFILL_EXACT mode: the decode kernel, 16 rows at a
  *   time; in FAST mode they are rounded once to f16 on the way in and take

@@ -292,7 +292,7 @@ def test_decode_rows_streamed_by_staying_workgroups(backend, bits, xdt, shape):
 @pytest.mark.parametrize("bits,N,K,pair", [(4, 14336, 4096, False), (4, 14341, 4064, False), (4, 8180, 3104, False), (4, 32000, 3200, False),
                                            (4, 28672, 4096, False), (4, 32784, 3200, False), (4, 10241, 3104, False), (4, 20480, 4096, True),
                                            (4, 6176, 3104, True), (4, 20480, 1792, True), (4, 6176, 1664, True), (8, 14336, 4096, False),
-                                           (8, 8224, 3104, True)])
+                                           (8, 8224, 3104, True), (4, 6144, 928, False), (4, 28640, 2048, True), (4, 28656, 4096, False), (8, 6144, 928, False)])
 @pytest.mark.parametrize("xdt", ["f16", "bf16"])
 def test_a_row_keeps_its_bits_from_3_to_32_rows(backend, bits, N, K, pair, xdt):
     g = torch.Generator(device="cuda").manual_seed(N + K)
