@@ -1,6 +1,6 @@
 // upload.hip - model load: interchange tensors in host memory -> native tiles in HBM.
 //
-// Bound by the host link (57 GB/s from pinned memory on the box this was measured on).  The source is pageable - a
+// Bound by the host link (57 GB/s from pinned memory where this was measured).  The source is pageable - a
 // mapped file, whose pages are also touched for the first time here - so somebody has to copy it into pinned memory:
 // one thread does that at 29 GB/s, four at 73, and the pages' faults are taken in parallel too.  The repack
 // kernel then reads the pinned slots itself: the bytes cross the bus once, coalesced, and leave the kernel as native
