@@ -523,8 +523,8 @@ class Backend:
         self._check(self._lib.cybq_debug_cache_read(self._ctx, _ptr(buf), nbytes, waves, in_flight, iters, stream))
 
     def set_gemm_tuning(self, rows_kernel: int = 0) -> None:
-        """Experiments only: 2 keeps prefill calls of up to 512 rows away from the K-splitting kernel, 1 sends
-        calls of up to 64 rows there whatever the output width, 0 restores the automatic choice."""
+        """Experiments only: 2 leaves FAST-mode prefill calls to the tiled kernels, 3 those of both modes, 1 sends calls of
+        up to 64 rows to the K-splitting kernel whatever the output width, 0 restores the automatic choice."""
         self._lib.cybq_debug_set_gemm_tuning(rows_kernel)
 
     def set_gemv_tuning(self, waves: int = 0, rows_kernel: int = 0, unroll: int = 0) -> None:

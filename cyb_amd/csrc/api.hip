@@ -496,12 +496,12 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
         if (e == hipSuccess) e = weight_is_wide(w, &is);
         return is;
     };
-    enum { kDecode, kTwoPasses, kPrefill, kWalk } way;
+    enum { kDecode, kTwoPasses, kPrefill, kPrefillExact, kWalk } way;
     if (M <= 16 || (M <= 32 && cybq::gemv_serves_32(v, (int)xdt, (int)M, ctx->num_cus, epi)))
         way = kDecode;
     else if (M <= 64 && (int64_t)w->N * w->K <= (int64_t)6144 * 4096 && cybq::gemv_serves_32(v, (int)xdt, 32, ctx->num_cus, epi) &&
              (ctx->prefill_exact || wide() || !cybq::gemm_rows_takes(v, (int)M, ctx->num_cus, epi)))
-        way = kTwoPasses;
+        way = (M > 32 && w->bits == 4 && xdt == CYBQ_BF16 && (w->K > 4096 || (w->K <= 512 && w->N >= 6144)) && !wide()) ? kPrefillExact : kTwoPasses;
     else if (!wide() && (xdt == CYBQ_F32 ? !ctx->prefill_exact : (M > 32 || (!ctx->prefill_exact && cybq::gemm_rows_takes(v, (int)M, ctx->num_cus, epi)))))
         way = kPrefill;
     else
@@ -520,10 +520,13 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
         e = cybq::launch_gemv(v, x, xdt, (int)M, y, ydt, ctx->num_cus, ctx->decode_exact, epi, dscr, dscr_bytes, st);
     } else if (way == kTwoPasses) {
         // 33..64 rows on a small weight (up to 4096 -> 6144) that the few-rows MFMA kernel does not take (exact
-        // mode, wide scales, K outside 2048 .. 8192, a folded SwiGLU): the tiled MFMA
-        // kernel would split K over workgroups and add the slabs in a second pass; two passes of the
-        // batched-rows decode kernel (32 rows, then the rest) are quicker although they stream the weights twice
-        // (4096 -> 4096 at 64 rows 21.8 -> 14.8 us; the few-rows kernel 13.1) - and exact
+        // mode, wide scales, K outside 2048 .. 8192): two passes of the batched-rows decode kernel (32 rows, then the rest) are
+        // quicker than a staging launch and a multiply although they stream the weights twice - and exact.  us per call, two passes
+        // / gemm_cols.hip with bf16 rows on Q4, at 33, 48, 64 rows: 4096 -> 4096 11.4, 12.6, 14.8 / 14.4, 14.9, 16.1, 2048 -> 6144 9.5, 9.6,
+        // 10.9 / 13.6, 14.1, 14.8.  Not with a longer K (8192 -> 512 15.0, 17.1, 20.6 / 12.7, 12.9, 13.3; 14336 -> 1024 25.9, 30.9, 38.0 /
+        // 16.9, 17.0, 17.9) nor with the shortest on a wide output (512 -> 14336 11.7, 15.8, 17.9 / 8.6, 8.8, 9.1): bf16 rows on Q4 go
+        // through the prefill path there, with exact operands whatever the mode (kPrefillExact; relative L2 against float64
+        // 7.6e-7 -> 2.2e-7; f16 rows 1.5e-7 -> 2.6e-7 and Q8 1.5e-7 -> 1.7e-6 stay).
         // (a context in CYBQ_PREFILL_EXACT mode asked for exact operands at this row count)
         const bool exact_ops = ctx->decode_exact || ctx->prefill_exact;
         const int64_t n_out = epi.kind == cybq::kEpiSwiglu ? w->N / 2 : w->N;
@@ -534,8 +537,8 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
         if (e == hipSuccess)
             e = cybq::launch_gemv(v, static_cast<const char*>(x) + (size_t)32 * w->K * dtype_size(xdt), xdt, (int)M - 32,
                                   static_cast<char*>(y) + yoff, ydt, ctx->num_cus, exact_ops, ec, dscr, dscr_bytes, st);
-    } else if (way == kPrefill) {
-        e = cybq::launch_gemm(v, x, xdt, (int)M, y, ydt, ctx->num_cus, ctx->prefill_exact, workspace, workspace_bytes,
+    } else if (way == kPrefill || way == kPrefillExact) {
+        e = cybq::launch_gemm(v, x, xdt, (int)M, y, ydt, ctx->num_cus, ctx->prefill_exact || way == kPrefillExact, workspace, workspace_bytes,
                               epi, st);
     } else {
         // fp32 activations keep full precision through the decode kernel's hi/lo split:

@@ -60,7 +60,17 @@ struct RowsPlan {
 RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi);
 hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, void* y, int ydt, const Epilogue& epi,
                             const float* ssq_part, int ssq_blocks, const float* unscale, const RowsPlan& plan, float* slabs, hipStream_t st);
-// test/bench hook: 2 = never take the few-rows kernel, 1 = whatever the width, 0 = automatic
+// the prefill kernel whose waves stand side by side along the columns (gemm_cols.hip).  mode: 0 FAST, 1 / 2 EXACT with f16 / bf16
+// operands; more than one split leaves fp32 slabs [splits][M][N] in `part` for the slab-adding pass
+struct ColsPlan {
+    int rb, cs, splits;      // row blocks of 16 per workgroup, strips per wave, workgroups that share out K (none of them empty)
+    float us;                // estimate of its time behind the staging pass
+};
+ColsPlan plan_gemm_cols(const WeightView& w, int mode, int M, int num_cus, size_t part_bytes);
+hipError_t launch_gemm_cols(const WeightView& w, const void* x_staged, int mode, int M, void* y, int ydt, const ColsPlan& plan, const Epilogue& epi,
+                            const float* ssq_part, int ssq_blocks, const float* unscale, float* part, hipStream_t st);
+// test/bench hook: 2 = in FAST mode the tiled kernels alone (neither the few-rows kernel nor gemm_cols.hip), 3 = in both modes,
+// 1 = the few-rows kernel whatever the width, 0 = automatic
 void set_gemm_tuning(int rows_kernel);
 // whether launch_gemm hands a FAST-mode call of M rows with this epilogue to the few-rows kernel (the hook included)
 bool gemm_rows_takes(const WeightView& w, int M, int num_cus, const Epilogue& epi);

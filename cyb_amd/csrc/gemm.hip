@@ -1,7 +1,7 @@
 // gemm.hip - prefill kernel: Y[M,N] = X[M,K] * W^T for M > 16 on MFMA.
 //
-// Workgroup = 8 or 4 waves, output tile 256 or 128 rows x (16*NF) columns; wave w owns
-// two row blocks of 16 against all NF column blocks.
+// Workgroup = 8 waves, output tile 256 (or 512) rows x (16*NF) columns; wave w owns
+// two (four) row blocks of 16 against all NF column blocks.  Fewer rows: gemm_rows.hip and gemm_cols.hip.
 //
 //   X  never touches LDS.  An MFMA A operand is 16 rows x 32 k with lane l
 //      holding row l%16, k 8*(l/16)..+8.  Read straight from a row-major X that is
@@ -48,6 +48,8 @@
 #include "cybq_internal.h"
 
 namespace cybq {
+
+int g_rows_kernel = 0;        // (set_gemm_tuning: 2 = the tiled kernels of this file alone in FAST mode, 3 = in both modes, 1 = the few-rows kernel whatever the width)
 
 namespace {
 
@@ -129,9 +131,9 @@ __device__ __forceinline__ void dequant_group_to_lds(const WRegs<BITS>& r, int j
 }
 
 // XBF = 1: X is bf16, 0: X is f16.  EXACT: see the header comment.
-// Wave wv of WAVES owns MF row blocks of 16 against all NF column blocks.
-template <int BITS, int XBF, int NF, bool EXACT, int MF, int WAVES>
-__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_kernel(const uint8_t* __restrict__ wbase, const u32x4_t* __restrict__ x, int KT_, int NT_, int x_row_blocks, int M,
+// Wave wv of eight owns MF row blocks of 16 against all NF column blocks.
+template <int BITS, int XBF, int NF, bool EXACT, int MF>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_kernel(const uint8_t* __restrict__ wbase, const u32x4_t* __restrict__ x, int KT_, int NT_, int x_row_blocks, int M,
                                                    int n_tiles, int m_tiles, int splits, int kt_per_split, int groups, int N_,
                                                    void* __restrict__ y, int ydt, int K_, float out_scale,
                                                    float* __restrict__ part, Epilogue epi, NormStats ns)
@@ -149,6 +151,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2
     const int split = item / (n_tiles * m_tiles);
     const int tile_m = (item - split * (n_tiles * m_tiles)) / n_tiles;
     const int tile_n = item - (split * m_tiles + tile_m) * n_tiles;
+    constexpr int WAVES = 8;
     constexpr int BM = WAVES * MF * 16;               // MF = row blocks (of 16) per wave
     constexpr int WT = (NF + WAVES - 1) / WAVES;      // weight tiles a wave stages per K tile
     constexpr int OPS = EXACT ? 2 : 1;                // B operands per scale group
@@ -281,8 +284,8 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2
         // spread between the MFMAs.  A wave issues in order: arithmetic queued behind a run of
         // MFMAs waits for all of them and the matrix pipe idles while it runs afterwards; and the
         // barrier keeps the two waves of a SIMD in the same phase, so they do not cover for each
-        // other.  (With one wave per SIMD, the 128-row shape, the same order measured slower.)
-        if constexpr (WAVES == 8 && !EXACT) {
+        // other.
+        if constexpr (!EXACT) {
             constexpr int READS = 4 * NF * OPS;
             __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);          // LDS reads run two ahead of their MFMAs
 #pragma unroll
@@ -716,123 +719,150 @@ hipError_t launch_reduce(const float* part, int splits, int M, int N, void* y, i
     return hipGetLastError();
 }
 
-template <int BITS, int XBF, int NF, bool EXACT, int MF, int WAVES>
-hipError_t launch_m(const WeightView& w, const void* x, int M, void* y, int ydt, float out_scale, float* part,
-                    size_t part_bytes, int num_cus, const Epilogue& epi, const NormStats& ns, hipStream_t st)
+template <int BITS, int XBF, int NF, bool EXACT, int MF>
+hipError_t launch_m(const WeightView& w, const void* x, int M, void* y, int ydt, float out_scale, float* part, int splits, const Epilogue& epi,
+                    const NormStats& ns, hipStream_t st)
 {
-    constexpr int BM = WAVES * MF * 16;
+    constexpr int BM = 8 * MF * 16;
     constexpr int lds = 2 * NF * (4 * (EXACT ? 2 : 1) * 64) * 16;     // operand buffers, 56 .. 128 KB
-    auto kern = gemm_kernel<BITS, XBF, NF, EXACT, MF, WAVES>;
-    (void)LdsRequest<&gemm_kernel<BITS, XBF, NF, EXACT, MF, WAVES>, lds>::registered;
+    auto kern = gemm_kernel<BITS, XBF, NF, EXACT, MF>;
+    (void)LdsRequest<&gemm_kernel<BITS, XBF, NF, EXACT, MF>, lds>::registered;
     const int n_tiles = (w.NT + NF - 1) / NF, m_tiles = (M + BM - 1) / BM;
-    // Too few tiles to fill the chip: split K over workgroups.  Every split adds its
-    // K range in fp32 into its own slab of `part`; a second kernel adds the slabs in
-    // a fixed order (no atomics: results are reproducible).
-    const int64_t tiles = (int64_t)n_tiles * m_tiles;
-    int splits = (int)std::min<int64_t>(kMaxSplits, num_cus / tiles);
-    splits = std::min(splits, w.KT / 4);                         // at least 4 K tiles per split
-    while (splits > 1 && (size_t)splits * M * w.N * 4 > part_bytes) splits--;
-    if (splits < 1) splits = 1;
     const int kt_per_split = (w.KT + splits - 1) / splits;
-    splits = (w.KT + kt_per_split - 1) / kt_per_split;          // no empty split
-    const unsigned groups = (unsigned)((tiles * splits + 7) / 8 * 8);
-    hipLaunchKernelGGL(kern, dim3(groups), dim3(WAVES * 64), lds, st, w.base, reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT,
+    const unsigned groups = (unsigned)(((int64_t)n_tiles * m_tiles * splits + 7) / 8 * 8);
+    hipLaunchKernelGGL(kern, dim3(groups), dim3(512), lds, st, w.base, reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT,
                        (M + 15) / 16, M, n_tiles, m_tiles, splits, kt_per_split, (int)groups, w.N, y, ydt, w.K, out_scale, part, epi, ns);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || splits == 1) return e;
     return launch_reduce(part, splits, M, w.N, y, ydt, out_scale, epi, ns, w.K, st);
 }
 
-// Workgroup shapes: every wave owns 2 row blocks.
-//   8 waves (256 rows): two waves per SIMD cover each other's waits and the tile's
-//       weights are dequantised once for all eight.
-//   4 waves (128 rows): twice the tiles, for few rows on grids that would leave CUs idle.
-//       From 256 rows up (a long K) or beyond, the 8-wave shape with a deeper K split is the
-//       quicker way to fill the chip (14336 -> 4096 at M = 512: 86.7 -> 74.6 us).
-template <int BITS, int XBF, int NF, bool EXACT>
-hipError_t launch_t(const WeightView& w, const void* x, int M, void* y, int ydt, float out_scale, float* part,
-                    size_t part_bytes, int num_cus, const Epilogue& epi, const NormStats& ns, hipStream_t st)
-{
-    const int64_t tiles256 = (int64_t)((w.NT + NF - 1) / NF) * ((M + 255) / 256);
-    const bool few_rows = M < 256 || (M == 256 && w.KT < 64);
-    // 512-row workgroups (four row blocks per wave: half the LDS operand reads per MFMA) once they
-    // fill the chip by themselves
-    if constexpr (!EXACT && NF == 7) {           // (eight column blocks x four row blocks spill)
-        const int64_t tiles512 = (int64_t)((w.NT + NF - 1) / NF) * ((M + 511) / 512);
-        const int rem = M % 512;                       // (a last tile at most half full: 256-row tiles waste less)
-        if (tiles512 >= num_cus && (rem == 0 || rem > 256))
-            return launch_m<BITS, XBF, NF, EXACT, 4, 8>(w, x, M, y, ydt, out_scale, part, part_bytes, num_cus, epi, ns, st);
-    }
-    // enough 256-row tiles to fill the chip without a K split: the role-split kernel
-    if constexpr (!EXACT) {
-        if (tiles256 >= num_cus) return launch_roles<BITS, NF, 2, 8, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
-    }
-    if (tiles256 < num_cus && few_rows) return launch_m<BITS, XBF, NF, EXACT, 2, 4>(w, x, M, y, ydt, out_scale, part, part_bytes, num_cus, epi, ns, st);
-    return launch_m<BITS, XBF, NF, EXACT, 2, 8>(w, x, M, y, ydt, out_scale, part, part_bytes, num_cus, epi, ns, st);
-}
+// What multiplies a staged chunk of M rows.
+//   kRoles   gemm_roles_kernel, mw multiplying waves (32 rows each), nf column blocks, no K split
+//   kTiles   gemm_kernel, mf row blocks per wave (256 or 512 rows), nf column blocks, K split over `splits` workgroups
+//   kCols    gemm_cols_kernel (gemm_cols.hip)
+struct TilePlan {
+    enum { kRoles, kTiles, kCols } kind;
+    int nf, mw, mf, splits;
+    ColsPlan cols;
+};
 
-template <int BITS, int XBF>
-hipError_t launch_nf(const WeightView& w, const void* x, int M, void* y, int ydt, bool exact, float out_scale,
-                     float* part, size_t part_bytes, int num_cus, const Epilogue& epi, const NormStats& ns, hipStream_t st)
+// The tiled kernels' way with a call, and an estimate of its time behind the staging pass in us (< 0: whatever the others take).
+// The estimates are fits to 1900 calls of 33 .. 600 rows on N of 512 .. 32768, K of 512 .. 14336 (Q4 and Q8, bf16; 4 - 8 % rms): a
+// round of workgroups costs a fixed part and so much per K tile, whatever the number of workgroups in it.
+static float tiled_plan(const WeightView& w, int M, bool exact, int num_cus, size_t part_bytes, const Epilogue& epi, TilePlan& plan)
 {
-    // 7 column blocks (BN = 112) tile N = 14336 = 128 * 112 exactly: with M = 512
-    // that is 256 workgroups, one per CU; 8 column blocks otherwise
-    const bool nf7 = w.NT % 7 == 0 && epi.kind != kEpiSwiglu;      // gate / up pairs need an even number of column blocks
-    if (exact) {
-        if (nf7) return launch_t<BITS, XBF, 7, true>(w, x, M, y, ydt, out_scale, part, part_bytes, num_cus, epi, ns, st);
-        return launch_t<BITS, XBF, 8, true>(w, x, M, y, ydt, out_scale, part, part_bytes, num_cus, epi, ns, st);
-    }
-    if constexpr (XBF == 0) {       // FAST multiplies in f16: bf16 activations were widened by the staging pass
-        // up to 128 rows on a wide output: 128 x 64 tiles fill most of the chip without a K split and
-        // its second pass over the partial sums
-        if (M <= 128 && epi.kind != kEpiSwiglu) {
-            const int64_t tiles64 = (w.NT + 3) / 4;                  // 64-column tiles
-            if (tiles64 * 2 >= 3 * num_cus) {        // more than one round of them: the plain kernel (48 against 58 us at N = 28672),
-                // up to 64 rows the role-split one with its smaller workgroups (41.5 -> 39.5 us)
-                if (M <= 64) return launch_roles<BITS, 4, 2, 2, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
-                return launch_m<BITS, 0, 4, false, 2, 4>(w, x, M, y, ydt, out_scale, part, part_bytes, num_cus, epi, ns, st);
-            }
-            if (tiles64 * 4 >= 3 * num_cus || (tiles64 * 2 >= num_cus && w.KT <= 48)) {      // (half a round still beats a K split on a short K)        // one round: the role-split kernel (30 against 34.5 us at N = 14336)
-                // (every workgroup streams all the rows of X from the L2, and that stream is what these
-                // calls wait for: two multiplying waves = 64 rows when that covers the batch)
-                if (M <= 64) return launch_roles<BITS, 4, 2, 2, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
-                return launch_roles<BITS, 4, 2, 4, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
-            }
+    const int64_t cus = num_cus;
+    const float out_mb = 4e-6f * (float)M * (float)w.N, kt = (float)w.KT;
+    auto roles = [&](int nf, int mw) { plan = {TilePlan::kRoles, nf, mw, 2, 1, {}}; };
+    if (!exact && epi.kind != kEpiSwiglu) {
+        const int64_t tiles64 = (w.NT + 3) / 4;                  // 64-column tiles
+        // up to 128 rows on a wide output: one round of 128 x 64 tiles (at least half of one where K is short) needs no K
+        // split and no second pass over partial sums; 64 rows where those cover the batch (every workgroup streams all the
+        // rows of X from the L2).  More than a round of them, or a long K, is gemm_cols.hip's: 4096 -> 28672 at 64 / 96 / 128 rows
+        // 32.7 / 42.5 / 46.6 -> 28.9 / 33.5 / 39.9 us, 14336 -> 14336 at 40 / 64 / 96 rows 58.5 / 56.4 / 64.7 -> 44.1 / 48.2 / 56.2
+        if (M <= 128 && tiles64 <= cus && w.KT <= 64 && (tiles64 * 4 >= 3 * cus || (tiles64 * 2 >= cus && w.KT <= 48))) {
+            roles(4, M <= 64 ? 2 : 4);
+            return -1.f;
         }
         // A narrow output with a short K (the attention projections at a prefill chunk): 256 x 112 tiles
         // would leave most CUs idle and get a K split with its second pass over the partial sums.
         // One round of 128-row tiles of the role-split kernel, as wide as still gives every CU a tile,
         // does without (X then crosses from the L2 once per column tile: K stays short for this).
-        if (epi.kind != kEpiSwiglu && w.KT <= 48 && M > 128) {
-            const int64_t tiles256 = (int64_t)((w.NT + 6) / 7) * ((M + 255) / 256);
-            if (tiles256 < num_cus) {
-                // (128-row tiles first, 64-row ones for batches they cannot spread over the chip; the
-                // width that fills most of one round, at least three quarters of it)
-                int best_nf = 0, best_mw = 0;
-                int64_t best_groups = 0;
-                for (int mw : {4, 2})
-                    for (int nf : {8, 6, 4}) {
-                        const int64_t g = (int64_t)((M + mw * 32 - 1) / (mw * 32)) * ((w.NT + nf - 1) / nf);
-                        if (g <= num_cus && g * 4 >= 3 * num_cus && (best_mw == 0 || (mw == best_mw && g > best_groups))) {
-                            best_nf = nf;
-                            best_mw = mw;
-                            best_groups = g;
-                        }
+        if (w.KT <= 48 && M > 128 && (int64_t)((w.NT + 6) / 7) * ((M + 255) / 256) < cus) {
+            // (128-row tiles first, 64-row ones for batches they cannot spread over the chip; the
+            // width that fills most of one round, at least three quarters of it)
+            int best_nf = 0, best_mw = 0;
+            int64_t best_groups = 0;
+            for (int mw : {4, 2})
+                for (int nf : {8, 6, 4}) {
+                    const int64_t g = (int64_t)((M + mw * 32 - 1) / (mw * 32)) * ((w.NT + nf - 1) / nf);
+                    if (g <= cus && g * 4 >= 3 * cus && (best_mw == 0 || (mw == best_mw && g > best_groups))) {
+                        best_nf = nf;
+                        best_mw = mw;
+                        best_groups = g;
                     }
-                if (best_mw == 4) {
-                    if (best_nf == 8) return launch_roles<BITS, 8, 2, 4, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
-                    if (best_nf == 6) return launch_roles<BITS, 6, 2, 4, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
-                    return launch_roles<BITS, 4, 2, 4, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
                 }
-                if (best_mw == 2) {
-                    if (best_nf == 8) return launch_roles<BITS, 8, 2, 2, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
-                    if (best_nf == 6) return launch_roles<BITS, 6, 2, 2, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
-                    return launch_roles<BITS, 4, 2, 2, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
-                }
+            if (best_mw) {
+                roles(best_nf, best_mw);
+                const float fixed = best_nf == 4 ? 1.4f : best_nf == 6 ? 2.0f : 2.4f;
+                const float per_kt = best_mw == 4 ? (best_nf == 4 ? 0.48f : best_nf == 6 ? 0.73f : 0.84f) : (best_nf == 4 ? 0.45f : best_nf == 6 ? 0.62f : 0.75f);
+                return fixed + per_kt * kt + 0.27f * out_mb;
             }
         }
-        if (nf7) return launch_t<BITS, 0, 7, false>(w, x, M, y, ydt, out_scale, part, part_bytes, num_cus, epi, ns, st);
-        return launch_t<BITS, 0, 8, false>(w, x, M, y, ydt, out_scale, part, part_bytes, num_cus, epi, ns, st);
+    }
+    // 7 column blocks (BN = 112) tile N = 14336 = 128 * 112 exactly: with M = 512
+    // that is 256 workgroups, one per CU; 8 column blocks otherwise
+    const int nf = w.NT % 7 == 0 && epi.kind != kEpiSwiglu ? 7 : 8;      // gate / up pairs need an even number of column blocks
+    // 512-row workgroups (four row blocks per wave: half the LDS operand reads per MFMA) once they
+    // fill the chip by themselves (eight column blocks x four row blocks spill)
+    if (!exact && nf == 7) {
+        const int64_t tiles512 = (int64_t)((w.NT + 6) / 7) * ((M + 511) / 512);
+        const int rem = M % 512;                       // (a last tile at most half full: 256-row tiles waste less)
+        if (tiles512 >= cus && (rem == 0 || rem > 256)) {
+            plan = {TilePlan::kTiles, 7, 8, 4, 1, {}};
+            return -1.f;
+        }
+    }
+    const int64_t tiles = (int64_t)((w.NT + nf - 1) / nf) * ((M + 255) / 256);
+    // enough 256-row tiles to fill the chip without a K split: the role-split kernel
+    if (!exact && tiles >= cus) {
+        roles(nf, 8);
+        return (float)((tiles + cus - 1) / cus) * (0.4f + 1.43f * kt) + 0.27f * out_mb;
+    }
+    // Too few tiles to fill the chip: split K over workgroups.  Every split adds its
+    // K range in fp32 into its own slab of `part`; a second kernel adds the slabs in
+    // a fixed order (no atomics: results are reproducible).
+    int splits = (int)std::min<int64_t>(kMaxSplits, cus / tiles);
+    splits = std::min(splits, w.KT / 4);                         // at least 4 K tiles per split
+    while (splits > 1 && (size_t)splits * M * w.N * 4 > part_bytes) splits--;
+    if (splits < 1) splits = 1;
+    const int per = (w.KT + splits - 1) / splits;
+    splits = (w.KT + per - 1) / per;                             // no empty split
+    plan = {TilePlan::kTiles, nf, 8, 2, splits, {}};
+    const float rounds = (float)((tiles * splits + cus - 1) / cus);
+    return rounds * (exact ? 0.9f + 2.75f * (float)per : 1.4f + 1.29f * (float)per) +
+           (splits > 1 ? 2.2f + 0.5f * ((float)splits + 0.5f) * out_mb : 0.27f * out_mb);
+}
+
+// The quicker of the tiled kernels and the one whose waves stand side by side (gemm_cols.hip), by their estimates
+static TilePlan plan_tiles(const WeightView& w, int M, bool exact, bool bf16, int num_cus, size_t part_bytes, const Epilogue& epi)
+{
+    TilePlan plan = {};
+    const float tiled = tiled_plan(w, M, exact, num_cus, part_bytes, epi, plan);
+    if (tiled < 0.f || g_rows_kernel == 3 || (g_rows_kernel == 2 && !exact)) return plan;
+    const ColsPlan cols = plan_gemm_cols(w, !exact ? 0 : bf16 ? 2 : 1, M, num_cus, part_bytes);
+    if (cols.us < 0.97f * tiled) plan = {TilePlan::kCols, 0, 0, 0, cols.splits, cols};
+    return plan;
+}
+
+template <int BITS, int XBF>
+hipError_t launch_tiles(const TilePlan& p, const WeightView& w, const void* x, int M, void* y, int ydt, bool exact, float out_scale, float* part,
+                        const Epilogue& epi, const NormStats& ns, hipStream_t st)
+{
+    if (p.kind == TilePlan::kCols) {
+        const hipError_t e = launch_gemm_cols(w, x, !exact ? 0 : XBF ? 2 : 1, M, y, ydt, p.cols, epi, ns.part, ns.nblk, ns.unscale, part, st);
+        if (e != hipSuccess || p.splits == 1) return e;
+        return launch_reduce(part, p.splits, M, w.N, y, ydt, out_scale, epi, ns, w.K, st);
+    }
+    if (exact) {
+        if (p.nf == 7) return launch_m<BITS, XBF, 7, true, 2>(w, x, M, y, ydt, out_scale, part, p.splits, epi, ns, st);
+        return launch_m<BITS, XBF, 8, true, 2>(w, x, M, y, ydt, out_scale, part, p.splits, epi, ns, st);
+    }
+    if constexpr (XBF == 0) {       // FAST multiplies in f16: bf16 activations were widened by the staging pass
+        if (p.kind == TilePlan::kRoles) {
+            if (p.mw == 8 && p.nf == 7) return launch_roles<BITS, 7, 2, 8, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
+            if (p.mw == 8) return launch_roles<BITS, 8, 2, 8, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
+            if (p.mw == 4 && p.nf == 8) return launch_roles<BITS, 8, 2, 4, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
+            if (p.mw == 4 && p.nf == 6) return launch_roles<BITS, 6, 2, 4, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
+            if (p.mw == 4) return launch_roles<BITS, 4, 2, 4, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
+            if (p.nf == 8) return launch_roles<BITS, 8, 2, 2, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
+            if (p.nf == 6) return launch_roles<BITS, 6, 2, 2, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
+            return launch_roles<BITS, 4, 2, 2, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
+        }
+        if (p.mf == 4) return launch_m<BITS, 0, 7, false, 4>(w, x, M, y, ydt, out_scale, part, 1, epi, ns, st);
+        if (p.nf == 7) return launch_m<BITS, 0, 7, false, 2>(w, x, M, y, ydt, out_scale, part, p.splits, epi, ns, st);
+        return launch_m<BITS, 0, 8, false, 2>(w, x, M, y, ydt, out_scale, part, p.splits, epi, ns, st);
     }
     return hipErrorInvalidValue;
 }
@@ -1111,13 +1141,12 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
 
 }  // namespace
 
-int g_rows_kernel = 0;        // (set_gemm_tuning: 2 = experiments switch the few-rows kernel off, 1 = on whatever the width)
 int g_touch = 2;              // (5 = the staging launch asks for no weights ahead of the multiply, 6 = only ahead of the few-rows kernel)
 void set_gemm_tuning(int rows_kernel) { g_rows_kernel = rows_kernel >= 5 ? 0 : rows_kernel; g_touch = rows_kernel == 5 ? 0 : rows_kernel == 6 ? 1 : 2; }
 
 static RowsPlan rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
-    if (g_rows_kernel == 2) return {0, 0};
+    if (g_rows_kernel == 2 || g_rows_kernel == 3) return {0, 0};
     return gemm_rows_plan(w, M, g_rows_kernel == 1 ? 1 : num_cus, epi);
 }
 
@@ -1135,12 +1164,12 @@ bool gemm_rows_takes(const WeightView& w, int M, int num_cus, const Epilogue& ep
 // at 64 / 128 rows 13.6 / 14.6 -> 12.4 / 13.4, 4096 -> 1024 13.1 -> 11.7, 8192 -> 4096 at 128 rows 25.1 -> 22.9.  Not
 // for f16 rows (their pass only reorders and is over before the reads are: 4096 -> 14336 at 64 rows 18.6 -> 19.1),
 // for 17 .. 32 fp32 rows (12.5 -> 13.4 on 4096 -> 8192) or for K up to 2048.
-// whether launch_nf gives a FAST-mode call of M rows the 64-column tiles (one row tile of up to 128 rows)
+// whether tiled_plan gives a FAST-mode call of M rows the 64-column tiles
 static bool few_rows_tiles64(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
+    TilePlan plan = {};
     if (M > 128 || epi.kind == kEpiSwiglu) return false;
-    const int64_t tiles64 = (w.NT + 3) / 4;
-    return tiles64 * 4 >= 3 * num_cus || (tiles64 * 2 >= num_cus && w.KT <= 48);
+    return tiled_plan(w, M, false, num_cus, 0, epi, plan) < 0.f && plan.kind == TilePlan::kRoles && plan.nf == 4;
 }
 
 static Touch plan_touch(const WeightView& w, int mc, int num_cus, const Epilogue& ec, bool exact, unsigned& grid_x)
@@ -1267,12 +1296,13 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
             if (e != hipSuccess) return e;
             continue;
         }
+        const TilePlan tp = plan_tiles(w, mc, exact, kdt == kBF16, num_cus, half, ec);
         if (w.bits == 4) {
-            e = kdt == kBF16 ? launch_nf<4, 1>(w, workspace, mc, yc, ydt, exact, out_scale, part, half, num_cus, ec, ns, st)
-                             : launch_nf<4, 0>(w, workspace, mc, yc, ydt, exact, out_scale, part, half, num_cus, ec, ns, st);
+            e = kdt == kBF16 ? launch_tiles<4, 1>(tp, w, workspace, mc, yc, ydt, exact, out_scale, part, ec, ns, st)
+                             : launch_tiles<4, 0>(tp, w, workspace, mc, yc, ydt, exact, out_scale, part, ec, ns, st);
         } else {
-            e = kdt == kBF16 ? launch_nf<8, 1>(w, workspace, mc, yc, ydt, exact, out_scale, part, half, num_cus, ec, ns, st)
-                             : launch_nf<8, 0>(w, workspace, mc, yc, ydt, exact, out_scale, part, half, num_cus, ec, ns, st);
+            e = kdt == kBF16 ? launch_tiles<8, 1>(tp, w, workspace, mc, yc, ydt, exact, out_scale, part, ec, ns, st)
+                             : launch_tiles<8, 0>(tp, w, workspace, mc, yc, ydt, exact, out_scale, part, ec, ns, st);
         }
         if (e != hipSuccess) return e;
     }

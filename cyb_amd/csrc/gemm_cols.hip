@@ -1,0 +1,476 @@
+// gemm_cols.hip - prefill kernel whose waves stand side by side along the columns and share out every K tile.
+//
+// Workgroup = 8 waves, output tile 16 * RB rows x 64 * CS columns.  Wave (col, kh) owns CS strips of 16 columns against ALL rows and,
+// of every K tile, the two scale groups of half kh; the halves' sums meet in LDS once at the end.
+//
+//   W  a native tile is multiplied by the two waves that hold its groups and by nobody else: its words go from LDS to registers,
+//      are dequantised there and are MFMA operands as they stand - no operand goes through LDS, none is made twice.
+//   X  (staged in operand order) is shared by the four columns of waves: copied to LDS once, read by each.
+//   Both come by global_load_lds, which needs no registers while in flight: 3 - 5 K tiles of X and up to 10 of packed weights
+//      are on their way, counted by hand (s_waitcnt vmcnt: copies retire in order), one barrier per K tile in its middle - the first
+//      half's operands are in registers when it is passed, the second half's arithmetic covers the reads behind it.
+//   EXACT mode: two operands per weight that add up to scale * q.  f16: the rounded product and what it lost (one fma).  bf16, Q4: the
+//      scale is cut into two parts of five significant bits, whose products with q are bf16 numbers as they stand; 36 vector
+//      instructions per eight weights where rounding the product and subtracting took 49.
+//
+// What bounds it: a SIMD's issue slots and LDS.  Per 16x16x32 MFMA (16 cycles of the matrix pipe) a SIMD issues two other vector
+// instructions for free, whatever the number of waves; the dequantisation of a strip's group is 16 (FAST) to 43 (EXACT bf16), which
+// only eight row blocks hide.  So the gain is where the tiled kernels of gemm.hip have few rows (their waves own 32 each, and every
+// weight operand crosses LDS for each of them) or EXACT's operands to make: K tile of 128 rows x 128 columns 1700 cycles in FAST,
+// 3230 in EXACT bf16, of which the MFMAs are 1024 and 2048.
+// us per call with the staging pass, before (128- / 64-row tiles of gemm.hip) and now.  EXACT, bf16 rows on Q4: 4096 -> 14336 at 64 / 128 /
+// 256 rows 47.7 / 50.5 / 80.6 -> 27.1 / 35.4 / 59.0, 14336 -> 4096 at 40 / 128 rows 46.2 / 50.1 -> 25.8 / 38.6, 4096 -> 4096 at 256 rows 35.5 ->
+// 26.9, 4096 -> 28672 at 64 rows 103 -> 43.6; f16 rows: 4096 -> 14336 at 256 rows 84.2 -> 53.5.  FAST: 4096 -> 28672 at 96 / 128 rows 42.5 /
+// 46.6 -> 33.5 / 39.9, with SwiGLU 48.9 / 49.8 -> 33.3 / 39.5, 14336 -> 14336 at 40 / 192 rows 58.5 / 124.5 -> 44.1 / 92.8, 4096 -> 14336 at 192 rows 39.4 ->
+// 33.7, 1024 -> 4096 at 128 rows 15.7 -> 10.1.
+// Tried: four waves of 128 x 64 on 32x32x16 MFMAs, every weight of a K tile dequantised by its wave (one wave per SIMD: MFMAs and
+// vector instructions add up, 2900 cycles a K tile for 2048 of MFMAs; 4096 -> 14336 at 512 rows 77 us against 60 of the role-split
+// kernel); deeper rings for the few-row forms (no change); words read from LDS a K tile earlier (3 % slower).
+#include <algorithm>
+#include <type_traits>
+
+#include "cybq_device.h"
+#include "cybq_internal.h"
+
+namespace cybq {
+
+namespace {
+
+#include "gemm_parts.h"
+
+template <int I, int N, class F>
+__device__ __forceinline__ void static_for(F&& f)
+{
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<I + 1, N>(f);
+    }
+}
+
+// 16 bytes per lane from base + off (the lane's own) to LDS bytes lds_off + 16 * lane, past the registers
+__device__ __forceinline__ void copy_to_lds(uint32_t lds_off, const void* base, uint32_t off)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds_off)), "v"(off), "s"(base));
+}
+// the same from the lanes of `lanes` alone (all 64 lanes are active around it; a branch would cut the scheduling region)
+__device__ __forceinline__ void copy_to_lds(uint32_t lds_off, const void* base, uint32_t off, uint64_t lanes)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1" ::"s"(__builtin_amdgcn_readfirstlane(lds_off)), "v"(off), "s"(base), "s"(lanes));
+}
+template <int N>
+__device__ __forceinline__ void wait_copies() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
+// MODE 0: FAST (one f16 operand per weight), 1 / 2: EXACT with f16 / bf16 operands (hi and lo)
+template <int BITS, int MODE, int RB, int CS>
+struct ColsShape {
+    static constexpr int OPS = MODE == 0 ? 1 : 2;
+    static constexpr int STRIPS = 4 * CS;
+    static constexpr int XTILE = RB * 4096;                                // bytes of a K tile of X
+    static constexpr int WSCALES = STRIPS * 1024 * (BITS / 4);             // scales behind the q words
+    static constexpr int WTILE = WSCALES + STRIPS * 128;
+    static constexpr bool FOLDED = BITS == 4 && CS == 1;                   // four waves copy q words, the other four scales
+    static constexpr int XCOPIES = (RB * 4 + 7) / 8;                       // per wave and K tile
+    static constexpr int QCOPIES = FOLDED ? 1 : STRIPS * (BITS / 4) / 8;
+    static constexpr int WCOPIES = FOLDED ? 1 : QCOPIES + 1;
+    static constexpr int BUDGET = 156 * 1024;
+    // K tiles of X in flight: three where a tile is long, up to five where it is short; weights get the rest
+    static constexpr int NX = RB >= 8 ? 3 : RB >= 6 ? (BITS * CS > 8 ? 3 : 4) : RB >= 4 && BITS * CS > 8 ? 4 : 5;
+    static constexpr int NWFIT = (BUDGET - NX * XTILE) / WTILE;
+    static constexpr int NW = NWFIT > 10 ? 10 : NWFIT;
+    // copies that may be outstanding when a K tile's X and words have to be there, `newer` batches behind the one with its X
+    static constexpr int allowed(int newer) { return newer * (XCOPIES + WCOPIES) + (NW > NX ? WCOPIES : 0); }
+    static constexpr int WBASE = NX * XTILE;
+    static constexpr int PITCH = STRIPS * 16 + 4;                          // floats, finished tile
+    static constexpr int TILE = RB * 16 * PITCH * 4;
+    static constexpr int LDS = WBASE + NW * WTILE > TILE + RB * 64 ? WBASE + NW * WTILE : TILE + RB * 64;
+    static_assert(NW >= NX && LDS <= 160 * 1024, "LDS");
+};
+
+template <int BITS, int MODE, int RB, int CS>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_cols_kernel(
+    const uint8_t* __restrict__ wbase, const uint8_t* __restrict__ x, int KT_, int NT, int x_row_blocks, int M, int n_tiles, int m_tiles,
+    int splits, int kt_per_split, int groups, int N, void* __restrict__ y, int ydt, int K, float* __restrict__ part, Epilogue epi, NormStats ns)
+{
+    using S = ColsShape<BITS, MODE, RB, CS>;
+    constexpr int NX = S::NX, NW = S::NW, XC = S::XCOPIES, WC = S::WCOPIES, OPS = S::OPS;
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int per_xcd = groups >> 3;
+    const int item = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
+    if (item >= n_tiles * m_tiles * splits) return;
+    // (divisions leave their results in vector registers: back to scalars, the copies' bases hang on them)
+    const int split = __builtin_amdgcn_readfirstlane(item / (n_tiles * m_tiles));
+    const int rest = item - split * (n_tiles * m_tiles);
+    const int tile_n = __builtin_amdgcn_readfirstlane(rest / m_tiles), tile_m = rest - tile_n * m_tiles;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = wave & 3, kh = wave >> 2;                  // my strips, my half of every K tile
+    const int m0 = tile_m * (RB * 16);
+    const int nt0 = tile_n * S::STRIPS;                        // first strip of the workgroup
+    const int kt_lo = split * kt_per_split;
+    const int KT = min(kt_per_split, KT_ - kt_lo);
+    const int kt0 = __builtin_amdgcn_readfirstlane(tile_n % KT);
+    const int G = K / kGroup;
+    auto rot = [&](int kt) {
+        const int r = min(kt, KT - 1) + kt0;
+        return kt_lo + (r >= KT ? r - KT : r);
+    };
+
+    // ---- copies into LDS.  X: block e = row block e / 4, group e % 4 of the K tile
+    uint32_t xrow[XC];
+    int xblk[XC];
+#pragma unroll
+    for (int c = 0; c < XC; c++) {
+        xblk[c] = min(c * 8 + wave, RB * 4 - 1);
+        xrow[c] = (uint32_t)min(m0 / 16 + (xblk[c] >> 2), x_row_blocks - 1) * (uint32_t)(G * 1024);
+    }
+    auto copy_x = [&](int kt, int buf, int c) {
+        const int g = min(rot(kt) * 4 + (xblk[c] & 3), G - 1);
+        copy_to_lds(buf * S::XTILE + xblk[c] * 1024, x, xrow[c] + (uint32_t)g * 1024u + (uint32_t)lane * 16u);
+    };
+    const int ntb = min(nt0, NT - 1);
+    const uint8_t* const wsrc = wbase + (int64_t)ntb * KT_ * kTileBytes<BITS>;
+    auto strip_at = [&](int s) { return (uint32_t)((min(nt0 + s, NT - 1) - ntb) * KT_) * (uint32_t)kTileBytes<BITS>; };
+    constexpr int PER_WAVE = S::STRIPS / 8 > 0 ? S::STRIPS / 8 : 1;                 // strips whose scales a wave copies
+    const int sfirst = (wave * PER_WAVE) % S::STRIPS;
+    const uint32_t sc_off = strip_at(sfirst + min(lane >> 3, PER_WAVE - 1)) + (uint32_t)(kTileQBytes<BITS> + (lane & 7) * 16);
+    uint32_t q_off[S::QCOPIES];
+    int q_dst[S::QCOPIES];
+#pragma unroll
+    for (int c = 0; c < S::QCOPIES; c++) {
+        const int e = S::FOLDED ? (wave & 3) : c * 8 + wave;                        // 1-KB block of the q words
+        q_dst[c] = e * 1024;
+        q_off[c] = strip_at(e / (BITS / 4)) + (uint32_t)(e % (BITS / 4)) * 1024u + (uint32_t)lane * 16u;
+    }
+    auto copy_w = [&](int kt, int buf, int c) {
+        const uint32_t at = (uint32_t)rot(kt) * (uint32_t)kTileBytes<BITS>;
+        const int dst = S::WBASE + buf * S::WTILE;
+        if (S::FOLDED) {
+            const bool sc = wave >= 4;
+            copy_to_lds(dst + (sc ? S::WSCALES + (wave - 4) * 128 : q_dst[0]), wsrc, (sc ? sc_off : q_off[0]) + at, sc ? 0xffull : ~0ull);
+        } else if (c < S::QCOPIES) {
+            copy_to_lds(dst + q_dst[c < S::QCOPIES ? c : 0], wsrc, q_off[c < S::QCOPIES ? c : 0] + at);
+        } else {
+            copy_to_lds(dst + S::WSCALES + sfirst * 128, wsrc, sc_off + at, (1ull << (8 * PER_WAVE)) - 1);
+        }
+    };
+
+    // ---- LDS -> registers
+    Frag16 a[2][RB], b[2][OPS][CS];
+    uint32_t wq[CS][BITS / 2], wn[CS][BITS / 2], sq[CS], sn[CS];           // packed weights and scales (my two groups): this K tile's, the next one's
+    auto read_a = [&](Frag16& dst, int buf, int j, int i) {               // j: 0 / 1 of my two groups
+        dst.u = *reinterpret_cast<const u32x4_t*>(smem + buf * S::XTILE + kh * 2048 + lane * 16 + (i * 4 + j) * 1024);
+    };
+    auto read_w = [&](int buf, uint32_t (&q)[CS][BITS / 2], uint32_t (&sc)[CS]) {
+        const uint8_t* p = smem + S::WBASE + buf * S::WTILE;
+#pragma unroll
+        for (int s = 0; s < CS; s++) {
+            if constexpr (BITS == 4) {
+                const u32x2_t v = *reinterpret_cast<const u32x2_t*>(p + (col * CS + s) * 1024 + lane * 16 + kh * 8);
+                q[s][0] = v[0];
+                q[s][1] = v[1];
+            } else {
+                const u32x4_t v = *reinterpret_cast<const u32x4_t*>(p + (col * CS + s) * 2048 + kh * 1024 + lane * 16);
+#pragma unroll
+                for (int e = 0; e < 4; e++) q[s][e & (BITS / 2 - 1)] = v[e];
+            }
+            sc[s] = *reinterpret_cast<const uint32_t*>(p + S::WSCALES + (col * CS + s) * 128 + (lane & 15) * 8 + kh * 4);
+        }
+    };
+    uint32_t magic_lo, magic_hi;
+    asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(magic_lo));
+    asm volatile("v_mov_b32 %0, 0x54005400" : "=v"(magic_hi));
+    // slots 2p, 2p + 1 of my group j in f16, plus a bias (kBias): 1024 + u, 64 + u (odd group of Q4) or 1024 + u with u = q + 128 (Q8)
+    auto biased = [&](const uint32_t (&q)[BITS / 2], int j, int p) {
+        if constexpr (BITS == 4) {
+            const uint32_t src = q[p >> 1] >> (8 * (p & 1));
+            return as_h2(j ? (src & 0x00F000F0u) | magic_hi : (src & 0x000F000Fu) | magic_lo);
+        } else {
+            return as_h2(__builtin_amdgcn_perm(0x64646464u, q[(2 * j + (p >> 1)) & (BITS / 2 - 1)], (p & 1) ? 0x04030402u : 0x04010400u));
+        }
+    };
+    auto operand = [&](const uint32_t (&q)[BITS / 2], uint32_t sc, int j, int p, int buf, int s) {
+        const half2_t v = biased(q, j, p);
+        const float bias = BITS == 8 ? -1152.0f : j ? -72.0f : -1032.0f;
+        const uint32_t bits16 = j ? sc >> 16 : sc & 0xffffu;
+        const _Float16 sh = __builtin_bit_cast(_Float16, (uint16_t)bits16);
+        if constexpr (MODE != 2) {
+            const half2_t s2 = {sh, sh}, n = v + (half2_t){(_Float16)bias, (_Float16)bias};          // exact integers
+            const half2_t hi = n * s2;
+            b[buf][0][s].u[p] = as_u32(hi);
+            if constexpr (MODE == 1) b[buf][OPS - 1][s].u[p] = as_u32(__builtin_elementwise_fma(n, s2, -hi));
+        } else if constexpr (BITS == 4) {
+            // scale = top + rest, five significant bits each (rest: at most 32 units of the scale's last place): with q of three
+            // bits (or -8) both products fit the eight bits of a bf16 operand, nothing is rounded
+            const _Float16 top = __builtin_bit_cast(_Float16, (uint16_t)((bits16 + 0x20u) & 0xffc0u)), rest = sh - top;
+            const float ft = (float)top, fr = (float)rest, ct = bias * ft, cr = bias * fr;
+            b[buf][0][s].u[p] = pack_bf16x2(fmaf((float)v.x, ft, ct), fmaf((float)v.y, ft, ct));
+            b[buf][OPS - 1][s].u[p] = pack_bf16x2(fmaf((float)v.x, fr, cr), fmaf((float)v.y, fr, cr));
+        } else {
+            const float f = (float)sh, c = bias * f, w0 = fmaf((float)v.x, f, c), w1 = fmaf((float)v.y, f, c);      // exact
+            const uint32_t hi = pack_bf16x2(w0, w1);
+            b[buf][0][s].u[p] = hi;
+            b[buf][OPS - 1][s].u[p] = pack_bf16x2(w0 - __builtin_bit_cast(float, hi << 16), w1 - __builtin_bit_cast(float, hi & 0xffff0000u));
+        }
+    };
+
+    float4_t acc[RB][CS];
+#pragma unroll
+    for (int i = 0; i < RB; i++)
+#pragma unroll
+        for (int s = 0; s < CS; s++) acc[i][s] = (float4_t){0.f, 0.f, 0.f, 0.f};
+
+    // ---- prologue: batch -n of the copies holds X of K tile NX - n and the weights of K tile NW - n
+    static_for<0, NW>([&](auto n_) {
+        constexpr int back = NW - decltype(n_)::value;         // NW .. 1
+        if constexpr (back <= NX) {
+#pragma unroll
+            for (int c = 0; c < XC; c++) copy_x(NX - back, NX - back, c);
+        }
+#pragma unroll
+        for (int c = 0; c < WC; c++) copy_w(NW - back, NW - back, c);
+    });
+    wait_copies<S::allowed(NX - 1)>();
+    asm volatile("s_barrier" ::: "memory");
+    read_w(0, wq, sq);
+#pragma unroll
+    for (int i = 0; i < RB; i++) read_a(a[0][i], 0, 0, i);
+#pragma unroll
+    for (int s = 0; s < CS; s++)
+#pragma unroll
+        for (int p = 0; p < 4; p++) operand(wq[s], sq[s], 0, p, 0, s);
+
+    int xbuf = 0, wbuf = 0;
+    // PHASE 0: copies of X and weights go out, 1: of X alone (the last NW K tiles), 2: none (the last NX)
+    auto k_tile = [&](int kt, auto phase_) {
+        constexpr int PHASE = decltype(phase_)::value;
+        const int xnext = xbuf + 1 == NX ? 0 : xbuf + 1, wnext = wbuf + 1 == NW ? 0 : wbuf + 1;
+        static_for<0, 2>([&](auto j_) {
+            constexpr int j = decltype(j_)::value, nxt = 1 - j;
+            if constexpr (j == 1) {
+                // all copies of the next K tile are in LDS, and nobody reads this one's any more
+                if constexpr (PHASE == 0) {
+                    wait_copies<S::allowed(NX - 2)>();
+                } else if constexpr (PHASE == 1) {
+                    wait_copies<(NX - 2) * XC>();
+                } else {
+                    const int left = min(NX - 2, KT - 2 - kt);         // K tiles of X requested after the next one's
+                    if (left == 3) wait_copies<3 * XC>();
+                    else if (left == 2) wait_copies<2 * XC>();
+                    else if (left == 1) wait_copies<XC>();
+                    else wait_copies<0>();
+                }
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                read_w(wnext, wn, sn);
+            }
+            constexpr int MMAS = RB * CS * OPS, PAIRS = 4 * CS;
+            static_for<0, MMAS>([&](auto m_) {
+                constexpr int m = decltype(m_)::value, i = m / (CS * OPS), o = (m / CS) % OPS, s = m % CS;
+                if constexpr (MODE == 2) acc[i][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j][i].b, b[j][o][s].b, acc[i][s], 0, 0, 0);
+                else acc[i][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j][i].h, b[j][o][s].h, acc[i][s], 0, 0, 0);
+                if constexpr (s == 0 && o == 0) read_a(a[nxt][i], j ? xnext : xbuf, nxt, i);
+                // (the next K tile's words have just been asked for: the second half of the group is theirs; a form that read them a
+                // K tile earlier and spread their arithmetic over the whole group was 3 % slower)
+                constexpr int F = j ? MMAS / 2 : 0, p0 = m < F ? 0 : (m - F) * PAIRS / (MMAS - F), p1 = m < F ? 0 : (m - F + 1) * PAIRS / (MMAS - F);
+                static_for<p0, p1>([&](auto q_) {
+                    constexpr int q = decltype(q_)::value, ds = q / 4, p = q & 3;
+                    if constexpr (j == 1) operand(wn[ds], sn[ds], 0, p, 0, ds);
+                    else operand(wq[ds], sq[ds], 1, p, 1, ds);
+                });
+                if constexpr (j == 1 && PHASE < 2) {
+                    constexpr int ALL = PHASE == 0 ? XC + WC : XC;
+                    static_for<m * ALL / MMAS, (m + 1) * ALL / MMAS>([&](auto c_) {
+                        constexpr int c = decltype(c_)::value;
+                        if constexpr (c < XC) copy_x(kt + NX, xbuf, c);
+                        else copy_w(kt + NW, wbuf, c - XC);
+                    });
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        });
+        xbuf = xnext;
+        wbuf = wnext;
+#pragma unroll
+        for (int s = 0; s < CS; s++) {
+            sq[s] = sn[s];
+#pragma unroll
+            for (int e = 0; e < BITS / 2; e++) wq[s][e] = wn[s][e];
+        }
+    };
+    int kt = 0;
+    for (; kt + NW < KT; kt++) k_tile(kt, std::integral_constant<int, 0>{});
+    for (; kt + NX < KT; kt++) k_tile(kt, std::integral_constant<int, 1>{});
+    for (; kt < KT; kt++) k_tile(kt, std::integral_constant<int, 2>{});
+
+    // ---- the two halves of K meet in LDS; then whole runs of a row, four elements per thread
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    float* const tile = reinterpret_cast<float*>(smem);
+    float* const rowf = reinterpret_cast<float*>(smem + S::TILE);
+    const bool slab = splits > 1;
+    const int row16 = lane & 15, oct = lane >> 4;
+    if (kh == 1) {
+#pragma unroll
+        for (int i = 0; i < RB; i++)
+#pragma unroll
+            for (int s = 0; s < CS; s++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) tile[(i * 16 + oct * 4 + r) * S::PITCH + (col * CS + s) * 16 + row16] = acc[i][s][r];
+    } else if (tid < RB * 16) {
+        rowf[tid] = slab || !(epi.gamma || ns.unscale) ? 1.0f : row_factor(ns, epi.gamma != nullptr, min(m0 + tid, M - 1), K, epi.eps);
+    }
+    __syncthreads();
+    if (kh == 0) {
+#pragma unroll
+        for (int i = 0; i < RB; i++)
+#pragma unroll
+            for (int s = 0; s < CS; s++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    float* t = &tile[(i * 16 + oct * 4 + r) * S::PITCH + (col * CS + s) * 16 + row16];
+                    *t = acc[i][s][r] + *t;
+                }
+    }
+    __syncthreads();
+    const bool swiglu = !slab && epi.kind == kEpiSwiglu, add = !slab && epi.kind == kEpiAdd;
+    if (slab) {
+        y = part + (int64_t)split * M * N;
+        ydt = kF32;
+    }
+    const int n_out = swiglu ? N >> 1 : N, n0 = swiglu ? nt0 * 8 : nt0 * 16;
+    const uintptr_t amask = ydt == kF32 ? 15u : 7u;
+    const bool aligned = (n_out & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & amask) == 0 &&
+                         (!add || (reinterpret_cast<uintptr_t>(epi.residual) & amask) == 0);
+    auto store4 = [&](float4_t v, int m, int n) {
+        const int64_t at = (int64_t)m * n_out + n;
+        if (!aligned) {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (n + e < n_out) {
+                    float o = v[e];
+                    if (add) o += load_out_g(epi.residual, ydt, at + e);
+                    store_out_g(y, ydt, at + e, o);
+                }
+        } else if (n < n_out) {
+            if (ydt == kF32) {
+                if (add) v += *reinterpret_cast<const float4_t*>(reinterpret_cast<const float*>(epi.residual) + at);
+                *reinterpret_cast<float4_t*>(reinterpret_cast<float*>(y) + at) = v;
+            } else {
+                if (add) {
+                    const u32x2_t rr = *reinterpret_cast<const u32x2_t*>(reinterpret_cast<const uint16_t*>(epi.residual) + at);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const uint32_t h = (e & 1) ? rr[e >> 1] >> 16 : rr[e >> 1] & 0xffffu;
+                        v[e] += ydt == kF16 ? f16_bits_to_f32(h) : __builtin_bit_cast(float, h << 16);
+                    }
+                }
+                u32x2_t o;
+                if (ydt == kF16) {
+                    const half2_t p = {(_Float16)v[0], (_Float16)v[1]}, q = {(_Float16)v[2], (_Float16)v[3]};
+                    o = (u32x2_t){as_u32(p), as_u32(q)};
+                } else {
+                    o = (u32x2_t){pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+                }
+                *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(y) + at) = o;
+            }
+        }
+    };
+    const int rows = min(RB * 16, M - m0);
+    if (swiglu) {                          // strips 2p / 2p + 1 are gate / up of output block (nt0 >> 1) + p
+        constexpr int V4 = S::STRIPS * 2;
+        for (int p = tid; p < rows * V4; p += 512) {
+            const int row = p / V4, c4 = p % V4;
+            const float* t = tile + row * S::PITCH + (c4 >> 2) * 32 + (c4 & 3) * 4;
+            const float f = rowf[row];
+            float4_t v;
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = silu_mul(t[e] * f, t[16 + e] * f);
+            store4(v, m0 + row, n0 + c4 * 4);
+        }
+    } else {
+        constexpr int V4 = S::STRIPS * 4;
+        for (int p = tid; p < rows * V4; p += 512) {
+            const int row = p / V4, c4 = p % V4;
+            store4(*reinterpret_cast<const float4_t*>(tile + row * S::PITCH + c4 * 4) * rowf[row], m0 + row, n0 + c4 * 4);
+        }
+    }
+}
+
+template <int BITS, int MODE, int RB, int CS>
+hipError_t launch_cols_t(const WeightView& w, const void* x, int M, void* y, int ydt, int splits, const Epilogue& epi, const NormStats& ns,
+                         float* part, hipStream_t st)
+{
+    using S = ColsShape<BITS, MODE, RB, CS>;
+    (void)LdsRequest<&gemm_cols_kernel<BITS, MODE, RB, CS>, S::LDS>::registered;
+    const int n_tiles = (w.NT + S::STRIPS - 1) / S::STRIPS, m_tiles = (M + 16 * RB - 1) / (16 * RB);
+    const int kt_per_split = (w.KT + splits - 1) / splits;
+    const unsigned groups = (unsigned)(((int64_t)n_tiles * m_tiles * splits + 7) / 8 * 8);
+    hipLaunchKernelGGL((gemm_cols_kernel<BITS, MODE, RB, CS>), dim3(groups), dim3(512), S::LDS, st, w.base, static_cast<const uint8_t*>(x),
+                       w.KT, w.NT, (M + 15) / 16, M, n_tiles, m_tiles, splits, kt_per_split, (int)groups, w.N, y, ydt, w.K, part, epi, ns);
+    return hipGetLastError();
+}
+
+constexpr int kColsSplits = 8;               // the slab-adding pass takes as many
+
+}  // namespace
+
+// Row blocks, strips per wave and splits with the shortest estimate.  A round of workgroups costs a fixed part and so much per K
+// tile (below, us; fits to 9000 forced calls of 33 .. 600 rows, N of 512 .. 32768, K of 512 .. 14336, Q4 and Q8: 3 - 5 % rms), a split
+// its slabs' way through memory.  Choosing by it costs 0.5 % against the best of all forms on these calls.
+ColsPlan plan_gemm_cols(const WeightView& w, int mode, int M, int num_cus, size_t part_bytes)
+{
+    struct Form {
+        int rb, cs;
+        float fixed[3], per_kt[3];           // FAST, EXACT f16, EXACT bf16
+    };
+    static const Form forms[] = {
+        {3, 1, {1.4f, 2.1f, 2.1f}, {0.384f, 0.407f, 0.527f}}, {4, 1, {1.7f, 1.8f, 1.9f}, {0.390f, 0.480f, 0.583f}},
+        {6, 1, {1.75f, 2.2f, 2.2f}, {0.450f, 0.550f, 0.656f}}, {8, 1, {1.9f, 2.2f, 2.2f}, {0.530f, 0.680f, 0.790f}},
+        {3, 2, {2.1f, 3.0f, 2.9f}, {0.516f, 0.620f, 0.900f}}, {4, 2, {2.2f, 2.5f, 2.5f}, {0.555f, 0.745f, 1.020f}},
+        {6, 2, {2.6f, 2.9f, 3.2f}, {0.650f, 0.910f, 1.150f}}, {8, 2, {3.0f, 3.0f, 3.3f}, {0.760f, 1.170f, 1.370f}},
+    };
+    const int need = (M + 15) / 16;          // row blocks
+    const float out_mb = 4e-6f * (float)M * (float)w.N;
+    ColsPlan best = {0, 0, 1, 1e30f};
+    for (const Form& f : forms) {
+        // up to 128 rows one row tile, the smallest that holds them; beyond, neither 48 rows nor many row tiles of 64
+        if (need <= 8 ? (f.rb < need || (f.rb > 3 && f.rb - (f.rb > 4 ? 2 : 1) >= need)) : (f.rb == 3 || (f.rb == 4 && need > 16))) continue;
+        const int64_t tiles = (int64_t)((w.NT + 4 * f.cs - 1) / (4 * f.cs)) * ((need + f.rb - 1) / f.rb);
+        for (int splits = 1; splits <= kColsSplits; splits++) {
+            const int per = (w.KT + splits - 1) / splits;
+            if (splits > 1 && (per < 4 || (w.KT + per - 1) / per != splits || (splits - 1) * tiles > num_cus ||
+                               (size_t)splits * M * w.N * 4 > part_bytes)) continue;
+            const float rounds = (float)((tiles * splits + num_cus - 1) / num_cus);
+            const float us = rounds * (f.fixed[mode] + f.per_kt[mode] * (float)per) +
+                             (splits > 1 ? 2.2f + 0.5f * ((float)splits + 0.5f) * out_mb : 0.27f * out_mb);
+            if (us < best.us) best = {f.rb, f.cs, splits, us};
+        }
+    }
+    return best;
+}
+
+hipError_t launch_gemm_cols(const WeightView& w, const void* x_staged, int mode, int M, void* y, int ydt, const ColsPlan& plan, const Epilogue& epi,
+                            const float* ssq_part, int ssq_blocks, const float* unscale, float* part, hipStream_t st)
+{
+    const NormStats ns = {ssq_part, ssq_blocks, unscale};
+    auto go = [&](auto bits, auto md, auto r, auto c) {
+        return launch_cols_t<decltype(bits)::value, decltype(md)::value, decltype(r)::value, decltype(c)::value>(w, x_staged, M, y, ydt, plan.splits, epi, ns, part, st);
+    };
+    using i0 = std::integral_constant<int, 0>;
+    using i1 = std::integral_constant<int, 1>;
+    using i2 = std::integral_constant<int, 2>;
+    using i3 = std::integral_constant<int, 3>;
+    using i4 = std::integral_constant<int, 4>;
+    using i6 = std::integral_constant<int, 6>;
+    using i8 = std::integral_constant<int, 8>;
+    auto rows = [&](auto bits, auto md, auto cs) {
+        if (plan.rb == 3) return go(bits, md, i3{}, cs);
+        if (plan.rb == 4) return go(bits, md, i4{}, cs);
+        if (plan.rb == 6) return go(bits, md, i6{}, cs);
+        if (plan.rb == 8) return go(bits, md, i8{}, cs);
+        return hipErrorInvalidValue;
+    };
+    auto shape = [&](auto bits, auto md) { return plan.cs == 1 ? rows(bits, md, i1{}) : rows(bits, md, i2{}); };
+    if (w.bits == 4) return mode == 0 ? shape(i4{}, i0{}) : mode == 1 ? shape(i4{}, i1{}) : shape(i4{}, i2{});
+    return mode == 0 ? shape(i8{}, i0{}) : mode == 1 ? shape(i8{}, i1{}) : shape(i8{}, i2{});
+}
+
+}  // namespace cybq

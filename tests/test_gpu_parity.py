@@ -1087,6 +1087,91 @@ def test_prefill_few_rows_long_k_shares(backend, oracle, bits, shape):
     qw.free()
 
 
+# (FAST needs K outside 2048 .. 8192 or more than 512 rows to get past the few-row kernel)
+COLS = [("exact", 1030, 33 * 128 - 32, 67), ("exact", 1024, 128, 97), ("exact", 4096, 4096, 128), ("exact", 14336, 288, 193),
+        ("exact", 520, 12 * 128 + 64, 260), ("exact", 9000, 640, 80), ("exact", 14400, 2048, 33),
+        ("fast", 1030, 9 * 128 - 32, 100), ("fast", 520, 128, 129), ("fast", 24640, 70 * 128 + 64, 48), ("fast", 30000, 1056, 64),
+        ("fast", 2064, 12288, 200), ("fast", 16400, 8320, 96), ("fast", 1040, 1920, 250)]
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("mode,N,K,M", COLS)
+def test_prefill_waves_side_by_side(backend, oracle, bits, mode, N, K, M):
+    """The kernel whose waves stand side by side and share out every K tile: one K tile, fewer than the copies reach ahead, a last
+    K tile that is a quarter, half, three quarters full, K shared out over workgroups, each of its row and column counts, a last row
+    and column tile that are not full, N that is no multiple of 16 or 4, y off its vector alignment, every epilogue.  Against
+    float64; against the tiled kernels (another order of summation: it did run); reproducible."""
+    q, s = _quant(oracle, bits, N, K, cfg=131)
+    qw = backend.upload_quantized(q, s, bits)
+    wd = torch.from_numpy(oracle.dequant(q, s)).cuda().double()
+    r = torch.from_numpy(synth.activations(133, M, N)).cuda()
+    bar = TIGHT if mode == "exact" else FAST
+    backend.set_prefill_mode(mode)
+    try:
+        for xdt in ("bf16", "f16"):
+            x = _x(M, K, xdt, cfg=132)
+            xd = x.double()
+            z = xd @ wd.T
+            y = _run(backend, qw, x)
+            assert ((y.double() - z).norm() / z.norm()).item() < bar, xdt
+            assert torch.equal(_run(backend, qw, x), y)
+            backend.set_gemm_tuning(3)
+            y_tiled = _run(backend, qw, x)
+            backend.set_gemm_tuning(0)
+            assert ((y - y_tiled).double().norm() / z.norm()).item() < (2e-6 if mode == "exact" else 2 * bar), xdt
+            if M > 64 or mode == "fast":                   # (up to 64 rows a small weight is two decode passes there)
+                assert K <= 256 or not torch.equal(y, y_tiled), xdt
+            for ydt, off in (("f32", 1), ("bf16", 0), ("f16", 3)):
+                y2 = torch.empty(M * N + 4, dtype=TDT[ydt], device="cuda")[off:off + M * N].view(M, N)
+                r2 = torch.empty_like(y2).copy_(r)
+                backend.matmul_ex(qw, x, y2, "add", r2)
+                want = z + r2.double()
+                assert ((y2.double() - want).norm() / want.norm()).item() < (bar if ydt == "f32" else 4e-3), (xdt, ydt)
+            gamma = (1.0 + 0.1 * torch.from_numpy(synth.activations(134, 1, K))[0]).cuda()
+            y3 = torch.empty((M, N), dtype=torch.float32, device="cuda")
+            backend.matmul_norm(qw, x, gamma, 1e-5, y3)
+            ref = (xd * torch.rsqrt((xd * xd).mean(dim=1, keepdim=True) + 1e-5) * gamma.double()) @ wd.T
+            assert ((y3.double() - ref).norm() / ref.norm()).item() < (4e-3 if mode == "exact" else 2 * FAST), xdt    # (x * gamma rounded)
+            if N % 16 == 0:
+                pair = backend.fuse_pairs(qw, qw)
+                y4 = torch.empty((M, N), dtype=torch.float32, device="cuda")
+                backend.matmul_ex(pair, x, y4, "swiglu")
+                ref = torch.nn.functional.silu(z) * z
+                assert ((y4.double() - ref).norm() / ref.norm()).item() < 4 * bar, xdt
+                pair.free()
+    finally:
+        backend.set_gemm_tuning(0)
+        backend.set_prefill_mode("fast")
+    qw.free()
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("xdt", ["bf16", "f16"])
+def test_prefill_exact_operands_over_all_scales(backend, bits, xdt):
+    """EXACT mode: the two operands of a weight add up to scale * q for subnormal, negative and large scales alike (every output
+    column has scales of one binade of its own; the largest keeps scale * q inside f16)."""
+    N, K, M = 37 * 16, 384, 80
+    rng = np.random.default_rng(7)
+    top = 11 if bits == 4 else 7                            # 2^12 * 8, 2^8 * 128
+    e = np.arange(N) % (top + 25) - 24
+    s = ((2.0 ** e)[:, None] * (1 + rng.random((N, K // 32))) * rng.choice([-1, 1], (N, K // 32))).astype(np.float16).view(np.uint16)
+    q = rng.integers(-(1 << (bits - 1)), 1 << (bits - 1), (N, K)).astype(np.int8)
+    qw = backend.upload_quantized(q, s, bits)
+    wd = torch.from_numpy(np.repeat(s.view(np.float16).astype(np.float64), 32, axis=1) * q).cuda()
+    x = _x(M, K, xdt, cfg=135)
+    backend.set_prefill_mode("exact")
+    try:
+        y = _run(backend, qw, x).double()
+    finally:
+        backend.set_prefill_mode("fast")
+    ref = x.double() @ wd.T
+    # fp32 sums: 1e-6; a Q8 weight's second bf16 operand is rounded to eight bits: 2^-17 of the weight; an f16 operand of the smallest
+    # scales is a subnormal with up to ten leading zeros, and the matrix pipe aligns its 24 bits by exponent fields: 2^(10 - 24)
+    bar = 6.2e-5 if xdt == "f16" else 1e-5 if bits == 8 else 2e-6
+    assert ((y - ref).norm(dim=0) / ref.norm(dim=0)).max().item() < bar
+    qw.free()
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("N,M,pair", [(28672, 300, True), (28672, 257, True), (32 * 1083, 512, True), (20000, 300, False),
                                       (24998, 700, False), (20016, 512, False)])
