@@ -54,18 +54,20 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
 // (gemm_rows.hip); ssq_part / ssq_blocks / unscale: the staging pass's per-row statistics
 struct RowsPlan {
     int nf;                  // column blocks of 16 per workgroup (1, 2 or 4); 0: the kernel does not take the call
-    int shares;              // > 0: K is cut into that many shares, one per wave; more than four go to shares - 3 slabs, fp32 [M][N]
     bool two_per_cu = false; // two workgroups share a CU (nf = 4, up to 48 rows)
 };
 RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi);
 hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, void* y, int ydt, const Epilogue& epi,
-                            const float* ssq_part, int ssq_blocks, const float* unscale, const RowsPlan& plan, float* slabs, hipStream_t st);
+                            const float* ssq_part, int ssq_blocks, const float* unscale, const RowsPlan& plan, hipStream_t st);
 // the prefill kernel whose waves stand side by side along the columns (gemm_cols.hip).  mode: 0 FAST, 1 / 2 EXACT with f16 / bf16
 // operands; more than one split leaves fp32 slabs [splits][M][N] in `part` for the slab-adding pass
 struct ColsPlan {
     int rb, cs, splits;      // row blocks of 16 per workgroup, strips per wave, workgroups that share out K (none of them empty)
+    bool whole_tiles;        // eight waves of one strip that take whole K tiles: the tiled kernels' order of sums, bit for bit
     float us;                // estimate of its time behind the staging pass
 };
+// FAST, a long K and few rows on an output that the tiled kernels split K for three ways or more (rb = 0: another call)
+ColsPlan plan_gemm_cols_long_k(const WeightView& w, int M, int num_cus, const Epilogue& epi);
 ColsPlan plan_gemm_cols(const WeightView& w, int mode, int M, int num_cus, size_t part_bytes);
 hipError_t launch_gemm_cols(const WeightView& w, const void* x_staged, int mode, int M, void* y, int ydt, const ColsPlan& plan, const Epilogue& epi,
                             const float* ssq_part, int ssq_blocks, const float* unscale, float* part, hipStream_t st);

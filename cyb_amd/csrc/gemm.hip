@@ -829,6 +829,10 @@ static float tiled_plan(const WeightView& w, int M, bool exact, int num_cus, siz
 static TilePlan plan_tiles(const WeightView& w, int M, bool exact, bool bf16, int num_cus, size_t part_bytes, const Epilogue& epi)
 {
     TilePlan plan = {};
+    if (!exact && g_rows_kernel < 2) {
+        const ColsPlan cols = plan_gemm_cols_long_k(w, M, num_cus, epi);
+        if (cols.rb) return {TilePlan::kCols, 0, 0, 0, cols.splits, cols};
+    }
     const float tiled = tiled_plan(w, M, exact, num_cus, part_bytes, epi, plan);
     if (tiled < 0.f || g_rows_kernel == 3 || (g_rows_kernel == 2 && !exact)) return plan;
     const ColsPlan cols = plan_gemm_cols(w, !exact ? 0 : bf16 ? 2 : 1, M, num_cus, part_bytes);
@@ -1146,15 +1150,13 @@ void set_gemm_tuning(int rows_kernel) { g_rows_kernel = rows_kernel >= 5 ? 0 : r
 
 static RowsPlan rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
-    if (g_rows_kernel == 2 || g_rows_kernel == 3) return {0, 0};
+    if (g_rows_kernel == 2 || g_rows_kernel == 3) return {0};
     return gemm_rows_plan(w, M, g_rows_kernel == 1 ? 1 : num_cus, epi);
 }
 
-// (the calls whose way here api.hip decides by this; a long K takes the kernel only where the tiled ones would have run)
 bool gemm_rows_takes(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
-    const RowsPlan plan = rows_plan(w, M, num_cus, epi);
-    return plan.nf != 0 && plan.shares == 0;
+    return rows_plan(w, M, num_cus, epi).nf != 0;
 }
 
 // the extra workgroups of a staging launch (grid_x grows by them) for a call of 33 rows or more that goes through the
@@ -1182,7 +1184,6 @@ static Touch plan_touch(const WeightView& w, int mc, int num_cus, const Epilogue
     if (plan.nf) {
         nf = plan.nf;
         groups = (w.NT + nf - 1) / nf;
-        if (plan.shares) return tc;
     } else if (g_touch >= 2 && per_k_tile * w.KT <= ((int64_t)40 << 20) && few_rows_tiles64(w, mc, num_cus, ec)) {
         // the 128 x 64 / 64 x 64 tiles of the tiled kernels (65 .. 128 rows on wide outputs; 4096 -> 14336 at 128 rows:
         // 27.5 us, 24.3 with the same tensor every call): 4096 -> 14336 at 65 / 100 / 128 rows 25.3 / 27.1 / 28.1 ->
@@ -1289,10 +1290,9 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         // few rows on a wide output, FAST mode: the kernel of gemm_rows.hip (waves split K, no LDS on the way)
-        const RowsPlan plan = !exact && kdt == kF16 ? rows_plan(w, mc, num_cus, ec) : RowsPlan{0, 0};
+        const RowsPlan plan = !exact && kdt == kF16 ? rows_plan(w, mc, num_cus, ec) : RowsPlan{0};
         if (plan.nf) {
-            e = launch_gemm_rows(w, workspace, mc, yc, ydt, ec, ns.part, ns.nblk, ns.unscale, plan, part, st);
-            if (e == hipSuccess && plan.shares > 4) e = launch_reduce(part, plan.shares - 3, mc, w.N, yc, ydt, out_scale, ec, ns, w.K, st);
+            e = launch_gemm_rows(w, workspace, mc, yc, ydt, ec, ns.part, ns.nblk, ns.unscale, plan, st);
             if (e != hipSuccess) return e;
             continue;
         }

@@ -1,7 +1,8 @@
 // gemm_cols.hip - prefill kernel whose waves stand side by side along the columns and share out every K tile.
 //
-// Workgroup = 8 waves, output tile 16 * RB rows x 64 * CS columns.  Wave (col, kh) owns CS strips of 16 columns against ALL rows and,
-// of every K tile, the two scale groups of half kh; the halves' sums meet in LDS once at the end.
+// Workgroup = 8 waves, output tile 16 * RB rows x 64 * CS columns (KH = 2).  Wave (col, kh) owns CS strips of 16 columns against ALL rows and,
+// of every K tile, the two scale groups of half kh; the halves' sums meet in LDS once at the end.  KH = 1: eight waves side by side,
+// whole K tiles (a long K on few rows, plan_gemm_cols_long_k).
 //
 //   W  a native tile is multiplied by the two waves that hold its groups and by nobody else: its words go from LDS to registers,
 //      are dequantised there and are MFMA operands as they stand - no operand goes through LDS, none is made twice.
@@ -61,20 +62,23 @@ template <int N>
 __device__ __forceinline__ void wait_copies() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
 // MODE 0: FAST (one f16 operand per weight), 1 / 2: EXACT with f16 / bf16 operands (hi and lo)
-template <int BITS, int MODE, int RB, int CS>
+template <int BITS, int MODE, int RB, int CS, int KH>
 struct ColsShape {
     static constexpr int OPS = MODE == 0 ? 1 : 2;
-    static constexpr int STRIPS = 4 * CS;
+    static constexpr int COLS = 8 / KH;                                    // waves side by side
+    static constexpr int STRIPS = COLS * CS;
+    static constexpr int GROUPS = 4 / KH;                                  // scale groups of a K tile per wave
+    static constexpr int WORDS = BITS / 2 * GROUPS / 2;                    // and packed words per lane
     static constexpr int XTILE = RB * 4096;                                // bytes of a K tile of X
     static constexpr int WSCALES = STRIPS * 1024 * (BITS / 4);             // scales behind the q words
     static constexpr int WTILE = WSCALES + STRIPS * 128;
-    static constexpr bool FOLDED = BITS == 4 && CS == 1;                   // four waves copy q words, the other four scales
+    static constexpr bool FOLDED = BITS == 4 && STRIPS == 4;               // four waves copy q words, the other four scales
     static constexpr int XCOPIES = (RB * 4 + 7) / 8;                       // per wave and K tile
     static constexpr int QCOPIES = FOLDED ? 1 : STRIPS * (BITS / 4) / 8;
     static constexpr int WCOPIES = FOLDED ? 1 : QCOPIES + 1;
     static constexpr int BUDGET = 156 * 1024;
     // K tiles of X in flight: three where a tile is long, up to five where it is short; weights get the rest
-    static constexpr int NX = RB >= 8 ? 3 : RB >= 6 ? (BITS * CS > 8 ? 3 : 4) : RB >= 4 && BITS * CS > 8 ? 4 : 5;
+    static constexpr int NX = RB >= 8 ? 3 : RB >= 6 ? (BITS * STRIPS > 32 ? 3 : 4) : RB >= 4 && BITS * STRIPS > 32 ? 4 : 5;
     static constexpr int NWFIT = (BUDGET - NX * XTILE) / WTILE;
     static constexpr int NW = NWFIT > 10 ? 10 : NWFIT;
     // copies that may be outstanding when a K tile's X and words have to be there, `newer` batches behind the one with its X
@@ -86,13 +90,13 @@ struct ColsShape {
     static_assert(NW >= NX && LDS <= 160 * 1024, "LDS");
 };
 
-template <int BITS, int MODE, int RB, int CS>
+template <int BITS, int MODE, int RB, int CS, int KH>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_cols_kernel(
     const uint8_t* __restrict__ wbase, const uint8_t* __restrict__ x, int KT_, int NT, int x_row_blocks, int M, int n_tiles, int m_tiles,
     int splits, int kt_per_split, int groups, int N, void* __restrict__ y, int ydt, int K, float* __restrict__ part, Epilogue epi, NormStats ns)
 {
-    using S = ColsShape<BITS, MODE, RB, CS>;
-    constexpr int NX = S::NX, NW = S::NW, XC = S::XCOPIES, WC = S::WCOPIES, OPS = S::OPS;
+    using S = ColsShape<BITS, MODE, RB, CS, KH>;
+    constexpr int NX = S::NX, NW = S::NW, XC = S::XCOPIES, WC = S::WCOPIES, OPS = S::OPS, GROUPS = S::GROUPS, WORDS = S::WORDS;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int per_xcd = groups >> 3;
     const int item = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
@@ -103,7 +107,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int tile_n = __builtin_amdgcn_readfirstlane(rest / m_tiles), tile_m = rest - tile_n * m_tiles;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int col = wave & 3, kh = wave >> 2;                  // my strips, my half of every K tile
+    const int col = wave % S::COLS, kh = wave / S::COLS;       // my strips, my half of every K tile (KH = 1: all of it)
     const int m0 = tile_m * (RB * 16);
     const int nt0 = tile_n * S::STRIPS;                        // first strip of the workgroup
     const int kt_lo = split * kt_per_split;
@@ -156,42 +160,48 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
     // ---- LDS -> registers
     Frag16 a[2][RB], b[2][OPS][CS];
-    uint32_t wq[CS][BITS / 2], wn[CS][BITS / 2], sq[CS], sn[CS];           // packed weights and scales (my two groups): this K tile's, the next one's
-    auto read_a = [&](Frag16& dst, int buf, int j, int i) {               // j: 0 / 1 of my two groups
-        dst.u = *reinterpret_cast<const u32x4_t*>(smem + buf * S::XTILE + kh * 2048 + lane * 16 + (i * 4 + j) * 1024);
+    uint32_t wq[CS][WORDS], wn[CS][WORDS], sq[CS][GROUPS / 2], sn[CS][GROUPS / 2];     // packed weights and scales of my groups: this K tile's, the next one's
+    auto read_a = [&](Frag16& dst, int buf, int j, int i) {               // j: which of my groups
+        dst.u = *reinterpret_cast<const u32x4_t*>(smem + buf * S::XTILE + kh * (GROUPS * 1024) + lane * 16 + (i * 4 + j) * 1024);
     };
-    auto read_w = [&](int buf, uint32_t (&q)[CS][BITS / 2], uint32_t (&sc)[CS]) {
+    auto read_w = [&](int buf, uint32_t (&q)[CS][WORDS], uint32_t (&sc)[CS][GROUPS / 2]) {
         const uint8_t* p = smem + S::WBASE + buf * S::WTILE;
 #pragma unroll
         for (int s = 0; s < CS; s++) {
-            if constexpr (BITS == 4) {
-                const u32x2_t v = *reinterpret_cast<const u32x2_t*>(p + (col * CS + s) * 1024 + lane * 16 + kh * 8);
+            const int strip = col * CS + s;
+            if constexpr (BITS == 4 && KH == 2) {
+                const u32x2_t v = *reinterpret_cast<const u32x2_t*>(p + strip * 1024 + lane * 16 + kh * 8);
                 q[s][0] = v[0];
                 q[s][1] = v[1];
             } else {
-                const u32x4_t v = *reinterpret_cast<const u32x4_t*>(p + (col * CS + s) * 2048 + kh * 1024 + lane * 16);
 #pragma unroll
-                for (int e = 0; e < 4; e++) q[s][e & (BITS / 2 - 1)] = v[e];
+                for (int h = 0; h < WORDS / 4; h++) {
+                    const u32x4_t v = *reinterpret_cast<const u32x4_t*>(p + strip * (1024 * (BITS / 4)) + (kh + h) * 1024 + lane * 16);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) q[s][(h * 4 + e) & (WORDS - 1)] = v[e];
+                }
             }
-            sc[s] = *reinterpret_cast<const uint32_t*>(p + S::WSCALES + (col * CS + s) * 128 + (lane & 15) * 8 + kh * 4);
+            const uint32_t* sp = reinterpret_cast<const uint32_t*>(p + S::WSCALES + strip * 128 + (lane & 15) * 8 + kh * 4);
+#pragma unroll
+            for (int g = 0; g < GROUPS / 2; g++) sc[s][g] = sp[g];
         }
     };
     uint32_t magic_lo, magic_hi;
     asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(magic_lo));
     asm volatile("v_mov_b32 %0, 0x54005400" : "=v"(magic_hi));
     // slots 2p, 2p + 1 of my group j in f16, plus a bias (kBias): 1024 + u, 64 + u (odd group of Q4) or 1024 + u with u = q + 128 (Q8)
-    auto biased = [&](const uint32_t (&q)[BITS / 2], int j, int p) {
+    auto biased = [&](const uint32_t (&q)[WORDS], int j, int p) {
         if constexpr (BITS == 4) {
-            const uint32_t src = q[p >> 1] >> (8 * (p & 1));
-            return as_h2(j ? (src & 0x00F000F0u) | magic_hi : (src & 0x000F000Fu) | magic_lo);
+            const uint32_t src = q[(2 * (j >> 1) + (p >> 1)) & (WORDS - 1)] >> (8 * (p & 1));
+            return as_h2((j & 1) ? (src & 0x00F000F0u) | magic_hi : (src & 0x000F000Fu) | magic_lo);
         } else {
-            return as_h2(__builtin_amdgcn_perm(0x64646464u, q[(2 * j + (p >> 1)) & (BITS / 2 - 1)], (p & 1) ? 0x04030402u : 0x04010400u));
+            return as_h2(__builtin_amdgcn_perm(0x64646464u, q[(2 * j + (p >> 1)) & (WORDS - 1)], (p & 1) ? 0x04030402u : 0x04010400u));
         }
     };
-    auto operand = [&](const uint32_t (&q)[BITS / 2], uint32_t sc, int j, int p, int buf, int s) {
+    auto operand = [&](const uint32_t (&q)[WORDS], const uint32_t (&sc)[GROUPS / 2], int j, int p, int buf, int s) {
         const half2_t v = biased(q, j, p);
-        const float bias = BITS == 8 ? -1152.0f : j ? -72.0f : -1032.0f;
-        const uint32_t bits16 = j ? sc >> 16 : sc & 0xffffu;
+        const float bias = BITS == 8 ? -1152.0f : (j & 1) ? -72.0f : -1032.0f;
+        const uint32_t bits16 = (j & 1) ? sc[j >> 1] >> 16 : sc[j >> 1] & 0xffffu;
         const _Float16 sh = __builtin_bit_cast(_Float16, (uint16_t)bits16);
         if constexpr (MODE != 2) {
             const half2_t s2 = {sh, sh}, n = v + (half2_t){(_Float16)bias, (_Float16)bias};          // exact integers
@@ -244,9 +254,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     auto k_tile = [&](int kt, auto phase_) {
         constexpr int PHASE = decltype(phase_)::value;
         const int xnext = xbuf + 1 == NX ? 0 : xbuf + 1, wnext = wbuf + 1 == NW ? 0 : wbuf + 1;
-        static_for<0, 2>([&](auto j_) {
-            constexpr int j = decltype(j_)::value, nxt = 1 - j;
-            if constexpr (j == 1) {
+        static_for<0, GROUPS>([&](auto j_) {
+            constexpr int j = decltype(j_)::value, cur = j & 1, nxt = 1 - cur;
+            constexpr bool last = j == GROUPS - 1;
+            if constexpr (last) {
                 // all copies of the next K tile are in LDS, and nobody reads this one's any more
                 if constexpr (PHASE == 0) {
                     wait_copies<S::allowed(NX - 2)>();
@@ -265,18 +276,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             constexpr int MMAS = RB * CS * OPS, PAIRS = 4 * CS;
             static_for<0, MMAS>([&](auto m_) {
                 constexpr int m = decltype(m_)::value, i = m / (CS * OPS), o = (m / CS) % OPS, s = m % CS;
-                if constexpr (MODE == 2) acc[i][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j][i].b, b[j][o][s].b, acc[i][s], 0, 0, 0);
-                else acc[i][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j][i].h, b[j][o][s].h, acc[i][s], 0, 0, 0);
-                if constexpr (s == 0 && o == 0) read_a(a[nxt][i], j ? xnext : xbuf, nxt, i);
+                if constexpr (MODE == 2) acc[i][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[cur][i].b, b[cur][o][s].b, acc[i][s], 0, 0, 0);
+                else acc[i][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[cur][i].h, b[cur][o][s].h, acc[i][s], 0, 0, 0);
+                if constexpr (s == 0 && o == 0) read_a(a[nxt][i], last ? xnext : xbuf, last ? 0 : j + 1, i);
                 // (the next K tile's words have just been asked for: the second half of the group is theirs; a form that read them a
                 // K tile earlier and spread their arithmetic over the whole group was 3 % slower)
-                constexpr int F = j ? MMAS / 2 : 0, p0 = m < F ? 0 : (m - F) * PAIRS / (MMAS - F), p1 = m < F ? 0 : (m - F + 1) * PAIRS / (MMAS - F);
+                constexpr int F = last ? MMAS / 2 : 0, p0 = m < F ? 0 : (m - F) * PAIRS / (MMAS - F), p1 = m < F ? 0 : (m - F + 1) * PAIRS / (MMAS - F);
                 static_for<p0, p1>([&](auto q_) {
                     constexpr int q = decltype(q_)::value, ds = q / 4, p = q & 3;
-                    if constexpr (j == 1) operand(wn[ds], sn[ds], 0, p, 0, ds);
-                    else operand(wq[ds], sq[ds], 1, p, 1, ds);
+                    if constexpr (last) operand(wn[ds], sn[ds], 0, p, nxt, ds);
+                    else operand(wq[ds], sq[ds], j + 1, p, nxt, ds);
                 });
-                if constexpr (j == 1 && PHASE < 2) {
+                if constexpr (last && PHASE < 2) {
                     constexpr int ALL = PHASE == 0 ? XC + WC : XC;
                     static_for<m * ALL / MMAS, (m + 1) * ALL / MMAS>([&](auto c_) {
                         constexpr int c = decltype(c_)::value;
@@ -291,9 +302,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         wbuf = wnext;
 #pragma unroll
         for (int s = 0; s < CS; s++) {
-            sq[s] = sn[s];
 #pragma unroll
-            for (int e = 0; e < BITS / 2; e++) wq[s][e] = wn[s][e];
+            for (int g = 0; g < GROUPS / 2; g++) sq[s][g] = sn[s][g];
+#pragma unroll
+            for (int e = 0; e < WORDS; e++) wq[s][e] = wn[s][e];
         }
     };
     int kt = 0;
@@ -307,29 +319,30 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     float* const rowf = reinterpret_cast<float*>(smem + S::TILE);
     const bool slab = splits > 1;
     const int row16 = lane & 15, oct = lane >> 4;
-    if (kh == 1) {
+    if (tid < RB * 16) rowf[tid] = slab || !(epi.gamma || ns.unscale) ? 1.0f : row_factor(ns, epi.gamma != nullptr, min(m0 + tid, M - 1), K, epi.eps);
+    if (kh == KH - 1) {
 #pragma unroll
         for (int i = 0; i < RB; i++)
 #pragma unroll
             for (int s = 0; s < CS; s++)
 #pragma unroll
                 for (int r = 0; r < 4; r++) tile[(i * 16 + oct * 4 + r) * S::PITCH + (col * CS + s) * 16 + row16] = acc[i][s][r];
-    } else if (tid < RB * 16) {
-        rowf[tid] = slab || !(epi.gamma || ns.unscale) ? 1.0f : row_factor(ns, epi.gamma != nullptr, min(m0 + tid, M - 1), K, epi.eps);
     }
     __syncthreads();
-    if (kh == 0) {
+    if constexpr (KH == 2) {
+        if (kh == 0) {
 #pragma unroll
-        for (int i = 0; i < RB; i++)
+            for (int i = 0; i < RB; i++)
 #pragma unroll
-            for (int s = 0; s < CS; s++)
+                for (int s = 0; s < CS; s++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    float* t = &tile[(i * 16 + oct * 4 + r) * S::PITCH + (col * CS + s) * 16 + row16];
-                    *t = acc[i][s][r] + *t;
-                }
+                    for (int r = 0; r < 4; r++) {
+                        float* t = &tile[(i * 16 + oct * 4 + r) * S::PITCH + (col * CS + s) * 16 + row16];
+                        *t = acc[i][s][r] + *t;
+                    }
+        }
+        __syncthreads();
     }
-    __syncthreads();
     const bool swiglu = !slab && epi.kind == kEpiSwiglu, add = !slab && epi.kind == kEpiAdd;
     if (slab) {
         y = part + (int64_t)split * M * N;
@@ -394,16 +407,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
-template <int BITS, int MODE, int RB, int CS>
+template <int BITS, int MODE, int RB, int CS, int KH>
 hipError_t launch_cols_t(const WeightView& w, const void* x, int M, void* y, int ydt, int splits, const Epilogue& epi, const NormStats& ns,
                          float* part, hipStream_t st)
 {
-    using S = ColsShape<BITS, MODE, RB, CS>;
-    (void)LdsRequest<&gemm_cols_kernel<BITS, MODE, RB, CS>, S::LDS>::registered;
+    using S = ColsShape<BITS, MODE, RB, CS, KH>;
+    (void)LdsRequest<&gemm_cols_kernel<BITS, MODE, RB, CS, KH>, S::LDS>::registered;
     const int n_tiles = (w.NT + S::STRIPS - 1) / S::STRIPS, m_tiles = (M + 16 * RB - 1) / (16 * RB);
     const int kt_per_split = (w.KT + splits - 1) / splits;
     const unsigned groups = (unsigned)(((int64_t)n_tiles * m_tiles * splits + 7) / 8 * 8);
-    hipLaunchKernelGGL((gemm_cols_kernel<BITS, MODE, RB, CS>), dim3(groups), dim3(512), S::LDS, st, w.base, static_cast<const uint8_t*>(x),
+    hipLaunchKernelGGL((gemm_cols_kernel<BITS, MODE, RB, CS, KH>), dim3(groups), dim3(512), S::LDS, st, w.base, static_cast<const uint8_t*>(x),
                        w.KT, w.NT, (M + 15) / 16, M, n_tiles, m_tiles, splits, kt_per_split, (int)groups, w.N, y, ydt, w.K, part, epi, ns);
     return hipGetLastError();
 }
@@ -429,7 +442,7 @@ ColsPlan plan_gemm_cols(const WeightView& w, int mode, int M, int num_cus, size_
     };
     const int need = (M + 15) / 16;          // row blocks
     const float out_mb = 4e-6f * (float)M * (float)w.N;
-    ColsPlan best = {0, 0, 1, 1e30f};
+    ColsPlan best = {0, 0, 1, false, 1e30f};
     for (const Form& f : forms) {
         // up to 128 rows one row tile, the smallest that holds them; beyond, neither 48 rows nor many row tiles of 64
         if (need <= 8 ? (f.rb < need || (f.rb > 3 && f.rb - (f.rb > 4 ? 2 : 1) >= need)) : (f.rb == 3 || (f.rb == 4 && need > 16))) continue;
@@ -441,10 +454,33 @@ ColsPlan plan_gemm_cols(const WeightView& w, int mode, int M, int num_cus, size_
             const float rounds = (float)((tiles * splits + num_cus - 1) / num_cus);
             const float us = rounds * (f.fixed[mode] + f.per_kt[mode] * (float)per) +
                              (splits > 1 ? 2.2f + 0.5f * ((float)splits + 0.5f) * out_mb : 0.27f * out_mb);
-            if (us < best.us) best = {f.rb, f.cs, splits, us};
+            if (us < best.us) best = {f.rb, f.cs, splits, false, us};
         }
     }
     return best;
+}
+
+// K of more than 64 tiles, up to 128 rows, where the tiled kernels split K three ways or more: that split, eight waves of one strip
+// that take whole K tiles of their share in the tiled kernels' order - their bits - and all shares as slabs.  A CU then takes in one
+// share of X for eight strips.  (Sums in another order are up to 5 % quicker, but through 32 layers of bf16 activations two such runs
+// end 1.3 % apart.)  us per call with all passes, against waves of the few-row kernel with a share each (X once per two strips): 14336 -> 4096
+// bf16 at 45 / 64 / 100 / 128 rows 25.8 / 28.7 / 33.3 / 35.8 -> 23.5 / 24.9 / 30.9 / 33.0, Q8 29.1 / 32.7 / 38.9 / 42.8 -> 25.0 / 26.5 / 32.3 / 34.2, fp32 at 24
+// rows 20.9 -> 20.5; 14336 -> 8192 35.1 / 41.1 / 45.5 / 49.3 -> 30.7 / 33.7 / 44.4 / 46.5; 12288 -> 6144 SwiGLU at 45 / 64 rows 33.8 / 37.7 -> 26.4 / 28.2.
+// Two row tiles beyond 64 rows where both fit one round: 9216 -> 1030 at 100 / 128 rows 22.9 / 24.8 -> 19.7 / 21.0.
+ColsPlan plan_gemm_cols_long_k(const WeightView& w, int M, int num_cus, const Epilogue& epi)
+{
+    const ColsPlan none = {0, 0, 1, false, 0.f};
+    const bool pairs = epi.kind == kEpiSwiglu;
+    if (M <= 16 || M > 128 || w.KT <= 64) return none;
+    if ((w.NT % 7 == 0 && !pairs) || (!pairs && (w.NT + 3) / 4 * 4 >= 3 * num_cus)) return none;
+    const int tiles = (w.NT + 7) / 8;
+    int shares = std::min(kColsSplits, num_cus / tiles);                  // the tiled kernels' K split
+    if (shares < 3) return none;
+    const int per = (w.KT + shares - 1) / shares;
+    shares = (w.KT + per - 1) / per;
+    const int need = (M + 15) / 16;
+    const int rb = need <= 2 ? 2 : need <= 4 ? need : 2 * tiles * shares <= num_cus ? (need <= 6 ? 3 : 4) : need <= 6 ? 6 : 8;
+    return {rb, 1, shares, true, 0.f};
 }
 
 hipError_t launch_gemm_cols(const WeightView& w, const void* x_staged, int mode, int M, void* y, int ydt, const ColsPlan& plan, const Epilogue& epi,
@@ -452,7 +488,7 @@ hipError_t launch_gemm_cols(const WeightView& w, const void* x_staged, int mode,
 {
     const NormStats ns = {ssq_part, ssq_blocks, unscale};
     auto go = [&](auto bits, auto md, auto r, auto c) {
-        return launch_cols_t<decltype(bits)::value, decltype(md)::value, decltype(r)::value, decltype(c)::value>(w, x_staged, M, y, ydt, plan.splits, epi, ns, part, st);
+        return launch_cols_t<decltype(bits)::value, decltype(md)::value, decltype(r)::value, decltype(c)::value, 2>(w, x_staged, M, y, ydt, plan.splits, epi, ns, part, st);
     };
     using i0 = std::integral_constant<int, 0>;
     using i1 = std::integral_constant<int, 1>;
@@ -461,6 +497,17 @@ hipError_t launch_gemm_cols(const WeightView& w, const void* x_staged, int mode,
     using i4 = std::integral_constant<int, 4>;
     using i6 = std::integral_constant<int, 6>;
     using i8 = std::integral_constant<int, 8>;
+    if (plan.whole_tiles) {
+        auto whole = [&](auto bits) {
+            constexpr int B = decltype(bits)::value;
+            if (plan.rb == 2) return launch_cols_t<B, 0, 2, 1, 1>(w, x_staged, M, y, ydt, plan.splits, epi, ns, part, st);
+            if (plan.rb == 3) return launch_cols_t<B, 0, 3, 1, 1>(w, x_staged, M, y, ydt, plan.splits, epi, ns, part, st);
+            if (plan.rb == 4) return launch_cols_t<B, 0, 4, 1, 1>(w, x_staged, M, y, ydt, plan.splits, epi, ns, part, st);
+            if (plan.rb == 6) return launch_cols_t<B, 0, 6, 1, 1>(w, x_staged, M, y, ydt, plan.splits, epi, ns, part, st);
+            return launch_cols_t<B, 0, 8, 1, 1>(w, x_staged, M, y, ydt, plan.splits, epi, ns, part, st);
+        };
+        return w.bits == 4 ? whole(i4{}) : whole(i8{});
+    }
     auto rows = [&](auto bits, auto md, auto cs) {
         if (plan.rb == 3) return go(bits, md, i3{}, cs);
         if (plan.rb == 4) return go(bits, md, i4{}, cs);

@@ -88,15 +88,11 @@ __device__ __forceinline__ void dequant_group(const WRegs<BITS>& r, int j, uint3
 
 // MF row blocks of 16 per workgroup (blockIdx.y-th MF * 16 rows of the call), NF column blocks per workgroup, WAVES
 // waves that split K, DEPTH K tiles of packed weights and XD K tiles of X in flight per wave.
-// SHARES: the K tiles are cut into `shares` runs of kt_per_share, and a wave walks one run (number blockIdx.z * WAVES + wave)
-// from the tile and in the order in which the tiled kernels' K split walks it; the runs' sums are added in their order, the
-// first four here, the others (blockIdx.z = 1: a slab each) with the first four's slab by the slab-adding pass.
-// The result is that of the tiled kernels bit for bit.
 // OCC: workgroups per CU.
-template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD, bool SHARES, int OCC = 1>
+template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD, int OCC = 1>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC * WAVES / 4, OCC * WAVES / 4))) void gemm_rows_kernel(
     const uint8_t* __restrict__ wbase, const u32x4_t* __restrict__ x, int KT_, int NT_, int x_row_blocks, int M, int N_,
-    void* __restrict__ y, int ydt, int K_, Epilogue epi, NormStats ns, int shares, int kt_per_share, float* __restrict__ slabs)
+    void* __restrict__ y, int ydt, int K_, Epilogue epi, NormStats ns)
 {
     const WeightView w = {wbase, N_, K_, NT_, KT_, BITS};
     constexpr int FR = MF * NF;                        // accumulator blocks per wave
@@ -109,20 +105,18 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC 
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nt0 = (int)blockIdx.x * NF;
     const int K = w.K, G = K / kGroup;
-    const int share = (int)blockIdx.z * WAVES + wv;
-    const int kt_lo = SHARES ? min(share * kt_per_share, w.KT - 1) : 0;
-    const int KT = SHARES ? min(kt_per_share, w.KT - kt_lo) : w.KT;      // my K tiles (SHARES: mine alone): kt_lo ..
+    const int KT = w.KT;
     const uint32_t magic = q4_magic_vgpr();
     // my K tiles: number t is tile wv + WAVES * t
-    const int T = SHARES ? (share < shares ? KT : 0) : KT > wv ? (KT - wv + WAVES - 1) / WAVES : 0;
+    const int T = KT > wv ? (KT - wv + WAVES - 1) / WAVES : 0;
     // Workgroups that run side by side read the same rows of X: walking K in the same order they would all
     // ask the same L2 channels for the same lines at the same moment, so every column tile starts its walk
     // at another K tile and wraps around (the order depends on the column tile only, not on M).
-    const int kt0 = SHARES ? (nt0 >> 3) % KT : (int)blockIdx.x % KT;      // (the tiled kernels' column tiles: eight blocks)
+    const int kt0 = (int)blockIdx.x % KT;
     // (a tile number past my last one is clamped to the last K tile: loaded again, never used)
     auto tile_of = [&](int t) __attribute__((always_inline)) {
-        const int kt = min(SHARES ? t : wv + WAVES * t, KT - 1) + kt0;
-        return kt_lo + (kt >= KT ? kt - KT : kt);
+        const int kt = min(wv + WAVES * t, KT - 1) + kt0;
+        return kt >= KT ? kt - KT : kt;
     };
     // (row blocks and column blocks past the end are clamped to the last real one: computed again, never
     // stored; the offsets are wave-uniform, the lane's part of an address is one register)
@@ -184,15 +178,6 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC 
         if (t + decltype(i)::value < T) k_tile(t + decltype(i)::value, i);
     });
 
-    if constexpr (SHARES) {
-        if (blockIdx.z > 0) {
-            const Epilogue plain = {kEpiNone, nullptr, nullptr, 0, 0.f};
-            if (share < shares)
-                write_rows<MF, NF>(acc, reinterpret_cast<float*>(smem) + wv * (16 * NF * 16), rb0 * 16, nt0, M, w.N,
-                                   slabs + (int64_t)(share - WAVES + 1) * M * w.N, kF32, 1.0f, plain, lane);
-            return;
-        }
-    }
     // ---- the partial sums meet: every wave leaves all of its blocks, waves 0 .. MF-1 finish a row block each
 #pragma unroll
     for (int i = 0; i < MF; i++)
@@ -210,13 +195,6 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC 
         tot[0][f] = s;
     }
     const int m0 = (rb0 + wv) * 16;
-    if constexpr (SHARES) {
-        if (shares > WAVES) {
-            const Epilogue plain = {kEpiNone, nullptr, nullptr, 0, 0.f};
-            write_rows<1, NF>(tot, stg + wv * (16 * NF * 16), m0, nt0, M, w.N, slabs, kF32, 1.0f, plain, lane);
-            return;
-        }
-    }
     if (epi.gamma || ns.unscale) {
 #pragma unroll
         for (int r4 = 0; r4 < 4; r4++) {
@@ -240,16 +218,14 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC 
     write_rows<1, NF>(tot, stg + wv * (16 * NF * 16), m0, nt0, M, w.N, y, ydt, 1.0f, epi, lane);
 }
 
-template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD, bool SHARES, int OCC = 1>
-hipError_t launch_rows_t(const WeightView& w, const void* x, int M, void* y, int ydt, const Epilogue& epi, const NormStats& ns, int shares,
-                         float* slabs, hipStream_t st)
+template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD, int OCC = 1>
+hipError_t launch_rows_t(const WeightView& w, const void* x, int M, void* y, int ydt, const Epilogue& epi, const NormStats& ns, hipStream_t st)
 {
     constexpr int lds = WAVES * MF * NF * 1024 + MF * 16 * NF * 16 * 4;
-    (void)LdsRequest<&gemm_rows_kernel<BITS, MF, NF, WAVES, DEPTH, XD, SHARES, OCC>, lds>::registered;
+    (void)LdsRequest<&gemm_rows_kernel<BITS, MF, NF, WAVES, DEPTH, XD, OCC>, lds>::registered;
     const unsigned groups = (unsigned)((w.NT + NF - 1) / NF), row_parts = (unsigned)((M + 16 * MF - 1) / (16 * MF));
-    hipLaunchKernelGGL((gemm_rows_kernel<BITS, MF, NF, WAVES, DEPTH, XD, SHARES, OCC>), dim3(groups, row_parts, SHARES ? (unsigned)((shares + WAVES - 1) / WAVES) : 1u), dim3(WAVES * 64), lds, st,
-                       w.base, reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT, (M + 15) / 16, M, w.N, y, ydt, w.K, epi, ns,
-                       shares, SHARES ? (w.KT + shares - 1) / shares : 0, slabs);
+    hipLaunchKernelGGL((gemm_rows_kernel<BITS, MF, NF, WAVES, DEPTH, XD, OCC>), dim3(groups, row_parts), dim3(WAVES * 64), lds, st,
+                       w.base, reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT, (M + 15) / 16, M, w.N, y, ydt, w.K, epi, ns);
     return hipGetLastError();
 }
 
@@ -262,48 +238,26 @@ hipError_t launch_rows_t(const WeightView& w, const void* x, int M, void* y, int
 // rows: 128 of one 11.6, the tiled kernels 17.5), at least a quarter of a round (4096 -> 1024 at 24 rows, 64
 // workgroups: 11.4 against 17.4), K of at least 16 tiles.  More than 64 rows are one workgroup per 64 rows and column
 // group: narrow outputs only, where all of them fit one round.
-// K of more than 64 tiles, up to 128 rows, where the tiled kernels split K three ways or more: the waves walk one share of
-// that split each, with the fewest column blocks that fit one round.  A CU then takes in its rows' part of K instead of
-// all of it, and no barrier stands between K tiles; same sums, same bits.  Fewer shares leave waves idle, more rows or a
-// wider output are not K-split there.  us per call with all passes, against the tiled kernels (their adding pass included
-// before it was made quicker): 14336 -> 4096 bf16 at 45 / 64 / 96 / 128 rows 26.6 / 30.1 / 33.1 / 36.8 against 36.5 / 37.7 /
-// 39.0 / 39.8, fp32 at 24 rows 21.9 against 36.2, f16 at 45 rows 24.3 against 30.2; 14336 -> 8192 at 45 rows 36.2 against
-// 50.2; 14336 -> 1024 at 100 rows 24.1 against 34.5 (23.4 against 27.6 with that pass as it is now), 12288 -> 512 at 100 / 128 rows
-// 17.3 / 21.6 against 22.0 / 24.7, 9216 -> 512 at 128 rows 15.1 against 18.6.  (Up to 64 rows of 16-bit activations on weights of up to
-// 6144 x 4096 are two decode passes and never get here.)
+// (A longer K: gemm_cols.hip.)
 RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
-    if (M <= 16 || M > 512 || w.KT < 16) return {0, 0};
+    if (M <= 16 || M > 512 || w.KT < 16 || w.KT > 64) return {0};
     const int64_t parts = (M + 63) / 64;
-    if (w.KT > 64) {
-        const bool pairs = epi.kind == kEpiSwiglu;
-        if (M > 128 || (w.NT % 7 == 0 && !pairs) || (!pairs && (w.NT + 3) / 4 * 4 >= 3 * num_cus)) return {0, 0};
-        const int64_t tiles = (w.NT + 7) / 8;
-        int shares = (int)std::min<int64_t>(8, num_cus / tiles);        // the tiled kernels' K split
-        if (shares < 3) return {0, 0};
-        const int per = (w.KT + shares - 1) / shares;
-        shares = (w.KT + per - 1) / per;
-        for (int nf : {1, 2, 4}) {
-            if (nf == 1 && pairs) continue;
-            if ((w.NT + nf - 1) / nf * parts * ((shares + 3) / 4) <= num_cus) return {nf, shares};
-        }
-        return {0, 0};
-    }
     for (int nf : {1, 2, 4}) {
         if (nf == 1 && epi.kind == kEpiSwiglu) continue;        // (a gate block and its up block sit in one workgroup)
         const int64_t groups = (w.NT + nf - 1) / nf * parts;
-        if (groups <= num_cus) return {groups * 4 >= num_cus ? nf : 0, 0};
+        if (groups <= num_cus) return {groups * 4 >= num_cus ? nf : 0};
     }
     // up to 64 rows a wide output may take more than one round.  Up to 48 rows two workgroups share a CU then (two or three
     // packed weight tiles in flight per wave instead of four, 256 registers): one's start and end overlap the other's
     // K loop (4096 -> 28672 bf16 norm + SwiGLU at 45 rows 35.0 -> 30.2 us, fp32 at 24 rows 28.3 -> 25.6, 2048 -> 20000 at 40
     // rows 20.5 -> 17.6, 2048 -> 128256 at 40 rows 71.0 -> 51.1).  With four row blocks they do not fit 256 registers
     // without giving up the lead of the weights: 38.3 against 38.1 us, 35.7 against 36.1.
-    return {parts == 1 ? 4 : 0, 0, parts == 1 && M <= 48};
+    return {parts == 1 ? 4 : 0, parts == 1 && M <= 48};
 }
 
 hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, void* y, int ydt, const Epilogue& epi,
-                            const float* ssq_part, int ssq_blocks, const float* unscale, const RowsPlan& plan, float* slabs, hipStream_t st)
+                            const float* ssq_part, int ssq_blocks, const float* unscale, const RowsPlan& plan, hipStream_t st)
 {
     const NormStats ns = {ssq_part, ssq_blocks, unscale};
     // four waves, one per SIMD with the whole register file: four K tiles of packed weights and one K tile of
@@ -315,33 +269,27 @@ hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, vo
     // Up to 48 rows the workgroup carries two or three row blocks instead of four: the rows of X are most of what
     // a CU takes in, and its L1 delivers 64 bytes a cycle.
     const int mf = M > 48 ? 4 : M > 32 ? 3 : 2;
-    auto go = [&](auto bits, auto nfc, auto split) {
+    auto go = [&](auto bits, auto nfc) {
         constexpr int B = decltype(bits)::value, F = decltype(nfc)::value;
-        constexpr bool S = decltype(split)::value;
-        if (mf == 2) return launch_rows_t<B, 2, F, 4, 4, 1, S>(w, x_staged, M, y, ydt, epi, ns, plan.shares, slabs, st);
-        if (mf == 3) return launch_rows_t<B, 3, F, 4, 4, 1, S>(w, x_staged, M, y, ydt, epi, ns, plan.shares, slabs, st);
-        return launch_rows_t<B, 4, F, 4, 4, 1, S>(w, x_staged, M, y, ydt, epi, ns, plan.shares, slabs, st);
+        if (mf == 2) return launch_rows_t<B, 2, F, 4, 4, 1>(w, x_staged, M, y, ydt, epi, ns, st);
+        if (mf == 3) return launch_rows_t<B, 3, F, 4, 4, 1>(w, x_staged, M, y, ydt, epi, ns, st);
+        return launch_rows_t<B, 4, F, 4, 4, 1>(w, x_staged, M, y, ydt, epi, ns, st);
     };
-    auto with_bits = [&](auto nfc, auto split) {
-        if (w.bits == 8) return go(std::integral_constant<int, 8>{}, nfc, split);
-        return go(std::integral_constant<int, 4>{}, nfc, split);
+    auto with_bits = [&](auto nfc) {
+        if (w.bits == 8) return go(std::integral_constant<int, 8>{}, nfc);
+        return go(std::integral_constant<int, 4>{}, nfc);
     };
     if (plan.two_per_cu) {
         if (w.bits == 8) {
-            if (mf == 2) return launch_rows_t<8, 2, 4, 4, 2, 1, false, 2>(w, x_staged, M, y, ydt, epi, ns, 0, slabs, st);
-            return launch_rows_t<8, 3, 4, 4, 2, 1, false, 2>(w, x_staged, M, y, ydt, epi, ns, 0, slabs, st);
+            if (mf == 2) return launch_rows_t<8, 2, 4, 4, 2, 1, 2>(w, x_staged, M, y, ydt, epi, ns, st);
+            return launch_rows_t<8, 3, 4, 4, 2, 1, 2>(w, x_staged, M, y, ydt, epi, ns, st);
         }
-        if (mf == 2) return launch_rows_t<4, 2, 4, 4, 3, 1, false, 2>(w, x_staged, M, y, ydt, epi, ns, 0, slabs, st);
-        return launch_rows_t<4, 3, 4, 4, 3, 1, false, 2>(w, x_staged, M, y, ydt, epi, ns, 0, slabs, st);
+        if (mf == 2) return launch_rows_t<4, 2, 4, 4, 3, 1, 2>(w, x_staged, M, y, ydt, epi, ns, st);
+        return launch_rows_t<4, 3, 4, 4, 3, 1, 2>(w, x_staged, M, y, ydt, epi, ns, st);
     }
-    if (plan.shares) {
-        if (plan.nf == 1) return with_bits(std::integral_constant<int, 1>{}, std::true_type{});
-        if (plan.nf == 2) return with_bits(std::integral_constant<int, 2>{}, std::true_type{});
-        return with_bits(std::integral_constant<int, 4>{}, std::true_type{});
-    }
-    if (plan.nf == 1) return with_bits(std::integral_constant<int, 1>{}, std::false_type{});
-    if (plan.nf == 2) return with_bits(std::integral_constant<int, 2>{}, std::false_type{});
-    return with_bits(std::integral_constant<int, 4>{}, std::false_type{});
+    if (plan.nf == 1) return with_bits(std::integral_constant<int, 1>{});
+    if (plan.nf == 2) return with_bits(std::integral_constant<int, 2>{});
+    return with_bits(std::integral_constant<int, 4>{});
 }
 
 }  // namespace cybq
