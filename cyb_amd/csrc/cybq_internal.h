@@ -55,6 +55,7 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
 struct RowsPlan {
     int nf;                  // column blocks of 16 per workgroup (1, 2 or 4); 0: the kernel does not take the call
     bool two_per_cu = false; // two workgroups share a CU (nf = 4, up to 48 rows)
+    bool pairs = false;      // one workgroup of eight waves does two column groups (nf = 4)
 };
 RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi);
 hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, void* y, int ydt, const Epilogue& epi,

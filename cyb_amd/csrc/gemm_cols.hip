@@ -48,11 +48,6 @@ __device__ __forceinline__ void static_for(F&& f)
     }
 }
 
-// 16 bytes per lane from base + off (the lane's own) to LDS bytes lds_off + 16 * lane, past the registers
-__device__ __forceinline__ void copy_to_lds(uint32_t lds_off, const void* base, uint32_t off)
-{
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds_off)), "v"(off), "s"(base));
-}
 // the same from the lanes of `lanes` alone (all 64 lanes are active around it; a branch would cut the scheduling region)
 __device__ __forceinline__ void copy_to_lds(uint32_t lds_off, const void* base, uint32_t off, uint64_t lanes)
 {

@@ -47,6 +47,12 @@ __device__ __forceinline__ float row_factor(const NormStats& ns, bool norm, int 
     return f;
 }
 
+// 16 bytes per lane from base + off (the lane's own) to LDS bytes lds_off + 16 * lane, past the registers
+__device__ __forceinline__ void copy_to_lds(uint32_t lds_off, const void* base, uint32_t off)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds_off)), "v"(off), "s"(base));
+}
+
 template <int BITS>
 struct WRegs {               // one native weight tile as loaded by one lane, and its 4 group scales
     u32x4_t q[BITS == 4 ? 1 : 2];

@@ -86,6 +86,34 @@ __device__ __forceinline__ void dequant_group(const WRegs<BITS>& r, int j, uint3
     for (int p = 0; p < 4; p++) b.u[p] = as_u32(as_h2(bw[p]) * s2);
 }
 
+// the finished sums of one row block (first row m0) on their way to y: row factors, SwiGLU, residual
+template <int NF>
+__device__ __forceinline__ void finish_row_block(float4_t (&tot)[1][NF], float* stg, int m0, int nt0, int M, const WeightView& w, void* y, int ydt, int K,
+                                                 const Epilogue& epi, const NormStats& ns, int lane)
+{
+    if (epi.gamma || ns.unscale) {
+#pragma unroll
+        for (int r4 = 0; r4 < 4; r4++) {
+            const float rs = row_factor(ns, epi.gamma != nullptr, min(m0 + (lane >> 4) * 4 + r4, M - 1), K, epi.eps);
+#pragma unroll
+            for (int f = 0; f < NF; f++) tot[0][f][r4] *= rs;
+        }
+    }
+    if constexpr (NF >= 2) {
+        if (epi.kind == kEpiSwiglu) {      // column blocks 2p / 2p+1 are gate / up of output block (nt0 >> 1) + p
+            float4_t act[1][NF / 2];
+#pragma unroll
+            for (int p = 0; p < NF / 2; p++)
+#pragma unroll
+                for (int r4 = 0; r4 < 4; r4++) act[0][p][r4] = silu_mul(tot[0][2 * p][r4], tot[0][2 * p + 1][r4]);
+            const Epilogue plain = {kEpiNone, nullptr, nullptr, 0, 0.f};
+            write_rows<1, NF / 2>(act, stg, m0, nt0 >> 1, M, w.N >> 1, y, ydt, 1.0f, plain, lane);
+            return;
+        }
+    }
+    write_rows<1, NF>(tot, stg, m0, nt0, M, w.N, y, ydt, 1.0f, epi, lane);
+}
+
 // MF row blocks of 16 per workgroup (blockIdx.y-th MF * 16 rows of the call), NF column blocks per workgroup, WAVES
 // waves that split K, DEPTH K tiles of packed weights and XD K tiles of X in flight per wave.
 // OCC: workgroups per CU.
@@ -194,28 +222,146 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC 
         for (int p = 1; p < WAVES; p++) s += part[(p * FR + blk) * 64 + lane];
         tot[0][f] = s;
     }
-    const int m0 = (rb0 + wv) * 16;
-    if (epi.gamma || ns.unscale) {
+    finish_row_block<NF>(tot, stg + wv * (16 * NF * 16), (rb0 + wv) * 16, nt0, M, w, y, ydt, K, epi, ns, lane);
+}
+
+// The same sums for outputs of more than a round of workgroups (up to 64 rows, four column blocks each): one workgroup of eight
+// waves does the work of two, column groups g and g + D.  D is a multiple of KT, so both walk the K tiles from the same one on and
+// wave wv of either half multiplies the same rows of X by its own weights: X comes once, by copies into LDS (a ring of RING steps
+// of four K tiles, each half of a tile copied by the two waves that use it), and the stream into the CUs is half of what two
+// workgroups draw.  What bounds it then is issue: per K tile a wave makes 16 operands of 13 vector instructions each, next to 32,
+// 48 or 64 MFMAs (4096 -> 28672 at 45 rows: 3.4 us before the first step, 8 steps of 3690 cycles in 15.4, 1.9 after).  Bit for
+// bit the result of gemm_rows_kernel.
+// (wbase without __restrict__: the waits below count the weight loads, so none of them may move over an asm that clobbers memory.)
+template <int BITS, int MF, int DEPTH, int RING>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_rows_pair_kernel(
+    const uint8_t* wbase, const uint8_t* x, int KT_, int NT_, int x_row_blocks, int M, int N_,
+    void* __restrict__ y, int ydt, int K_, int D, Epilogue epi, NormStats ns)
+{
+    const WeightView w = {wbase, N_, K_, NT_, KT_, BITS};
+    constexpr int NF = 4, FR = MF * NF;
+    constexpr int XC = 2 * MF;                         // copies of X per wave and step
+    constexpr int WL = NF * (BITS == 4 ? 2 : 3);       // weight loads per wave and step
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w8 = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int half = w8 >> 2, wv = w8 & 3;
+    const int nt0 = ((int)blockIdx.x + half * D) * NF;         // (a second half past the last column group computes and stores nothing of use)
+    const int K = w.K, G = K / kGroup, KT = w.KT;
+    const uint32_t magic = q4_magic_vgpr();
+    const int steps = (KT + 3) / 4, T = KT > wv ? (KT - wv + 3) / 4 : 0;
+    const int kt0 = (int)blockIdx.x % KT;
+    auto tile_of = [&](int t) __attribute__((always_inline)) {
+        const int kt = min(wv + 4 * t, KT - 1) + kt0;
+        return kt >= KT ? kt - KT : kt;
+    };
+    // block e of a K tile of X = row block e / 4, group e % 4; this wave copies 2 * MF of its tile's 4 * MF
+    uint32_t xrow[XC];
 #pragma unroll
-        for (int r4 = 0; r4 < 4; r4++) {
-            const float rs = row_factor(ns, epi.gamma != nullptr, min(m0 + (lane >> 4) * 4 + r4, M - 1), K, epi.eps);
+    for (int c = 0; c < XC; c++) xrow[c] = (uint32_t)min((half * XC + c) >> 2, x_row_blocks - 1) * (uint32_t)(G * 1024);
+    auto copy_x = [&](int t, int ring) __attribute__((always_inline)) {
+        const int kt = tile_of(t);
 #pragma unroll
-            for (int f = 0; f < NF; f++) tot[0][f][r4] *= rs;
+        for (int c = 0; c < XC; c++) {
+            const int e = half * XC + c;
+            copy_to_lds((ring * 4 + wv) * (MF * 4096) + e * 1024, x, xrow[c] + (uint32_t)min(kt * 4 + (e & 3), G - 1) * 1024u + (uint32_t)lane * 16u);
         }
-    }
-    if constexpr (NF >= 2) {
-        if (epi.kind == kEpiSwiglu) {      // column blocks 2p / 2p+1 are gate / up of output block (nt0 >> 1) + p
-            float4_t act[1][NF / 2];
+    };
+    int64_t wtile[NF];
 #pragma unroll
-            for (int p = 0; p < NF / 2; p++)
+    for (int f = 0; f < NF; f++) wtile[f] = (int64_t)min(nt0 + f, w.NT - 1) * w.KT;
+    auto fetch = [&](WRegs<BITS> (&dst)[NF], int t) __attribute__((always_inline)) {
+        const int kt = tile_of(t);
 #pragma unroll
-                for (int r4 = 0; r4 < 4; r4++) act[0][p][r4] = silu_mul(tot[0][2 * p][r4], tot[0][2 * p + 1][r4]);
-            const Epilogue plain = {kEpiNone, nullptr, nullptr, 0, 0.f};
-            write_rows<1, NF / 2>(act, stg + wv * (16 * NF * 16), m0, nt0 >> 1, M, w.N >> 1, y, ydt, 1.0f, plain, lane);
-            return;
+        for (int f = 0; f < NF; f++) load_wtile<BITS>(dst[f], w, wtile[f] + kt, lane);
+    };
+    float4_t acc[MF][NF];
+#pragma unroll
+    for (int i = 0; i < MF; i++)
+#pragma unroll
+        for (int f = 0; f < NF; f++) acc[i][f] = (float4_t){0.f, 0.f, 0.f, 0.f};
+
+    WRegs<BITS> wreg[DEPTH][NF];
+#pragma unroll
+    for (int r = 0; r < RING - 1; r++) copy_x(r, r);
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++) fetch(wreg[d], d);
+    // (a wait for all but the weights asked for behind it)
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(DEPTH * WL > 63 ? 63 : DEPTH * WL) : "memory");
+
+    int ring = 0;
+    auto step = [&](int t, auto residue, bool mine) __attribute__((always_inline)) {
+        constexpr int R = decltype(residue)::value;
+        const int far = ring == 0 ? RING - 1 : ring - 1;       // the step before this one's place: X of step t + RING - 1
+        copy_x(t + RING - 1, far);
+        const uint8_t* xl = smem + (ring * 4 + wv) * (MF * 4096) + lane * 16;
+        if (mine) {
+            Frag16 xa[2][MF];
+#pragma unroll
+            for (int i = 0; i < MF; i++) xa[0][i].u = *reinterpret_cast<const u32x4_t*>(xl + i * 4096);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (j < 3) {
+#pragma unroll
+                    for (int i = 0; i < MF; i++) xa[(j + 1) & 1][i].u = *reinterpret_cast<const u32x4_t*>(xl + i * 4096 + (j + 1) * 1024);
+                }
+#pragma unroll
+                for (int f = 0; f < NF; f++) {
+                    Frag16 b;
+                    dequant_group<BITS>(wreg[R][f], j, magic, b);
+#pragma unroll
+                    for (int i = 0; i < MF; i++) acc[i][f] = mma<0>(xa[j & 1][i], b, acc[i][f]);
+                }
+                __builtin_amdgcn_sched_barrier(0);             // (left alone the scheduler makes all operands of a K tile first and spills)
+            }
         }
+        fetch(wreg[R], t + DEPTH);
+        // X of the next step is there: newer than its copies are the weights of this step and, with three places, of the one before
+        // and the copies of this step
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(RING == 2 ? WL : (RING - 1) * WL + (RING - 2) * XC) : "memory");
+        ring = ring + 1 == RING ? 0 : ring + 1;
+    };
+    int t = 0;
+    for (; t + DEPTH < steps; t += DEPTH)
+        static_for_r<0, DEPTH>([&](auto i) __attribute__((always_inline)) { step(t + decltype(i)::value, i, true); });
+    static_for_r<0, DEPTH>([&](auto i) __attribute__((always_inline)) {       // (in the last step not every wave has a K tile)
+        if (t + decltype(i)::value < steps) step(t + decltype(i)::value, i, t + decltype(i)::value < T);
+    });
+
+    // ---- as in gemm_rows_kernel, each half for itself
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");       // (copies past the last step)
+    float4_t* const part = reinterpret_cast<float4_t*>(smem) + half * (4 * FR * 64);
+    float* const stg = reinterpret_cast<float*>(smem + 8 * FR * 1024) + half * (MF * 16 * NF * 16);
+#pragma unroll
+    for (int i = 0; i < MF; i++)
+#pragma unroll
+        for (int f = 0; f < NF; f++) part[(wv * FR + i * NF + f) * 64 + lane] = acc[i][f];
+    __syncthreads();
+    if (wv >= MF) return;
+    float4_t tot[1][NF];
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+        const int blk = wv * NF + f;
+        float4_t s = part[blk * 64 + lane];
+#pragma unroll
+        for (int p = 1; p < 4; p++) s += part[(p * FR + blk) * 64 + lane];
+        tot[0][f] = s;
     }
-    write_rows<1, NF>(tot, stg + wv * (16 * NF * 16), m0, nt0, M, w.N, y, ydt, 1.0f, epi, lane);
+    finish_row_block<NF>(tot, stg + wv * (16 * NF * 16), wv * 16, nt0, M, w, y, ydt, K, epi, ns, lane);
+}
+
+template <int BITS, int MF, int DEPTH, int RING>
+hipError_t launch_pair_t(const WeightView& w, const void* x, int M, void* y, int ydt, const Epilogue& epi, const NormStats& ns, hipStream_t st)
+{
+    constexpr int lds_ring = RING * 4 * MF * 4096, lds_end = 8 * MF * 4 * 1024 + 2 * MF * 16 * 64 * 4;
+    constexpr int lds = lds_ring > lds_end ? lds_ring : lds_end;
+    static_assert(lds <= 160 * 1024, "LDS");
+    (void)LdsRequest<&gemm_rows_pair_kernel<BITS, MF, DEPTH, RING>, lds>::registered;
+    const int groups = (w.NT + 3) / 4, D = ((groups + 1) / 2 + w.KT - 1) / w.KT * w.KT;
+    hipLaunchKernelGGL((gemm_rows_pair_kernel<BITS, MF, DEPTH, RING>), dim3((unsigned)D), dim3(512), lds, st, w.base,
+                       static_cast<const uint8_t*>(x), w.KT, w.NT, (M + 15) / 16, M, w.N, y, ydt, w.K, D, epi, ns);
+    return hipGetLastError();
 }
 
 template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD, int OCC = 1>
@@ -251,9 +397,15 @@ RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue&
     // up to 64 rows a wide output may take more than one round.  Up to 48 rows two workgroups share a CU then (two or three
     // packed weight tiles in flight per wave instead of four, 256 registers): one's start and end overlap the other's
     // K loop (4096 -> 28672 bf16 norm + SwiGLU at 45 rows 35.0 -> 30.2 us, fp32 at 24 rows 28.3 -> 25.6, 2048 -> 20000 at 40
-    // rows 20.5 -> 17.6, 2048 -> 128256 at 40 rows 71.0 -> 51.1).  With four row blocks they do not fit 256 registers
-    // without giving up the lead of the weights: 38.3 against 38.1 us, 35.7 against 36.1.
-    return {parts == 1 ? 4 : 0, parts == 1 && M <= 48};
+    // rows 20.5 -> 17.6, 2048 -> 128256 at 40 rows 71.0 -> 51.1).
+    // Beyond 48 rows one workgroup of eight waves does two column groups that share X (gemm_rows_pair_kernel): 4096 -> 28672 norm +
+    // SwiGLU at 64 rows 36.2 -> 33.2 us, Q8 44.6 -> 38.4, 2048 -> 20000 Q8 24.9 -> 20.1, 4096 -> 128256 120.3 -> 112.8.  Up to 48
+    // rows it pays where the groups fit one round and a step is long, Q8 or many K tiles (Q8 4096 -> 28672 at 45 rows 40.2 -> 37.1,
+    // Q8 8192 -> 16640 at 40 rows 55.2 -> 46.3, Q4 44.1 -> 40.0); not else (Q4 4096 -> 28672 at 45 rows 29.6 / 29.7, 2048 -> 128256
+    // at 40 rows 49.5 / 62.9, Q8 76.2 / 81.6).
+    const int groups4 = (w.NT + 3) / 4, rounds_of_two = ((groups4 + 1) / 2 + w.KT - 1) / w.KT * w.KT;
+    const bool pairs = parts == 1 && num_cus > 1 && (M > 48 || (rounds_of_two <= num_cus && (w.bits == 8 || w.KT > 48)));
+    return {parts == 1 ? 4 : 0, parts == 1 && M <= 48 && !pairs, pairs};
 }
 
 hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, void* y, int ydt, const Epilogue& epi,
@@ -279,6 +431,16 @@ hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, vo
         if (w.bits == 8) return go(std::integral_constant<int, 8>{}, nfc);
         return go(std::integral_constant<int, 4>{}, nfc);
     };
+    if (plan.pairs) {
+        if (w.bits == 4) {
+            if (mf == 2) return launch_pair_t<4, 2, 4, 3>(w, x_staged, M, y, ydt, epi, ns, st);
+            if (mf == 3) return launch_pair_t<4, 3, 4, 3>(w, x_staged, M, y, ydt, epi, ns, st);
+            return launch_pair_t<4, 4, 4, 2>(w, x_staged, M, y, ydt, epi, ns, st);
+        }
+        if (mf == 2) return launch_pair_t<8, 2, 3, 3>(w, x_staged, M, y, ydt, epi, ns, st);
+        if (mf == 3) return launch_pair_t<8, 3, 3, 3>(w, x_staged, M, y, ydt, epi, ns, st);
+        return launch_pair_t<8, 4, 2, 2>(w, x_staged, M, y, ydt, epi, ns, st);
+    }
     if (plan.two_per_cu) {
         if (w.bits == 8) {
             if (mf == 2) return launch_rows_t<8, 2, 4, 4, 2, 1, 2>(w, x_staged, M, y, ydt, epi, ns, st);

@@ -1087,6 +1087,48 @@ def test_prefill_few_rows_long_k_shares(backend, oracle, bits, shape):
     qw.free()
 
 
+@pytest.mark.parametrize("bits,N,K,M", [(4, 16400, 17 * 128, 49), (4, 16384 + 64, 18 * 128 - 32, 64), (4, 33000, 19 * 128 - 96, 63),
+                                        (8, 16400, 20 * 128, 17), (8, 24002, 21 * 128 + 64, 48), (8, 16448, 62 * 128, 64), (4, 17000, 63 * 128 + 32, 33)])
+def test_prefill_few_rows_two_column_groups_per_workgroup(backend, oracle, bits, N, K, M):
+    """More than a round of workgroups: two column groups to a workgroup that walk the K tiles together.  A last group that is not full or
+    has no partner, K tiles that leave waves without one in the last step, N that is no multiple of 16 or 4: bit for bit the kernel with a
+    group to a workgroup; against float64; the epilogues."""
+    q, s = _quant(oracle, bits, N, K, cfg=137)
+    qw = backend.upload_quantized(q, s, bits)
+    wd = torch.from_numpy(oracle.dequant(q, s)).cuda().double()
+    r = torch.from_numpy(synth.activations(138, M, N)).cuda()
+    try:
+        for xdt in ("bf16", "f16") if M > 32 else ("f32",):
+            x = _x(M, K, xdt, cfg=139)
+            y = _run(backend, qw, x)
+            ref = x.double() @ wd.T
+            assert ((y.double() - ref).norm() / ref.norm()).item() < FAST
+            backend.set_gemm_tuning(1)
+            assert torch.equal(_run(backend, qw, x), y), xdt
+            backend.set_gemm_tuning(0)
+            y2 = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+            backend.matmul_ex(qw, x, y2, "add", r.bfloat16())
+            want = ref + r.bfloat16().double()
+            assert ((y2.double() - want).norm() / want.norm()).item() < 4e-3
+        if N % 16 == 0:
+            h = torch.arange(N // 2 // 16 * 16, device="cuda")
+            half = backend.upload_quantized(q[: N // 2 // 16 * 16], s[: N // 2 // 16 * 16], bits)
+            pair = backend.fuse_pairs(half, half)
+            gamma = (1.0 + 0.1 * torch.from_numpy(synth.activations(140, 1, K))[0]).cuda()
+            y3 = torch.empty((M, len(h)), dtype=torch.float32, device="cuda")
+            y4 = torch.empty_like(y3)
+            backend.matmul_norm(pair, x, gamma, 1e-5, y3, "swiglu")
+            backend.set_gemm_tuning(1)
+            backend.matmul_norm(pair, x, gamma, 1e-5, y4, "swiglu")
+            torch.cuda.synchronize()
+            assert torch.equal(y3, y4)
+            pair.free()
+            half.free()
+    finally:
+        backend.set_gemm_tuning(0)
+    qw.free()
+
+
 # (FAST needs K outside 2048 .. 8192 or more than 512 rows to get past the few-row kernel)
 COLS = [("exact", 1030, 33 * 128 - 32, 67), ("exact", 1024, 128, 97), ("exact", 4096, 4096, 128), ("exact", 14336, 288, 193),
         ("exact", 520, 12 * 128 + 64, 260), ("exact", 9000, 640, 80), ("exact", 14400, 2048, 33),
