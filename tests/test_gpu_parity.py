@@ -324,6 +324,45 @@ def test_a_row_keeps_its_bits_from_3_to_32_rows(backend, bits, N, K, pair, xdt):
         backend.set_decode_mode("stream")
 
 
+# a folded norm on wide outputs, up to 16 rows (Q4: by tile), the three load patterns: two, three and four K tiles per wave with waves that
+# have one less, four waves, ragged K and N, a half-filled last pair; more than two steps per workgroup.  gamma is a power of two, so x * gamma is
+# exact and what is left is the sums: up to 128 products per fp32 step with the bias in them (8 .. 128 times the weights), 1e-6 and less
+@pytest.mark.parametrize("bits,N,K,pair", [(4, 6149, 4064, False), (4, 12288, 3104, True), (4, 20000, 4096, True), (4, 32784, 4096, False),
+                                           (4, 14341, 3488, False), (4, 6176, 2080, True), (4, 28689, 3072, False), (4, 8200, 1120, False),
+                                           (4, 6149, 1664, False), (8, 6149, 4064, False), (8, 12320, 1120, True)])
+@pytest.mark.parametrize("xdt", ["f16", "bf16"])
+def test_staying_workgroups_with_a_folded_norm(backend, bits, N, K, pair, xdt):
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    rows, parts, wd = N // 2 if pair else N, [], []
+    for _ in range(2 if pair else 1):
+        w = torch.empty((rows, K), device="cuda").normal_(0.0, 0.02, generator=g)
+        qd = torch.empty(rows * K * bits // 8, dtype=torch.uint8, device="cuda")
+        sd = torch.empty(rows * (K // 32), dtype=torch.int16, device="cuda")
+        backend.quantize(bits, w, rows, K, qd, sd)
+        parts.append(backend.weight_from_device(bits, rows, K, qd, sd))
+        backend.dequant(parts[-1], w)
+        wd.append(w.double())
+    qw = backend.fuse_pairs(*parts) if pair else parts[0]
+    gamma = torch.exp2(torch.randint(-1, 2, (K,), device="cuda", generator=g).float())
+    try:
+        for mode in ("stream", "exact"):
+            backend.set_decode_mode(mode)
+            for i, M in enumerate((3, 4, 5, 8, 9, 16)):
+                x = torch.empty((M, K), device="cuda").normal_(generator=g).to(TDT[xdt])
+                xn = x.double() * gamma.double() / (x.double().square().mean(1, keepdim=True) + 1e-5).sqrt()
+                ref = xn @ wd[0].t()
+                if pair:
+                    ref = torch.nn.functional.silu(ref) * (xn @ wd[1].t())
+                y = torch.full((M, rows), float("nan"), device="cuda")
+                gd = (torch.float16, torch.float32, torch.bfloat16)[i % 3]
+                backend.matmul_norm(qw, x, gamma.to(gd), 1e-5, y, "swiglu" if pair else "none")
+                # (a pair's error is u silu'(g) dg + silu(g) du with |silu'| <= 1.1 and |silu(g)| <= |g|, against |silu(g) u|, which for normal g is
+                # about 0.6 |g u|: at most 2.1 / 0.6 = 3.5 times that of its sums)
+                assert ((y.double() - ref).norm() / ref.norm()).item() < (7e-6 if pair else 2e-6), (mode, M)
+    finally:
+        backend.set_decode_mode("stream")
+
+
 # with the same operands (f16 rows and exact integers; Q8) the staying workgroups and the batched-rows kernel (decode tuning 5: the
 # former never) give the same bits: every epilogue and output type, a folded norm where both load the rows alike
 # (Q4 bf16 rows: another order of sums; the test above has the shapes that the kernels share)
