@@ -15,7 +15,7 @@ extern "C" {
 
 /* Overrides the decode kernels' launch heuristics for experiments: waves per
  * workgroup (1..16); which decode kernel runs (0 automatic, 1 always the
- * x-in-registers kernel, 2 never, 5: automatic without the kernel of gemv_stream.hip); tiles in flight per wave of the streaming
+ * x-in-registers kernel (fp32 rows too), 2 never, 5: automatic without the kernel of gemv_stream.hip); tiles in flight per wave of the streaming
  * variant (2 or 4).  0 restores the automatic choice.  Any non-zero value also keeps
  * one-row calls away from the kernel of gemv1.hip. */
 int cybq_debug_set_gemv_tuning(int waves_per_group, int rows_kernel, int unroll);

@@ -16,6 +16,7 @@
 #include <type_traits>
 #include "cybq_device.h"
 #include "cybq_internal.h"
+#include <type_traits>
 #include "gemv_parts.h"
 
 namespace cybq {
@@ -456,7 +457,7 @@ __global__ __launch_bounds__(1024) void gemv_kernel(const uint8_t* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// Batch rows 3..16: x operands live in REGISTERS and are reused across strips.
+// Batch rows 3..16: x operands live in REGISTERS and are reused across strips.  (16-bit rows; fp32 rows where rows_kernel_has_f32 says so.)
 //
 // With more than a few batch rows the LDS kernel above spends its time moving
 // x: every 16-row strip's workgroup stages all M rows of x (128 KB at M = 16,
@@ -484,6 +485,8 @@ __global__ __launch_bounds__(1024) void gemv_kernel(const uint8_t* __restrict__ 
 // 4u * 2^-24 / 64u * 2^-24 (six vector instructions per eight weights instead of nine), the bias comes off
 // through the MFMA's C operand like with bf16 activations, 1/16 for the odd groups rides on their scale
 // and 2^22 on the final sums.
+// XF32: fp32 rows, as the LDS kernel multiplies them: every value is split into the f16 nearest to it and the f16 nearest to what that leaves,
+// and a weight operand (the exact integers) meets both, into the same sums.  A row's bits do not depend on its batch of 3 .. 16 rows here.
 // KS: K is split over `splits` workgroups per strip group (few strips and a long K: with one workgroup per
 // strip every CU pulls all of x out of the L2, M x K x 2 bytes against its 37 KB x strips of weights).  Workgroup
 // (group, split) walks the K tiles [split * kt_per_split, ...) of the group's NS strips and leaves its sums in
@@ -493,8 +496,8 @@ __global__ __launch_bounds__(1024) void gemv_kernel(const uint8_t* __restrict__ 
 // The ticket is left at zero again for the next launch; launches that share `slabs` must not overlap.
 template <int BITS, int XMODE, int TS, int NS, bool NORM, int XR, int MB = 1, bool SUB = false, bool KS = false>
 // (waves_per_eu: the scheduler would otherwise trade the up-front loads for occupancy)
-__global__ __launch_bounds__((TS <= 2 && MB == 1 && !NORM) ? 1024 : 512)
-__attribute__((amdgpu_waves_per_eu(2, (TS <= 2 && MB == 1 && !NORM) ? 4 : 2)))
+__global__ __launch_bounds__((TS <= 2 && MB == 1 && !NORM && XMODE != XF32) ? 1024 : 512)
+__attribute__((amdgpu_waves_per_eu(2, (TS <= 2 && MB == 1 && !NORM && XMODE != XF32) ? 4 : 2)))
 void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restrict__ x, const void* __restrict__ gamma, int KT_, int K,
                       int NT, int M, int nwaves, int gamma_dt, int N, void* __restrict__ y, int ydt, Epilogue epi, int splits,
                       int kt_per_split, float* __restrict__ slabs, unsigned* __restrict__ tickets)
@@ -525,7 +528,9 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
     constexpr int P = 64 / XR;                  // 16 B pieces per row and load
     constexpr int L = 16 / P;                   // loads per tile: 1, 2, 4
     constexpr int GPL = 4 / L;                  // scale groups per load
-    static_assert(MB == 1 || (XR == 16 && !NORM), "two row blocks: full loads, no folded norm");
+    static_assert(MB == 1 || (XR == 16 && !NORM && XMODE != XF32), "two row blocks: full loads, 16-bit rows, no folded norm");
+    constexpr int PL = XMODE == XF32 ? 2 : 1;   // fp32 rows: the high halves and what they leave, two f16 operands
+    static_assert(PL == 1 || !SUB, "fp32 rows: exact integers");
     const uint16_t* xrow = x + (int64_t)min(lane / P, M - 1) * w.K + (lane % P) * 8;
     const int64_t xblock = MB > 1 ? (int64_t)(min(16 + lane / P, M - 1) - min(lane / P, M - 1)) * w.K : 0;     // to my row of the second block
     const int klast = w.K - 8 - (lane % P) * 8;          // last start at which this lane's piece is inside the row
@@ -556,7 +561,7 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
         // my K tiles of this slab and their x operands (clamped past the end; such tiles get scale 0)
         int kt[TS];
         bool valid[TS];
-        Frag16 a[MB][TS][4];
+        Frag16 a[MB * PL][TS][4];
         u32x4_t graw[NORM ? TS : 1];        // NORM: gamma of my tiles, 8 values in each of 16 lanes (4 in each of 32: fp32)
 #pragma unroll
         for (int u = 0; u < TS; u++) {
@@ -570,7 +575,11 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
             for (int h = 0; h < L; h++) {
                 // (past the end of K: any x inside the row will do, the padded weights are zero)
                 const int k0 = kt[u] * kTileK + h * (GPL * 32);
-                if (XR == 16) {
+                if constexpr (XMODE == XF32) {
+                    const float* from = reinterpret_cast<const float*>(x) + (xrow - x) + (XR == 16 ? min(k0, w.K - 32) : min(k0, klast));
+                    a[0][u][h].u = reinterpret_cast<const u32x4_t*>(from)[0];
+                    a[1][u][h].u = reinterpret_cast<const u32x4_t*>(from)[1];
+                } else if (XR == 16) {
 #pragma unroll
                     for (int b = 0; b < MB; b++)
                         a[b][u][h].u = *reinterpret_cast<const u32x4_t*>(xrow + b * xblock + min(k0, w.K - 32));
@@ -592,6 +601,16 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
         constexpr int WU = NS == 4 ? (TS < 2 ? TS : 2) : TS;       // BY_TILE: K tiles requested ahead (about eight weight tiles)
         TileRegs<BITS> buf[NS][TS];
         constexpr int AHEAD = NS < 2 ? NS : 2;
+        // (fp32 rows: a tile's four groups first, then the tiles - eight waves add up to 56 groups each where the LDS kernel's sixteen add 28;
+        // error against 64 bits, 14336 -> 4101: 1.42e-7 there, 1.62e-7 here without this, 1.21e-7 with it)
+        auto fold = [&](u32x2_t sc, const float4_t (&d)[4], float (&sum)[4]) __attribute__((always_inline)) {
+            if constexpr (XMODE == XF32) {
+                float t[4] = {0.f, 0.f, 0.f, 0.f};
+                tile_accum<4>(sc, d, t);
+#pragma unroll
+                for (int r = 0; r < 4; r++) sum[r] += t[r];
+            } else tile_accum<4>(sc, d, sum);
+        };
         if constexpr (BY_TILE) {
 #pragma unroll
             for (int u = 0; u < WU; u++)
@@ -649,7 +668,18 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
                         counts[h] = valid[u] && kp < w.K;
                     }
 #pragma unroll
-                    for (int h = 0; h < L; h++) norm_piece<XMODE, GH>(a[0][u][h].u, g[h], counts[h], ssq);
+                    for (int h = 0; h < L; h++) {
+                        if constexpr (XMODE == XF32) {
+                            float sq = ssq;
+#pragma unroll
+                            for (int i = 0; i < 8; i++) {
+                                const float v = __builtin_bit_cast(float, (uint32_t)a[i >> 2][u][h].u[i & 3]);
+                                sq = fmaf(v, v, sq);
+                                a[i >> 2][u][h].u[i & 3] = __builtin_bit_cast(uint32_t, v * __builtin_bit_cast(float, (uint32_t)(i < 4 ? g[h].lo : g[h].hi)[i & 3]));
+                            }
+                            ssq = counts[h] ? sq : ssq;
+                        } else norm_piece<XMODE, GH>(a[0][u][h].u, g[h], counts[h], ssq);
+                    }
                 }
             };
             if constexpr (XMODE == XF16) {
@@ -657,8 +687,27 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
                 else norm_all(std::false_type{});
             } else norm_all(std::false_type{});
         }
+        if constexpr (XMODE == XF32) {              // eight values as loaded -> their halves
 #pragma unroll
-        for (int b = 0; b < MB; b++)
+            for (int u = 0; u < TS; u++)
+#pragma unroll
+                for (int h = 0; h < L; h++) {
+                    Frag16 hi, lo;
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        float v = __builtin_bit_cast(float, (uint32_t)a[i >> 2][u][h].u[i & 3]);
+                        // (x * gamma rounded to fp32 once: the compiler would round the product to f16 in one step for the operand and in two
+                        // for the difference, and where these disagree the low half is off by a bit of the high one: 6e-6)
+                        if (NORM) asm("" : "+v"(v));
+                        hi.h[i] = (_Float16)v;
+                        lo.h[i] = (_Float16)(v - (float)hi.h[i]);
+                    }
+                    a[0][u][h] = hi;
+                    a[1][u][h] = lo;
+                }
+        }
+#pragma unroll
+        for (int b = 0; b < MB * PL; b++)
 #pragma unroll
             for (int u = 0; u < TS; u++) {
                 u32x4_t raw[L];
@@ -722,19 +771,23 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
                 tile_operands<BITS, XMODE>(buf[s][u], magic, bop);
 #pragma unroll
                 for (int b = 0; b < MB; b++) tile_multiply<BITS, XMODE>(a[b][u], bop, d[b]);
+                if constexpr (PL == 2) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) d[0][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[1][u][j].h, bop[j].h, d[0][j], 0, 0, 0);
+                }
                 u32x2_t sc = buf[s][u].s;
                 sc[0] = valid[u] ? sc[0] : 0u;
                 sc[1] = valid[u] ? sc[1] : 0u;
 #pragma unroll
                 for (int b = 0; b < MB; b++) {
-                    tile_accum<4>(sprev, dprev[b], acc[s][b]);
+                    fold(sprev, dprev[b], acc[s][b]);
 #pragma unroll
                     for (int j = 0; j < 4; j++) dprev[b][j] = d[b][j];
                 }
                 sprev = sc;
             }
 #pragma unroll
-            for (int b = 0; b < MB; b++) tile_accum<4>(sprev, dprev[b], acc[s][b]);
+            for (int b = 0; b < MB; b++) fold(sprev, dprev[b], acc[s][b]);
         }
     }
 
@@ -848,7 +901,7 @@ hipError_t launch_rows_x(const WeightView& w, const void* x, int M, void* y, int
 {
     size_t lds = (size_t)NS * MB * nwaves * 4 * 64 * sizeof(float) + 8 * 16 * sizeof(float);
     const unsigned groups = (unsigned)((w.NT + NS - 1) / NS);
-    if constexpr (MB == 1) {
+    if constexpr (MB == 1 && !(XMODE == XF32 && TS == 4)) {
         if (epi.gamma) {
             lds += (size_t)nwaves * TS * kTileK * sizeof(float);            // each wave's tiles of gamma as fp32
             auto kern = gemv_rows_kernel<BITS, XMODE, TS, NS, true, XR>;
@@ -1005,6 +1058,56 @@ hipError_t launch_rows(const WeightView& w, const void* x, int M, void* y, int y
     return launch_rows_t<BITS, XMODE, 4, 1>(w, x, M, y, ydt, nwaves, epi, sub, st);
 }
 
+// fp32 rows: two operands per K tile.  Four K tiles per wave and slab fit the registers where a load takes up to eight rows of them, without
+// gamma and with few strips; where they leave more of the last slab empty, two (2048 -> 4096 at 8 rows 6.1 -> 4.4 us).
+template <int BITS>
+hipError_t launch_rows_f32(const WeightView& w, const void* x, int M, void* y, int ydt, int num_cus, const Epilogue& epi, hipStream_t st)
+{
+    const int ns = strips_per_group(w, num_cus, epi);
+    int nwaves = 8;
+    while (nwaves > 1 && nwaves * 2 > w.KT) nwaves >>= 1;
+    auto padded = [&](int ts) { return (w.KT + nwaves * ts - 1) / (nwaves * ts) * (nwaves * ts); };
+    const bool four = w.KT > 2 * nwaves && padded(4) <= padded(2) && !epi.gamma;
+    auto go = [&](auto strips) {
+        constexpr int NS = decltype(strips)::value, TS = NS == 1 || (NS == 2 && BITS == 4) ? 4 : 2;
+        if (M > 8) return launch_rows_x<BITS, XF32, 2, NS, 16>(w, x, M, y, ydt, nwaves, epi, false, st);
+        if constexpr (TS == 4) {
+            if (four && M <= 4) return launch_rows_x<BITS, XF32, TS, NS, 4>(w, x, M, y, ydt, nwaves, epi, false, st);
+            if (four) return launch_rows_x<BITS, XF32, TS, NS, 8>(w, x, M, y, ydt, nwaves, epi, false, st);
+        }
+        if (M <= 4) return launch_rows_x<BITS, XF32, 2, NS, 4>(w, x, M, y, ydt, nwaves, epi, false, st);
+        return launch_rows_x<BITS, XF32, 2, NS, 8>(w, x, M, y, ydt, nwaves, epi, false, st);
+    };
+    if constexpr (BITS == 4) {
+        if (ns == 4) return go(std::integral_constant<int, 4>{});
+    }
+    if (ns >= 2) return go(std::integral_constant<int, 2>{});
+    return go(std::integral_constant<int, 1>{});
+}
+
+// Whether fp32 rows take the batched-rows kernel.  The LDS kernel stages and splits all rows of x once per strip, so it grows with rows x K
+// and strips; a slab that the K tiles leave partly empty is what it saves.  us per call, LDS kernel / this one, Q4: 4096 -> 4096 at
+// 3 / 8 / 16 rows 6.2 / 5.8, 8.1 / 6.2, 14.5 / 7.4; 4096 -> 32768 27.4 / 18.5, 32.2 / 20.2, 59.0 / 23.7; 14336 -> 32768 100 / 53, 193 / 61,
+// 250 / 71; 14336 -> 4096 14.4 / 14.5, 25.8 / 17.4, 32.9 / 19.4; 2048 -> 4096 at 4 / 8 / 16 rows 3.7 / 5.5, 5.0 / 4.4, 8.4 / 5.1; 1024 -> 32768
+// at 4 / 8 rows 7.4 / 7.1, 13.0 / 7.5; 512 -> 4096 at 16 rows 3.2 / 3.4; 8192 -> 4096 at 3 / 6 / 8 rows 8.5 / 9.4, 11.4 / 10.0, 16.5 / 10.2;
+// 5120 -> 4096 at 6 rows 8.5 / 10.1; 3072 -> 20000 (24 of 32 K tiles) at 8 / 16 rows 17.1 / 18.6, 30.1 / 21.2; Q8 3072 -> 11008 at 8 / 16 rows
+// 12.4 / 15.5, 21.0 / 18.2; Q8 pairs of 4096 -> 28672 at 8 / 16 rows 29.6 / 31.2, 51.5 / 35.5.  With a norm always: 256 -> 300 at 3 rows 6.3 / 4.2,
+// 4096 -> 4096 at 16 rows 87 / 10.5, 14336 -> 32000 789 / 86.
+bool rows_kernel_has_f32(const WeightView& w, int M, int num_cus, const Epilogue& epi)
+{
+    if (M < 3) return false;
+    if (epi.gamma) return true;
+    const bool pair = epi.kind == kEpiSwiglu, narrow = w.NT <= 2 * num_cus, widest = w.NT >= 8 * num_cus;
+    if (M < 4 && (pair || (w.KT > 96 && w.NT <= num_cus))) return false;
+    if (w.KT > 32 && w.KT <= 96 && M < (narrow ? 8 : 4)) return false;
+    if (w.bits == 8 && pair && !narrow && M < 10) return false;
+    int slab = 16;                                           // K tiles of a slab of two per wave
+    while (slab > 2 && slab > w.KT) slab >>= 1;
+    const int padded = (w.KT + slab - 1) / slab * slab;
+    if (w.KT * 4 <= padded * 3 && M < (w.bits == 8 || narrow ? 12 : widest || w.KT <= 16 ? 6 : 10)) return false;
+    return M * w.KT >= (widest ? 48 : 96);
+}
+
 // 17 .. 32 rows: two activation operands per weight operand.  Two tiles of x per wave and slab
 // (a wave holds 2 x 2 x 4 operand fragments) when a workgroup has several strips, four with one.
 template <int BITS, int XMODE>
@@ -1148,7 +1251,7 @@ hipError_t launch_gemv(const WeightView& w, const void* x, int xdt, int M, void*
         unroll = 2;
     }
 
-    // three or more batch rows (16-bit activations): x in registers, shared across strips
+    // three or more batch rows: x in registers, shared across strips
     // (Q8 on wide outputs: up to four rows the LDS kernel is still the quicker one, 24.0 against
     // 27.6 us at 4096 -> 28672)
     const bool wide_q8 = w.bits == 8 && (w.NT + num_cus / 2) / num_cus >= 3;
@@ -1172,6 +1275,10 @@ hipError_t launch_gemv(const WeightView& w, const void* x, int xdt, int M, void*
         }
         if (xdt == kF16) return launch_rows2<8, XF16>(w, x, M, y, ydt, g_tune_waves, num_cus, epi, !exact_operands, st);
         return launch_rows2<8, XBF16>(w, x, M, y, ydt, g_tune_waves, num_cus, epi, !exact_operands, st);
+    }
+    if (xdt == kF32 && (g_tune_rows == 1 || (gemv_is_automatic() && rows_kernel_has_f32(w, M, num_cus, epi)))) {
+        if (w.bits == 4) return launch_rows_f32<4>(w, x, M, y, ydt, num_cus, epi, st);
+        return launch_rows_f32<8>(w, x, M, y, ydt, num_cus, epi, st);
     }
     if (rows_kernel && xdt != kF32) {
         if (w.bits == 4) {

@@ -363,6 +363,52 @@ def test_staying_workgroups_with_a_folded_norm(backend, bits, N, K, pair, xdt):
         backend.set_decode_mode("stream")
 
 
+# fp32 rows in the batched-rows kernel (decode tuning 1 forces it) and wherever the library sends them: one, two and four strips to a workgroup, two and
+# four K tiles per wave, slabs partly filled, one K tile, ragged K and N, each load pattern.  The two halves of a row keep 22 bits of every value
+# (2^-23 of it left out at most) and the sums are fp32: 1e-6; a pair's error is at most 3.5 times that (above), and the same rows alone or
+# in a larger batch have the same bits
+@pytest.mark.parametrize("bits,N,K", [(4, 33, 96), (4, 500, 1056), (4, 4096, 2048 + 32), (4, 6149, 4064), (4, 12304, 3104), (4, 4101, 14336), (8, 33, 160),
+                                      (8, 4096, 4096 + 96), (8, 12304, 1120), (8, 6160, 8192)])
+def test_batched_rows_of_fp32(backend, bits, N, K):
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    w = torch.empty((N, K), device="cuda").normal_(0.0, 0.02, generator=g)
+    qd = torch.empty(N * K * bits // 8, dtype=torch.uint8, device="cuda")
+    sd = torch.empty(N * (K // 32), dtype=torch.int16, device="cuda")
+    backend.quantize(bits, w, N, K, qd, sd)
+    qw = backend.weight_from_device(bits, N, K, qd, sd)
+    backend.dequant(qw, w)
+    x = torch.empty((16, K), device="cuda").normal_(generator=g)
+    gamma = 1.0 + 0.25 * torch.empty(K, device="cuda").normal_(generator=g)
+    res = torch.empty((16, N), device="cuda").normal_(generator=g)
+    rms = (x.double().square().mean(1, keepdim=True) + 1e-5).sqrt()
+    plain, normed = x.double() @ w.double().t(), (x.double() * gamma.double() / rms) @ w.double().t()
+    rel = lambda y, ref: ((y.double() - ref).norm() / ref.norm()).item()
+    half = N // 2 // 16 * 16
+    parts = [backend.weight_from_device(bits, half, K, qd[i * half * K * bits // 8:], sd[i * half * (K // 32):]) for i in (0, 1)] if half else []
+    pair = backend.fuse_pairs(*parts) if half else None
+    first = None
+    try:
+        for tuning in (1, 0):
+            backend.set_gemv_tuning(0, tuning, 0)
+            for M in (16, 9, 8, 5, 4, 3):
+                y = torch.full((M, N), float("nan"), device="cuda")
+                backend.matmul(qw, x[:M].contiguous(), y)
+                assert rel(y, plain[:M]) < 1e-6, (tuning, M)
+                if tuning == 1:
+                    first = y if first is None else first
+                    assert torch.equal(y, first[:M]), M
+                y = torch.full((M, N), float("nan"), device="cuda")
+                backend.matmul_norm(qw, x[:M].contiguous(), gamma, 1e-5, y, "add", res[:M].contiguous())
+                assert rel(y, normed[:M] + res[:M].double()) < 1e-6, (tuning, M)
+                if pair is not None:
+                    y = torch.full((M, half), float("nan"), device="cuda")
+                    backend.matmul_ex(pair, x[:M].contiguous(), y, "swiglu")
+                    ref = torch.nn.functional.silu(plain[:M, :half]) * plain[:M, half:2 * half]
+                    assert rel(y, ref) < 3.5e-6, (tuning, M)
+    finally:
+        backend.set_gemv_tuning(0, 0, 0)
+
+
 # with the same operands (f16 rows and exact integers; Q8) the staying workgroups and the batched-rows kernel (decode tuning 5: the
 # former never) give the same bits: every epilogue and output type, a folded norm where both load the rows alike
 # (Q4 bf16 rows: another order of sums; the test above has the shapes that the kernels share)
