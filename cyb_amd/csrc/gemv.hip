@@ -946,8 +946,9 @@ bool rows_split_plan(const WeightView& w, int xdt, int M, int num_cus, const Epi
 {
     if (w.bits != 4 || xdt == kF32 || epi.gamma || epi.kind == kEpiSwiglu) return false;
     // a long K and about one strip per CU (14336 -> 4096 on 256 CUs: 12.6 against 13.9 us at 16 rows, 17.4 against
-    // 21.5 at 32; with K = 11008 or a quarter of the strips the split only costs: its slabs and ticket add 2.5 - 3 us)
-    if (w.KT < 96 || (int64_t)w.NT * 2 > (int64_t)num_cus * 3 || (int64_t)w.NT * 4 < (int64_t)num_cus * 3) return false;
+    // 21.5 at 32; with K = 11008 or a quarter of the strips the split only costs: its slabs and ticket add 2.5 - 3 us;
+    // with more strips than CUs its workgroups take two rounds: 12288 -> 5120 at 16 / 32 rows 20.0 / 27.7, two whole strips each 14.6 / 22.1)
+    if (w.KT < 96 || w.NT > num_cus || (int64_t)w.NT * 4 < (int64_t)num_cus * 3) return false;
     sp.splits = kSplitWays;
     sp.kt_per_split = (w.KT + sp.splits - 1) / sp.splits;
     sp.splits = (w.KT + sp.kt_per_split - 1) / sp.kt_per_split;                         // no empty split
@@ -1004,11 +1005,20 @@ hipError_t launch_rows_t(const WeightView& w, const void* x, int M, void* y, int
     return launch_rows_x<BITS, XMODE, TS, NS, 16>(w, x, M, y, ydt, nwaves, epi, sub, st);
 }
 
-// strips per workgroup: as many as keeps about one workgroup per CU, at most 4
-int strips_per_group(const WeightView& w, int num_cus, const Epilogue& epi)
+// strips per workgroup: as many as keeps about one workgroup per CU, at most 4.  Two from one strip per CU on: workgroups of eight
+// waves have a CU to themselves, so a few more of them than CUs take two rounds.  us per call, one strip / two: Q4 f16 4096 -> 4224 at
+// 8 / 16 / 32 rows 7.0 / 5.2, 8.0 / 5.9, 11.7 / 9.4, 11008 -> 6000 15.8 / 12.5, 19.8 / 14.4, 30.7 / 21.6, fp32 4096 -> 5120 at 16 rows with a
+// norm 18.0 / 10.9, Q8 f16 14336 -> 4224 at 8 / 32 rows 23.6 / 18.7, 39.5 / 28.6.  Not with four waves, two of whose workgroups share a CU (1024 ->
+// 5120 at 8 rows 4.1 / 4.3, Q8 4.3 / 4.8; 17 .. 32 rows of Q4 6.6 / 4.7), nor for nine or more f16 rows of Q8 with a norm (14336 -> 4224 31.1 / 33.4).
+// Likewise four of Q4 from two per CU on, two / four, f16: 8192 -> 9216 at 8 / 16 / 32 rows 16.9 / 13.4, 19.7 / 15.1, 28.1 / 21.2, 14336 -> 9216 with a
+// norm at 16 rows 37.7 / 29.4, bf16 46.1 / 31.8 (16-bit rows of K up to 4096 run the kernel of gemv_stream.hip there).
+int strips_per_group(const WeightView& w, int xdt, int M, int num_cus, const Epilogue& epi)
 {
     int ns = (w.NT + num_cus / 2) / num_cus;
     ns = ns >= 3 ? 4 : (ns >= 2 ? 2 : 1);
+    const bool two = w.KT >= 16 ? !(w.bits == 8 && xdt == kF16 && epi.gamma && M > 8) : w.bits == 4 && M > 16;
+    if (w.NT > num_cus && two && ns < 2) ns = 2;
+    if (w.NT > 2 * num_cus && ns < 4 && w.bits == 4 && (w.KT > 32 || (xdt == kF32 && w.KT >= 16))) ns = 4;
     if (epi.kind == kEpiSwiglu && ns < 2) ns = 2;          // a gate strip and its up strip share a workgroup
     return ns;
 }
@@ -1018,7 +1028,7 @@ hipError_t launch_rows(const WeightView& w, const void* x, int M, void* y, int y
                        const Epilogue& epi, bool sub, hipStream_t st)
 {
     // 8 waves split K (fewer when the strip has fewer tiles), 4 tiles of x per wave and slab
-    const int ns = strips_per_group(w, num_cus, epi);
+    const int ns = strips_per_group(w, XMODE == XF16 ? kF16 : kBF16, M, num_cus, epi);
     // seven strips per workgroup when that is exactly one workgroup per CU (N = 28672 on 256 CUs:
     // with four strips the 448 workgroups need a second, mostly empty round); SwiGLU pairs need an
     // even count: eight strips there, 224 workgroups in one round
@@ -1063,7 +1073,7 @@ hipError_t launch_rows(const WeightView& w, const void* x, int M, void* y, int y
 template <int BITS>
 hipError_t launch_rows_f32(const WeightView& w, const void* x, int M, void* y, int ydt, int num_cus, const Epilogue& epi, hipStream_t st)
 {
-    const int ns = strips_per_group(w, num_cus, epi);
+    const int ns = strips_per_group(w, kF32, M, num_cus, epi);
     int nwaves = 8;
     while (nwaves > 1 && nwaves * 2 > w.KT) nwaves >>= 1;
     auto padded = [&](int ts) { return (w.KT + nwaves * ts - 1) / (nwaves * ts) * (nwaves * ts); };
@@ -1114,7 +1124,7 @@ template <int BITS, int XMODE>
 hipError_t launch_rows2(const WeightView& w, const void* x, int M, void* y, int ydt, int tuned_waves, int num_cus,
                         const Epilogue& epi, bool sub, hipStream_t st)
 {
-    const int ns = strips_per_group(w, num_cus, epi);
+    const int ns = strips_per_group(w, XMODE == XF16 ? kF16 : kBF16, M, num_cus, epi);
     int nwaves = tuned_waves > 0 ? min(tuned_waves, 8) : 8;
     while (nwaves > 1 && nwaves * 2 > w.KT) nwaves >>= 1;
     if constexpr (BITS == 4) {

@@ -409,6 +409,28 @@ def test_batched_rows_of_fp32(backend, bits, N, K):
         backend.set_gemv_tuning(0, 0, 0)
 
 
+# a few strips more than CUs, or than twice as many (256 CUs: two and four strips to a workgroup), and K split over workgroups up to one per CU: an odd
+# last strip, ragged N and K, up to 32 rows
+@pytest.mark.parametrize("bits,N,K", [(4, 4096, 12288), (4, 4100, 12288), (4, 4112, 2048), (4, 6128, 4096 + 32), (4, 4130, 1024), (4, 8200, 4128), (4, 10224, 4128),
+                                      (8, 4130, 2080), (8, 6128, 4128)])
+@pytest.mark.parametrize("xdt", ["f16", "bf16", "f32"])
+def test_decode_a_few_strips_more_than_cus(backend, bits, N, K, xdt):
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    w = torch.empty((N, K), device="cuda").normal_(0.0, 0.02, generator=g)
+    qd = torch.empty(N * K * bits // 8, dtype=torch.uint8, device="cuda")
+    sd = torch.empty(N * (K // 32), dtype=torch.int16, device="cuda")
+    backend.quantize(bits, w, N, K, qd, sd)
+    qw = backend.weight_from_device(bits, N, K, qd, sd)
+    backend.dequant(qw, w)
+    for M in (3, 8, 16) + ((17, 32) if xdt != "f32" else ()):
+        x = torch.empty((M, K), device="cuda").normal_(generator=g).to(TDT[xdt])
+        r = torch.empty((M, N), device="cuda").normal_(generator=g)
+        y = torch.full((M, N), float("nan"), device="cuda")
+        backend.matmul_ex(qw, x, y, "add", r)
+        ref = x.double() @ w.double().t() + r.double()
+        assert ((y.double() - ref).norm() / ref.norm()).item() < TIGHT, M
+
+
 # with the same operands (f16 rows and exact integers; Q8) the staying workgroups and the batched-rows kernel (decode tuning 5: the
 # former never) give the same bits: every epilogue and output type, a folded norm where both load the rows alike
 # (Q4 bf16 rows: another order of sums; the test above has the shapes that the kernels share)
