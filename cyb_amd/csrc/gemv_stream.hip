@@ -12,9 +12,8 @@
 // Which wave owns which K tile, and the order of every sum, is that of gemv.hip's kernel with the same waves, with its plain
 // operands (f16 rows: exact integers) or, where that kernel shares a shape by row count and walks it by tile, with those of that
 // walk (TILE): a row's bits do not depend on the batch of 3 .. 32 rows it travels in.  (With a folded norm the squares are summed as
-// loaded, so they do: 3 .. 4, 5 .. 8, 9 .. 32 rows; and up to 16 rows Q4 goes by tile, whatever the shape: six vector instructions instead of
-// nine unpack eight weights, and on long outputs these kept the weights waiting: 4096 -> 32768 at 8 f16 rows 18.0 -> 16.2 us, a step of
-// two strips per CU 3.6 -> 3.05 us, 5.2 -> 6.2 TB/s.)
+// loaded, so they do: 3 .. 4, 5 .. 8, 9 .. 32 rows.  The operands are the plain ones then: by tile 4096 -> 32768 at 8 f16 rows takes 16.2 us
+// instead of 18.0, but its sums carry the bias: 5e-7 of relative L2 against float64 where the integers have 1e-7.)
 // (f16 rows, us per call before -> after: Q8 2560 -> 32003 at 8 / 27 rows 20.1 -> 16.1, 36.4 -> 17.9 (12.4 at 7 TB/s); Q4 2048 ->
 // 20000 with a norm 17.6 -> 8.2, 22.0 -> 10.6; Q4 4096 -> 128256 at 27 rows 92.6 -> 66.2.  Two or three pairs ahead
 // instead of one changed nothing on long outputs and cost 2 us on short ones.)
@@ -28,15 +27,14 @@ namespace {
 // S: strips of a step, 2 or (where the registers do not hold two) 1.
 // TILE (Q4): the operands and the order of sums of the batched-rows kernel's walk by tile - the product of the activations
 // with the constant that takes the bias off comes first, one for all strips of a step, and f16 activations meet subnormal
-// weights (gemv_rows_kernel, SUB).  For shapes where that kernel has the calls with fewer, or more, rows, so that a row keeps its bits, and for
-// a folded norm, where it is the quicker walk (by_tile).
+// weights (gemv_rows_kernel, SUB).  For shapes where that kernel has the calls with fewer, or more, rows: a row keeps its bits.
 template <int BITS, int XMODE, int W, int TS, int MB, int XR, bool NORM, int S, bool TILE>
 __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemv_stream_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restrict__ x, const void* __restrict__ gamma, int KT, int K, int NT,
                         int M, int gamma_dt, int steps, int N, void* __restrict__ y, int ydt, Epilogue epi)
 {
     static_assert(W == 4 || W == 8, "a wave finishes output registers of one row in four");
-    static_assert(!TILE || BITS == 4, "by tile: Q4");
+    static_assert(!TILE || (BITS == 4 && !NORM), "by tile: Q4, no folded norm");
     const WeightView w = {wbase, N, K, NT, KT, BITS};
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const uint32_t magic = (BITS == 4 && XMODE == XBF16) ? q4_magic_vgpr_bf16() : q4_magic_vgpr();
@@ -177,7 +175,7 @@ void gemv_stream_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __res
                 float t = 0.f;
 #pragma unroll
                 for (int k = 0; k < W; k++) t += ssq_part[(b * W + k) * 16 + 4 * oct + (wv & 3)];
-                scale[b] *= __builtin_amdgcn_rsqf(fmaf(t, __builtin_amdgcn_rcpf((float)K), epi.eps));
+                scale[b] = __builtin_amdgcn_rsqf(fmaf(t, __builtin_amdgcn_rcpf((float)K), epi.eps));
             }
         }
 
@@ -277,8 +275,7 @@ hipError_t launch_k(const WeightView& w, const void* x, int M, void* y, int ydt,
 template <int BITS, int XMODE, int W, int TS, bool NORM, bool TILE>
 hipError_t launch_m(const WeightView& w, const void* x, int M, void* y, int ydt, int num_cus, const Epilogue& epi, hipStream_t st)
 {
-    // (17 .. 32 rows: a norm only of f16 rows and up to three tiles per wave, and not by tile - two row blocks, three tiles, gamma and the
-    // bias do not fit the registers, and with two tiles it is 0 - 1.3 us slower; pairs of four tiles go elsewhere; by tile never with four waves)
+    // (17 .. 32 rows: a norm only of f16 rows and up to three tiles per wave; by tile never with four waves)
     if (M > 16) {
         if constexpr (!NORM) return launch_k<BITS, XMODE, W, TS, 2, 16, false, TILE && W == 8>(w, x, M, y, ydt, num_cus, epi, st);
         else if constexpr (TS < 4 && XMODE == XF16) return launch_k<BITS, XMODE, W, TS, 2, 16, true>(w, x, M, y, ydt, num_cus, epi, st);
@@ -305,43 +302,40 @@ bool rows_kernel_by_tile(const WeightView& w, int num_cus)
     return groups * 5 >= rounds * num_cus * 4;
 }
 
-// Whether the batched-rows kernel is the quicker one up to 16 rows: nine rows or more where its workgroups are one nearly full round of
-// four strips, or with a norm of two, and, but for pairs, the widest outputs.  It gives every wave four K tiles to walk whether they are there
+// Whether the batched-rows kernel is the quicker one up to 16 rows.  Without a norm: nine rows or more where its workgroups are one nearly
+// full round of four strips, and, but for pairs, the widest outputs.  It gives every wave four K tiles to walk whether they are there
 // or not, so a shorter K is never its.  us per call, this kernel / that one, f16 rows (bf16).  K = 4096: 14336 at 4 / 8 / 16 rows 8.3 / 8.3,
-// 8.5 / 8.5, 9.7 / 9.0 (8.4 / 8.4, 9.0 / 9.0, 10.3 / 9.4), 16384 8.9 / 8.7, 9.0 / 9.7, 10.5 / 9.6; with a norm 6144 at 4 / 8 / 16 rows
-// 6.1 / 6.4, 6.7 / 6.9, 7.5 / 7.3 (6.7 / 7.2, 7.5 / 7.6, 8.8 / 8.5), 14336 9.1 / 9.7, 9.4 / 10.0, 10.2 / 10.8, 24576 at 8 rows 13.2 / 18.5
-// (13.9 / 18.9), 32768 16.2 / 19.6, 49152 22.4 / 28.4, 28672, exactly seven strips per CU, 15.3 / 15.1, 16.1 / 16.3 at 16; 28672 without a norm
-// 15.7 / 14.6, pairs 14.1 / 14.4, pairs of 128256 48.7 / 53.1.  K = 3456: 14336 at 8 / 16 rows 7.4 / 8.6, 8.9 / 8.9, 32768 14.2 / 15.0,
-// 15.0 / 16.3; K = 3712: 28672 at 8 rows 15.3 / 14.2.
+// 8.5 / 8.5, 9.7 / 9.0 (8.4 / 8.4, 9.0 / 9.0, 10.3 / 9.4), 16384 8.9 / 8.7, 9.0 / 9.7, 10.5 / 9.6, 28672 15.7 / 14.6, pairs 14.1 / 14.4, pairs
+// of 128256 48.7 / 53.1.  K = 3456: 14336 at 8 / 16 rows 7.4 / 8.6, 8.9 / 8.9, 32768 14.2 / 15.0, 15.0 / 16.3; K = 3712: 28672 at 8 rows 15.3 / 14.2.
+// With a norm: nearly full rounds, whatever the rows and K, and the widest outputs.
 bool leaves_few_rows(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
-    if (w.bits != 4 || waves_of(w) != 8 || tiles_per_wave(w) != 4 || w.KT < 28) return false;
-    if (epi.gamma) return M > 8 && w.NT <= 2 * num_cus;
-    if (w.NT >= 8 * num_cus || w.NT == 7 * num_cus) return epi.kind != kEpiSwiglu;
+    if (w.bits != 4 || waves_of(w) != 8 || tiles_per_wave(w) != 4) return false;
+    const bool widest = w.NT >= 8 * num_cus || w.NT == 7 * num_cus;
+    if (epi.gamma) {
+        const int ns = (w.NT + num_cus / 2) / num_cus >= 3 ? 4 : 2;
+        const int groups = (w.NT + ns - 1) / ns, rounds = (groups + num_cus - 1) / num_cus;
+        return widest || groups * 4 >= rounds * num_cus * 3;
+    }
+    if (w.KT < 28) return false;
+    if (widest) return epi.kind != kEpiSwiglu;
     return M > 8 && w.NT * 5 >= num_cus * 16 && w.NT <= num_cus * 4;
 }
 
-// By tile (TILE), besides those: gate / up pairs of four tiles per wave (17 .. 32 rows of them run the batched-rows kernel, by tile), and every
-// call with a folded norm, where a row's bits go with the batch anyhow.  f16 rows only in decode mode STREAM.
-// us per call, plain / by tile, with a norm at 8 f16 rows (bf16): 4096 -> 14336 10.1 / 9.4 (10.3 / 10.2), 24576 14.4 / 13.1, 28672 17.0 / 15.3
-// (16.5 / 16.3), 65536 32.1 / 28.4; 3072 -> 28672 13.6 / 12.6, 2048 -> 28672 9.9 / 9.5 (10.3 / 9.9).  Without a norm, 17 .. 32 rows go the
-// same way and lose by it (4096 -> 14336 at 24 rows 11.8 / 12.7), so only the shapes whose rows that keeps together do.
+// By tile (TILE), besides those: gate / up pairs of four tiles per wave (17 .. 32 rows of them run the batched-rows kernel, by tile).  f16
+// rows only in decode mode STREAM.  17 .. 32 rows go the same way and lose by it (4096 -> 14336 at 24 rows 11.8 / 12.7 us), so only the
+// shapes whose rows that keeps together do.
 bool by_tile(const WeightView& w, int xdt, int num_cus, bool exact_operands, const Epilogue& epi)
 {
-    if (w.bits != 4 || (xdt == kF16 && exact_operands)) return false;
-    if (epi.gamma) return true;
-    return tiles_per_wave(w) == 4 && (epi.kind == kEpiSwiglu || rows_kernel_by_tile(w, num_cus));
+    if (w.bits != 4 || tiles_per_wave(w) != 4 || epi.gamma || (xdt == kF16 && exact_operands)) return false;
+    return epi.kind == kEpiSwiglu || rows_kernel_by_tile(w, num_cus);
 }
 
 template <int BITS, int XMODE, int W, bool NORM>
 hipError_t launch_w(const WeightView& w, const void* x, int M, void* y, int ydt, int num_cus, bool tile, const Epilogue& epi, hipStream_t st)
 {
     const int ts = tiles_per_wave(w);
-    if constexpr (BITS == 4) {
-        if constexpr (NORM) {
-            if (ts == 2 && tile) return launch_m<BITS, XMODE, W, 2, true, true>(w, x, M, y, ydt, num_cus, epi, st);
-            if (ts == 3 && tile) return launch_m<BITS, XMODE, W, 3, true, true>(w, x, M, y, ydt, num_cus, epi, st);
-        }
+    if constexpr (BITS == 4 && !NORM) {
         if (ts == 4 && tile) return launch_m<BITS, XMODE, W, 4, NORM, true>(w, x, M, y, ydt, num_cus, epi, st);
     }
     if (ts == 2) return launch_m<BITS, XMODE, W, 2, NORM, false>(w, x, M, y, ydt, num_cus, epi, st);

@@ -96,9 +96,9 @@ typedef enum cybq_prefill_mode { CYBQ_PREFILL_FAST = 0, CYBQ_PREFILL_EXACT = 1 }
  * f16 group scale in fp32 and stays far inside the 1e-3 tolerance.  Which form runs:
  *   f16 activations   1 - 2 rows: STREAM -> subnormal operands, EXACT -> exact integers.
  *                     3 - 32 rows (and the 33 - 64-row walk): EXACT -> exact integers.  STREAM -> subnormal
- *                     operands for Q4 where the kernel that has the shape takes a weight tile's two to four
- *                     16-row strips together (with a folded norm up to 16 rows), exact integers otherwise (both
- *                     well inside the tolerance; the kernel goes with N, K and the epilogue).
+ *                     operands for Q4 without a folded norm where the kernel that has the shape takes a
+ *                     weight tile's two to four 16-row strips together, exact integers otherwise (both well
+ *                     inside the tolerance; the kernel goes with N, K and the epilogue).
  *   bf16 activations  any row count, either mode: the bf16 numbers 128 + (q + bias) with the bias
  *                     removed inside the accumulation (bf16 has no packed add to take it off
  *                     beforehand); the mode only chooses the kernel for 1 - 2 rows.

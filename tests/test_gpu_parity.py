@@ -324,9 +324,10 @@ def test_a_row_keeps_its_bits_from_3_to_32_rows(backend, bits, N, K, pair, xdt):
         backend.set_decode_mode("stream")
 
 
-# a folded norm on wide outputs, up to 16 rows (Q4: by tile), the three load patterns: two, three and four K tiles per wave with waves that
+# a folded norm on wide outputs, up to 16 rows, every load pattern: two, three and four K tiles per wave with waves that
 # have one less, four waves, ragged K and N, a half-filled last pair; more than two steps per workgroup.  gamma is a power of two, so x * gamma is
-# exact and what is left is the sums: up to 128 products per fp32 step with the bias in them (8 .. 128 times the weights), 1e-6 and less
+# exact and what is left is the sums: up to 128 products per fp32 step, for bf16 rows with the bias in them (8 .. 128 times the weights), 1e-6 and
+# less; f16 rows meet the exact integers in either mode, whatever kernel has the shape: the same bits, and a weight of zeros gives exact zeros
 @pytest.mark.parametrize("bits,N,K,pair", [(4, 6149, 4064, False), (4, 12288, 3104, True), (4, 20000, 4096, True), (4, 32784, 4096, False),
                                            (4, 14341, 3488, False), (4, 6176, 2080, True), (4, 28689, 3072, False), (4, 8200, 1120, False),
                                            (4, 6149, 1664, False), (8, 6149, 4064, False), (8, 12320, 1120, True)])
@@ -344,11 +345,13 @@ def test_staying_workgroups_with_a_folded_norm(backend, bits, N, K, pair, xdt):
         wd.append(w.double())
     qw = backend.fuse_pairs(*parts) if pair else parts[0]
     gamma = torch.exp2(torch.randint(-1, 2, (K,), device="cuda", generator=g).float())
+    zero = backend.weight_from_device(bits, rows, K, torch.zeros_like(qd), sd)
+    first = {}
     try:
         for mode in ("stream", "exact"):
             backend.set_decode_mode(mode)
             for i, M in enumerate((3, 4, 5, 8, 9, 16)):
-                x = torch.empty((M, K), device="cuda").normal_(generator=g).to(TDT[xdt])
+                x = torch.empty((M, K), device="cuda").normal_(generator=g.manual_seed(M)).to(TDT[xdt])
                 xn = x.double() * gamma.double() / (x.double().square().mean(1, keepdim=True) + 1e-5).sqrt()
                 ref = xn @ wd[0].t()
                 if pair:
@@ -359,6 +362,11 @@ def test_staying_workgroups_with_a_folded_norm(backend, bits, N, K, pair, xdt):
                 # (a pair's error is u silu'(g) dg + silu(g) du with |silu'| <= 1.1 and |silu(g)| <= |g|, against |silu(g) u|, which for normal g is
                 # about 0.6 |g u|: at most 2.1 / 0.6 = 3.5 times that of its sums)
                 assert ((y.double() - ref).norm() / ref.norm()).item() < (7e-6 if pair else 2e-6), (mode, M)
+                if xdt == "f16":
+                    assert torch.equal(y, first.setdefault(M, y)), (mode, M)
+                    y0 = torch.full((M, rows), float("nan"), device="cuda")
+                    backend.matmul_norm(zero, x, gamma.to(gd), 1e-5, y0)
+                    assert (y0 == 0).all(), (mode, M)
     finally:
         backend.set_decode_mode("stream")
 
