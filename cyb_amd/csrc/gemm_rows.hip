@@ -232,7 +232,9 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC 
 // workgroups draw.  What bounds it then is issue: per K tile a wave makes 16 operands of 13 vector instructions each, next to 32,
 // 48 or 64 MFMAs (4096 -> 28672 at 45 rows: 3.4 us before the first step, 8 steps of 3690 cycles in 15.4, 1.9 after).  Bit for
 // bit the result of gemm_rows_kernel.
-// (wbase without __restrict__: the waits below count the weight loads, so none of them may move over an asm that clobbers memory.)
+// (wbase without __restrict__: the waits below count the weight loads, so none of them may move over an asm that clobbers memory.  A load
+// whose value nobody reads is removed, and a wait that counted it lets the copies pass: the last DEPTH steps ask for no weights and
+// wait for the copies alone.)
 template <int BITS, int MF, int DEPTH, int RING>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_rows_pair_kernel(
     const uint8_t* wbase, const uint8_t* x, int KT_, int NT_, int x_row_blocks, int M, int N_,
@@ -291,10 +293,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(DEPTH * WL > 63 ? 63 : DEPTH * WL) : "memory");
 
     int ring = 0;
-    auto step = [&](int t, auto residue, bool mine) __attribute__((always_inline)) {
+    auto step = [&](int t, auto residue, auto more, bool mine) __attribute__((always_inline)) {
         constexpr int R = decltype(residue)::value;
+        constexpr bool MORE = decltype(more)::value;           // there are weights left to ask for
         const int far = ring == 0 ? RING - 1 : ring - 1;       // the step before this one's place: X of step t + RING - 1
         copy_x(t + RING - 1, far);
+        asm volatile("" ::: "memory");                         // (the weights behind the copies)
         const uint8_t* xl = smem + (ring * 4 + wv) * (MF * 4096) + lane * 16;
         if (mine) {
             Frag16 xa[2][MF];
@@ -316,17 +320,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 __builtin_amdgcn_sched_barrier(0);             // (left alone the scheduler makes all operands of a K tile first and spills)
             }
         }
-        fetch(wreg[R], t + DEPTH);
+        if constexpr (MORE) fetch(wreg[R], t + DEPTH);
         // X of the next step is there: newer than its copies are the weights of this step and, with three places, of the one before
-        // and the copies of this step
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(RING == 2 ? WL : (RING - 1) * WL + (RING - 2) * XC) : "memory");
+        // and the copies of this step; without weights those copies alone
+        constexpr int NEWER = !MORE ? (RING - 2) * XC : RING == 2 ? WL : (RING - 1) * WL + (RING - 2) * XC;
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NEWER) : "memory");
         ring = ring + 1 == RING ? 0 : ring + 1;
     };
     int t = 0;
     for (; t + DEPTH < steps; t += DEPTH)
-        static_for_r<0, DEPTH>([&](auto i) __attribute__((always_inline)) { step(t + decltype(i)::value, i, true); });
+        static_for_r<0, DEPTH>([&](auto i) __attribute__((always_inline)) { step(t + decltype(i)::value, i, std::true_type{}, true); });
     static_for_r<0, DEPTH>([&](auto i) __attribute__((always_inline)) {       // (in the last step not every wave has a K tile)
-        if (t + decltype(i)::value < steps) step(t + decltype(i)::value, i, t + decltype(i)::value < T);
+        if (t + decltype(i)::value < steps) step(t + decltype(i)::value, i, std::false_type{}, t + decltype(i)::value < T);
     });
 
     // ---- as in gemm_rows_kernel, each half for itself
@@ -399,9 +404,9 @@ RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue&
     // K loop (4096 -> 28672 bf16 norm + SwiGLU at 45 rows 35.0 -> 30.2 us, fp32 at 24 rows 28.3 -> 25.6, 2048 -> 20000 at 40
     // rows 20.5 -> 17.6, 2048 -> 128256 at 40 rows 71.0 -> 51.1).
     // Beyond 48 rows one workgroup of eight waves does two column groups that share X (gemm_rows_pair_kernel): 4096 -> 28672 norm +
-    // SwiGLU at 64 rows 36.2 -> 33.2 us, Q8 44.6 -> 38.4, 2048 -> 20000 Q8 24.9 -> 20.1, 4096 -> 128256 120.3 -> 112.8.  Up to 48
-    // rows it pays where the groups fit one round and a step is long, Q8 or many K tiles (Q8 4096 -> 28672 at 45 rows 40.2 -> 37.1,
-    // Q8 8192 -> 16640 at 40 rows 55.2 -> 46.3, Q4 44.1 -> 40.0); not else (Q4 4096 -> 28672 at 45 rows 29.6 / 29.7, 2048 -> 128256
+    // SwiGLU at 64 rows 36.5 -> 34.1 us, Q8 45.0 -> 38.5, 2048 -> 20000 Q8 25.3 -> 20.6, 4096 -> 128256 122.5 -> 116.3.  Up to 48
+    // rows it pays where the groups fit one round and a step is long, Q8 or many K tiles (Q8 4096 -> 28672 at 45 rows 41.0 -> 38.0,
+    // Q8 8192 -> 16640 at 40 rows 59.7 -> 49.1, Q4 44.1 -> 40.6); not else (Q4 4096 -> 28672 at 45 rows 29.6 / 29.7, 2048 -> 128256
     // at 40 rows 49.5 / 62.9, Q8 76.2 / 81.6).
     const int groups4 = (w.NT + 3) / 4, rounds_of_two = ((groups4 + 1) / 2 + w.KT - 1) / w.KT * w.KT;
     const bool pairs = parts == 1 && num_cus > 1 && (M > 48 || (rounds_of_two <= num_cus && (w.bits == 8 || w.KT > 48)));
