@@ -494,7 +494,8 @@ __global__ __launch_bounds__(1024) void gemv_kernel(const uint8_t* __restrict__ 
 // order - a fixed order whoever arrives when - and writes y.  Slabs and ticket travel past the caches (stores
 // and loads at system scope, waited for before the ticket is taken): nothing is flushed, nothing invalidated.
 // The ticket is left at zero again for the next launch; launches that share `slabs` must not overlap.
-template <int BITS, int XMODE, int TS, int NS, bool NORM, int XR, int MB = 1, bool SUB = false, bool KS = false>
+// STRIPS: strip by strip, also where the walk goes by tile otherwise (BY_TILE).
+template <int BITS, int XMODE, int TS, int NS, bool NORM, int XR, int MB = 1, bool SUB = false, bool KS = false, bool STRIPS = false>
 // (waves_per_eu: the scheduler would otherwise trade the up-front loads for occupancy)
 __global__ __launch_bounds__((TS <= 2 && MB == 1 && !NORM && XMODE != XF32) ? 1024 : 512)
 __attribute__((amdgpu_waves_per_eu(2, (TS <= 2 && MB == 1 && !NORM && XMODE != XF32) ? 4 : 2)))
@@ -596,7 +597,7 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
         // second product does not depend on the strip, so the tiles are walked K tile by K tile with all
         // strips of a tile behind one bias product (its result is the C operand of their MFMAs):
         // 4 + 4 NS instead of 8 NS MFMAs per tile.  Each strip still sums its tiles in the same order.
-        constexpr bool BY_TILE = (XMODE == XBF16 || SUB) && BITS == 4 && NS >= 2 && NS <= 4 && (TS == 4 || MB == 2);       // (the others would spill)
+        constexpr bool BY_TILE = !STRIPS && (XMODE == XBF16 || SUB) && BITS == 4 && NS >= 2 && NS <= 4 && (TS == 4 || MB == 2);       // (the others would spill)
         static_assert(!SUB || (BY_TILE && XMODE == XF16 && !NORM), "subnormal operands: f16 activations, walked by tile");
         constexpr int WU = NS == 4 ? (TS < 2 ? TS : 2) : TS;       // BY_TILE: K tiles requested ahead (about eight weight tiles)
         TileRegs<BITS> buf[NS][TS];
@@ -895,7 +896,7 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
     }
 }
 
-template <int BITS, int XMODE, int TS, int NS, int XR, int MB = 1>
+template <int BITS, int XMODE, int TS, int NS, int XR, int MB = 1, bool STRIPS = false>
 hipError_t launch_rows_x(const WeightView& w, const void* x, int M, void* y, int ydt, int nwaves, const Epilogue& epi,
                          bool sub, hipStream_t st)
 {
@@ -928,8 +929,8 @@ hipError_t launch_rows_x(const WeightView& w, const void* x, int M, void* y, int
     }
     // (the exchange area alone passes 64 KB with eight strips, or four strips and two row blocks)
     if constexpr (NS * MB * 8 * 1024 + 512 > 64 * 1024)
-        (void)LdsRequest<&gemv_rows_kernel<BITS, XMODE, TS, NS, false, XR, MB>, 150 * 1024>::registered;
-    hipLaunchKernelGGL((gemv_rows_kernel<BITS, XMODE, TS, NS, false, XR, MB>), dim3(groups), dim3(nwaves * 64), lds, st, w.base,
+        (void)LdsRequest<&gemv_rows_kernel<BITS, XMODE, TS, NS, false, XR, MB, false, false, STRIPS>, 150 * 1024>::registered;
+    hipLaunchKernelGGL((gemv_rows_kernel<BITS, XMODE, TS, NS, false, XR, MB, false, false, STRIPS>), dim3(groups), dim3(nwaves * 64), lds, st, w.base,
                        reinterpret_cast<const uint16_t*>(x), nullptr, w.KT, w.K, w.NT, M, nwaves, 0, w.N, y, ydt, epi, 1, 0, nullptr, nullptr);
     return hipGetLastError();
 }
@@ -1007,9 +1008,9 @@ hipError_t launch_rows_t(const WeightView& w, const void* x, int M, void* y, int
 
 // strips per workgroup: as many as keeps about one workgroup per CU, at most 4.  Two from one strip per CU on: workgroups of eight
 // waves have a CU to themselves, so a few more of them than CUs take two rounds.  us per call, one strip / two: Q4 f16 4096 -> 4224 at
-// 8 / 16 / 32 rows 7.0 / 5.2, 8.0 / 5.9, 11.7 / 9.4, 11008 -> 6000 15.8 / 12.5, 19.8 / 14.4, 30.7 / 21.6, fp32 4096 -> 5120 at 16 rows with a
+// 8 / 16 / 32 rows 7.0 / 5.8, 8.0 / 6.3, 11.7 / 9.7, 11008 -> 6000 15.8 / 13.6, 19.8 / 15.0, 30.7 / 22.2, fp32 4096 -> 5120 at 16 rows with a
 // norm 18.0 / 10.9, Q8 f16 14336 -> 4224 at 8 / 32 rows 23.6 / 18.7, 39.5 / 28.6.  Not with four waves, two of whose workgroups share a CU (1024 ->
-// 5120 at 8 rows 4.1 / 4.3, Q8 4.3 / 4.8; 17 .. 32 rows of Q4 6.6 / 4.7), nor for nine or more f16 rows of Q8 with a norm (14336 -> 4224 31.1 / 33.4).
+// 5120 at 8 rows 4.1 / 4.3, Q8 4.3 / 4.8; 17 .. 32 rows of Q4 6.6 / 5.2), nor for nine or more f16 rows of Q8 with a norm (14336 -> 4224 31.1 / 33.4).
 // Likewise four of Q4 from two per CU on, two / four, f16: 8192 -> 9216 at 8 / 16 / 32 rows 16.9 / 13.4, 19.7 / 15.1, 28.1 / 21.2, 14336 -> 9216 with a
 // norm at 16 rows 37.7 / 29.4, bf16 46.1 / 31.8 (16-bit rows of K up to 4096 run the kernel of gemv_stream.hip there).
 int strips_per_group(const WeightView& w, int xdt, int M, int num_cus, const Epilogue& epi)
@@ -1023,12 +1024,23 @@ int strips_per_group(const WeightView& w, int xdt, int M, int num_cus, const Epi
     return ns;
 }
 
+// Which outputs go by tile where their workgroups have two strips or more (f16 rows: with subnormal operands): from one and a half strips per
+// CU on, and pairs.  Below that a workgroup has two strips for the sake of its rounds alone; a row goes strip by strip there, in any batch of
+// 3 .. 32, as it does with one: f16 rows with exact integers (9e-8 against 5e-7 of relative L2 at K = 4096), 8 / 16 / 32 rows of 4096 -> 4224
+// 5.8 / 6.3 / 9.7 us where the walk by tile takes 5.5 / 6.1 / 9.7, of 14336 -> 4224 14.6 / 18.6 / 24.2 and 15.0 / 18.2 / 23.8; 17 / 32 bf16 rows of
+// 1024 -> 5120 5.5 / 5.7 and 4.9 / 5.1.  (bf16 rows of 16 K tiles and more go by tile in any batch all the same: 7.5e-7 -> 5e-7.)
+bool goes_by_tile(const WeightView& w, int num_cus, const Epilogue& epi)
+{
+    return epi.kind == kEpiSwiglu || w.NT + num_cus / 2 >= 2 * num_cus;
+}
+
 template <int BITS, int XMODE>
 hipError_t launch_rows(const WeightView& w, const void* x, int M, void* y, int ydt, int tuned_waves, int num_cus,
                        const Epilogue& epi, bool sub, hipStream_t st)
 {
     // 8 waves split K (fewer when the strip has fewer tiles), 4 tiles of x per wave and slab
     const int ns = strips_per_group(w, XMODE == XF16 ? kF16 : kBF16, M, num_cus, epi);
+    sub = sub && goes_by_tile(w, num_cus, epi);
     // seven strips per workgroup when that is exactly one workgroup per CU (N = 28672 on 256 CUs:
     // with four strips the 448 workgroups need a second, mostly empty round); SwiGLU pairs need an
     // even count: eight strips there, 224 workgroups in one round
@@ -1125,8 +1137,13 @@ hipError_t launch_rows2(const WeightView& w, const void* x, int M, void* y, int 
                         const Epilogue& epi, bool sub, hipStream_t st)
 {
     const int ns = strips_per_group(w, XMODE == XF16 ? kF16 : kBF16, M, num_cus, epi);
+    sub = sub && goes_by_tile(w, num_cus, epi);
     int nwaves = tuned_waves > 0 ? min(tuned_waves, 8) : 8;
     while (nwaves > 1 && nwaves * 2 > w.KT) nwaves >>= 1;
+    if constexpr (BITS == 4 && XMODE == XBF16) {        // (up to 16 rows of so short a K have one strip to a workgroup)
+        if (w.KT < 16 && ns == 2 && !goes_by_tile(w, num_cus, epi))
+            return launch_rows_x<BITS, XMODE, 2, 2, 16, 2, true>(w, x, M, y, ydt, nwaves, epi, sub, st);
+    }
     if constexpr (BITS == 4) {
         if (w.NT == 7 * num_cus && epi.kind != kEpiSwiglu)
             return launch_rows_x<BITS, XMODE, 2, 7, 16, 2>(w, x, M, y, ydt, nwaves, epi, sub, st);

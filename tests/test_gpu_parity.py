@@ -288,11 +288,13 @@ def test_decode_rows_streamed_by_staying_workgroups(backend, bits, xdt, shape):
 
 # two kernels share these shapes by row count: full rounds of four and two strips up to 16 rows and staying workgroups beyond (an odd
 # last strip, a ragged K tile, waves with three and four K tiles), the reverse for gate / up pairs (four waves too),
-# seven strips per CU, several rounds per CU, and shapes that one kernel has for itself
+# seven strips per CU, several rounds per CU, and shapes that one kernel has for itself; a few strips more than CUs, with two strips to a
+# workgroup from 17 rows or from three
 @pytest.mark.parametrize("bits,N,K,pair", [(4, 14336, 4096, False), (4, 14341, 4064, False), (4, 8180, 3104, False), (4, 32000, 3200, False),
                                            (4, 28672, 4096, False), (4, 32784, 3200, False), (4, 10241, 3104, False), (4, 20480, 4096, True),
                                            (4, 6176, 3104, True), (4, 20480, 1792, True), (4, 6176, 1664, True), (8, 14336, 4096, False),
-                                           (8, 8224, 3104, True), (4, 6144, 928, False), (4, 28640, 2048, True), (4, 28656, 4096, False), (8, 6144, 928, False)])
+                                           (8, 8224, 3104, True), (4, 6144, 928, False), (4, 28640, 2048, True), (4, 28656, 4096, False), (8, 6144, 928, False),
+                                           (4, 4130, 1024, False), (4, 5120, 4096, False), (4, 6127, 12320, False)])
 @pytest.mark.parametrize("xdt", ["f16", "bf16"])
 def test_a_row_keeps_its_bits_from_3_to_32_rows(backend, bits, N, K, pair, xdt):
     g = torch.Generator(device="cuda").manual_seed(N + K)
@@ -473,6 +475,31 @@ def test_staying_workgroups_against_the_batched_rows_kernel(backend, bits, N, K,
                     assert torch.equal(a, b) or a.isnan().all() and b.isnan().all(), (M, ydt)
     finally:
         backend.set_gemv_tuning(0, 0, 0)
+        backend.set_decode_mode("stream")
+
+
+# f16 rows that meet the exact integers in either decode mode, two strips to a workgroup or not: fewer than one and a half strips per CU (the
+# shortest K from 17 rows).  The same bits in both modes, and zeros from zeros
+@pytest.mark.parametrize("N,K,pair", [(4112, 160, False), (4224, 1024, False), (5120, 4096, False), (6127, 2080, False), (4224, 12320, False)])
+def test_f16_rows_with_integers_in_either_mode(backend, N, K, pair):
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    rows = N // 2 if pair else N
+    qd = torch.randint(0, 256, (rows * K // 2,), dtype=torch.uint8, device="cuda", generator=g)
+    sd = (0.01 * torch.rand(rows * (K // 32), device="cuda", generator=g)).half().view(torch.int16)
+    ws = [[backend.weight_from_device(4, rows, K, q, sd) for _ in range(2 if pair else 1)] for q in (qd, torch.zeros_like(qd))]
+    w, zero = [backend.fuse_pairs(*p) if pair else p[0] for p in ws]
+    try:
+        for M in (3, 8, 9, 16) + (() if pair else (17, 32)):
+            x = torch.empty((M, K), device="cuda").normal_(generator=g).half()
+            ys = []
+            for mode in ("stream", "exact"):
+                backend.set_decode_mode(mode)
+                for v in (w, zero):
+                    y = torch.full((M, rows), float("nan"), device="cuda")
+                    backend.matmul_ex(v, x, y, "swiglu" if pair else "none")
+                    ys.append(y)
+            assert torch.equal(ys[0], ys[2]) and (ys[1] == 0).all() and (ys[3] == 0).all(), M
+    finally:
         backend.set_decode_mode("stream")
 
 
