@@ -292,43 +292,47 @@ hipError_t launch_m(const WeightView& w, const void* x, int M, void* y, int ydt,
 int waves_of(const WeightView& w) { return w.KT < 16 ? 4 : 8; }
 int tiles_per_wave(const WeightView& w) { return (w.KT + waves_of(w) - 1) / waves_of(w); }
 
+// seven strips per CU, or eight and more: the batched-rows kernel goes strip by strip there
+bool is_widest(const WeightView& w, int num_cus) { return w.NT >= 8 * num_cus || w.NT == 7 * num_cus; }
+
 // Q4, four K tiles per wave: whether the batched-rows kernel's workgroups (four strips, or two) come in nearly full rounds.  It walks
 // such a shape by tile (gemv_rows_kernel, BY_TILE), and so does this kernel then, whichever of the two has a call: a row keeps its bits.
 bool rows_kernel_by_tile(const WeightView& w, int num_cus)
 {
-    if (w.bits != 4 || waves_of(w) != 8 || tiles_per_wave(w) != 4 || w.NT >= 8 * num_cus || w.NT == 7 * num_cus) return false;
+    if (w.bits != 4 || waves_of(w) != 8 || tiles_per_wave(w) != 4 || is_widest(w, num_cus)) return false;
     const int ns = (w.NT + num_cus / 2) / num_cus >= 3 ? 4 : 2;
     const int groups = (w.NT + ns - 1) / ns, rounds = (groups + num_cus - 1) / num_cus;
     return groups * 5 >= rounds * num_cus * 4;
 }
 
 // Whether the batched-rows kernel is the quicker one up to 16 rows.  Without a norm: nine rows or more where its workgroups are one nearly
-// full round of four strips, and, but for pairs, the widest outputs.  It gives every wave four K tiles to walk whether they are there
+// full round of four strips, and, but for pairs of bf16 rows, the widest outputs.  It gives every wave four K tiles to walk whether they are there
 // or not, so a shorter K is never its.  us per call, this kernel / that one, f16 rows (bf16).  K = 4096: 14336 at 4 / 8 / 16 rows 8.3 / 8.3,
-// 8.5 / 8.5, 9.7 / 9.0 (8.4 / 8.4, 9.0 / 9.0, 10.3 / 9.4), 16384 8.9 / 8.7, 9.0 / 9.7, 10.5 / 9.6, 28672 15.7 / 14.6, pairs 14.1 / 14.4, pairs
-// of 128256 48.7 / 53.1.  K = 3456: 14336 at 8 / 16 rows 7.4 / 8.6, 8.9 / 8.9, 32768 14.2 / 15.0, 15.0 / 16.3; K = 3712: 28672 at 8 rows 15.3 / 14.2.
+// 8.5 / 8.5, 9.7 / 9.0 (8.4 / 8.4, 9.0 / 9.0, 10.3 / 9.4), 16384 8.9 / 8.7, 9.0 / 9.7, 10.5 / 9.6, 28672 15.7 / 14.6, pairs at 4 / 8 / 16
+// rows 16.4 / 14.6, 16.9 / 15.1, 16.7 / 16.0 (14.5 / 14.6, 14.7 / 16.0, 15.9 / 16.3), of 128256 57.1 / 51.1, 58.5 / 53.2, 56.3 / 57.5 (49.6 / 52.7,
+// 51.6 / 56.4, 52.2 / 59.2).  K = 3456: 14336 at 8 / 16 rows 7.4 / 8.6, 8.9 / 8.9, 32768 14.2 / 15.0, 15.0 / 16.3; K = 3712: 28672 at 8 rows 15.3 / 14.2.
 // With a norm: nearly full rounds, whatever the rows and K, and the widest outputs.
-bool leaves_few_rows(const WeightView& w, int M, int num_cus, const Epilogue& epi)
+bool leaves_few_rows(const WeightView& w, int xdt, int M, int num_cus, const Epilogue& epi)
 {
     if (w.bits != 4 || waves_of(w) != 8 || tiles_per_wave(w) != 4) return false;
-    const bool widest = w.NT >= 8 * num_cus || w.NT == 7 * num_cus;
     if (epi.gamma) {
         const int ns = (w.NT + num_cus / 2) / num_cus >= 3 ? 4 : 2;
         const int groups = (w.NT + ns - 1) / ns, rounds = (groups + num_cus - 1) / num_cus;
-        return widest || groups * 4 >= rounds * num_cus * 3;
+        return is_widest(w, num_cus) || groups * 4 >= rounds * num_cus * 3;
     }
     if (w.KT < 28) return false;
-    if (widest) return epi.kind != kEpiSwiglu;
+    if (is_widest(w, num_cus)) return epi.kind != kEpiSwiglu || xdt == kF16;
     return M > 8 && w.NT * 5 >= num_cus * 16 && w.NT <= num_cus * 4;
 }
 
-// By tile (TILE), besides those: gate / up pairs of four tiles per wave (17 .. 32 rows of them run the batched-rows kernel, by tile).  f16
-// rows only in decode mode STREAM.  17 .. 32 rows go the same way and lose by it (4096 -> 14336 at 24 rows 11.8 / 12.7 us), so only the
-// shapes whose rows that keeps together do.
+// By tile (TILE), besides those: gate / up pairs of four tiles per wave (17 .. 32 rows of them run the batched-rows kernel, by tile), but for
+// f16 rows of the widest, which keep their integers (1.5e-7 against 8e-7 of relative L2).  f16 rows only in decode mode STREAM.  17 .. 32 rows
+// go the same way and lose by it (4096 -> 14336 at 24 rows 11.8 / 12.7 us), so only the shapes whose rows that keeps together do.
 bool by_tile(const WeightView& w, int xdt, int num_cus, bool exact_operands, const Epilogue& epi)
 {
     if (w.bits != 4 || tiles_per_wave(w) != 4 || epi.gamma || (xdt == kF16 && exact_operands)) return false;
-    return epi.kind == kEpiSwiglu || rows_kernel_by_tile(w, num_cus);
+    if (epi.kind == kEpiSwiglu) return xdt == kBF16 || !is_widest(w, num_cus);
+    return rows_kernel_by_tile(w, num_cus);
 }
 
 template <int BITS, int XMODE, int W, bool NORM>
@@ -365,7 +369,7 @@ bool gemv_stream_serves(const WeightView& w, int xdt, int M, int num_cus, const 
     if (tiles_per_wave(w) == 4 && M > 16 && (epi.kind == kEpiSwiglu || epi.gamma)) return false;          // (pairs, or gamma, do not fit them)
     // (x * gamma is rounded to the operand type: the prefill kernels, which take these calls otherwise, round it to f16)
     if (M > 16 && epi.gamma && xdt == kBF16) return false;
-    return M > 16 || !leaves_few_rows(w, M, num_cus, epi);
+    return M > 16 || !leaves_few_rows(w, xdt, M, num_cus, epi);
 }
 
 hipError_t launch_gemv_stream(const WeightView& w, const void* x, int xdt, int M, void* y, int ydt, int num_cus, bool exact_operands,

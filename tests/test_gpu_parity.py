@@ -479,8 +479,9 @@ def test_staying_workgroups_against_the_batched_rows_kernel(backend, bits, N, K,
 
 
 # f16 rows that meet the exact integers in either decode mode, two strips to a workgroup or not: fewer than one and a half strips per CU (the
-# shortest K from 17 rows).  The same bits in both modes, and zeros from zeros
-@pytest.mark.parametrize("N,K,pair", [(4112, 160, False), (4224, 1024, False), (5120, 4096, False), (6127, 2080, False), (4224, 12320, False)])
+# shortest K from 17 rows), and pairs of seven strips per CU or eight and more.  The same bits in both modes, and zeros from zeros
+@pytest.mark.parametrize("N,K,pair", [(4112, 160, False), (4224, 1024, False), (5120, 4096, False), (6127, 2080, False), (4224, 12320, False),
+                                      (28672, 4096, True), (32800, 3104, True), (40000, 3616, True)])
 def test_f16_rows_with_integers_in_either_mode(backend, N, K, pair):
     g = torch.Generator(device="cuda").manual_seed(N + K)
     rows = N // 2 if pair else N
