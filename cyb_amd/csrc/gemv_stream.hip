@@ -12,7 +12,7 @@
 // Which wave owns which K tile, and the order of every sum, is that of gemv.hip's kernel with the same waves, with its plain
 // operands (f16 rows: exact integers) or, where that kernel shares a shape by row count and walks it by tile, with those of that
 // walk (TILE): a row's bits do not depend on the batch of 3 .. 32 rows it travels in.  (With a folded norm the squares are summed as
-// loaded, so they do: 3 .. 4, 5 .. 8, 9 .. 32 rows.  The operands are the plain ones then: by tile 4096 -> 32768 at 8 f16 rows takes 16.2 us
+// loaded, so they do: 3 .. 8, 9 .. 32 rows here, up to 4, 8, 16 in gemv.hip.  The operands are the plain ones then: by tile 4096 -> 32768 at 8 f16 rows takes 16.2 us
 // instead of 18.0, but its sums carry the bias: 5e-7 of relative L2 against float64 where the integers have 1e-7.)
 // (f16 rows, us per call before -> after: Q8 2560 -> 32003 at 8 / 27 rows 20.1 -> 16.1, 36.4 -> 17.9 (12.4 at 7 TB/s); Q4 2048 ->
 // 20000 with a norm 17.6 -> 8.2, 22.0 -> 10.6; Q4 4096 -> 128256 at 27 rows 92.6 -> 66.2.  Two or three pairs ahead
@@ -271,7 +271,7 @@ hipError_t launch_k(const WeightView& w, const void* x, int M, void* y, int ydt,
 }
 
 // (the x load pattern follows the batch: up to 4, up to 8, up to 16 rows per load.  f16 rows, 4 rows, eight / four to a load: 4096 -> 6144
-// 5.4 / 4.9 us, with a norm 6.6 / 6.1, bf16 7.4 / 6.7; 4096 -> 28672 with a norm 15.2 / 14.9)
+// 5.4 / 4.9 us.  With a folded norm the squares are summed as loaded: eight to a load, so that 3 .. 8 rows share a row's bits; Q8 8.9 / 8.5, bf16 9.6 / 9.0)
 template <int BITS, int XMODE, int W, int TS, bool NORM, bool TILE>
 hipError_t launch_m(const WeightView& w, const void* x, int M, void* y, int ydt, int num_cus, const Epilogue& epi, hipStream_t st)
 {
@@ -282,7 +282,9 @@ hipError_t launch_m(const WeightView& w, const void* x, int M, void* y, int ydt,
         else return hipErrorInvalidValue;        // gemv_stream_serves() said no
     }
     if constexpr (W == 8) {
-        if (M <= 4) return launch_k<BITS, XMODE, W, TS, 1, 4, NORM, TILE>(w, x, M, y, ydt, num_cus, epi, st);
+        if constexpr (!NORM) {
+            if (M <= 4) return launch_k<BITS, XMODE, W, TS, 1, 4, false, TILE>(w, x, M, y, ydt, num_cus, epi, st);
+        }
         if (M <= 8) return launch_k<BITS, XMODE, W, TS, 1, 8, NORM, TILE>(w, x, M, y, ydt, num_cus, epi, st);
     }
     return launch_k<BITS, XMODE, W, TS, 1, 16, NORM, TILE>(w, x, M, y, ydt, num_cus, epi, st);

@@ -478,6 +478,24 @@ def test_staying_workgroups_against_the_batched_rows_kernel(backend, bits, N, K,
         backend.set_decode_mode("stream")
 
 
+# a folded norm: the squares of a row are summed as the row is loaded, and the workgroups that stay load 3 .. 8 rows in one form
+@pytest.mark.parametrize("bits,N,K", [(4, 6149, 2080), (4, 12288, 3072), (4, 20000, 4096), (8, 6149, 4064), (8, 8192, 2048)])
+@pytest.mark.parametrize("xdt", ["f16", "bf16"])
+def test_a_row_keeps_its_bits_from_3_to_8_rows_with_a_folded_norm(backend, bits, N, K, xdt):
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    qd = torch.randint(0, 256, (N * K * bits // 8,), dtype=torch.uint8, device="cuda", generator=g)
+    sd = (0.01 * torch.rand(N * (K // 32), device="cuda", generator=g)).half().view(torch.int16)
+    w = backend.weight_from_device(bits, N, K, qd, sd)
+    x = torch.empty((8, K), device="cuda").normal_(generator=g).to(TDT[xdt])
+    gamma = 1.0 + 0.25 * torch.empty(K, device="cuda").normal_(generator=g)
+    full = torch.full((8, N), float("nan"), device="cuda")
+    backend.matmul_norm(w, x, gamma, 1e-5, full)
+    for M in (3, 4, 5):
+        y = torch.full((M, N), float("nan"), device="cuda")
+        backend.matmul_norm(w, x[:M].contiguous(), gamma, 1e-5, y)
+        assert torch.equal(y, full[:M]), M
+
+
 # f16 rows that meet the exact integers in either decode mode, two strips to a workgroup or not: fewer than one and a half strips per CU (the
 # shortest K from 17 rows), and pairs of seven strips per CU or eight and more.  The same bits in both modes, and zeros from zeros
 @pytest.mark.parametrize("N,K,pair", [(4112, 160, False), (4224, 1024, False), (5120, 4096, False), (6127, 2080, False), (4224, 12320, False),
