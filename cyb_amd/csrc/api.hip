@@ -496,26 +496,24 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
         if (e == hipSuccess) e = weight_is_wide(w, &is);
         return is;
     };
+    // the tail of the scratch belongs to the decode kernels (tickets and slabs of a K split), the rest to prefill
+    const bool split = workspace && workspace_bytes > 2 * cybq::kDecodeScratchBytes;
+    const size_t prefill_bytes = !workspace ? 0 : split ? workspace_bytes - cybq::kDecodeScratchBytes : workspace_bytes;
+    void* const dscr = split ? static_cast<char*>(workspace) + prefill_bytes : nullptr;
+    const size_t dscr_bytes = split ? cybq::kDecodeScratchBytes : 0;
     enum { kDecode, kTwoPasses, kPrefill, kPrefillExact, kWalk } way;
     if (M <= 16 || (M <= 32 && cybq::gemv_serves_32(v, (int)xdt, (int)M, ctx->num_cus, epi)))
         way = kDecode;
     else if (M <= 64 && (int64_t)w->N * w->K <= (int64_t)6144 * 4096 && cybq::gemv_serves_32(v, (int)xdt, 32, ctx->num_cus, epi) &&
              (ctx->prefill_exact || wide() || !cybq::gemm_rows_takes(v, (int)M, ctx->num_cus, epi)))
-        way = (M > 32 && w->bits == 4 && xdt == CYBQ_BF16 && (w->K > 4096 || (w->K <= 512 && w->N >= 6144)) && !wide()) ? kPrefillExact : kTwoPasses;
+        way = (M > 32 && w->bits == 4 && xdt == CYBQ_BF16 && (w->K > 4096 || (w->K <= 512 && w->N >= 6144)) && !wide() &&
+               cybq::gemm_stages(v, prefill_bytes)) ? kPrefillExact : kTwoPasses;
     else if (!wide() && (xdt == CYBQ_F32 ? !ctx->prefill_exact : (M > 32 || (!ctx->prefill_exact && cybq::gemm_rows_takes(v, (int)M, ctx->num_cus, epi)))))
         way = kPrefill;
     else
         way = kWalk;
     if (e != hipSuccess) return fail_hip(ctx, e, "scale scan");
     mark_use(w, stream);
-    // the tail of the scratch belongs to the decode kernels (tickets and slabs of a K split), the rest to prefill
-    void* dscr = nullptr;
-    size_t dscr_bytes = 0;
-    if (workspace && workspace_bytes > 2 * cybq::kDecodeScratchBytes) {
-        workspace_bytes -= cybq::kDecodeScratchBytes;
-        dscr = static_cast<char*>(workspace) + workspace_bytes;
-        dscr_bytes = cybq::kDecodeScratchBytes;
-    }
     if (way == kDecode) {
         e = cybq::launch_gemv(v, x, xdt, (int)M, y, ydt, ctx->num_cus, ctx->decode_exact, epi, dscr, dscr_bytes, st);
     } else if (way == kTwoPasses) {
@@ -524,9 +522,9 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
         // quicker than a staging launch and a multiply although they stream the weights twice - and exact.  us per call, two passes
         // / gemm_cols.hip with bf16 rows on Q4, at 33, 48, 64 rows: 4096 -> 4096 11.4, 12.6, 14.8 / 14.4, 14.9, 16.1, 2048 -> 6144 9.5, 9.6,
         // 10.9 / 13.6, 14.1, 14.8.  Not with a longer K (8192 -> 512 15.0, 17.1, 20.6 / 12.7, 12.9, 13.3; 14336 -> 1024 25.9, 30.9, 38.0 /
-        // 16.9, 17.0, 17.9) nor with the shortest on a wide output (512 -> 14336 11.7, 15.8, 17.9 / 8.6, 8.8, 9.1): bf16 rows on Q4 go
-        // through the prefill path there, with exact operands whatever the mode (kPrefillExact; relative L2 against float64
-        // 7.6e-7 -> 2.2e-7; f16 rows 1.5e-7 -> 2.6e-7 and Q8 1.5e-7 -> 1.7e-6 stay).
+        // 16.9, 17.0, 17.9) nor with the shortest on a wide output (512 -> 14336 11.7, 15.8, 17.9 / 8.6, 8.8, 9.1): bf16 rows on Q4
+        // go through the prefill path there, with exact operands whatever the mode (kPrefillExact; relative L2 against float64 7.6e-7 -> 2.2e-7; f16 rows
+        // 1.5e-7 -> 2.6e-7 and Q8 1.5e-7 -> 1.7e-6 stay), unless K is so long (251 936 and more) that the scratch does not hold 256 staged rows.
         // (a context in CYBQ_PREFILL_EXACT mode asked for exact operands at this row count)
         const bool exact_ops = ctx->decode_exact || ctx->prefill_exact;
         const int64_t n_out = epi.kind == cybq::kEpiSwiglu ? w->N / 2 : w->N;
@@ -538,7 +536,7 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
             e = cybq::launch_gemv(v, static_cast<const char*>(x) + (size_t)32 * w->K * dtype_size(xdt), xdt, (int)M - 32,
                                   static_cast<char*>(y) + yoff, ydt, ctx->num_cus, exact_ops, ec, dscr, dscr_bytes, st);
     } else if (way == kPrefill || way == kPrefillExact) {
-        e = cybq::launch_gemm(v, x, xdt, (int)M, y, ydt, ctx->num_cus, ctx->prefill_exact || way == kPrefillExact, workspace, workspace_bytes,
+        e = cybq::launch_gemm(v, x, xdt, (int)M, y, ydt, ctx->num_cus, ctx->prefill_exact || way == kPrefillExact, workspace, prefill_bytes,
                               epi, st);
     } else {
         // fp32 activations keep full precision through the decode kernel's hi/lo split:

@@ -60,6 +60,8 @@ struct RowsPlan {
 RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi);
 hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, void* y, int ydt, const Epilogue& epi,
                             const float* ssq_part, int ssq_blocks, const float* unscale, const RowsPlan& plan, hipStream_t st);
+// whether a scratch of this size holds enough staged rows of w's K for launch_gemm (which refuses the call otherwise)
+bool gemm_stages(const WeightView& w, size_t workspace_bytes);
 // the prefill kernel whose waves stand side by side along the columns (gemm_cols.hip).  mode: 0 FAST, 1 / 2 EXACT with f16 / bf16
 // operands; more than one split leaves fp32 slabs [splits][M][N] in `part` for the slab-adding pass
 struct ColsPlan {

@@ -1203,6 +1203,21 @@ static Touch plan_touch(const WeightView& w, int mc, int num_cus, const Epilogue
     return tc;
 }
 
+// The last MiB of the scratch's first half: per-row statistics - partial sums of squares of a folded
+// RMSNorm (rows of a chunk x K / 512 floats: less than half / 256 bytes) and, in its last
+// quarter, the per-row power of two of widened activations (at most 65536 rows per chunk).
+constexpr size_t kStatsBytes = (size_t)1 << 20;
+
+// rows of K 16-bit elements the first half holds in front of them, in whole row tiles
+static int64_t staged_rows(const WeightView& w, size_t workspace_bytes)
+{
+    const size_t half = workspace_bytes / 2;
+    if (half <= kStatsBytes) return 0;
+    return std::min<int64_t>(65536, (int64_t)((half - kStatsBytes) / ((size_t)w.K * 2)) / 256 * 256);
+}
+
+bool gemm_stages(const WeightView& w, size_t workspace_bytes) { return staged_rows(w, workspace_bytes) >= 256; }
+
 hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void* y, int ydt,
                        int num_cus, bool exact, void* workspace, size_t workspace_bytes, const Epilogue& epi,
                        hipStream_t st)
@@ -1218,17 +1233,11 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
     // First half of the workspace: staged X; second half: partial sums of a K split.
     const size_t half = workspace_bytes / 2;
     float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + half);
-    // The last MiB of the first half: per-row statistics - partial sums of squares of a folded
-    // RMSNorm (rows of a chunk x K / 512 floats: less than half / 256 bytes) and, in its last
-    // quarter, the per-row power of two of widened activations (at most 65536 rows per chunk).
-    const size_t stats_bytes = (size_t)1 << 20;
-    if (!workspace || half <= stats_bytes) return hipErrorOutOfMemory;
-    float* ssq_part = reinterpret_cast<float*>(static_cast<char*>(workspace) + half - stats_bytes);
-    float* unscale = reinterpret_cast<float*>(static_cast<char*>(workspace) + half - stats_bytes / 4);
+    const int64_t max_rows = staged_rows(w, workspace_bytes);
+    if (!workspace || max_rows < 256) return hipErrorOutOfMemory;
+    float* ssq_part = reinterpret_cast<float*>(static_cast<char*>(workspace) + half - kStatsBytes);
+    float* unscale = reinterpret_cast<float*>(static_cast<char*>(workspace) + half - kStatsBytes / 4);
     const int64_t row_bytes = (int64_t)w.K * (xdt == kF32 ? 4 : 2);        // a row of the caller's X
-    const int64_t max_rows =
-        std::min<int64_t>(65536, (int64_t)((half - stats_bytes) / (size_t)(w.K * 2)) / 256 * 256);    // staged rows are 16-bit
-    if (max_rows < 256) return hipErrorOutOfMemory;
     const size_t ysize = ydt == kF32 ? 4 : 2;
     for (int64_t m_lo = 0; m_lo < M; m_lo += max_rows) {
         const int mc = (int)((M - m_lo) < max_rows ? (M - m_lo) : max_rows);

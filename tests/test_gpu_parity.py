@@ -2245,6 +2245,28 @@ def test_rows_33_to_64_on_a_small_weight_are_two_decode_passes(backend, oracle, 
         wz.free()
 
 
+def _two_passes(backend, w, x):
+    return torch.cat([_run(backend, w, x[:32].contiguous()), _run(backend, w, x[32:].contiguous())])
+
+
+def test_rows_33_to_64_with_a_k_that_the_scratch_does_not_hold(backend):
+    """256 staged rows of a K over 251 904 pass the scratch: 33..64 bf16 rows of Q4 stay two decode passes there; just below they are one
+    prefill call with exact operands."""
+    N, M = 48, 45
+    g = torch.Generator(device="cuda").manual_seed(17)
+    for K, fits in ((262144 + 32, False), (131072, True)):
+        qd = torch.randint(0, 256, (N * K // 2,), dtype=torch.uint8, device="cuda", generator=g)
+        sd = (0.01 * torch.rand(N * (K // 32), device="cuda", generator=g)).half().view(torch.int16)
+        w = backend.weight_from_device(4, N, K, qd, sd)
+        wd = torch.empty((N, K), device="cuda")
+        backend.dequant(w, wd)
+        x = torch.empty((M, K), device="cuda").normal_(generator=g).bfloat16()
+        y = _run(backend, w, x)
+        ref = x.double() @ wd.double().t()
+        assert ((y.double() - ref).norm() / ref.norm()).item() < TIGHT
+        assert torch.equal(y, _two_passes(backend, w, x)) == (not fits)
+
+
 def _node_reference(oracle, st, node, epi, edges, rows=None):
     """float64 oracle output of one stack node from the PLANAR buffers the stack kept."""
     qd, sd = st.planar[node.w]
