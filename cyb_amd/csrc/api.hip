@@ -506,7 +506,9 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
         way = kDecode;
     else if (M <= 64 && (int64_t)w->N * w->K <= (int64_t)6144 * 4096 && cybq::gemv_serves_32(v, (int)xdt, 32, ctx->num_cus, epi) &&
              (ctx->prefill_exact || wide() || !cybq::gemm_rows_takes(v, (int)M, ctx->num_cus, epi)))
-        way = (M > 32 && w->bits == 4 && xdt == CYBQ_BF16 && (w->K > 4096 || (w->K <= 512 && w->N >= 6144)) && !wide() &&
+        // (in FAST mode, where the line above has asked whether the scales are wide: EXACT calls of these rows never did, and their first one on
+        // a weight from device memory may sit in a capture, where the answer cannot be waited for)
+        way = (M > 32 && w->bits == 4 && xdt == CYBQ_BF16 && (w->K > 4096 || (w->K <= 512 && w->N >= 6144)) && !ctx->prefill_exact && !wide() &&
                cybq::gemm_stages(v, prefill_bytes)) ? kPrefillExact : kTwoPasses;
     else if (!wide() && (xdt == CYBQ_F32 ? !ctx->prefill_exact : (M > 32 || (!ctx->prefill_exact && cybq::gemm_rows_takes(v, (int)M, ctx->num_cus, epi)))))
         way = kPrefill;
@@ -522,8 +524,8 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
         // quicker than a staging launch and a multiply although they stream the weights twice - and exact.  us per call, two passes
         // / gemm_cols.hip with bf16 rows on Q4, at 33, 48, 64 rows: 4096 -> 4096 11.4, 12.6, 14.8 / 14.4, 14.9, 16.1, 2048 -> 6144 9.5, 9.6,
         // 10.9 / 13.6, 14.1, 14.8.  Not with a longer K (8192 -> 512 15.0, 17.1, 20.6 / 12.7, 12.9, 13.3; 14336 -> 1024 25.9, 30.9, 38.0 /
-        // 16.9, 17.0, 17.9) nor with the shortest on a wide output (512 -> 14336 11.7, 15.8, 17.9 / 8.6, 8.8, 9.1): bf16 rows on Q4
-        // go through the prefill path there, with exact operands whatever the mode (kPrefillExact; relative L2 against float64 7.6e-7 -> 2.2e-7; f16 rows
+        // 16.9, 17.0, 17.9) nor with the shortest on a wide output (512 -> 14336 11.7, 15.8, 17.9 / 8.6, 8.8, 9.1): in FAST mode bf16 rows on Q4
+        // go through the prefill path there, with exact operands (kPrefillExact; relative L2 against float64 7.6e-7 -> 2.2e-7; f16 rows
         // 1.5e-7 -> 2.6e-7 and Q8 1.5e-7 -> 1.7e-6 stay), unless K is so long (251 936 and more) that the scratch does not hold 256 staged rows.
         // (a context in CYBQ_PREFILL_EXACT mode asked for exact operands at this row count)
         const bool exact_ops = ctx->decode_exact || ctx->prefill_exact;

@@ -78,9 +78,10 @@ typedef enum cybq_dtype { CYBQ_F32 = 0, CYBQ_F16 = 1, CYBQ_BF16 = 2 } cybq_dtype
  * activations with a folded RMSNorm on weights with K of 2048 .. 8192, unless the decode kernels have them in
  * one pass, see cybq_matmul) feed the matrix cores.  Both stay inside the operator's 1e-3 relative-L2
  * tolerance.  (Calls of up to 16 rows, other calls of up to 32 rows, and 33 .. 64 rows on weights of up to
- * 6144 x 4096 that the FAST kernels do not take - with CYBQ_PREFILL_EXACT all but bf16 rows on Q4 with K over
- * 4096, or of up to 512 on N of 6144 and more; it gives them the decode kernels' EXACT operands - take the
- * decode kernels, whose operand form cybq_decode_mode describes.)
+ * 6144 x 4096 that the FAST kernels do not take - always so with CYBQ_PREFILL_EXACT, which gives them the
+ * decode kernels' EXACT operands - take the decode kernels, whose operand form cybq_decode_mode describes.  In
+ * FAST mode bf16 rows of the latter kind on Q4 with K over 4096, or of up to 512 on N of 6144 and more, take the
+ * prefill kernels with EXACT operands instead, where the scratch holds them.)
  *   FAST   (default) one f16 MFMA per 32-group; the weight operand is
  *          round_f16(scale * q), relative error <= 2^-11 per weight (about 2e-4
  *          relative L2 on y).  bf16 and fp32 activations become f16 operands behind a

@@ -2267,6 +2267,36 @@ def test_rows_33_to_64_with_a_k_that_the_scratch_does_not_hold(backend):
         assert torch.equal(y, _two_passes(backend, w, x)) == (not fits)
 
 
+def test_rows_33_to_64_in_exact_mode_may_be_captured_first(backend):
+    """EXACT mode, 33..64 bf16 rows of Q4 on a small weight with a long K: the first call on a weight made from device memory sits in a
+    capture, so nothing in it may wait for the scan of the weight's scales."""
+    N, K, M = 528, 4640, 45
+    g = torch.Generator(device="cuda").manual_seed(18)
+    qd = torch.randint(0, 256, (N * K // 2,), dtype=torch.uint8, device="cuda", generator=g)
+    sd = (0.01 * torch.rand(N * (K // 32), device="cuda", generator=g)).half().view(torch.int16)
+    x = torch.empty((M, K), device="cuda").normal_(generator=g).bfloat16()
+    y = torch.zeros((M, N), device="cuda")
+    w = backend.weight_from_device(4, N, K, qd, sd)
+    torch.cuda.synchronize()
+    backend.set_prefill_mode("exact")
+    try:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+            backend.matmul(w, x, y, stream=torch.cuda.current_stream().cuda_stream)
+        for _ in range(2):
+            y.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, _run(backend, w, x))
+        wd = torch.empty((N, K), device="cuda")
+        backend.dequant(w, wd)
+        ref = x.double() @ wd.double().t()
+        assert ((y.double() - ref).norm() / ref.norm()).item() < TIGHT
+    finally:
+        backend.set_prefill_mode("fast")
+
+
 def _node_reference(oracle, st, node, epi, edges, rows=None):
     """float64 oracle output of one stack node from the PLANAR buffers the stack kept."""
     qd, sd = st.planar[node.w]
