@@ -553,13 +553,15 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
         // time where the batched-rows kernel takes them in one pass: the weights stream once per 32 rows.
         const int64_t n_out = epi.kind == cybq::kEpiSwiglu ? w->N / 2 : w->N;
         const int64_t step = cybq::gemv_serves_32(v, (int)xdt, 32, ctx->num_cus, epi) ? 32 : 16;
-        for (int64_t m0 = 0; m0 < M && e == hipSuccess; m0 += step) {
-            int mm = (int)((M - m0) < step ? (M - m0) : step);
+        for (int64_t m0 = 0, mm; m0 < M && e == hipSuccess; m0 += mm) {
+            mm = (M - m0) < step ? (M - m0) : step;
+            // (with a norm one or two fp32 rows have sums of squares in another order than 3 .. 16: none are left over)
+            if (xdt == CYBQ_F32 && gamma && M - m0 > step && M - m0 < step + 3) mm = step - 2;
             const char* xp = static_cast<const char*>(x) + (size_t)m0 * w->K * dtype_size(xdt);
             const size_t yoff = (size_t)m0 * n_out * dtype_size(ydt);
             cybq::Epilogue ec = epi;
             if (epi.kind == cybq::kEpiAdd) ec.residual = static_cast<const char*>(residual) + yoff;
-            e = cybq::launch_gemv(v, xp, xdt, mm, static_cast<char*>(y) + yoff, ydt, ctx->num_cus, ctx->decode_exact, ec, dscr, dscr_bytes, st);
+            e = cybq::launch_gemv(v, xp, xdt, (int)mm, static_cast<char*>(y) + yoff, ydt, ctx->num_cus, ctx->decode_exact, ec, dscr, dscr_bytes, st);
         }
     }
     if (e != hipSuccess) return fail_hip(ctx, e, "matmul launch");

@@ -12,11 +12,11 @@
 // f16 scale is applied in fp32 on the MFMA result, so the weight operand stays
 // an exact small integer and the only rounding is the fp32 accumulation.
 // Split-K partials meet in LDS in a fixed order: results are deterministic and
-// row m of a batch is bit-identical to the same row run alone.
+// within this kernel row m of a batch is bit-identical to the same row run alone
+// (a folded norm: where x is staged in one slab).
 #include <type_traits>
 #include "cybq_device.h"
 #include "cybq_internal.h"
-#include <type_traits>
 #include "gemv_parts.h"
 
 namespace cybq {
@@ -486,7 +486,9 @@ __global__ __launch_bounds__(1024) void gemv_kernel(const uint8_t* __restrict__ 
 // through the MFMA's C operand like with bf16 activations, 1/16 for the odd groups rides on their scale
 // and 2^22 on the final sums.
 // XF32: fp32 rows, as the LDS kernel multiplies them: every value is split into the f16 nearest to it and the f16 nearest to what that leaves,
-// and a weight operand (the exact integers) meets both, into the same sums.  A row's bits do not depend on its batch of 3 .. 16 rows here.
+// and a weight operand (the exact integers) meets both, into the same sums.  The K tiles are shared out over as many sums as that kernel has waves
+// (lds_waves; up to eight waves here, with SUMS of them each), every sum in its order: a row has the same bits in both, alone or in a batch of up to
+// 16 (eight waves whatever K would take 11.0 instead of 12.2 us at 4 rows of 4096 -> 14336, 8.5 instead of 8.9 at 16 of 4096 -> 4096).  With a norm, whose squares that kernel adds up slab by slab, this one has eight waves and an order of its own, the same for 3 .. 16 rows.
 // KS: K is split over `splits` workgroups per strip group (few strips and a long K: with one workgroup per
 // strip every CU pulls all of x out of the L2, M x K x 2 bytes against its 37 KB x strips of weights).  Workgroup
 // (group, split) walks the K tiles [split * kt_per_split, ...) of the group's NS strips and leaves its sums in
@@ -495,7 +497,7 @@ __global__ __launch_bounds__(1024) void gemv_kernel(const uint8_t* __restrict__ 
 // and loads at system scope, waited for before the ticket is taken): nothing is flushed, nothing invalidated.
 // The ticket is left at zero again for the next launch; launches that share `slabs` must not overlap.
 // STRIPS: strip by strip, also where the walk goes by tile otherwise (BY_TILE).
-template <int BITS, int XMODE, int TS, int NS, bool NORM, int XR, int MB = 1, bool SUB = false, bool KS = false, bool STRIPS = false>
+template <int BITS, int XMODE, int TS, int NS, bool NORM, int XR, int MB = 1, bool SUB = false, bool KS = false, bool STRIPS = false, int SUMS = 1>
 // (waves_per_eu: the scheduler would otherwise trade the up-front loads for occupancy)
 __global__ __launch_bounds__((TS <= 2 && MB == 1 && !NORM && XMODE != XF32) ? 1024 : 512)
 __attribute__((amdgpu_waves_per_eu(2, (TS <= 2 && MB == 1 && !NORM && XMODE != XF32) ? 4 : 2)))
@@ -532,27 +534,29 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
     static_assert(MB == 1 || (XR == 16 && !NORM && XMODE != XF32), "two row blocks: full loads, 16-bit rows, no folded norm");
     constexpr int PL = XMODE == XF32 ? 2 : 1;   // fp32 rows: the high halves and what they leave, two f16 operands
     static_assert(PL == 1 || !SUB, "fp32 rows: exact integers");
+    static_assert(SUMS == 1 || (PL == 2 && TS % SUMS == 0), "tile u of a slab belongs to sum u % SUMS of its wave");
     const uint16_t* xrow = x + (int64_t)min(lane / P, M - 1) * w.K + (lane % P) * 8;
     const int64_t xblock = MB > 1 ? (int64_t)(min(16 + lane / P, M - 1) - min(lane / P, M - 1)) * w.K : 0;     // to my row of the second block
     const int klast = w.K - 8 - (lane % P) * 8;          // last start at which this lane's piece is inside the row
     const int from_lane = ((((lane & 15) & (XR - 1)) * P) | oct) << 2;       // byte address for ds_bpermute (+ 16 per group)
     // NORM: each wave keeps the gamma of the K tiles it is working on in an LDS area of its own,
     // behind the exchange areas
-    uint8_t* gamma_lds = smem + ((size_t)NS * MB * nwaves * 4 * 64 + 8 * 16 + (size_t)wv * TS * kTileK) * sizeof(float);
+    uint8_t* gamma_lds = smem + ((size_t)NS * MB * SUMS * nwaves * 4 * 64 + 8 * 16 + (size_t)wv * TS * kTileK) * sizeof(float);
     const bool gamma_h = NORM && XMODE == XF16 && gamma_dt == kF16;
     const bool gamma_f32 = NORM && gamma_dt == kF32;
     const int g_count = gamma_f32 ? 4 : 8;               // values of a tile's gamma a lane loads,
     const int g_first = (lane & (gamma_f32 ? 31 : 15)) * g_count;       // the first of them,
     const int g_shift = gamma_f32 ? 2 : 1;               // log2 of their size
 
-    float acc[NS][MB][4];
+    float acc[NS][MB * SUMS][4];
 #pragma unroll
     for (int s = 0; s < NS; s++)
 #pragma unroll
-        for (int b = 0; b < MB; b++)
+        for (int b = 0; b < MB * SUMS; b++)
 #pragma unroll
             for (int r = 0; r < 4; r++) acc[s][b][r] = 0.f;
     float ssq = 0.f;          // NORM: squares of the x values this lane loaded (row lane / P)
+    float ssq_of[L] = {};     // fp32 rows: of each load
 
     int64_t sbase[NS];
 #pragma unroll
@@ -602,10 +606,10 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
         constexpr int WU = NS == 4 ? (TS < 2 ? TS : 2) : TS;       // BY_TILE: K tiles requested ahead (about eight weight tiles)
         TileRegs<BITS> buf[NS][TS];
         constexpr int AHEAD = NS < 2 ? NS : 2;
-        // (fp32 rows: a tile's four groups first, then the tiles - eight waves add up to 56 groups each where the LDS kernel's sixteen add 28;
-        // error against 64 bits, 14336 -> 4101: 1.42e-7 there, 1.62e-7 here without this, 1.21e-7 with it)
+        // (fp32 rows with a norm: a tile's four groups first, then the tiles - eight waves add up to 56 groups each where the LDS kernel's sixteen
+        // add 28; error against 64 bits, 14336 -> 4101: 1.42e-7 there, 1.62e-7 here without this, 1.21e-7 with it)
         auto fold = [&](u32x2_t sc, const float4_t (&d)[4], float (&sum)[4]) __attribute__((always_inline)) {
-            if constexpr (XMODE == XF32) {
+            if constexpr (XMODE == XF32 && NORM) {
                 float t[4] = {0.f, 0.f, 0.f, 0.f};
                 tile_accum<4>(sc, d, t);
 #pragma unroll
@@ -671,14 +675,14 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
 #pragma unroll
                     for (int h = 0; h < L; h++) {
                         if constexpr (XMODE == XF32) {
-                            float sq = ssq;
+                            float sq = ssq_of[h];
 #pragma unroll
                             for (int i = 0; i < 8; i++) {
                                 const float v = __builtin_bit_cast(float, (uint32_t)a[i >> 2][u][h].u[i & 3]);
                                 sq = fmaf(v, v, sq);
                                 a[i >> 2][u][h].u[i & 3] = __builtin_bit_cast(uint32_t, v * __builtin_bit_cast(float, (uint32_t)(i < 4 ? g[h].lo : g[h].hi)[i & 3]));
                             }
-                            ssq = counts[h] ? sq : ssq;
+                            ssq_of[h] = counts[h] ? sq : ssq_of[h];
                         } else norm_piece<XMODE, GH>(a[0][u][h].u, g[h], counts[h], ssq);
                     }
                 }
@@ -781,34 +785,47 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
                 sc[1] = valid[u] ? sc[1] : 0u;
 #pragma unroll
                 for (int b = 0; b < MB; b++) {
-                    fold(sprev, dprev[b], acc[s][b]);
+                    fold(sprev, dprev[b], acc[s][SUMS == 1 ? b : (u + SUMS - 1) % SUMS]);
 #pragma unroll
                     for (int j = 0; j < 4; j++) dprev[b][j] = d[b][j];
                 }
                 sprev = sc;
             }
 #pragma unroll
-            for (int b = 0; b < MB; b++) fold(sprev, dprev[b], acc[s][b]);
+            for (int b = 0; b < MB; b++) fold(sprev, dprev[b], acc[s][SUMS == 1 ? b : (TS - 1) % SUMS]);
         }
     }
 
     // split-K partials -> LDS, summed in wave order
     // (slot = strip * MB + row block)
     float* red = reinterpret_cast<float*>(smem);
+    const int sums = SUMS * nwaves;
 #pragma unroll
     for (int s = 0; s < NS; s++)
 #pragma unroll
-        for (int b = 0; b < MB; b++)
+        for (int b = 0; b < MB * SUMS; b++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) red[(((s * MB + b) * nwaves + wv) * 4 + r) * 64 + lane] = acc[s][b][r];
-    float* ssq_part = red + NS * MB * nwaves * 4 * 64;      // [wave][row]
+            for (int r = 0; r < 4; r++)
+                red[((SUMS == 1 ? (s * MB + b) * nwaves + wv : s * sums + b * nwaves + wv) * 4 + r) * 64 + lane] = acc[s][b][r];
+    float* ssq_part = red + NS * MB * sums * 4 * 64;        // [wave][row]
+    if constexpr (NORM && XMODE == XF32) {
+        // (fp32 rows: a row's sixteen pieces of a tile meet eight, then four apart, then within the quad, whether a load has them all in its
+        // lanes or in registers; the lanes that hand a row's sum on are the first of its P)
+        ssq = L == 4 ? (ssq_of[0] + ssq_of[2 % L]) + (ssq_of[1 % L] + ssq_of[3 % L]) : L == 2 ? ssq_of[0] + ssq_of[1 % L] : ssq_of[0];
+        if (P >= 16) ssq += lane_cross<0x128>(ssq);
+        if (P >= 8) ssq += lane_cross<0x12C>(ssq);
+        ssq += lane_cross<0xB1>(ssq);
+        ssq += lane_cross<0x4E>(ssq);
+    }
     if (NORM) {
         // lane l holds pieces of row l / P: sum over each run of P lanes with lane-crossing moves
         // inside the ALU (pairs, quads, then the mirror images within 8 and within 16 lanes)
-        ssq += lane_cross<0xB1>(ssq);
-        ssq += lane_cross<0x4E>(ssq);
-        if (P >= 8) ssq += lane_cross<0x141>(ssq);
-        if (P >= 16) ssq += lane_cross<0x140>(ssq);
+        if constexpr (XMODE != XF32) {
+            ssq += lane_cross<0xB1>(ssq);
+            ssq += lane_cross<0x4E>(ssq);
+            if (P >= 8) ssq += lane_cross<0x141>(ssq);
+            if (P >= 16) ssq += lane_cross<0x140>(ssq);
+        }
         if (lane % P == 0) {
             ssq_part[wv * 16 + lane / P] = ssq;
             if (wv == 0) {                              // the slots of waves this launch does not have
@@ -831,7 +848,16 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
         // and root are some 140 instructions here, half a microsecond between the barrier and the stores)
         const float inv_k = __builtin_amdgcn_rcpf((float)w.K);
 #pragma unroll
-        for (int r = 0; r < 4; r++) rstd[r] = __builtin_amdgcn_rsqf(fmaf(t[r], inv_k, epi.eps));
+        for (int r = 0; r < 4; r++) {
+            if constexpr (XMODE == XF32) {
+                // (fp32 rows: a correction step each, half an ulp; sums near the smallest floats are scaled out of the way, infinity stays)
+                const float q = t[r] * inv_k, v = fmaf(fmaf(-q, (float)w.K, t[r]), inv_k, q) + epi.eps;
+                const bool tiny = v < 0x1p-100f;
+                const float vs = tiny ? fmaf(t[r] * 0x1p100f, inv_k, epi.eps * 0x1p100f) : v, y0 = __builtin_amdgcn_rsqf(vs), vy = vs * y0;
+                const float y1 = fmaf(0.5f * y0, fmaf(-y0, vy, fmaf(-y0, fmaf(vs, y0, -vy), 1.f)), y0);
+                rstd[r] = !(v < 0x1p100f) ? y0 : tiny ? y1 * 0x1p50f : y1;
+            } else rstd[r] = __builtin_amdgcn_rsqf(fmaf(t[r], inv_k, epi.eps));
+        }
     }
     // wave v finishes (strip, output register) pairs v, v + waves, ...
     if (NS >= 2 && epi.kind == kEpiSwiglu) {       // strips 2j / 2j+1 of the group are gate / up of output strip (strip0 >> 1) + j
@@ -840,8 +866,8 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
             const int r = p & 3, b = (p >> 2) % MB, j = (p >> 2) / MB;
             const int nt = (strip0 >> 1) + j;
             const int n = nt * 16 + (lane & 15);
-            const float g = sum_partials(red + (((2 * j) * MB + b) * nwaves * 4 + r) * 64 + lane, nwaves, 4 * 64) * rstd[r];
-            const float u = sum_partials(red + (((2 * j + 1) * MB + b) * nwaves * 4 + r) * 64 + lane, nwaves, 4 * 64) * rstd[r];
+            const float g = sum_partials(red + (((2 * j) * MB + b) * sums * 4 + r) * 64 + lane, sums, 4 * 64) * rstd[r];
+            const float u = sum_partials(red + (((2 * j + 1) * MB + b) * sums * 4 + r) * 64 + lane, sums, 4 * 64) * rstd[r];
             const int m = 16 * b + 4 * oct + r;
             if (2 * nt + 1 < w.NT && m < M && n < n_out) store_out(y, ydt, (int64_t)m * n_out + n, silu_mul(g, u));
         }
@@ -890,19 +916,19 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
         const int r = p & 3, b = (p >> 2) % MB, s = (p >> 2) / MB;
         const int nt = strip0 + s;
         const int n = nt * 16 + (lane & 15);
-        const float v = sum_partials(red + ((s * MB + b) * nwaves * 4 + r) * 64 + lane, nwaves, 4 * 64) * rstd[r];
+        const float v = sum_partials(red + ((s * MB + b) * sums * 4 + r) * 64 + lane, sums, 4 * 64) * rstd[r];
         const int m = 16 * b + 4 * oct + r;
         if (nt < w.NT && m < M && n < w.N) emit(y, ydt, epi, (int64_t)m * w.N + n, v);
     }
 }
 
-template <int BITS, int XMODE, int TS, int NS, int XR, int MB = 1, bool STRIPS = false>
+template <int BITS, int XMODE, int TS, int NS, int XR, int MB = 1, bool STRIPS = false, int SUMS = 1>
 hipError_t launch_rows_x(const WeightView& w, const void* x, int M, void* y, int ydt, int nwaves, const Epilogue& epi,
                          bool sub, hipStream_t st)
 {
-    size_t lds = (size_t)NS * MB * nwaves * 4 * 64 * sizeof(float) + 8 * 16 * sizeof(float);
+    size_t lds = (size_t)NS * MB * SUMS * nwaves * 4 * 64 * sizeof(float) + 8 * 16 * sizeof(float);
     const unsigned groups = (unsigned)((w.NT + NS - 1) / NS);
-    if constexpr (MB == 1 && !(XMODE == XF32 && TS == 4)) {
+    if constexpr (MB == 1 && SUMS == 1 && !(XMODE == XF32 && TS == 4)) {
         if (epi.gamma) {
             lds += (size_t)nwaves * TS * kTileK * sizeof(float);            // each wave's tiles of gamma as fp32
             auto kern = gemv_rows_kernel<BITS, XMODE, TS, NS, true, XR>;
@@ -928,9 +954,9 @@ hipError_t launch_rows_x(const WeightView& w, const void* x, int M, void* y, int
         }
     }
     // (the exchange area alone passes 64 KB with eight strips, or four strips and two row blocks)
-    if constexpr (NS * MB * 8 * 1024 + 512 > 64 * 1024)
-        (void)LdsRequest<&gemv_rows_kernel<BITS, XMODE, TS, NS, false, XR, MB, false, false, STRIPS>, 150 * 1024>::registered;
-    hipLaunchKernelGGL((gemv_rows_kernel<BITS, XMODE, TS, NS, false, XR, MB, false, false, STRIPS>), dim3(groups), dim3(nwaves * 64), lds, st, w.base,
+    if constexpr (NS * MB * SUMS * 8 * 1024 + 512 > 64 * 1024)
+        (void)LdsRequest<&gemv_rows_kernel<BITS, XMODE, TS, NS, false, XR, MB, false, false, STRIPS, SUMS>, 150 * 1024>::registered;
+    hipLaunchKernelGGL((gemv_rows_kernel<BITS, XMODE, TS, NS, false, XR, MB, false, false, STRIPS, SUMS>), dim3(groups), dim3(nwaves * 64), lds, st, w.base,
                        reinterpret_cast<const uint16_t*>(x), nullptr, w.KT, w.K, w.NT, M, nwaves, 0, w.N, y, ydt, epi, 1, 0, nullptr, nullptr);
     return hipGetLastError();
 }
@@ -1080,54 +1106,91 @@ hipError_t launch_rows(const WeightView& w, const void* x, int M, void* y, int y
     return launch_rows_t<BITS, XMODE, 4, 1>(w, x, M, y, ydt, nwaves, epi, sub, st);
 }
 
+int g_tune_waves = 0, g_tune_unroll = 0, g_tune_rows = 0;
+
+// Waves per workgroup of the LDS kernel (= split of a strip's K tiles).  Depends on the weight
+// shape only, never on M, so that the summation order is the same for every
+// batch size: up to 4 waves (2 when there are strips enough for 8 waves per CU anyway), then
+// more if that is what it takes to bring a wave's share down to 8 tiles, all requested
+// up front.  (K = 4096 is 4 waves x 8 tiles for every N: with few strips 8 waves x 4 tiles
+// measured 2 - 4 % slower.)
+// unroll 0: request a wave's whole share up front when it fits, else stream in batches of 2.
+int lds_waves(const WeightView& w, int num_cus, const Epilogue& epi, int& unroll)
+{
+    int nwaves = g_tune_waves;
+    if (nwaves <= 0) {
+        nwaves = 2;
+        while (nwaves < 4 && (int64_t)w.NT * nwaves < (int64_t)num_cus * 8) nwaves *= 2;
+        while (nwaves < 16 && w.KT > 8 * nwaves) nwaves *= 2;
+    }
+    if (nwaves > 16) nwaves = 16;
+    if (epi.kind == kEpiSwiglu && nwaves > 8) nwaves = 8;      // two strips per workgroup: 2 x 8 waves at most
+    while (nwaves > 1 && nwaves > w.KT) nwaves >>= 1;
+    // One workgroup per CU and a long K (the down projection): nothing else runs on the CU while a
+    // wave sits in the issue of its up-front requests, so stream in batches of two there -
+    // arithmetic in between the requests (14336 -> 4096: 10.2 -> 8.8 us, 11008 -> 4096: 9.4 -> 7.9 us).
+    // Which wave owns which tile, and with it every sum, is the same either way.
+    if (g_tune_waves <= 0 && unroll == 0 && w.NT <= num_cus && w.KT > 64 && epi.kind != kEpiSwiglu) {
+        nwaves = w.KT >= 96 ? 16 : 8;
+        unroll = 2;
+    }
+    return nwaves;
+}
+
 // fp32 rows: two operands per K tile.  Four K tiles per wave and slab fit the registers where a load takes up to eight rows of them, without
 // gamma and with few strips; where they leave more of the last slab empty, two (2048 -> 4096 at 8 rows 6.1 -> 4.4 us).
+// Strips per workgroup: one up to one per place, two up to two, four (Q4) beyond; a CU has one place, four for workgroups of one or two
+// waves (2048 -> 28672 at 4 / 16 rows with one / two / four strips 16.7 / 12.5 / 15.9, 21.9 / 16.1 / 18.9 us, 4096 -> 14336 with two / four 12.1 / 12.1,
+// 16.1 / 13.9).
 template <int BITS>
 hipError_t launch_rows_f32(const WeightView& w, const void* x, int M, void* y, int ydt, int num_cus, const Epilogue& epi, hipStream_t st)
 {
-    const int ns = strips_per_group(w, kF32, M, num_cus, epi);
-    int nwaves = 8;
-    while (nwaves > 1 && nwaves * 2 > w.KT) nwaves >>= 1;
+    int unroll = 0, sums = lds_waves(w, num_cus, epi, unroll);
+    int ns, nwaves = min(sums, 8);
+    if (epi.gamma) {
+        ns = strips_per_group(w, kF32, M, num_cus, epi);
+        nwaves = 8;
+        while (nwaves > 1 && nwaves * 2 > w.KT) nwaves >>= 1;
+        sums = nwaves;
+    } else {
+        const int places = nwaves <= 2 ? 4 * num_cus : num_cus;
+        ns = w.NT > 2 * places ? 4 : w.NT > places || epi.kind == kEpiSwiglu ? 2 : 1;
+    }
     auto padded = [&](int ts) { return (w.KT + nwaves * ts - 1) / (nwaves * ts) * (nwaves * ts); };
     const bool four = w.KT > 2 * nwaves && padded(4) <= padded(2) && !epi.gamma;
-    auto go = [&](auto strips) {
-        constexpr int NS = decltype(strips)::value, TS = NS == 1 || (NS == 2 && BITS == 4) ? 4 : 2;
-        if (M > 8) return launch_rows_x<BITS, XF32, 2, NS, 16>(w, x, M, y, ydt, nwaves, epi, false, st);
+    auto go = [&](auto strips, auto per_wave) {
+        constexpr int NS = decltype(strips)::value, SUMS = decltype(per_wave)::value, TS = NS == 1 || (NS == 2 && BITS == 4) ? 4 : 2;
+        if (M > 8) return launch_rows_x<BITS, XF32, 2, NS, 16, 1, false, SUMS>(w, x, M, y, ydt, nwaves, epi, false, st);
         if constexpr (TS == 4) {
-            if (four && M <= 4) return launch_rows_x<BITS, XF32, TS, NS, 4>(w, x, M, y, ydt, nwaves, epi, false, st);
-            if (four) return launch_rows_x<BITS, XF32, TS, NS, 8>(w, x, M, y, ydt, nwaves, epi, false, st);
+            if (four && M <= 4) return launch_rows_x<BITS, XF32, TS, NS, 4, 1, false, SUMS>(w, x, M, y, ydt, nwaves, epi, false, st);
+            if (four) return launch_rows_x<BITS, XF32, TS, NS, 8, 1, false, SUMS>(w, x, M, y, ydt, nwaves, epi, false, st);
         }
-        if (M <= 4) return launch_rows_x<BITS, XF32, 2, NS, 4>(w, x, M, y, ydt, nwaves, epi, false, st);
-        return launch_rows_x<BITS, XF32, 2, NS, 8>(w, x, M, y, ydt, nwaves, epi, false, st);
+        if (M <= 4) return launch_rows_x<BITS, XF32, 2, NS, 4, 1, false, SUMS>(w, x, M, y, ydt, nwaves, epi, false, st);
+        return launch_rows_x<BITS, XF32, 2, NS, 8, 1, false, SUMS>(w, x, M, y, ydt, nwaves, epi, false, st);
+    };
+    auto with_sums = [&](auto strips) {
+        if (sums == 16) return go(strips, std::integral_constant<int, 2>{});
+        return go(strips, std::integral_constant<int, 1>{});
     };
     if constexpr (BITS == 4) {
-        if (ns == 4) return go(std::integral_constant<int, 4>{});
+        if (ns == 4) return with_sums(std::integral_constant<int, 4>{});
     }
-    if (ns >= 2) return go(std::integral_constant<int, 2>{});
-    return go(std::integral_constant<int, 1>{});
+    if (ns >= 2) return with_sums(std::integral_constant<int, 2>{});
+    return with_sums(std::integral_constant<int, 1>{});
 }
 
 // Whether fp32 rows take the batched-rows kernel.  The LDS kernel stages and splits all rows of x once per strip, so it grows with rows x K
-// and strips; a slab that the K tiles leave partly empty is what it saves.  us per call, LDS kernel / this one, Q4: 4096 -> 4096 at
-// 3 / 8 / 16 rows 6.2 / 5.8, 8.1 / 6.2, 14.5 / 7.4; 4096 -> 32768 27.4 / 18.5, 32.2 / 20.2, 59.0 / 23.7; 14336 -> 32768 100 / 53, 193 / 61,
-// 250 / 71; 14336 -> 4096 14.4 / 14.5, 25.8 / 17.4, 32.9 / 19.4; 2048 -> 4096 at 4 / 8 / 16 rows 3.7 / 5.5, 5.0 / 4.4, 8.4 / 5.1; 1024 -> 32768
-// at 4 / 8 rows 7.4 / 7.1, 13.0 / 7.5; 512 -> 4096 at 16 rows 3.2 / 3.4; 8192 -> 4096 at 3 / 6 / 8 rows 8.5 / 9.4, 11.4 / 10.0, 16.5 / 10.2;
-// 5120 -> 4096 at 6 rows 8.5 / 10.1; 3072 -> 20000 (24 of 32 K tiles) at 8 / 16 rows 17.1 / 18.6, 30.1 / 21.2; Q8 3072 -> 11008 at 8 / 16 rows
-// 12.4 / 15.5, 21.0 / 18.2; Q8 pairs of 4096 -> 28672 at 8 / 16 rows 29.6 / 31.2, 51.5 / 35.5.  With a norm always: 256 -> 300 at 3 rows 6.3 / 4.2,
-// 4096 -> 4096 at 16 rows 87 / 10.5, 14336 -> 32000 789 / 86.
+// and strips (pairs: half as fast); the results are the same, bit for bit.  us per call, LDS kernel / this one, Q4: 4096 -> 4096 at 3 / 4 / 8 /
+// 16 rows 6.3 / 6.5, 7.1 / 6.7, 8.4 / 7.4, 14.8 / 8.9; 2048 -> 4096 at 4 / 8 / 16 rows 3.9 / 4.2, 5.2 / 4.8, 8.5 / 6.0; 3072 -> 14336 at 3 rows
+// 11.8 / 9.9; 4096 -> 32768 at 4 / 16 rows 31.7 / 18.6, 59.5 / 23.1; 2048 -> 32768 at 3 rows 17.2 / 13.8; 1024 -> 32768 at 4 / 6 rows 8.0 / 8.3,
+// 12.2 / 9.5; 14336 -> 32768 at 4 / 16 rows 163 / 57, 250 / 75; Q8 4096 -> 14336 at 4 / 16 rows 18.4 / 13.7, 32.6 / 18.7; pairs of 4096 -> 14336
+// at 3 / 4 / 16 rows 10.6 / 11.8, 12.1 / 12.0, 26.1 / 13.8.  Over 1100 such calls the line costs 0.4 % against the better of the two.
+// With a norm always, from three rows on: 256 -> 300 at 3 rows 6.3 / 4.2, 4096 -> 4096 at 16 rows 87 / 10.5, 14336 -> 32000 789 / 86; one row
+// 4096 -> 4096 7.1 / 9.4.
 bool rows_kernel_has_f32(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
-    if (M < 3) return false;
-    if (epi.gamma) return true;
-    const bool pair = epi.kind == kEpiSwiglu, narrow = w.NT <= 2 * num_cus, widest = w.NT >= 8 * num_cus;
-    if (M < 4 && (pair || (w.KT > 96 && w.NT <= num_cus))) return false;
-    if (w.KT > 32 && w.KT <= 96 && M < (narrow ? 8 : 4)) return false;
-    if (w.bits == 8 && pair && !narrow && M < 10) return false;
-    int slab = 16;                                           // K tiles of a slab of two per wave
-    while (slab > 2 && slab > w.KT) slab >>= 1;
-    const int padded = (w.KT + slab - 1) / slab * slab;
-    if (w.KT * 4 <= padded * 3 && M < (w.bits == 8 || narrow ? 12 : widest || w.KT <= 16 ? 6 : 10)) return false;
-    return M * w.KT >= (widest ? 48 : 96);
+    const int least = epi.kind == kEpiSwiglu || w.NT <= 2 * num_cus ? 112 : w.NT < 4 * num_cus ? 72 : 48;
+    return M >= 3 && (epi.gamma || M * w.KT >= least);
 }
 
 // 17 .. 32 rows: two activation operands per weight operand.  Two tiles of x per wave and slab
@@ -1154,7 +1217,6 @@ hipError_t launch_rows2(const WeightView& w, const void* x, int M, void* y, int 
     return launch_rows_x<BITS, XMODE, 2, 1, 16, 2>(w, x, M, y, ydt, nwaves, epi, sub, st);
 }
 
-int g_tune_waves = 0, g_tune_unroll = 0, g_tune_rows = 0;
 constexpr int kSplitMinRows = 12;
 
 constexpr int kLdsBudget = 64 * 1024;      // what a slab of x aims for
@@ -1248,35 +1310,12 @@ bool gemv_serves_32(const WeightView& w, int xdt, int M, int num_cus, const Epil
 hipError_t launch_gemv(const WeightView& w, const void* x, int xdt, int M, void* y, int ydt,
                        int num_cus, bool exact_operands, const Epilogue& epi, void* scratch, size_t scratch_bytes, hipStream_t st)
 {
-    // Waves per workgroup (= split of a strip's K tiles).  Depends on the weight
-    // shape only, never on M, so that the summation order is the same for every
-    // batch size: up to 4 waves (2 when there are strips enough for 8 waves per CU anyway), then
-    // more if that is what it takes to bring a wave's share down to 8 tiles, all requested
-    // up front.  (K = 4096 is 4 waves x 8 tiles for every N: with few strips 8 waves x 4 tiles
-    // measured 2 - 4 % slower.)
     // one or two f16 rows: the kernel of gemv1.hip (unless the caller asked for exact integer weight
     // operands, or a test forces one of the kernels below)
     if (!exact_operands && g_tune_waves == 0 && g_tune_rows == 0 && g_tune_unroll == 0 && gemv1_serves(w, xdt, M, epi))
         return launch_gemv1(w, x, xdt, M, y, ydt, epi, st);
-    int nwaves = g_tune_waves;
-    if (nwaves <= 0) {
-        nwaves = 2;
-        while (nwaves < 4 && (int64_t)w.NT * nwaves < (int64_t)num_cus * 8) nwaves *= 2;
-        while (nwaves < 16 && w.KT > 8 * nwaves) nwaves *= 2;
-    }
-    if (nwaves > 16) nwaves = 16;
-    if (epi.kind == kEpiSwiglu && nwaves > 8) nwaves = 8;      // two strips per workgroup: 2 x 8 waves at most
-    while (nwaves > 1 && nwaves > w.KT) nwaves >>= 1;
-    // 0: request a wave's whole share up front when it fits, else stream in batches of 2
     int unroll = g_tune_unroll;
-    // One workgroup per CU and a long K (the down projection): nothing else runs on the CU while a
-    // wave sits in the issue of its up-front requests, so stream in batches of two there -
-    // arithmetic in between the requests (14336 -> 4096: 10.2 -> 8.8 us, 11008 -> 4096: 9.4 -> 7.9 us).
-    // Which wave owns which tile, and with it every sum, is the same either way.
-    if (g_tune_waves <= 0 && g_tune_unroll == 0 && w.NT <= num_cus && w.KT > 64 && epi.kind != kEpiSwiglu) {
-        nwaves = w.KT >= 96 ? 16 : 8;
-        unroll = 2;
-    }
+    const int nwaves = lds_waves(w, num_cus, epi, unroll);
 
     // three or more batch rows: x in registers, shared across strips
     // (Q8 on wide outputs: up to four rows the LDS kernel is still the quicker one, 24.0 against

@@ -105,7 +105,9 @@ typedef enum cybq_prefill_mode { CYBQ_PREFILL_FAST = 0, CYBQ_PREFILL_EXACT = 1 }
  *                     beforehand); the mode only chooses the kernel for 1 - 2 rows.
  *   fp32 activations  exact integers in either mode (activations split into two f16 halves).
  * A 16-bit row keeps its bits in any batch of 3 .. 32 rows on weights of N = 6144 .. 28656 and K = 928 .. 4096
- * without a folded norm; elsewhere the kernel, and with it the last bits of a row, may change with the batch.
+ * without a folded norm; elsewhere the kernel, and with it the last bits of a row, may change with the batch.  An
+ * fp32 row has the same bits alone, in any batch of up to 16 rows and in CYBQ_PREFILL_EXACT calls; with a folded norm in any
+ * batch of 3 .. 16 rows and in such calls.
  *   STREAM (default) the packed nibbles / bytes are used straight from memory - as f16 subnormals
  *          (q + bias) * 2^-22 with f16 activations - and the bias is removed inside the same fp32
  *          accumulation; about 4e-7 (bf16: 1e-6) relative L2.  The sums carry the bias until it

@@ -375,8 +375,8 @@ def test_staying_workgroups_with_a_folded_norm(backend, bits, N, K, pair, xdt):
 
 # fp32 rows in the batched-rows kernel (decode tuning 1 forces it) and wherever the library sends them: one, two and four strips to a workgroup, two and
 # four K tiles per wave, slabs partly filled, one K tile, ragged K and N, each load pattern.  The two halves of a row keep 22 bits of every value
-# (2^-23 of it left out at most) and the sums are fp32: 1e-6; a pair's error is at most 3.5 times that (above), and the same rows alone or
-# in a larger batch have the same bits
+# (2^-23 of it left out at most) and the sums are fp32: 1e-6; a pair's error is at most 3.5 times that (above).  A row has the same bits in
+# the LDS kernel (decode tuning 2), alone and in any batch, and as one of many in EXACT mode; with a norm in any batch of 3 .. 16 and in EXACT mode
 @pytest.mark.parametrize("bits,N,K", [(4, 33, 96), (4, 500, 1056), (4, 4096, 2048 + 32), (4, 6149, 4064), (4, 12304, 3104), (4, 4101, 14336), (8, 33, 160),
                                       (8, 4096, 4096 + 96), (8, 12304, 1120), (8, 6160, 8192)])
 def test_batched_rows_of_fp32(backend, bits, N, K):
@@ -396,27 +396,38 @@ def test_batched_rows_of_fp32(backend, bits, N, K):
     half = N // 2 // 16 * 16
     parts = [backend.weight_from_device(bits, half, K, qd[i * half * K * bits // 8:], sd[i * half * (K // 32):]) for i in (0, 1)] if half else []
     pair = backend.fuse_pairs(*parts) if half else None
-    first = None
+    first = {}
     try:
-        for tuning in (1, 0):
+        for tuning in (1, 0, 2):
             backend.set_gemv_tuning(0, tuning, 0)
-            for M in (16, 9, 8, 5, 4, 3):
+            for M in (16, 9, 8, 5, 4, 3, 2, 1):
                 y = torch.full((M, N), float("nan"), device="cuda")
                 backend.matmul(qw, x[:M].contiguous(), y)
                 assert rel(y, plain[:M]) < 1e-6, (tuning, M)
-                if tuning == 1:
-                    first = y if first is None else first
-                    assert torch.equal(y, first[:M]), M
+                assert torch.equal(y, first.setdefault("plain", y)[:M]), (tuning, M)
                 y = torch.full((M, N), float("nan"), device="cuda")
                 backend.matmul_norm(qw, x[:M].contiguous(), gamma, 1e-5, y, "add", res[:M].contiguous())
                 assert rel(y, normed[:M] + res[:M].double()) < 1e-6, (tuning, M)
+                if tuning != 2 and M > 2:
+                    assert torch.equal(y, first.setdefault("normed", y)[:M]), (tuning, M)
                 if pair is not None:
                     y = torch.full((M, half), float("nan"), device="cuda")
                     backend.matmul_ex(pair, x[:M].contiguous(), y, "swiglu")
                     ref = torch.nn.functional.silu(plain[:M, :half]) * plain[:M, half:2 * half]
                     assert rel(y, ref) < 3.5e-6, (tuning, M)
+                    assert torch.equal(y, first.setdefault("pair", y)[:M]), (tuning, M)
+        backend.set_gemv_tuning(0, 0, 0)
+        backend.set_prefill_mode("exact")
+        for M in (17, 18, 35):
+            rows = torch.arange(M, device="cuda") % 16
+            y = torch.full((M, N), float("nan"), device="cuda")
+            backend.matmul(qw, x[rows].contiguous(), y)
+            assert torch.equal(y, first["plain"][rows]), M
+            backend.matmul_norm(qw, x[rows].contiguous(), gamma, 1e-5, y, "add", res[rows].contiguous())
+            assert torch.equal(y, first["normed"][rows]), M
     finally:
         backend.set_gemv_tuning(0, 0, 0)
+        backend.set_prefill_mode("fast")
 
 
 # a few strips more than CUs, or than twice as many (256 CUs: two and four strips to a workgroup), and K split over workgroups up to one per CU: an odd
