@@ -57,7 +57,8 @@ struct RowsPlan {
     bool two_per_cu = false; // two workgroups share a CU (nf = 4, up to 48 rows)
     bool pairs = false;      // one workgroup of eight waves does two column groups (nf = 4)
 };
-RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi);
+// (any_width: a group to a workgroup, up to 64 rows, however many rounds that makes)
+RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi, bool any_width);
 hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, void* y, int ydt, const Epilogue& epi,
                             const float* ssq_part, int ssq_blocks, const float* unscale, const RowsPlan& plan, hipStream_t st);
 // whether a scratch of this size holds enough staged rows of w's K for launch_gemm (which refuses the call otherwise)

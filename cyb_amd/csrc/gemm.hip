@@ -1151,7 +1151,7 @@ void set_gemm_tuning(int rows_kernel) { g_rows_kernel = rows_kernel >= 5 ? 0 : r
 static RowsPlan rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
     if (g_rows_kernel == 2 || g_rows_kernel == 3) return {0};
-    return gemm_rows_plan(w, M, g_rows_kernel == 1 ? 1 : num_cus, epi);
+    return gemm_rows_plan(w, M, num_cus, epi, g_rows_kernel == 1);
 }
 
 bool gemm_rows_takes(const WeightView& w, int M, int num_cus, const Epilogue& epi)

@@ -390,11 +390,12 @@ hipError_t launch_rows_t(const WeightView& w, const void* x, int M, void* y, int
 // workgroups: 11.4 against 17.4), K of at least 16 tiles.  More than 64 rows are one workgroup per 64 rows and column
 // group: narrow outputs only, where all of them fit one round.
 // (A longer K: gemm_cols.hip.)
-RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi)
+RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi, bool any_width)
 {
     if (M <= 16 || M > 512 || w.KT < 16 || w.KT > 64) return {0};
     const int64_t parts = (M + 63) / 64;
     for (int nf : {1, 2, 4}) {
+        if (any_width) break;
         if (nf == 1 && epi.kind == kEpiSwiglu) continue;        // (a gate block and its up block sit in one workgroup)
         const int64_t groups = (w.NT + nf - 1) / nf * parts;
         if (groups <= num_cus) return {groups * 4 >= num_cus ? nf : 0};
@@ -404,12 +405,16 @@ RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue&
     // K loop (4096 -> 28672 bf16 norm + SwiGLU at 45 rows 35.0 -> 30.2 us, fp32 at 24 rows 28.3 -> 25.6, 2048 -> 20000 at 40
     // rows 20.5 -> 17.6, 2048 -> 128256 at 40 rows 71.0 -> 51.1).
     // Beyond 48 rows one workgroup of eight waves does two column groups that share X (gemm_rows_pair_kernel): 4096 -> 28672 norm +
-    // SwiGLU at 64 rows 36.5 -> 34.1 us, Q8 45.0 -> 38.5, 2048 -> 20000 Q8 25.3 -> 20.6, 4096 -> 128256 122.5 -> 116.3.  Up to 48
-    // rows it pays where the groups fit one round and a step is long, Q8 or many K tiles (Q8 4096 -> 28672 at 45 rows 41.0 -> 38.0,
-    // Q8 8192 -> 16640 at 40 rows 59.7 -> 49.1, Q4 44.1 -> 40.6); not else (Q4 4096 -> 28672 at 45 rows 29.6 / 29.7, 2048 -> 128256
-    // at 40 rows 49.5 / 62.9, Q8 76.2 / 81.6).
-    const int groups4 = (w.NT + 3) / 4, rounds_of_two = ((groups4 + 1) / 2 + w.KT - 1) / w.KT * w.KT;
-    const bool pairs = parts == 1 && num_cus > 1 && (M > 48 || (rounds_of_two <= num_cus && (w.bits == 8 || w.KT > 48)));
+    // SwiGLU at 64 rows 36.5 -> 34.1 us, Q8 45.0 -> 38.5, 2048 -> 20000 Q8 25.3 -> 20.6, 4096 -> 128256 122.5 -> 116.3.  Its workgroups are
+    // a multiple of the K tiles, and a round of them takes 1.7 times as long as one of single groups: not where the multiple, or
+    // the last round, costs the rounds it saves (single groups / pairs, rounds in brackets, Q4: 5120 -> 32000 at 63 rows 41 (2) / 61 (2), 2176 ->
+    // 33882 at 54 rows 36.8 (3) / 41.5 (2), 4256 -> 40987 at 61 rows 55.1 (3) / 63.8 (2); 49 - 64 rows by rounds 2 / 1 0.92, 4 / 2 0.88, 6 / 3 0.92, 7 / 4
+    // 0.91, Q8 0.85, 0.83, 0.83, 0.91).  Up to 48 rows it pays where the groups fit one round and a step is long, Q8 or many K tiles (Q8 4096 ->
+    // 28672 at 45 rows 41.0 -> 38.0, Q8 8192 -> 16640 at 40 rows 59.7 -> 49.1, Q4 44.1 -> 40.6); not else (Q4 4096 -> 28672 at 45 rows
+    // 29.6 / 29.7, 2048 -> 128256 at 40 rows 49.5 / 62.9, Q8 76.2 / 81.6).
+    const int groups4 = (w.NT + 3) / 4, pair_groups = ((groups4 + 1) / 2 + w.KT - 1) / w.KT * w.KT;
+    const int rounds = (groups4 + num_cus - 1) / num_cus, pair_rounds = (pair_groups + num_cus - 1) / num_cus;
+    const bool pairs = parts == 1 && !any_width && (M > 48 ? pair_rounds * 17 <= rounds * 10 : pair_rounds == 1 && (w.bits == 8 || w.KT > 48));
     return {parts == 1 ? 4 : 0, parts == 1 && M <= 48 && !pairs, pairs};
 }
 

@@ -1260,7 +1260,7 @@ def test_prefill_few_rows_long_k_shares(backend, oracle, bits, shape):
 
 
 @pytest.mark.parametrize("bits,N,K,M", [(4, 16400, 17 * 128, 49), (4, 16384 + 64, 18 * 128 - 32, 64), (4, 33000, 19 * 128 - 96, 63),
-                                        (8, 16400, 20 * 128, 17), (8, 24002, 21 * 128 + 64, 48), (8, 16448, 62 * 128, 64), (4, 17000, 63 * 128 + 32, 33)])
+                                        (4, 49172, 16 * 128, 50), (8, 16400, 20 * 128, 17), (8, 24002, 21 * 128 + 64, 48), (8, 16448, 62 * 128, 64), (4, 17000, 63 * 128 + 32, 33)])
 def test_prefill_few_rows_two_column_groups_per_workgroup(backend, oracle, bits, N, K, M):
     """More than a round of workgroups: two column groups to a workgroup that walk the K tiles together.  A last group that is not full or
     has no partner, K tiles that leave waves without one in the last step, N that is no multiple of 16 or 4: bit for bit the kernel with a
