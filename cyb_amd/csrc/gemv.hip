@@ -1036,14 +1036,15 @@ hipError_t launch_rows_t(const WeightView& w, const void* x, int M, void* y, int
 // waves have a CU to themselves, so a few more of them than CUs take two rounds.  us per call, one strip / two: Q4 f16 4096 -> 4224 at
 // 8 / 16 / 32 rows 7.0 / 5.8, 8.0 / 6.3, 11.7 / 9.7, 11008 -> 6000 15.8 / 13.6, 19.8 / 15.0, 30.7 / 22.2, fp32 4096 -> 5120 at 16 rows with a
 // norm 18.0 / 10.9, Q8 f16 14336 -> 4224 at 8 / 32 rows 23.6 / 18.7, 39.5 / 28.6.  Not with four waves, two of whose workgroups share a CU (1024 ->
-// 5120 at 8 rows 4.1 / 4.3, Q8 4.3 / 4.8; 17 .. 32 rows of Q4 6.6 / 5.2), nor for nine or more f16 rows of Q8 with a norm (14336 -> 4224 31.1 / 33.4).
+// 5120 at 8 rows 4.1 / 4.3, Q8 4.3 / 4.8; 17 .. 32 rows of Q4 6.6 / 5.5, but with one or two waves, K under 1024, 320 -> 4819 at 31 rows 7.2 / 11.5,
+// 800 -> 4862 at 18 rows 6.5 / 8.1), nor for nine or more f16 rows of Q8 with a norm (14336 -> 4224 31.1 / 33.4).
 // Likewise four of Q4 from two per CU on, two / four, f16: 8192 -> 9216 at 8 / 16 / 32 rows 16.9 / 13.4, 19.7 / 15.1, 28.1 / 21.2, 14336 -> 9216 with a
 // norm at 16 rows 37.7 / 29.4, bf16 46.1 / 31.8 (16-bit rows of K up to 4096 run the kernel of gemv_stream.hip there).
 int strips_per_group(const WeightView& w, int xdt, int M, int num_cus, const Epilogue& epi)
 {
     int ns = (w.NT + num_cus / 2) / num_cus;
     ns = ns >= 3 ? 4 : (ns >= 2 ? 2 : 1);
-    const bool two = w.KT >= 16 ? !(w.bits == 8 && xdt == kF16 && epi.gamma && M > 8) : w.bits == 4 && M > 16;
+    const bool two = w.KT >= 16 ? !(w.bits == 8 && xdt == kF16 && epi.gamma && M > 8) : w.KT >= 8 && w.bits == 4 && M > 16;
     if (w.NT > num_cus && two && ns < 2) ns = 2;
     if (w.NT > 2 * num_cus && ns < 4 && w.bits == 4 && (w.KT > 32 || (xdt == kF32 && w.KT >= 16))) ns = 4;
     if (epi.kind == kEpiSwiglu && ns < 2) ns = 2;          // a gate strip and its up strip share a workgroup
