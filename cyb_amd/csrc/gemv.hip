@@ -1182,7 +1182,7 @@ hipError_t launch_rows_f32(const WeightView& w, const void* x, int M, void* y, i
 
 // Whether fp32 rows take the batched-rows kernel.  The LDS kernel stages and splits all rows of x once per strip, so it grows with rows x K
 // and strips (pairs: half as fast); the results are the same, bit for bit.  us per call, LDS kernel / this one, Q4: 4096 -> 4096 at 3 / 4 / 8 /
-// 16 rows 6.3 / 6.5, 7.1 / 6.7, 8.4 / 7.4, 14.8 / 8.9; 2048 -> 4096 at 4 / 8 / 16 rows 3.9 / 4.2, 5.2 / 4.8, 8.5 / 6.0; 3072 -> 14336 at 3 rows
+// 16 rows 6.3 / 6.5, 7.1 / 6.7, 8.4 / 7.4, 14.8 / 8.9; 9888 -> 799 at 3 rows 9.0 / 10.7, 14176 -> 694 12.6 / 14.0, 3200 -> 3770 at 5 rows 6.8 / 7.8; 2048 -> 4096 at 4 / 8 / 16 rows 3.9 / 4.2, 5.2 / 4.8, 8.5 / 6.0; 3072 -> 14336 at 3 rows
 // 11.8 / 9.9; 4096 -> 32768 at 4 / 16 rows 31.7 / 18.6, 59.5 / 23.1; 2048 -> 32768 at 3 rows 17.2 / 13.8; 1024 -> 32768 at 4 / 6 rows 8.0 / 8.3,
 // 12.2 / 9.5; 14336 -> 32768 at 4 / 16 rows 163 / 57, 250 / 75; Q8 4096 -> 14336 at 4 / 16 rows 18.4 / 13.7, 32.6 / 18.7; pairs of 4096 -> 14336
 // at 3 / 4 / 16 rows 10.6 / 11.8, 12.1 / 12.0, 26.1 / 13.8.  Over 1100 such calls the line costs 0.4 % against the better of the two.
@@ -1190,6 +1190,8 @@ hipError_t launch_rows_f32(const WeightView& w, const void* x, int M, void* y, i
 // 4096 -> 4096 7.1 / 9.4.
 bool rows_kernel_has_f32(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
+    // (the load patterns hold 4, 8 and 16 rows: where a workgroup has one strip to load them for, 3 and 5 rows are the LDS kernel's)
+    if (!epi.gamma && epi.kind != kEpiSwiglu && w.NT <= num_cus && (M == 3 || M == 5)) return false;
     const int least = epi.kind == kEpiSwiglu || w.NT <= 2 * num_cus ? 112 : w.NT < 4 * num_cus ? 72 : 48;
     return M >= 3 && (epi.gamma || M * w.KT >= least);
 }
