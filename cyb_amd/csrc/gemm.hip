@@ -1159,13 +1159,6 @@ bool gemm_rows_takes(const WeightView& w, int M, int num_cus, const Epilogue& ep
     return rows_plan(w, M, num_cus, epi).nf != 0;
 }
 
-// the extra workgroups of a staging launch (grid_x grows by them) for a call of 33 rows or more that goes through the
-// row-scaling pass (bf16 / fp32 rows) and on to the few-row kernel or to the tiled kernels' 64-column tiles: up to
-// 16 MB of the tensor, from the K tile every column group starts at.  Per call: 4096 -> 14336 at 64 rows 19.6 -> 18.7
-// us with 16 of the 32 K tiles (no gain with all of them: the launch then takes as long as the reads), 4096 -> 4096
-// at 64 / 128 rows 13.6 / 14.6 -> 12.4 / 13.4, 4096 -> 1024 13.1 -> 11.7, 8192 -> 4096 at 128 rows 25.1 -> 22.9.  Not
-// for f16 rows (their pass only reorders and is over before the reads are: 4096 -> 14336 at 64 rows 18.6 -> 19.1),
-// for 17 .. 32 fp32 rows (12.5 -> 13.4 on 4096 -> 8192) or for K up to 2048.
 // whether tiled_plan gives a FAST-mode call of M rows the 64-column tiles
 static bool few_rows_tiles64(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
@@ -1174,6 +1167,13 @@ static bool few_rows_tiles64(const WeightView& w, int M, int num_cus, const Epil
     return tiled_plan(w, M, false, num_cus, 0, epi, plan) < 0.f && plan.kind == TilePlan::kRoles && plan.nf == 4;
 }
 
+// the extra workgroups of a staging launch (grid_x grows by them) for a call of 33 rows or more that goes through the
+// row-scaling pass (bf16 / fp32 rows) and on to the few-row kernel or to the tiled kernels' 64-column tiles: up to
+// 16 MB of the tensor, from the K tile every column group starts at.  Per call: 4096 -> 14336 at 64 rows 19.6 -> 18.7
+// us with 16 of the 32 K tiles (no gain with all of them: the launch then takes as long as the reads), 4096 -> 4096
+// at 64 / 128 rows 13.6 / 14.6 -> 12.4 / 13.4, 4096 -> 1024 13.1 -> 11.7, 8192 -> 4096 at 128 rows 25.1 -> 22.9.  Not
+// for f16 rows (their pass only reorders and is over before the reads are: 4096 -> 14336 at 64 rows 18.6 -> 19.1),
+// for 17 .. 32 fp32 rows (12.5 -> 13.4 on 4096 -> 8192) or for K up to 2048.
 static Touch plan_touch(const WeightView& w, int mc, int num_cus, const Epilogue& ec, bool exact, unsigned& grid_x)
 {
     Touch tc = {nullptr, 0x7fffffff, w.NT, w.KT, 1, tile_bytes(w.bits), 0, 0, 0};

@@ -32,25 +32,10 @@
 //   4096 ->  6144 at 64 / 128 rows       14.3 / 17.6 against 19.3 / 26.8     8192 -> 14336 at 33 .. 64 rows 30 - 32 against 36.5 - 38
 //   4096 ->  1024 at 128 / 256 / 512 rows 12.9 / 14.2 / 20.7 against 18.7 / 21.6 / 27.6
 //   fp32 rows, 17 .. 32: 4096 -> 14336 15.9 against 21, 4096 -> 4096 10.7 against 18
-// The same kernel on v_mfma_f32_32x32x16_f16 (one wave per SIMD issues a 16x16x32 MFMA only every ~27 cycles, a
-// 32x32x16 one back to back; both operands load in that shape from the same layouts as four 256-byte runs) measured
-// the same to 0.3 us on every shape: the MFMAs are a quarter of a wave's cycles.  Two workgroups of two column
-// blocks per CU (two waves per SIMD, twice the rows of X into every CU): 23.9 against 19.6 us.
-// Two waves per SIMD (eight waves; wave (k share, half) takes two of the four scale groups of each of its K tiles:
-// half the X registers, half of every tile record, nothing loaded or dequantised twice, eight partial sums at the
-// end) is slower on every shape: 4096 -> 4096 at 64 rows 14.2 against 13.1 us, 4096 -> 8192 16.9 against 14.9,
-// 4096 -> 1024 at 128 rows 13.9 against 12.8 (and it spills with four column blocks).
-// Eight column blocks per workgroup on 32x32x16 (64 rows x 128 columns: 65 .. 128 rows on 4096 -> 14336 in one round,
-// 0.8 MB into a CU instead of the tiled kernel's 1.15): 31.4 against 27.6 us at 128 rows, 30.3 against 24.5 at 65 -
-// one wave's MFMAs, dequantisation and loads then add up instead of overlapping.
-// With eight row blocks per wave (65 .. 128 rows in one workgroup, for wide outputs whose 64-row pieces would
-// need two rounds) a wave has twice the MFMAs to issue per K tile next to the same dequantisation and the
-// kernel is no quicker than the tiled one (X a whole K tile ahead: the operands no longer fit the register
-// file next to 128 accumulator registers, 31 against 27 us; X half a K tile ahead: 27.5 against 27.4 at 128
-// rows, 25.3 against 24.2 at 65): those calls stay there.
-// Reading f16 rows where the caller has them (row-major: sixteen 64-byte runs per operand load instead of one
-// KB) to save the restaging launch is slower, not quicker: 4096 -> 14336 at 64 rows 23.7 against 18.3 us with
-// the pass, 4096 -> 4096 at 128 rows 21.9 against 15.9.
+// Not kept, us per call there / here: 32x32x16 MFMAs (the same to 0.3 on every shape: the MFMAs are a quarter of a wave's cycles); two waves
+// per SIMD by scale groups of a K tile 14.2 / 13.1 (4096 -> 4096 at 64 rows); eight column blocks for 65 .. 128 rows 31.4 / the tiled
+// kernel's 27.6, eight row blocks 27.5 / 27.4; rows read where the caller has them, without the staging launch, 23.7 / 18.3 (sixteen
+// 64-byte runs per operand load instead of one KB).
 #include <algorithm>
 #include <type_traits>
 
