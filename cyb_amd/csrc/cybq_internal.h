@@ -56,11 +56,14 @@ struct RowsPlan {
     int nf;                  // column blocks of 16 per workgroup (1, 2 or 4); 0: the kernel does not take the call
     bool two_per_cu = false; // two workgroups share a CU (nf = 4, up to 48 rows)
     bool pairs = false;      // one workgroup of eight waves does two column groups (nf = 4)
+    int shares = 0;          // > 0: K is cut into that many shares, one per wave; more than four go to shares - 3 slabs, fp32 [M][N]
 };
 // (any_width: a group to a workgroup, up to 64 rows, however many rounds that makes)
 RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi, bool any_width);
 hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, void* y, int ydt, const Epilogue& epi,
-                            const float* ssq_part, int ssq_blocks, const float* unscale, const RowsPlan& plan, hipStream_t st);
+                            const float* ssq_part, int ssq_blocks, const float* unscale, const RowsPlan& plan, float* slabs, hipStream_t st);
+// the calls of plan_gemm_cols_long_k (below) that are this kernel's, a share of K per wave
+RowsPlan gemm_rows_plan_long_k(const WeightView& w, int M, int num_cus, const Epilogue& epi);
 // whether a scratch of this size holds enough staged rows of w's K for launch_gemm (which refuses the call otherwise)
 bool gemm_stages(const WeightView& w, size_t workspace_bytes);
 // the prefill kernel whose waves stand side by side along the columns (gemm_cols.hip).  mode: 0 FAST, 1 / 2 EXACT with f16 / bf16

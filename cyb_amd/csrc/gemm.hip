@@ -1299,9 +1299,11 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         // few rows on a wide output, FAST mode: the kernel of gemm_rows.hip (waves split K, no LDS on the way)
-        const RowsPlan plan = !exact && kdt == kF16 ? rows_plan(w, mc, num_cus, ec) : RowsPlan{0};
+        RowsPlan plan = !exact && kdt == kF16 ? rows_plan(w, mc, num_cus, ec) : RowsPlan{0};
+        if (!plan.nf && !exact && kdt == kF16 && g_rows_kernel < 2) plan = gemm_rows_plan_long_k(w, mc, num_cus, ec);
         if (plan.nf) {
-            e = launch_gemm_rows(w, workspace, mc, yc, ydt, ec, ns.part, ns.nblk, ns.unscale, plan, st);
+            e = launch_gemm_rows(w, workspace, mc, yc, ydt, ec, ns.part, ns.nblk, ns.unscale, plan, part, st);
+            if (e == hipSuccess && plan.shares > 4) e = launch_reduce(part, plan.shares - 3, mc, w.N, yc, ydt, out_scale, ec, ns, w.K, st);
             if (e != hipSuccess) return e;
             continue;
         }

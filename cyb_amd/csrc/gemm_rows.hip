@@ -102,10 +102,14 @@ __device__ __forceinline__ void finish_row_block(float4_t (&tot)[1][NF], float* 
 // MF row blocks of 16 per workgroup (blockIdx.y-th MF * 16 rows of the call), NF column blocks per workgroup, WAVES
 // waves that split K, DEPTH K tiles of packed weights and XD K tiles of X in flight per wave.
 // OCC: workgroups per CU.
-template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD, int OCC = 1>
+// SHARES: the K tiles are cut into `shares` runs of kt_per_share, and a wave walks one run (number blockIdx.z * WAVES + wave)
+// from the tile and in the order in which the tiled kernels' K split walks it; the runs' sums are added in their order, the
+// first four here, the others (blockIdx.z = 1: a slab each) with the first four's slab by the slab-adding pass.
+// The result is that of the tiled kernels bit for bit.
+template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD, int OCC = 1, bool SHARES = false>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC * WAVES / 4, OCC * WAVES / 4))) void gemm_rows_kernel(
     const uint8_t* __restrict__ wbase, const u32x4_t* __restrict__ x, int KT_, int NT_, int x_row_blocks, int M, int N_,
-    void* __restrict__ y, int ydt, int K_, Epilogue epi, NormStats ns)
+    void* __restrict__ y, int ydt, int K_, Epilogue epi, NormStats ns, int shares, int kt_per_share, float* __restrict__ slabs)
 {
     const WeightView w = {wbase, N_, K_, NT_, KT_, BITS};
     constexpr int FR = MF * NF;                        // accumulator blocks per wave
@@ -118,18 +122,20 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC 
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nt0 = (int)blockIdx.x * NF;
     const int K = w.K, G = K / kGroup;
-    const int KT = w.KT;
+    const int share = (int)blockIdx.z * WAVES + wv;
+    const int kt_lo = SHARES ? min(share * kt_per_share, w.KT - 1) : 0;
+    const int KT = SHARES ? min(kt_per_share, w.KT - kt_lo) : w.KT;      // my K tiles (SHARES: mine alone): kt_lo ..
     const uint32_t magic = q4_magic_vgpr();
     // my K tiles: number t is tile wv + WAVES * t
-    const int T = KT > wv ? (KT - wv + WAVES - 1) / WAVES : 0;
+    const int T = SHARES ? (share < shares ? KT : 0) : KT > wv ? (KT - wv + WAVES - 1) / WAVES : 0;
     // Workgroups that run side by side read the same rows of X: walking K in the same order they would all
     // ask the same L2 channels for the same lines at the same moment, so every column tile starts its walk
     // at another K tile and wraps around (the order depends on the column tile only, not on M).
-    const int kt0 = (int)blockIdx.x % KT;
+    const int kt0 = SHARES ? (nt0 >> 3) % KT : (int)blockIdx.x % KT;      // (the tiled kernels' column tiles: eight blocks)
     // (a tile number past my last one is clamped to the last K tile: loaded again, never used)
     auto tile_of = [&](int t) __attribute__((always_inline)) {
-        const int kt = min(wv + WAVES * t, KT - 1) + kt0;
-        return kt >= KT ? kt - KT : kt;
+        const int kt = min(SHARES ? t : wv + WAVES * t, KT - 1) + kt0;
+        return kt_lo + (kt >= KT ? kt - KT : kt);
     };
     // (row blocks and column blocks past the end are clamped to the last real one: computed again, never
     // stored; the offsets are wave-uniform, the lane's part of an address is one register)
@@ -191,6 +197,15 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC 
         if (t + decltype(i)::value < T) k_tile(t + decltype(i)::value, i);
     });
 
+    const Epilogue plain = {kEpiNone, nullptr, nullptr, 0, 0.f};
+    if constexpr (SHARES) {
+        if (blockIdx.z > 0) {
+            if (share < shares)
+                write_rows<MF, NF>(acc, reinterpret_cast<float*>(smem) + wv * (16 * NF * 16), rb0 * 16, nt0, M, w.N,
+                                   slabs + (int64_t)(share - WAVES + 1) * M * w.N, kF32, 1.0f, plain, lane);
+            return;
+        }
+    }
     // ---- the partial sums meet: every wave leaves all of its blocks, waves 0 .. MF-1 finish a row block each
 #pragma unroll
     for (int i = 0; i < MF; i++)
@@ -206,6 +221,12 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC 
 #pragma unroll
         for (int p = 1; p < WAVES; p++) s += part[(p * FR + blk) * 64 + lane];
         tot[0][f] = s;
+    }
+    if constexpr (SHARES) {
+        if (shares > WAVES) {
+            write_rows<1, NF>(tot, stg + wv * (16 * NF * 16), (rb0 + wv) * 16, nt0, M, w.N, slabs, kF32, 1.0f, plain, lane);
+            return;
+        }
     }
     finish_row_block<NF>(tot, stg + wv * (16 * NF * 16), (rb0 + wv) * 16, nt0, M, w, y, ydt, K, epi, ns, lane);
 }
@@ -354,14 +375,17 @@ hipError_t launch_pair_t(const WeightView& w, const void* x, int M, void* y, int
     return hipGetLastError();
 }
 
-template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD, int OCC = 1>
-hipError_t launch_rows_t(const WeightView& w, const void* x, int M, void* y, int ydt, const Epilogue& epi, const NormStats& ns, hipStream_t st)
+template <int BITS, int MF, int NF, int WAVES, int DEPTH, int XD, int OCC = 1, bool SHARES = false>
+hipError_t launch_rows_t(const WeightView& w, const void* x, int M, void* y, int ydt, const Epilogue& epi, const NormStats& ns, hipStream_t st,
+                         int shares = 0, float* slabs = nullptr)
 {
     constexpr int lds = WAVES * MF * NF * 1024 + MF * 16 * NF * 16 * 4;
-    (void)LdsRequest<&gemm_rows_kernel<BITS, MF, NF, WAVES, DEPTH, XD, OCC>, lds>::registered;
+    (void)LdsRequest<&gemm_rows_kernel<BITS, MF, NF, WAVES, DEPTH, XD, OCC, SHARES>, lds>::registered;
     const unsigned groups = (unsigned)((w.NT + NF - 1) / NF), row_parts = (unsigned)((M + 16 * MF - 1) / (16 * MF));
-    hipLaunchKernelGGL((gemm_rows_kernel<BITS, MF, NF, WAVES, DEPTH, XD, OCC>), dim3(groups, row_parts), dim3(WAVES * 64), lds, st,
-                       w.base, reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT, (M + 15) / 16, M, w.N, y, ydt, w.K, epi, ns);
+    hipLaunchKernelGGL((gemm_rows_kernel<BITS, MF, NF, WAVES, DEPTH, XD, OCC, SHARES>),
+                       dim3(groups, row_parts, SHARES ? (unsigned)((shares + WAVES - 1) / WAVES) : 1u), dim3(WAVES * 64), lds, st,
+                       w.base, reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT, (M + 15) / 16, M, w.N, y, ydt, w.K, epi, ns,
+                       shares, SHARES ? (w.KT + shares - 1) / shares : 0, slabs);
     return hipGetLastError();
 }
 
@@ -374,7 +398,7 @@ hipError_t launch_rows_t(const WeightView& w, const void* x, int M, void* y, int
 // rows: 128 of one 11.6, the tiled kernels 17.5), at least a quarter of a round (4096 -> 1024 at 24 rows, 64
 // workgroups: 11.4 against 17.4), K of at least 16 tiles.  More than 64 rows are one workgroup per 64 rows and column
 // group: narrow outputs only, where all of them fit one round.
-// (A longer K: gemm_cols.hip.)
+// (A longer K: gemm_rows_plan_long_k and gemm_cols.hip.)
 RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi, bool any_width)
 {
     if (M <= 16 || M > 512 || w.KT < 16 || w.KT > 64) return {0};
@@ -403,8 +427,25 @@ RowsPlan gemm_rows_plan(const WeightView& w, int M, int num_cus, const Epilogue&
     return {parts == 1 ? 4 : 0, parts == 1 && M <= 48 && !pairs, pairs};
 }
 
+// K of more than 64 tiles (plan_gemm_cols_long_k says which calls): a share of K per wave where a round of workgroups has one column
+// block each, or two of Q4, and the rows are few: nothing to share X with then, and five slabs instead of eight.  The same bits.  us per
+// call, weights in the L2s (from HBM), eight strips side by side / here, Q4 fp32 rows: 11136 -> 192 at 19 rows 14.9 / 13.2 (0.95 of the
+// time), 10592 -> 496 at 28 15.3 / 13.3 (0.90), 13216 -> 368 at 21 16.2 / 14.8 (0.97), Q8 10400 -> 656 at 31 15.6 / 13.5 (0.93), 10208 -> 400 at 43
+// 16.5 / 14.7 (0.93), two blocks: 10944 -> 3856 at 32 17.9 / 16.3 (0.96).  Not there: pairs 13664 -> 320 at 31 rows 16.6 / 16.1 (1.03), Q8 11808 ->
+// 1344 at 34 17.3 / 17.8 (1.14); a longer K with more to take in, Q8 12544 -> 160 at 33 17.0 / 16.9 (1.08), 14144 -> 2272 at 28 18.0 / 17.3 (1.05);
+// 49 rows and more, 13440 -> 256 at 49 19.8 / 19.9 (1.06); four blocks 11072 -> 4896 at 18 19.0 / 21.6 (1.13).
+RowsPlan gemm_rows_plan_long_k(const WeightView& w, int M, int num_cus, const Epilogue& epi)
+{
+    const ColsPlan cols = plan_gemm_cols_long_k(w, M, num_cus, epi);
+    if (!cols.rb || M > 48 || epi.kind == kEpiSwiglu) return {0};
+    const int parts = (cols.splits + 3) / 4;               // workgroups per column group, four shares each
+    if (w.NT * parts <= num_cus && (M <= 32 || w.KT <= 96)) return {1, false, false, cols.splits};
+    if ((w.NT + 1) / 2 * parts <= num_cus && w.bits == 4 && M <= 32 && w.KT <= 96) return {2, false, false, cols.splits};
+    return {0};
+}
+
 hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, void* y, int ydt, const Epilogue& epi,
-                            const float* ssq_part, int ssq_blocks, const float* unscale, const RowsPlan& plan, hipStream_t st)
+                            const float* ssq_part, int ssq_blocks, const float* unscale, const RowsPlan& plan, float* slabs, hipStream_t st)
 {
     const NormStats ns = {ssq_part, ssq_blocks, unscale};
     // four waves, one per SIMD with the whole register file: four K tiles of packed weights and one K tile of
@@ -426,6 +467,15 @@ hipError_t launch_gemm_rows(const WeightView& w, const void* x_staged, int M, vo
         if (w.bits == 8) return go(std::integral_constant<int, 8>{}, nfc);
         return go(std::integral_constant<int, 4>{}, nfc);
     };
+    if (plan.shares) {
+        if (plan.nf == 2) return launch_rows_t<4, 2, 2, 4, 4, 1, 1, true>(w, x_staged, M, y, ydt, epi, ns, st, plan.shares, slabs);
+        if (w.bits == 8) {
+            if (mf == 2) return launch_rows_t<8, 2, 1, 4, 4, 1, 1, true>(w, x_staged, M, y, ydt, epi, ns, st, plan.shares, slabs);
+            return launch_rows_t<8, 3, 1, 4, 4, 1, 1, true>(w, x_staged, M, y, ydt, epi, ns, st, plan.shares, slabs);
+        }
+        if (mf == 2) return launch_rows_t<4, 2, 1, 4, 4, 1, 1, true>(w, x_staged, M, y, ydt, epi, ns, st, plan.shares, slabs);
+        return launch_rows_t<4, 3, 1, 4, 4, 1, 1, true>(w, x_staged, M, y, ydt, epi, ns, st, plan.shares, slabs);
+    }
     if (plan.pairs) {
         if (w.bits == 4) {
             if (mf == 2) return launch_pair_t<4, 2, 4, 3>(w, x_staged, M, y, ydt, epi, ns, st);

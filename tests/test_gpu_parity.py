@@ -1206,11 +1206,12 @@ def test_prefill_few_rows_waves_split_k(backend, oracle, bits, shape):
 
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("shape", [(4096, 14336, 45), (992, 65 * 128, 64), (16, 16384 + 32, 128), (1030, 9216 + 64, 100),
-                                   (2048, 8192 + 32, 33), (4096, 65 * 128 - 32, 17), (8224, 65 * 128, 40), (10000, 8192 + 128, 60)])
+                                   (2048, 8192 + 32, 33), (4096, 65 * 128 - 32, 17), (8224, 65 * 128, 40), (10000, 8192 + 128, 60),
+                                   (500, 96 * 128, 48), (500, 96 * 128 + 32, 33), (2050, 112 * 128, 32), (3850, 65 * 128, 31), (3850, 96 * 128, 19)])
 def test_prefill_few_rows_long_k_shares(backend, oracle, bits, shape):
-    """FAST mode, up to 128 rows, K of more than 64 tiles: each wave of the few-row kernel walks one share of K as the tiled
-    kernels' K split does, so the results are the tiled kernels' bit for bit.  Eight, seven, four, three shares, the fewest K
-    tiles, a last share shorter than the others, one strip, N that ends inside a column block and is no multiple of four,
+    """FAST mode, up to 128 rows, K of more than 64 tiles: each wave of the few-row kernel, or each workgroup of eight
+    strips, walks one share of K as the tiled kernels' K split does, so the results are the tiled kernels' bit for bit.  Eight,
+    seven, four, three shares, both sides of 96 tiles, of 32 and 48 rows and of one column block per workgroup, the fewest K tiles, a last share shorter than the others, one strip, N that ends inside a column block and is no multiple of four,
     y off its vector alignment, every epilogue; 17 rows are fp32 (16-bit rows that few keep the decode kernels)."""
     N, K, M = shape
     q, s = _quant(oracle, bits, N, K, cfg=65)
