@@ -1190,8 +1190,9 @@ hipError_t launch_rows_f32(const WeightView& w, const void* x, int M, void* y, i
 // 4096 -> 4096 7.1 / 9.4.
 bool rows_kernel_has_f32(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
-    // (the load patterns hold 4, 8 and 16 rows: where a workgroup has one strip to load them for, 3 and 5 rows are the LDS kernel's)
-    if (!epi.gamma && epi.kind != kEpiSwiglu && w.NT <= num_cus && (M == 3 || M == 5)) return false;
+    // (the load patterns hold 4, 8 and 16 rows: where a workgroup has one strip to load them for, 3 and 5 rows are the LDS kernel's; but from 96 K
+    // tiles on that has sixteen waves and a slab of one tile each: 12800 -> 300 at 5 rows 19.4 / 14.0, 12160 -> 480 12.2 / 12.5)
+    if (!epi.gamma && epi.kind != kEpiSwiglu && w.NT <= num_cus && (M == 3 || (M == 5 && w.KT < 96))) return false;
     const int least = epi.kind == kEpiSwiglu || w.NT <= 2 * num_cus ? 112 : w.NT < 4 * num_cus ? 72 : 48;
     return M >= 3 && (epi.gamma || M * w.KT >= least);
 }

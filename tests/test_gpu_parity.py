@@ -377,7 +377,7 @@ def test_staying_workgroups_with_a_folded_norm(backend, bits, N, K, pair, xdt):
 # four K tiles per wave, slabs partly filled, one K tile, ragged K and N, each load pattern.  The two halves of a row keep 22 bits of every value
 # (2^-23 of it left out at most) and the sums are fp32: 1e-6; a pair's error is at most 3.5 times that (above).  A row has the same bits in
 # the LDS kernel (decode tuning 2), alone and in any batch, and as one of many in EXACT mode; with a norm in any batch of 3 .. 16 and in EXACT mode
-@pytest.mark.parametrize("bits,N,K", [(4, 33, 96), (4, 500, 1056), (4, 4096, 2048 + 32), (4, 6149, 4064), (4, 12304, 3104), (4, 4101, 14336), (8, 33, 160),
+@pytest.mark.parametrize("bits,N,K", [(4, 33, 96), (4, 500, 1056), (4, 4096, 2048 + 32), (4, 6149, 4064), (4, 12304, 3104), (4, 4101, 14336), (4, 300, 12384), (8, 33, 160),
                                       (8, 4096, 4096 + 96), (8, 12304, 1120), (8, 6160, 8192)])
 def test_batched_rows_of_fp32(backend, bits, N, K):
     g = torch.Generator(device="cuda").manual_seed(N + K)
