@@ -524,7 +524,7 @@ class Backend:
 
     def set_gemm_tuning(self, rows_kernel: int = 0) -> None:
         """Experiments only: 2 leaves FAST-mode prefill calls to the tiled kernels, 3 those of both modes, 1 sends calls of
-        up to 64 rows to the K-splitting kernel whatever the output width, 0 restores the automatic choice."""
+        up to 64 rows to the K-splitting kernel whatever the output width, 4 has all rows staged before the multiply, 0 restores the automatic choice."""
         self._lib.cybq_debug_set_gemm_tuning(rows_kernel)
 
     def set_gemv_tuning(self, waves: int = 0, rows_kernel: int = 0, unroll: int = 0) -> None:

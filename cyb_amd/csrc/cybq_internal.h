@@ -76,7 +76,8 @@ struct ColsPlan {
 // FAST, a long K and few rows on an output that the tiled kernels split K for three ways or more (rb = 0: another call)
 ColsPlan plan_gemm_cols_long_k(const WeightView& w, int M, int num_cus, const Epilogue& epi);
 ColsPlan plan_gemm_cols(const WeightView& w, int mode, int M, int num_cus, size_t part_bytes);
-hipError_t launch_gemm_cols(const WeightView& w, const void* x_staged, int mode, int M, void* y, int ydt, const ColsPlan& plan, const Epilogue& epi,
+// raw: x is the caller's, row major in the operands' type (no norm), instead of staged operands
+hipError_t launch_gemm_cols(const WeightView& w, const void* x, bool raw, int mode, int M, void* y, int ydt, const ColsPlan& plan, const Epilogue& epi,
                             const float* ssq_part, int ssq_blocks, const float* unscale, float* part, hipStream_t st);
 // test/bench hook: 2 = in FAST mode the tiled kernels alone (neither the few-rows kernel nor gemm_cols.hip), 3 = in both modes,
 // 1 = the few-rows kernel whatever the width, 0 = automatic

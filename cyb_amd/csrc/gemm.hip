@@ -841,11 +841,11 @@ static TilePlan plan_tiles(const WeightView& w, int M, bool exact, bool bf16, in
 }
 
 template <int BITS, int XBF>
-hipError_t launch_tiles(const TilePlan& p, const WeightView& w, const void* x, int M, void* y, int ydt, bool exact, float out_scale, float* part,
+hipError_t launch_tiles(const TilePlan& p, const WeightView& w, const void* x, bool raw, int M, void* y, int ydt, bool exact, float out_scale, float* part,
                         const Epilogue& epi, const NormStats& ns, hipStream_t st)
 {
     if (p.kind == TilePlan::kCols) {
-        const hipError_t e = launch_gemm_cols(w, x, !exact ? 0 : XBF ? 2 : 1, M, y, ydt, p.cols, epi, ns.part, ns.nblk, ns.unscale, part, st);
+        const hipError_t e = launch_gemm_cols(w, x, raw, !exact ? 0 : XBF ? 2 : 1, M, y, ydt, p.cols, epi, ns.part, ns.nblk, ns.unscale, part, st);
         if (e != hipSuccess || p.splits == 1) return e;
         return launch_reduce(part, p.splits, M, w.N, y, ydt, out_scale, epi, ns, w.K, st);
     }
@@ -1145,8 +1145,14 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
 
 }  // namespace
 
+bool g_raw = true;            // (4 = gemm_cols.hip reads staged rows only)
 int g_touch = 2;              // (5 = the staging launch asks for no weights ahead of the multiply, 6 = only ahead of the few-rows kernel)
-void set_gemm_tuning(int rows_kernel) { g_rows_kernel = rows_kernel >= 5 ? 0 : rows_kernel; g_touch = rows_kernel == 5 ? 0 : rows_kernel == 6 ? 1 : 2; }
+void set_gemm_tuning(int rows_kernel)
+{
+    g_rows_kernel = rows_kernel >= 4 ? 0 : rows_kernel;
+    g_raw = rows_kernel != 4;
+    g_touch = rows_kernel == 5 ? 0 : rows_kernel == 6 ? 1 : 2;
+}
 
 static RowsPlan rows_plan(const WeightView& w, int M, int num_cus, const Epilogue& epi)
 {
@@ -1246,11 +1252,24 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
         void* yc = static_cast<char*>(y) + (size_t)m_lo * n_out * ysize;
         Epilogue ec = epi;                 // this row chunk's slice of the residual
         if (epi.kind == kEpiAdd) ec.residual = static_cast<const char*>(epi.residual) + (size_t)m_lo * n_out * ysize;
+        // few rows on a wide output, FAST mode: the kernel of gemm_rows.hip (waves split K, no LDS on the way)
+        RowsPlan plan = !exact && kdt == kF16 ? rows_plan(w, mc, num_cus, ec) : RowsPlan{0};
+        if (!plan.nf && !exact && kdt == kF16 && g_rows_kernel < 2) plan = gemm_rows_plan_long_k(w, mc, num_cus, ec);
+        const TilePlan tp = plan.nf ? TilePlan{} : plan_tiles(w, mc, exact, kdt == kBF16, num_cus, half, ec);
+        // gemm_cols.hip takes rows that are operands as they stand from where the caller has them: no staging launch (not where y is
+        // written over them).  us per call with / without it, EXACT: bf16 4096 -> 14336 at 64 / 256 rows 26.8 / 23.5, 57.7 / 53.9, 512 -> 1000
+        // at 100 rows 9.9 / 7.6, 7008 -> 800 at 200 rows 17.8 / 14.0, f16 4096 -> 6144 at 512 rows 51.9 / 45.6; FAST f16 14336 -> 4096 at 45 / 128
+        // rows 21.2 / 17.6, 30.9 / 26.6.
+        const char *xb = reinterpret_cast<const char*>(xs), *yb = static_cast<const char*>(yc);
+        const bool apart = xb + (size_t)mc * w.K * 2 <= yb || yb + (size_t)mc * n_out * ysize <= xb;
+        const bool raw = !plan.nf && tp.kind == TilePlan::kCols && !widen && !epi.gamma && apart && g_raw;
         const int K8 = w.K / 8;
         const dim3 grid((unsigned)((mc + 15) / 16), (unsigned)((K8 / 4 + kStageGroups - 1) / kStageGroups));
         u32x4_t* xst = reinterpret_cast<u32x4_t*>(workspace);
         NormStats ns = {ssq_part, (int)grid.y, nullptr};
-        if (widen) {
+        if (raw) {
+            ns = NormStats{nullptr, 0, nullptr};
+        } else if (widen) {
             // per-row scaled f16 operands; one sum of squares per row
             ns = NormStats{ssq_part, 1, unscale};
             // Rows per workgroup of sixteen waves: with few of them one workgroup per four rows leaves the chip idle and a
@@ -1298,22 +1317,19 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
         }
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-        // few rows on a wide output, FAST mode: the kernel of gemm_rows.hip (waves split K, no LDS on the way)
-        RowsPlan plan = !exact && kdt == kF16 ? rows_plan(w, mc, num_cus, ec) : RowsPlan{0};
-        if (!plan.nf && !exact && kdt == kF16 && g_rows_kernel < 2) plan = gemm_rows_plan_long_k(w, mc, num_cus, ec);
         if (plan.nf) {
             e = launch_gemm_rows(w, workspace, mc, yc, ydt, ec, ns.part, ns.nblk, ns.unscale, plan, part, st);
             if (e == hipSuccess && plan.shares > 4) e = launch_reduce(part, plan.shares - 3, mc, w.N, yc, ydt, out_scale, ec, ns, w.K, st);
             if (e != hipSuccess) return e;
             continue;
         }
-        const TilePlan tp = plan_tiles(w, mc, exact, kdt == kBF16, num_cus, half, ec);
+        const void* const from = raw ? static_cast<const void*>(xs) : workspace;
         if (w.bits == 4) {
-            e = kdt == kBF16 ? launch_tiles<4, 1>(tp, w, workspace, mc, yc, ydt, exact, out_scale, part, ec, ns, st)
-                             : launch_tiles<4, 0>(tp, w, workspace, mc, yc, ydt, exact, out_scale, part, ec, ns, st);
+            e = kdt == kBF16 ? launch_tiles<4, 1>(tp, w, from, raw, mc, yc, ydt, exact, out_scale, part, ec, ns, st)
+                             : launch_tiles<4, 0>(tp, w, from, raw, mc, yc, ydt, exact, out_scale, part, ec, ns, st);
         } else {
-            e = kdt == kBF16 ? launch_tiles<8, 1>(tp, w, workspace, mc, yc, ydt, exact, out_scale, part, ec, ns, st)
-                             : launch_tiles<8, 0>(tp, w, workspace, mc, yc, ydt, exact, out_scale, part, ec, ns, st);
+            e = kdt == kBF16 ? launch_tiles<8, 1>(tp, w, from, raw, mc, yc, ydt, exact, out_scale, part, ec, ns, st)
+                             : launch_tiles<8, 0>(tp, w, from, raw, mc, yc, ydt, exact, out_scale, part, ec, ns, st);
         }
         if (e != hipSuccess) return e;
     }

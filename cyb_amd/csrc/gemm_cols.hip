@@ -6,7 +6,9 @@
 //
 //   W  a native tile is multiplied by the two waves that hold its groups and by nobody else: its words go from LDS to registers,
 //      are dequantised there and are MFMA operands as they stand - no operand goes through LDS, none is made twice.
-//   X  (staged in operand order) is shared by the four columns of waves: copied to LDS once, read by each.
+//   X  is shared by the four columns of waves: copied to LDS once, read by each.  Rows that are operands as they stand (16-bit, no norm,
+//      FAST mode: f16) come from where the caller has them (RAW), whole lines of a row per copy, their pieces permuted so that
+//      reads meet no bank conflicts: as quick as copies of staged operands, and the staging launch (2.4 us and 1 us a megabyte) is gone.
 //   Both come by global_load_lds, which needs no registers while in flight: 3 - 5 K tiles of X and up to 10 of packed weights
 //      are on their way, counted by hand (s_waitcnt vmcnt: copies retire in order), one barrier per K tile in its middle - the first
 //      half's operands are in registers when it is passed, the second half's arithmetic covers the reads behind it.
@@ -85,7 +87,8 @@ struct ColsShape {
     static_assert(NW >= NX && LDS <= 160 * 1024, "LDS");
 };
 
-template <int BITS, int MODE, int RB, int CS, int KH>
+// RAW: X as the caller has it, row major, of the operands' type (no staging launch before the multiply)
+template <int BITS, int MODE, int RB, int CS, int KH, bool RAW>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_cols_kernel(
     const uint8_t* __restrict__ wbase, const uint8_t* __restrict__ x, int KT_, int NT, int x_row_blocks, int M, int n_tiles, int m_tiles,
     int splits, int kt_per_split, int groups, int N, void* __restrict__ y, int ydt, int K, float* __restrict__ part, Epilogue epi, NormStats ns)
@@ -114,17 +117,31 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         return kt_lo + (r >= KT ? r - KT : r);
     };
 
-    // ---- copies into LDS.  X: block e = row block e / 4, group e % 4 of the K tile
+    // ---- copies into LDS.  X: block e = row block e / 4, group e % 4 of the K tile.  RAW: block e = rows 8 * (e / 2) .. + 8, half e % 2 of
+    // the K tile: whole 128-byte lines, eight lanes to a row, with piece p of row r in slot p ^ r of the row: the sixteen lanes that read
+    // one piece of sixteen rows then meet sixteen different slots.
+    const int raw_row = lane >> 3, raw_piece = (lane & 7) ^ raw_row;
     uint32_t xrow[XC];
     int xblk[XC];
 #pragma unroll
     for (int c = 0; c < XC; c++) {
-        xblk[c] = min(c * 8 + wave, RB * 4 - 1);
-        xrow[c] = (uint32_t)min(m0 / 16 + (xblk[c] >> 2), x_row_blocks - 1) * (uint32_t)(G * 1024);
+        if constexpr (RAW) {
+            xblk[c] = min(c * 8 + wave, RB * 4 - 2 + (wave & 1));
+            xrow[c] = (uint32_t)min(m0 + (xblk[c] >> 1) * 8 + raw_row, M - 1) * (uint32_t)(K * 2) + (uint32_t)(raw_piece & 3) * 16u;
+        } else {
+            xblk[c] = min(c * 8 + wave, RB * 4 - 1);
+            xrow[c] = (uint32_t)min(m0 / 16 + (xblk[c] >> 2), x_row_blocks - 1) * (uint32_t)(G * 1024);
+        }
     }
     auto copy_x = [&](int kt, int buf, int c) {
-        const int g = min(rot(kt) * 4 + (xblk[c] & 3), G - 1);
-        copy_to_lds(buf * S::XTILE + xblk[c] * 1024, x, xrow[c] + (uint32_t)g * 1024u + (uint32_t)lane * 16u);
+        if constexpr (RAW) {
+            // (groups past the end of a row: its last one, against weights of zero)
+            const int g = min(rot(kt) * 4 + ((wave & 1) * 2 + (raw_piece >> 2)), G - 1);
+            copy_to_lds(buf * S::XTILE + (xblk[c] & 1) * (RB * 2048) + (xblk[c] >> 1) * 1024, x, xrow[c] + (uint32_t)g * 64u);
+        } else {
+            const int g = min(rot(kt) * 4 + (xblk[c] & 3), G - 1);
+            copy_to_lds(buf * S::XTILE + xblk[c] * 1024, x, xrow[c] + (uint32_t)g * 1024u + (uint32_t)lane * 16u);
+        }
     };
     const int ntb = min(nt0, NT - 1);
     const uint8_t* const wsrc = wbase + (int64_t)ntb * KT_ * kTileBytes<BITS>;
@@ -156,8 +173,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // ---- LDS -> registers
     Frag16 a[2][RB], b[2][OPS][CS];
     uint32_t wq[CS][WORDS], wn[CS][WORDS], sq[CS][GROUPS / 2], sn[CS][GROUPS / 2];     // packed weights and scales of my groups: this K tile's, the next one's
+    const uint32_t raw_lane = (uint32_t)(((lane >> 3) & 1) * 1024 + (lane & 7) * 128 + (((lane >> 4) ^ (lane & 7)) * 16));
     auto read_a = [&](Frag16& dst, int buf, int j, int i) {               // j: which of my groups
-        dst.u = *reinterpret_cast<const u32x4_t*>(smem + buf * S::XTILE + kh * (GROUPS * 1024) + lane * 16 + (i * 4 + j) * 1024);
+        if constexpr (RAW) {
+            const int half = KH == 2 ? kh : j >> 1;
+            dst.u = *reinterpret_cast<const u32x4_t*>(smem + buf * S::XTILE + half * (RB * 2048) + i * 2048 + ((j & 1) ? raw_lane ^ 64u : raw_lane));
+        } else dst.u = *reinterpret_cast<const u32x4_t*>(smem + buf * S::XTILE + kh * (GROUPS * 1024) + lane * 16 + (i * 4 + j) * 1024);
     };
     auto read_w = [&](int buf, uint32_t (&q)[CS][WORDS], uint32_t (&sc)[CS][GROUPS / 2]) {
         const uint8_t* p = smem + S::WBASE + buf * S::WTILE;
@@ -402,16 +423,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
-template <int BITS, int MODE, int RB, int CS, int KH>
+template <int BITS, int MODE, int RB, int CS, int KH, bool RAW>
 hipError_t launch_cols_t(const WeightView& w, const void* x, int M, void* y, int ydt, int splits, const Epilogue& epi, const NormStats& ns,
                          float* part, hipStream_t st)
 {
     using S = ColsShape<BITS, MODE, RB, CS, KH>;
-    (void)LdsRequest<&gemm_cols_kernel<BITS, MODE, RB, CS, KH>, S::LDS>::registered;
+    (void)LdsRequest<&gemm_cols_kernel<BITS, MODE, RB, CS, KH, RAW>, S::LDS>::registered;
     const int n_tiles = (w.NT + S::STRIPS - 1) / S::STRIPS, m_tiles = (M + 16 * RB - 1) / (16 * RB);
     const int kt_per_split = (w.KT + splits - 1) / splits;
     const unsigned groups = (unsigned)(((int64_t)n_tiles * m_tiles * splits + 7) / 8 * 8);
-    hipLaunchKernelGGL((gemm_cols_kernel<BITS, MODE, RB, CS, KH>), dim3(groups), dim3(512), S::LDS, st, w.base, static_cast<const uint8_t*>(x),
+    hipLaunchKernelGGL((gemm_cols_kernel<BITS, MODE, RB, CS, KH, RAW>), dim3(groups), dim3(512), S::LDS, st, w.base, static_cast<const uint8_t*>(x),
                        w.KT, w.NT, (M + 15) / 16, M, n_tiles, m_tiles, splits, kt_per_split, (int)groups, w.N, y, ydt, w.K, part, epi, ns);
     return hipGetLastError();
 }
@@ -478,12 +499,14 @@ ColsPlan plan_gemm_cols_long_k(const WeightView& w, int M, int num_cus, const Ep
     return {rb, 1, shares, true, 0.f};
 }
 
-hipError_t launch_gemm_cols(const WeightView& w, const void* x_staged, int mode, int M, void* y, int ydt, const ColsPlan& plan, const Epilogue& epi,
+hipError_t launch_gemm_cols(const WeightView& w, const void* x, bool raw, int mode, int M, void* y, int ydt, const ColsPlan& plan, const Epilogue& epi,
                             const float* ssq_part, int ssq_blocks, const float* unscale, float* part, hipStream_t st)
 {
     const NormStats ns = {ssq_part, ssq_blocks, unscale};
-    auto go = [&](auto bits, auto md, auto r, auto c) {
-        return launch_cols_t<decltype(bits)::value, decltype(md)::value, decltype(r)::value, decltype(c)::value, 2>(w, x_staged, M, y, ydt, plan.splits, epi, ns, part, st);
+    auto go = [&](auto bits, auto md, auto r, auto c, auto kh) {
+        constexpr int B = decltype(bits)::value, MD = decltype(md)::value, R = decltype(r)::value, C = decltype(c)::value, KH = decltype(kh)::value;
+        return raw ? launch_cols_t<B, MD, R, C, KH, true>(w, x, M, y, ydt, plan.splits, epi, ns, part, st)
+                   : launch_cols_t<B, MD, R, C, KH, false>(w, x, M, y, ydt, plan.splits, epi, ns, part, st);
     };
     using i0 = std::integral_constant<int, 0>;
     using i1 = std::integral_constant<int, 1>;
@@ -494,20 +517,19 @@ hipError_t launch_gemm_cols(const WeightView& w, const void* x_staged, int mode,
     using i8 = std::integral_constant<int, 8>;
     if (plan.whole_tiles) {
         auto whole = [&](auto bits) {
-            constexpr int B = decltype(bits)::value;
-            if (plan.rb == 2) return launch_cols_t<B, 0, 2, 1, 1>(w, x_staged, M, y, ydt, plan.splits, epi, ns, part, st);
-            if (plan.rb == 3) return launch_cols_t<B, 0, 3, 1, 1>(w, x_staged, M, y, ydt, plan.splits, epi, ns, part, st);
-            if (plan.rb == 4) return launch_cols_t<B, 0, 4, 1, 1>(w, x_staged, M, y, ydt, plan.splits, epi, ns, part, st);
-            if (plan.rb == 6) return launch_cols_t<B, 0, 6, 1, 1>(w, x_staged, M, y, ydt, plan.splits, epi, ns, part, st);
-            return launch_cols_t<B, 0, 8, 1, 1>(w, x_staged, M, y, ydt, plan.splits, epi, ns, part, st);
+            if (plan.rb == 2) return go(bits, i0{}, i2{}, i1{}, i1{});
+            if (plan.rb == 3) return go(bits, i0{}, i3{}, i1{}, i1{});
+            if (plan.rb == 4) return go(bits, i0{}, i4{}, i1{}, i1{});
+            if (plan.rb == 6) return go(bits, i0{}, i6{}, i1{}, i1{});
+            return go(bits, i0{}, i8{}, i1{}, i1{});
         };
         return w.bits == 4 ? whole(i4{}) : whole(i8{});
     }
     auto rows = [&](auto bits, auto md, auto cs) {
-        if (plan.rb == 3) return go(bits, md, i3{}, cs);
-        if (plan.rb == 4) return go(bits, md, i4{}, cs);
-        if (plan.rb == 6) return go(bits, md, i6{}, cs);
-        if (plan.rb == 8) return go(bits, md, i8{}, cs);
+        if (plan.rb == 3) return go(bits, md, i3{}, cs, i2{});
+        if (plan.rb == 4) return go(bits, md, i4{}, cs, i2{});
+        if (plan.rb == 6) return go(bits, md, i6{}, cs, i2{});
+        if (plan.rb == 8) return go(bits, md, i8{}, cs, i2{});
         return hipErrorInvalidValue;
     };
     auto shape = [&](auto bits, auto md) { return plan.cs == 1 ? rows(bits, md, i1{}) : rows(bits, md, i2{}); };

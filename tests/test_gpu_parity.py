@@ -1361,6 +1361,44 @@ def test_prefill_waves_side_by_side(backend, oracle, bits, mode, N, K, M):
 
 
 @pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("mode,N,K,M", [("exact", 1030, 128, 97), ("exact", 530, 352, 65), ("exact", 14336, 288, 193), ("exact", 4096, 1056, 130),
+                                        ("exact", 96, 4096, 519), ("fast", 520, 96, 129), ("fast", 1030, 9 * 128 - 32, 100), ("fast", 24640, 576, 47),
+                                        ("fast", 1030, 70 * 128 + 64, 33), ("fast", 1030, 66 * 128 + 32, 128)])
+def test_prefill_rows_read_in_place(backend, oracle, bits, mode, N, K, M):
+    """Rows that are operands as they stand are multiplied from where the caller has them: the bits of the same call behind a staging
+    launch, over row counts and K that leave a last row block and a last K tile of every fill, whatever lies behind the last row; and
+    rows that y is written over are staged."""
+    q, s = _quant(oracle, bits, N, K, cfg=141)
+    qw = backend.upload_quantized(q, s, bits)
+    backend.set_prefill_mode(mode)
+    try:
+        for xdt in ("f16", "bf16"):
+            big = torch.full((M + 40, K), float("nan"), dtype=TDT[xdt], device="cuda")
+            x = big[:M].copy_(_x(M, K, xdt, cfg=142))
+            y = _run(backend, qw, x)
+            backend.set_gemm_tuning(4)
+            staged = _run(backend, qw, x)
+            backend.set_gemm_tuning(0)
+            ref = oracle.matmul_f64(q, s, x.float().cpu().numpy())
+            assert oracle.rel_l2(y.cpu().numpy(), ref) < _bar(mode), xdt
+            if mode == "exact" or xdt == "f16":
+                assert torch.equal(y, staged), xdt
+            if N <= K:                                     # y over the rows it is made from
+                both = torch.zeros((M * K + 8,), dtype=TDT[xdt], device="cuda")
+                xo, yo = both[:M * K].view(M, K), both[8:8 + M * N].view(M, N)
+                xo.copy_(x)
+                backend.matmul(qw, xo, yo)
+                apart = torch.empty((M, N), dtype=TDT[xdt], device="cuda")
+                backend.matmul(qw, x, apart)
+                torch.cuda.synchronize()
+                assert ((yo.float() - apart.float()).norm() / apart.float().norm()).item() < 1e-2, xdt
+    finally:
+        backend.set_gemm_tuning(0)
+        backend.set_prefill_mode("fast")
+    qw.free()
+
+
+@pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("xdt", ["bf16", "f16"])
 def test_prefill_exact_operands_over_all_scales(backend, bits, xdt):
     """EXACT mode: the two operands of a weight add up to scale * q for subnormal, negative and large scales alike (every output
