@@ -12,20 +12,21 @@
 //   Both come by global_load_lds, which needs no registers while in flight: 3 - 5 K tiles of X and up to 10 of packed weights
 //      are on their way, counted by hand (s_waitcnt vmcnt: copies retire in order), one barrier per K tile in its middle - the first
 //      half's operands are in registers when it is passed, the second half's arithmetic covers the reads behind it.
-//   EXACT mode: two operands per weight that add up to scale * q.  f16: the rounded product and what it lost (one fma).  bf16, Q4: the
-//      scale is cut into two parts of five significant bits, whose products with q are bf16 numbers as they stand; 36 vector
-//      instructions per eight weights where rounding the product and subtracting took 49.
+//   EXACT mode: the operands are the integers q, one MFMA of a strip and group starts from zero and its sums are scaled on their way
+//      into the fp32 accumulators, two MFMAs later: four FMAs per MFMA.  Nothing is rounded before fp32 and no scale leaves its range.
+//      (Until now w = scale * q was cut into two operands: twice the MFMAs, 18 (f16) to 43 (bf16) vector instructions to make them.)
+//      f16 integers take 10 vector instructions per eight weights (Q8: 8), bf16 ones 15 (a signed byte to fp32, whose upper half it is).
 //
 // What bounds it: a SIMD's issue slots and LDS.  Per 16x16x32 MFMA (16 cycles of the matrix pipe) a SIMD issues two other vector
-// instructions for free, whatever the number of waves; the dequantisation of a strip's group is 16 (FAST) to 43 (EXACT bf16), which
-// only eight row blocks hide.  So the gain is where the tiled kernels of gemm.hip have few rows (their waves own 32 each, and every
-// weight operand crosses LDS for each of them) or EXACT's operands to make: K tile of 128 rows x 128 columns 1700 cycles in FAST,
-// 3230 in EXACT bf16, of which the MFMAs are 1024 and 2048.
-// us per call with the staging pass, before (128- / 64-row tiles of gemm.hip) and now.  EXACT, bf16 rows on Q4: 4096 -> 14336 at 64 / 128 /
-// 256 rows 47.7 / 50.5 / 80.6 -> 27.1 / 35.4 / 59.0, 14336 -> 4096 at 40 / 128 rows 46.2 / 50.1 -> 25.8 / 38.6, 4096 -> 4096 at 256 rows 35.5 ->
-// 26.9, 4096 -> 28672 at 64 rows 103 -> 43.6; f16 rows: 4096 -> 14336 at 256 rows 84.2 -> 53.5.  FAST: 4096 -> 28672 at 96 / 128 rows 42.5 /
-// 46.6 -> 33.5 / 39.9, with SwiGLU 48.9 / 49.8 -> 33.3 / 39.5, 14336 -> 14336 at 40 / 192 rows 58.5 / 124.5 -> 44.1 / 92.8, 4096 -> 14336 at 192 rows 39.4 ->
-// 33.7, 1024 -> 4096 at 128 rows 15.7 -> 10.1.
+// instructions for free, whatever the number of waves; per strip and group FAST has 14 of them and EXACT 11 - 16 and four per row block.
+// So the gain is where the tiled kernels of gemm.hip have few rows (their waves own 32 each, and every weight operand crosses LDS for
+// each of them) or EXACT's operands to make.  A K tile of 128 rows x 128 columns takes 1700 cycles in FAST, 1024 of them MFMAs.
+// us per call, hi / lo operands (with a staging launch) -> integers (rows in place), EXACT on Q4: bf16 4096 -> 14336 at 40 / 64 / 256 rows 24.4 /
+// 26.6 / 58.4 -> 17.2 / 19.8 / 44.3, 14336 -> 4096 at 128 rows 38.1 -> 29.1, 4096 -> 4096 at 256 rows 27.5 -> 19.2, 4096 -> 6144 at 512 rows 58.4 ->
+// 43.5; f16 4096 -> 14336 at 256 rows 53.4 -> 43.2, 4096 -> 4096 at 256 rows 24.4 -> 19.8.  Relative L2 against float64, same calls and Q8: bf16 1.2e-7 -
+// 3e-7 (Q8 1.7e-6) -> 6e-8 - 1.4e-7, f16 1.4e-7 - 3.9e-7 -> 6e-8 - 1.4e-7.  FAST, tiled kernels -> this one, both behind a staging launch: 4096 ->
+// 28672 at 96 / 128 rows 42.5 / 46.6 -> 33.5 / 39.9, with SwiGLU 48.9 / 49.8 -> 33.3 / 39.5, 14336 -> 14336 at 40 / 192 rows 58.5 / 124.5 -> 44.1 / 92.8,
+// 4096 -> 14336 at 192 rows 39.4 -> 33.7, 1024 -> 4096 at 128 rows 15.7 -> 10.1.
 // Tried: four waves of 128 x 64 on 32x32x16 MFMAs, every weight of a K tile dequantised by its wave (one wave per SIMD: MFMAs and
 // vector instructions add up, 2900 cycles a K tile for 2048 of MFMAs; 4096 -> 14336 at 512 rows 77 us against 60 of the role-split
 // kernel); deeper rings for the few-row forms (no change); words read from LDS a K tile earlier (3 % slower).
@@ -58,10 +59,9 @@ __device__ __forceinline__ void copy_to_lds(uint32_t lds_off, const void* base, 
 template <int N>
 __device__ __forceinline__ void wait_copies() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
-// MODE 0: FAST (one f16 operand per weight), 1 / 2: EXACT with f16 / bf16 operands (hi and lo)
+// MODE 0: FAST (operands round_f16(scale * q)), 1 / 2: EXACT with f16 / bf16 rows (operands the integers q, the scale on each group's sums)
 template <int BITS, int MODE, int RB, int CS, int KH>
 struct ColsShape {
-    static constexpr int OPS = MODE == 0 ? 1 : 2;
     static constexpr int COLS = 8 / KH;                                    // waves side by side
     static constexpr int STRIPS = COLS * CS;
     static constexpr int GROUPS = 4 / KH;                                  // scale groups of a K tile per wave
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     int splits, int kt_per_split, int groups, int N, void* __restrict__ y, int ydt, int K, float* __restrict__ part, Epilogue epi, NormStats ns)
 {
     using S = ColsShape<BITS, MODE, RB, CS, KH>;
-    constexpr int NX = S::NX, NW = S::NW, XC = S::XCOPIES, WC = S::WCOPIES, OPS = S::OPS, GROUPS = S::GROUPS, WORDS = S::WORDS;
+    constexpr int NX = S::NX, NW = S::NW, XC = S::XCOPIES, WC = S::WCOPIES, GROUPS = S::GROUPS, WORDS = S::WORDS;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int per_xcd = groups >> 3;
     const int item = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     };
 
     // ---- LDS -> registers
-    Frag16 a[2][RB], b[2][OPS][CS];
+    Frag16 a[2][RB], b[2][CS];
     uint32_t wq[CS][WORDS], wn[CS][WORDS], sq[CS][GROUPS / 2], sn[CS][GROUPS / 2];     // packed weights and scales of my groups: this K tile's, the next one's
     const uint32_t raw_lane = (uint32_t)(((lane >> 3) & 1) * 1024 + (lane & 7) * 128 + (((lane >> 4) ^ (lane & 7)) * 16));
     auto read_a = [&](Frag16& dst, int buf, int j, int i) {               // j: which of my groups
@@ -214,28 +214,29 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             return as_h2(__builtin_amdgcn_perm(0x64646464u, q[(2 * j + (p >> 1)) & (WORDS - 1)], (p & 1) ? 0x04030402u : 0x04010400u));
         }
     };
+    // bf16 rows: slots 2p, 2p + 1 as bf16 integers, 16 q for Q4 (a nibble in the upper half of a signed byte): byte to fp32 to its upper half
+    auto integers_bf16 = [&](const uint32_t (&q)[WORDS], int j, int p) {
+        uint32_t src = q[BITS == 4 ? (2 * (j >> 1) + (p >> 1)) & (WORDS - 1) : (2 * j + (p >> 1)) & (WORDS - 1)];
+        if constexpr (BITS == 4) src = (((j & 1) ? src : src << 4) & 0xf0f0f0f0u) ^ 0x80808080u;
+        else src ^= 0x80808080u;
+        const int lo = BITS == 4 ? 8 * (p & 1) : 16 * (p & 1), hi = lo + (BITS == 4 ? 16 : 8);
+        const float f0 = (float)(int8_t)(src >> lo), f1 = (float)(int8_t)(src >> hi);
+        return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f1), __builtin_bit_cast(uint32_t, f0), 0x07060302u);
+    };
+    auto scale_of = [&](const uint32_t (&sc)[GROUPS / 2], int j) {
+        return __builtin_bit_cast(_Float16, (uint16_t)((j & 1) ? sc[j >> 1] >> 16 : sc[j >> 1] & 0xffffu));
+    };
     auto operand = [&](const uint32_t (&q)[WORDS], const uint32_t (&sc)[GROUPS / 2], int j, int p, int buf, int s) {
-        const half2_t v = biased(q, j, p);
-        const float bias = BITS == 8 ? -1152.0f : (j & 1) ? -72.0f : -1032.0f;
-        const uint32_t bits16 = (j & 1) ? sc[j >> 1] >> 16 : sc[j >> 1] & 0xffffu;
-        const _Float16 sh = __builtin_bit_cast(_Float16, (uint16_t)bits16);
-        if constexpr (MODE != 2) {
-            const half2_t s2 = {sh, sh}, n = v + (half2_t){(_Float16)bias, (_Float16)bias};          // exact integers
-            const half2_t hi = n * s2;
-            b[buf][0][s].u[p] = as_u32(hi);
-            if constexpr (MODE == 1) b[buf][OPS - 1][s].u[p] = as_u32(__builtin_elementwise_fma(n, s2, -hi));
-        } else if constexpr (BITS == 4) {
-            // scale = top + rest, five significant bits each (rest: at most 32 units of the scale's last place): with q of three
-            // bits (or -8) both products fit the eight bits of a bf16 operand, nothing is rounded
-            const _Float16 top = __builtin_bit_cast(_Float16, (uint16_t)((bits16 + 0x20u) & 0xffc0u)), rest = sh - top;
-            const float ft = (float)top, fr = (float)rest, ct = bias * ft, cr = bias * fr;
-            b[buf][0][s].u[p] = pack_bf16x2(fmaf((float)v.x, ft, ct), fmaf((float)v.y, ft, ct));
-            b[buf][OPS - 1][s].u[p] = pack_bf16x2(fmaf((float)v.x, fr, cr), fmaf((float)v.y, fr, cr));
+        if constexpr (MODE == 2) {
+            b[buf][s].u[p] = integers_bf16(q, j, p);
         } else {
-            const float f = (float)sh, c = bias * f, w0 = fmaf((float)v.x, f, c), w1 = fmaf((float)v.y, f, c);      // exact
-            const uint32_t hi = pack_bf16x2(w0, w1);
-            b[buf][0][s].u[p] = hi;
-            b[buf][OPS - 1][s].u[p] = pack_bf16x2(w0 - __builtin_bit_cast(float, hi << 16), w1 - __builtin_bit_cast(float, hi & 0xffff0000u));
+            const _Float16 bias = (_Float16)(BITS == 8 ? -1152.0f : (j & 1) ? -72.0f : -1032.0f);
+            half2_t n = biased(q, j, p) + (half2_t){bias, bias};          // exact integers
+            if constexpr (MODE == 0) {
+                const _Float16 sh = scale_of(sc, j);
+                n *= (half2_t){sh, sh};
+            }
+            b[buf][s].u[p] = as_u32(n);
         }
     };
 
@@ -244,6 +245,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int i = 0; i < RB; i++)
 #pragma unroll
         for (int s = 0; s < CS; s++) acc[i][s] = (float4_t){0.f, 0.f, 0.f, 0.f};
+    // EXACT: the sums of one strip and group, on their way for two MFMAs before the scale is applied, and the scales of this group and the last
+    float4_t d[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    float scf[2][CS] = {};
+    auto apply = [&](float4_t& sum, float f, const float4_t& v) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) sum[r] = fmaf(f, v[r], sum[r]);
+    };
 
     // ---- prologue: batch -n of the copies holds X of K tile NX - n and the weights of K tile NW - n
     static_for<0, NW>([&](auto n_) {
@@ -289,12 +297,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
                 read_w(wnext, wn, sn);
             }
-            constexpr int MMAS = RB * CS * OPS, PAIRS = 4 * CS;
+            constexpr int MMAS = RB * CS, PAIRS = 4 * CS;
+            if constexpr (MODE != 0) {
+#pragma unroll
+                for (int s = 0; s < CS; s++) scf[cur][s] = (float)scale_of(sq[s], j) * (MODE == 2 && BITS == 4 ? 0.0625f : 1.0f);
+            }
             static_for<0, MMAS>([&](auto m_) {
-                constexpr int m = decltype(m_)::value, i = m / (CS * OPS), o = (m / CS) % OPS, s = m % CS;
-                if constexpr (MODE == 2) acc[i][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[cur][i].b, b[cur][o][s].b, acc[i][s], 0, 0, 0);
-                else acc[i][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[cur][i].h, b[cur][o][s].h, acc[i][s], 0, 0, 0);
-                if constexpr (s == 0 && o == 0) read_a(a[nxt][i], last ? xnext : xbuf, last ? 0 : j + 1, i);
+                constexpr int m = decltype(m_)::value, i = m / CS, s = m % CS;
+                if constexpr (MODE == 0) {
+                    acc[i][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[cur][i].h, b[cur][s].h, acc[i][s], 0, 0, 0);
+                } else {
+                    constexpr int slot = (j * MMAS + m) & 1, before = (m + MMAS - 2) % MMAS;      // two MFMAs ago: perhaps of the last group
+                    apply(acc[before / CS][before % CS], scf[m < 2 ? nxt : cur][before % CS], d[slot]);
+                    d[slot] = mma<MODE == 2>(a[cur][i], b[cur][s], (float4_t){0.f, 0.f, 0.f, 0.f});
+                }
+                if constexpr (s == 0) read_a(a[nxt][i], last ? xnext : xbuf, last ? 0 : j + 1, i);
                 // (the next K tile's words have just been asked for: the second half of the group is theirs; a form that read them a
                 // K tile earlier and spread their arithmetic over the whole group was 3 % slower)
                 constexpr int F = last ? MMAS / 2 : 0, p0 = m < F ? 0 : (m - F) * PAIRS / (MMAS - F), p1 = m < F ? 0 : (m - F + 1) * PAIRS / (MMAS - F);
@@ -328,6 +345,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (; kt + NW < KT; kt++) k_tile(kt, std::integral_constant<int, 0>{});
     for (; kt + NX < KT; kt++) k_tile(kt, std::integral_constant<int, 1>{});
     for (; kt < KT; kt++) k_tile(kt, std::integral_constant<int, 2>{});
+    if constexpr (MODE != 0) {
+#pragma unroll
+        for (int m = RB * CS - 2; m < RB * CS; m++) apply(acc[m / CS][m % CS], scf[(GROUPS - 1) & 1][m % CS], d[((GROUPS - 1) * RB * CS + m) & 1]);
+    }
 
     // ---- the two halves of K meet in LDS; then whole runs of a row, four elements per thread
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
