@@ -369,7 +369,8 @@ __global__ __launch_bounds__((MW + 4) * 64) __attribute__((amdgpu_waves_per_eu((
 {
     const WeightView w = {wbase, N_, K_, NT_, KT_, BITS};
     constexpr int SW = 4;                             // staging waves
-    constexpr int WT = (NF + SW - 1) / SW;            // weight tiles a staging wave handles per K tile
+    constexpr bool HALF = NF % SW == 2;
+    constexpr int WT = HALF ? NF / SW : (NF + SW - 1) / SW;            // weight tiles a staging wave handles per K tile (and half of one)
     constexpr int TILE16 = 4 * 64;                    // u32x4 per column block per K tile
     constexpr int BUF16 = NF * TILE16;
     // K tiles of packed weights in flight per staging wave (8 measured the same at 64 and 128 rows, 16
@@ -404,16 +405,42 @@ __global__ __launch_bounds__((MW + 4) * 64) __attribute__((amdgpu_waves_per_eu((
             wdst[t] = f * TILE16;
             wtile[t] = (int64_t)min(nt0 + f, w.NT - 1) * w.KT;
         }
-        WRegs<BITS> wreg[DEPTH][WT];
-        auto fetch = [&](WRegs<BITS> (&dst)[WT], int kt) {
-#pragma unroll
-            for (int t = 0; t < WT; t++) load_wtile<BITS>(dst[t], w, wtile[t] + rot(kt), lane);
+        // Six blocks: the last two in halves (two scale groups each).  A K tile waits for the last of these waves, and two blocks to a wave were
+        // eight's work.  us per call, before / after, bf16: 4096 -> 6144 at 512 rows 43.4 / 41.2, Q8 44.5 / 41.7, 4096 -> 12288 at 256 rows 41.1 / 39.3,
+        // 2048 -> 3072 at 1000 rows 25.3 / 24.1, 2880 -> 5760 at 512 rows 30.3 / 28.7.  (Seven blocks in equal parts, three groups of a block to
+        // three waves and their fourth groups to the last: 4096 -> 14336 at 512 rows 69.0 / 69.0, with a norm 69.7 / 70.9; not done.  Eight
+        // staging waves: 41.5 / 42.0, 4096 -> 6144 at 256 rows 27.6 / 28.5.)
+        const int half = pw & 1, hf = min(WT * SW + (pw >> 1), NF - 1), hdst = hf * TILE16 + half * 128;
+        const int64_t htile = (int64_t)min(nt0 + hf, w.NT - 1) * w.KT;
+        struct Staged {
+            WRegs<BITS> whole[WT];
+            WRegs<BITS> half;             // (its first two groups' registers)
         };
-        auto stage = [&](WRegs<BITS> (&src)[WT], u32x4_t* buf) {
+        Staged wreg[DEPTH];
+        auto fetch = [&](Staged& dst, int kt) {
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+            for (int t = 0; t < WT; t++) load_wtile<BITS>(dst.whole[t], w, wtile[t] + rot(kt), lane);
+            if constexpr (HALF) {
+                const int64_t tile = htile + rot(kt);
+                if constexpr (BITS == 4) {
+                    const u32x2_t q = reinterpret_cast<const u32x2_t*>(tile_q<BITS>(w, tile))[lane * 2 + half];
+                    dst.half.q[0][0] = q[0];
+                    dst.half.q[0][1] = q[1];
+                } else {
+                    dst.half.q[0] = tile_q<BITS>(w, tile)[half * 64 + lane];
+                }
+                dst.half.s[0] = reinterpret_cast<const uint32_t*>(tile_s<BITS>(w, tile))[(lane & 15) * 2 + half];
+            }
+        };
+        auto stage = [&](Staged& src, u32x4_t* buf) {
 #pragma unroll
-                for (int t = 0; t < WT; t++) dequant_group_to_lds<BITS, 0, false>(src[t], j, magic, buf + wdst[t], lane);
+            for (int j = 0; j < 4; j++) {
+#pragma unroll
+                for (int t = 0; t < WT; t++) dequant_group_to_lds<BITS, 0, false>(src.whole[t], j, magic, buf + wdst[t], lane);
+                if constexpr (HALF) {
+                    if (j < 2) dequant_group_to_lds<BITS, 0, false>(src.half, j, magic, buf + hdst, lane);
+                }
+            }
         };
 #pragma unroll
         for (int d = 0; d < DEPTH; d++) fetch(wreg[d], d);

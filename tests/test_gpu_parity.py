@@ -1399,6 +1399,27 @@ def test_prefill_rows_read_in_place(backend, oracle, bits, mode, N, K, M):
 
 
 @pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("N,K,M", [(1536, 128, 2000), (1530, 352, 1999), (1441, 544, 2000), (5600, 1184, 250), (5590, 96, 193)])
+def test_prefill_six_column_blocks_per_workgroup(backend, oracle, bits, N, K, M):
+    """Shapes whose tiles of six column blocks fill most of a round (128 rows, the last two 64): two of the blocks are shared out in halves
+    among the four waves that stage weights.  One to ten K tiles, a last tile of every fill, a last column tile that is not whole."""
+    q, s = _quant(oracle, bits, N, K, cfg=151)
+    qw = backend.upload_quantized(q, s, bits)
+    w = torch.empty((N, K), dtype=torch.float32, device="cuda")
+    backend.dequant(qw, w)
+    try:
+        backend.set_gemm_tuning(2)                                     # (a short K is gemm_cols.hip's otherwise)
+        for xdt in ("bf16", "f16"):
+            x = _x(M, K, xdt, cfg=152)
+            y = _run(backend, qw, x)
+            ref = x.double() @ w.double().t()
+            assert ((y.double() - ref).norm() / ref.norm()).item() < FAST, xdt
+    finally:
+        backend.set_gemm_tuning(0)
+    qw.free()
+
+
+@pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("xdt", ["bf16", "f16"])
 def test_prefill_exact_operands_over_all_scales(backend, bits, xdt):
     """EXACT mode: the two operands of a weight add up to scale * q for subnormal, negative and large scales alike (every output
