@@ -848,7 +848,12 @@ static float tiled_plan(const WeightView& w, int M, bool exact, int num_cus, siz
     splits = (w.KT + per - 1) / per;                             // no empty split
     plan = {TilePlan::kTiles, nf, 8, 2, splits, {}};
     const float rounds = (float)((tiles * splits + cus - 1) / cus);
-    return rounds * (exact ? 0.9f + 2.75f * (float)per : 1.4f + 1.29f * (float)per) +
+    // (EXACT: fits to 254 calls of 33 .. 2048 rows on N of 256 .. 32768, 10 - 12 % rms, taken when gemm_cols.hip went over to integer operands; with
+    // the lines from before, 0.9 + 2.75 per K tile, wide outputs of a short K and the odd large call stayed here that are quicker there.  us per
+    // call here / there: f16 640 -> 14364 at 327 rows 27.7 / 21.1, 1120 -> 7768 at 1015 rows 46.6 / 37.2, bf16 Q8 1248 -> 30164 at 174 rows 43.7 /
+    // 32.6, Q4 4544 -> 13471 at 452 rows 124 / 104)
+    const float round = exact ? (nf == 7 ? 2.4f + 2.77f * (float)per : 2.7f + 3.03f * (float)per) : 1.4f + 1.29f * (float)per;
+    return rounds * round +
            (splits > 1 ? 2.2f + 0.5f * ((float)splits + 0.5f) * out_mb : 0.27f * out_mb);
 }
 

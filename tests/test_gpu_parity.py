@@ -1420,6 +1420,31 @@ def test_prefill_six_column_blocks_per_workgroup(backend, oracle, bits, N, K, M)
 
 
 @pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("N,K,M", [(14364, 640, 327), (30164, 1248, 174), (7768, 1120, 1015), (15093, 512, 579)])
+def test_prefill_exact_on_wide_outputs_of_a_short_k(backend, oracle, bits, N, K, M):
+    """EXACT calls between the tiled kernels and the one whose waves stand side by side: both stay within what fp32 sums leave."""
+    rng = np.random.default_rng(161)
+    q = rng.integers(-8 if bits == 4 else -128, 8 if bits == 4 else 128, size=(N, K), dtype=np.int8)
+    s = (rng.random((N, K // 32), dtype=np.float32) * 0.01).astype(np.float16).view(np.uint16)
+    qw = backend.upload_quantized(q, s, bits)
+    w = torch.empty((N, K), dtype=torch.float32, device="cuda")
+    backend.dequant(qw, w)
+    backend.set_prefill_mode("exact")
+    try:
+        for xdt in ("bf16", "f16"):
+            x = _x(M, K, xdt, cfg=162)
+            ref = x.double() @ w.double().t()
+            for tuning in (0, 3):
+                backend.set_gemm_tuning(tuning)
+                y = _run(backend, qw, x)
+                assert ((y.double() - ref).norm() / ref.norm()).item() < TIGHT, (xdt, tuning)
+    finally:
+        backend.set_gemm_tuning(0)
+        backend.set_prefill_mode("fast")
+    qw.free()
+
+
+@pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("xdt", ["bf16", "f16"])
 def test_prefill_exact_operands_over_all_scales(backend, bits, xdt):
     """EXACT mode: the two operands of a weight add up to scale * q for subnormal, negative and large scales alike (every output
