@@ -487,7 +487,7 @@ class Backend:
 
     def set_prefill_mode(self, mode: str) -> None:
         """'fast' (default): one f16 MFMA per group, weights rounded once to f16;
-        'exact': lossless hi/lo split, two MFMAs per group."""
+        'exact': integer operands, fp32 scales on each group's sums (the largest calls: lossless hi/lo split, two MFMAs per group)."""
         codes = {"fast": 0, "exact": 1}
         if mode not in codes:
             raise CybqError(-1, "invalid argument", f"prefill mode {mode!r}")
