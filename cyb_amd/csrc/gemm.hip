@@ -1047,7 +1047,7 @@ __device__ __forceinline__ void row_chunk_values(const RowChunk<XT>& c, float v[
     }
 }
 
-// A workgroup of sixteen waves owns ROWS rows (4, 2 or 1) and gives every row PW = 16 / ROWS waves: wave (r, p) takes the
+// A workgroup of sixteen waves owns ROWS rows (8, 4, 2 or 1) and gives every row PW = 16 / ROWS waves: wave (r, p) takes the
 // pieces of 512 k numbered p, p + PW, ... of row r (CH of them at most stay in registers between the two steps), the parts
 // of a row meet once through LDS for the row's largest magnitude (and sum of squares).  One wave per row took 5 - 7 us for
 // 512 rows of 4096 and 10 - 12 us for rows of 14336, most of it the latency of one wave walking its row.
@@ -1314,7 +1314,13 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
             // 8192 -> 4096 at 45 rows 18.7 / 17.2 / 17.1, at 64 rows 21.4 / 20.0 / 19.8, at 100 rows 21.8 / 21.6 / 21.6; 4096 -> 4096 at 45 rows
             // 11.2 / 10.9 / 11.3, fp32 at 24 rows 10.5 / 10.1 / 10.4; 4096 -> 14336 at 45 / 64 rows 17.2 / 17.2 / 17.6, 18.8 / 19.0 / 19.4.
             // (A folded norm: always four, one order of its sums.)
-            const int stage_rows = epi.gamma ? 4 : w.K > 8192 ? (mc <= 128 ? 1 : mc <= (xdt == kF32 ? 512 : 384) ? 2 : 4) : (mc <= 48 ? 2 : 4);
+            // Eight where that makes one workgroup per CU of a second round of four-row ones: all rows go at once then, and out in whole 128-byte
+            // lines.  bf16 of K up to 4096 at more than 6 and up to 8 rows per CU, us per call, 4 / 8 rows: 4096 -> 4096 at 1900 / 2048 rows 74.1 /
+            // 69.8, 73.8 / 67.8, Q8 78.2 / 74.4, 4096 -> 1024 at 1560 / 2048 rows 31.8 / 29.8, 35.2 / 30.8 (the pass alone 15.1 / 9.7), 2048 ->
+            // 1024 21.3 / 20.5, 22.7 / 21.4, 4096 -> 14336 at 2048 rows 205 / 204.  Outside: 4096 -> 1024 at 1400 / 1500 / 2100 / 2700 rows
+            // 29.7 / 31.5, 30.5 / 32.6, 38.1 / 40.8, 44.2 / 45.3, 14336 -> 1024 at 3000 rows 135 / 155, fp32 4096 -> 1024 at 2048 rows 33.3 / 34.1.
+            const bool eight = !epi.gamma && xdt == kBF16 && w.K <= 4096 && mc > 6 * num_cus && mc <= 8 * num_cus;
+            const int stage_rows = eight ? 8 : epi.gamma ? 4 : w.K > 8192 ? (mc <= 128 ? 1 : mc <= (xdt == kF32 ? 512 : 384) ? 2 : 4) : (mc <= 48 ? 2 : 4);
             dim3 rgrid((unsigned)((mc + 15) / 16) * (16 / stage_rows));
             const Touch touch = plan_touch(w, mc, num_cus, ec, exact, rgrid.x);
             // pieces of 512 k a lane keeps in registers: the whole row when it has at most 16384 (bf16) or 8192 (fp32)
@@ -1334,7 +1340,10 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
         else if (stage_rows == 2) CYBQ_STAGE_ROWS_CH(XT, false, 2, 1, 2, 4);               \
         else CYBQ_STAGE_ROWS_CH(XT, NORM, 4, (XT == 2 ? 1 : 2), (XT == 2 ? 2 : 4), (XT == 2 ? 4 : 8)); \
     } while (0)
-            if (xdt == kF32 && epi.gamma) CYBQ_STAGE_ROWS_N(2, true);
+            if (eight) {
+                if (batches <= 2) CYBQ_STAGE_ROWS(1, false, 2, 8);
+                else CYBQ_STAGE_ROWS(1, false, 4, 8);
+            } else if (xdt == kF32 && epi.gamma) CYBQ_STAGE_ROWS_N(2, true);
             else if (xdt == kF32) CYBQ_STAGE_ROWS_N(2, false);
             else if (epi.gamma) CYBQ_STAGE_ROWS_N(1, true);
             else CYBQ_STAGE_ROWS_N(1, false);

@@ -1444,6 +1444,25 @@ def test_prefill_exact_on_wide_outputs_of_a_short_k(backend, oracle, bits, N, K,
     qw.free()
 
 
+@pytest.mark.parametrize("N,K,M", [(300, 4096, 1537), (272, 4064, 1545), (530, 1056, 2047), (1024, 2080, 2048), (64, 32, 1551), (300, 4096, 1536), (300, 4128, 2048)])
+def test_prefill_rows_staged_eight_to_a_workgroup(backend, oracle, N, K, M):
+    """bf16 rows at and around the counts that are staged eight to a workgroup: last workgroups of one to eight rows, last pieces of every fill,
+    rows of very different magnitudes (each has a power of two of its own)."""
+    q, s = _quant(oracle, 4, N, K, cfg=171)
+    qw = backend.upload_quantized(q, s, 4)
+    w = torch.empty((N, K), dtype=torch.float32, device="cuda")
+    backend.dequant(qw, w)
+    x = _x(M, K, "f32", cfg=172)
+    x *= torch.pow(2.0, (torch.arange(M, device="cuda") % 61 - 30).float())[:, None]
+    x = x.to(torch.bfloat16)
+    y = _run(backend, qw, x)
+    ref = x.double() @ w.double().t()
+    err = (y.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    # a row by itself: the mode's 2e-4 and, where N outputs are few, their spread; a row with a neighbour's power of two would be off by half and more
+    assert err.max().item() < 1e-2 and err.mean().item() < FAST
+    qw.free()
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("xdt", ["bf16", "f16"])
 def test_prefill_exact_operands_over_all_scales(backend, bits, xdt):
