@@ -12,18 +12,20 @@
 //   Both come by global_load_lds, which needs no registers while in flight: 3 - 5 K tiles of X and up to 10 of packed weights
 //      are on their way, counted by hand (s_waitcnt vmcnt: copies retire in order), one barrier per K tile in its middle - the first
 //      half's operands are in registers when it is passed, the second half's arithmetic covers the reads behind it.
-//   EXACT mode: the operands are the integers q, one MFMA of a strip and group starts from zero and its sums are scaled on their way
-//      into the fp32 accumulators, two MFMAs later: four FMAs per MFMA.  Nothing is rounded before fp32 and no scale leaves its range.
-//      (Until now w = scale * q was cut into two operands: twice the MFMAs, 18 (f16) to 43 (bf16) vector instructions to make them.)
-//      f16 integers take 10 vector instructions per eight weights (Q8: 8), bf16 ones 15 (a signed byte to fp32, whose upper half it is).
+//   EXACT mode: the operands are the integers q (bf16 rows: times the power of two of the group's scale, so that no sum leaves fp32's range
+//      before the scale is on it), one MFMA of a strip and group starts from zero and its sums are scaled on their way into the fp32
+//      accumulators, two MFMAs later: four FMAs per MFMA.  Nothing is rounded before fp32.  (w = scale * q cut into two operands took
+//      twice the MFMAs and 18 (f16) to 43 (bf16) vector instructions to make them.)
+//      f16 integers take 10 vector instructions per eight weights (Q8: 8), bf16 operands 16.
 //
 // What bounds it: a SIMD's issue slots and LDS.  Per 16x16x32 MFMA (16 cycles of the matrix pipe) a SIMD issues two other vector
-// instructions for free, whatever the number of waves; per strip and group FAST has 14 of them and EXACT 11 - 16 and four per row block.
+// instructions for free, whatever the number of waves; per strip and group FAST has 14 of them and EXACT 11 - 18 and four per row block.
 // So the gain is where the tiled kernels of gemm.hip have few rows (their waves own 32 each, and every weight operand crosses LDS for
 // each of them) or EXACT's operands to make.  A K tile of 128 rows x 128 columns takes 1700 cycles in FAST, 1024 of them MFMAs.
-// us per call, hi / lo operands (with a staging launch) -> integers (rows in place), EXACT on Q4: bf16 4096 -> 14336 at 40 / 64 / 256 rows 24.4 /
-// 26.6 / 58.4 -> 17.2 / 19.8 / 44.3, 14336 -> 4096 at 128 rows 38.1 -> 29.1, 4096 -> 4096 at 256 rows 27.5 -> 19.2, 4096 -> 6144 at 512 rows 58.4 ->
-// 43.5; f16 4096 -> 14336 at 256 rows 53.4 -> 43.2, 4096 -> 4096 at 256 rows 24.4 -> 19.8.  Relative L2 against float64, same calls and Q8: bf16 1.2e-7 -
+// us per call, weights from HBM, hi / lo operands with a staging launch -> now, EXACT: bf16 Q4 4096 -> 14336 at 40 / 64 / 256 rows 27.6 / 28.7 / 60.2 ->
+// 20.6 / 22.1 / 45.3, 14336 -> 4096 at 128 rows 39.8 -> 31.0, 4096 -> 4096 at 256 rows 27.8 -> 19.4, 4096 -> 6144 at 512 rows 59.1 -> 43.4; Q8
+// 4096 -> 14336 at 64 / 256 rows 30.0 / 68.9 -> 24.4 / 54.1; f16 Q4 4096 -> 14336 at 256 rows 61.0 -> 49.5, 4096 -> 4096 at 256 rows 26.5 -> 21.1.  (The
+// powers of two: nothing to 4 %, 40 rows 19.7 -> 20.6, Q8 53.1 -> 54.1.)  Relative L2 against float64, same calls and Q8: bf16 1.2e-7 -
 // 3e-7 (Q8 1.7e-6) -> 6e-8 - 1.4e-7, f16 1.4e-7 - 3.9e-7 -> 6e-8 - 1.4e-7.  FAST, tiled kernels -> this one, both behind a staging launch: 4096 ->
 // 28672 at 96 / 128 rows 42.5 / 46.6 -> 33.5 / 39.9, with SwiGLU 48.9 / 49.8 -> 33.3 / 39.5, 14336 -> 14336 at 40 / 192 rows 58.5 / 124.5 -> 44.1 / 92.8,
 // 4096 -> 14336 at 192 rows 39.4 -> 33.7, 1024 -> 4096 at 128 rows 15.7 -> 10.1.
@@ -59,7 +61,8 @@ __device__ __forceinline__ void copy_to_lds(uint32_t lds_off, const void* base, 
 template <int N>
 __device__ __forceinline__ void wait_copies() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
-// MODE 0: FAST (operands round_f16(scale * q)), 1 / 2: EXACT with f16 / bf16 rows (operands the integers q, the scale on each group's sums)
+// MODE 0: FAST (operands round_f16(scale * q)), 1 / 2: EXACT with f16 / bf16 rows (operands q / q * 2^e, the scale / the rest of it on each
+// group's sums)
 template <int BITS, int MODE, int RB, int CS, int KH>
 struct ColsShape {
     static constexpr int COLS = 8 / KH;                                    // waves side by side
@@ -214,24 +217,32 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             return as_h2(__builtin_amdgcn_perm(0x64646464u, q[(2 * j + (p >> 1)) & (WORDS - 1)], (p & 1) ? 0x04030402u : 0x04010400u));
         }
     };
-    // bf16 rows: slots 2p, 2p + 1 as bf16 integers, 16 q for Q4 (a nibble in the upper half of a signed byte): byte to fp32 to its upper half
-    auto integers_bf16 = [&](const uint32_t (&q)[WORDS], int j, int p) {
-        uint32_t src = q[BITS == 4 ? (2 * (j >> 1) + (p >> 1)) & (WORDS - 1) : (2 * j + (p >> 1)) & (WORDS - 1)];
-        if constexpr (BITS == 4) src = (((j & 1) ? src : src << 4) & 0xf0f0f0f0u) ^ 0x80808080u;
-        else src ^= 0x80808080u;
-        const int lo = BITS == 4 ? 8 * (p & 1) : 16 * (p & 1), hi = lo + (BITS == 4 ? 16 : 8);
-        const float f0 = (float)(int8_t)(src >> lo), f1 = (float)(int8_t)(src >> hi);
-        return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f1), __builtin_bit_cast(uint32_t, f0), 0x07060302u);
-    };
     auto scale_of = [&](const uint32_t (&sc)[GROUPS / 2], int j) {
         return __builtin_bit_cast(_Float16, (uint16_t)((j & 1) ? sc[j >> 1] >> 16 : sc[j >> 1] & 0xffffu));
     };
+    // bf16 rows: a group's operands are q * 2^e with 2^e the power of two of its scale (exact: eight significant bits), its sums are multiplied
+    // by scale / 2^e, 1 to 2: they leave fp32's range where the group's own contribution to y does.  (Sums of q itself were Inf from |x| of
+    // 8e34 on, whatever the scale.)  Q4: |q| up to 8 fits the upper byte of an f16 number, and a pair of such bytes is converted with the
+    // exponent of the scale (zero: 2^-127) in one instruction; 16 vector instructions per eight weights.  Q8: one fma to fp32 each, 16.
+    uint32_t pend[2] = {};
     auto operand = [&](const uint32_t (&q)[WORDS], const uint32_t (&sc)[GROUPS / 2], int j, int p, int buf, int s) {
-        if constexpr (MODE == 2) {
-            b[buf][s].u[p] = integers_bf16(q, j, p);
+        const float bias = BITS == 8 ? -1152.0f : (j & 1) ? -72.0f : -1032.0f;
+        auto integers = [&]() { return biased(q, j, p) + (half2_t){(_Float16)bias, (_Float16)bias}; };          // exact
+        if constexpr (MODE == 2 && BITS == 4) {
+            pend[p & 1] = as_u32(integers());
+            if (p & 1) {
+                const uint32_t bytes = __builtin_amdgcn_perm(pend[1], pend[0], 0x07050301u);
+                const float f = (float)scale_of(sc, j);
+                b[buf][s].u[p - 1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(bytes, f, false));
+                b[buf][s].u[p] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(bytes, f, true));
+            }
+        } else if constexpr (MODE == 2) {
+            const half2_t v = biased(q, j, p);
+            const float f = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, (float)scale_of(sc, j)) & 0x7f800000u), c = bias * f;
+            const float w0 = fmaf((float)v.x, f, c), w1 = fmaf((float)v.y, f, c);
+            b[buf][s].u[p] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, w1), __builtin_bit_cast(uint32_t, w0), 0x07060302u);
         } else {
-            const _Float16 bias = (_Float16)(BITS == 8 ? -1152.0f : (j & 1) ? -72.0f : -1032.0f);
-            half2_t n = biased(q, j, p) + (half2_t){bias, bias};          // exact integers
+            half2_t n = integers();
             if constexpr (MODE == 0) {
                 const _Float16 sh = scale_of(sc, j);
                 n *= (half2_t){sh, sh};
@@ -300,7 +311,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             constexpr int MMAS = RB * CS, PAIRS = 4 * CS;
             if constexpr (MODE != 0) {
 #pragma unroll
-                for (int s = 0; s < CS; s++) scf[cur][s] = (float)scale_of(sq[s], j) * (MODE == 2 && BITS == 4 ? 0.0625f : 1.0f);
+                for (int s = 0; s < CS; s++) {
+                    const float f = (float)scale_of(sq[s], j);
+                    scf[cur][s] = MODE == 1 ? f : 2.0f * __builtin_amdgcn_frexp_mantf(f);
+                }
             }
             static_for<0, MMAS>([&](auto m_) {
                 constexpr int m = decltype(m_)::value, i = m / CS, s = m % CS;

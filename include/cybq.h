@@ -89,9 +89,10 @@ typedef enum cybq_dtype { CYBQ_F32 = 0, CYBQ_F16 = 1, CYBQ_BF16 = 2 } cybq_dtype
  *          output): rows of any finite magnitude keep that accuracy; within a row, elements
  *          below 2^-27 of the largest lose bits.  f16 activations are used as they are.
  *   EXACT  nothing is rounded on the way to the fp32 sums, so y differs from the fp32 CPU path only by
- *          accumulation order (about 1e-7 relative L2).  The operands are the integers q, each group's fp32 scale is
- *          applied to its sums; the largest calls multiply scale * q as a high and a low 16-bit operand, two
- *          MFMAs per 32-group (the low one rounded for Q8: 2e-6). */
+ *          accumulation order (about 1e-7 relative L2), for rows of any finite magnitude.  The operands are the
+ *          integers q (bf16 rows: times the power of two of the group's scale), each group's scale (what is left
+ *          of it) is applied to its sums in fp32; the largest calls multiply scale * q as a high and a low 16-bit
+ *          operand, two MFMAs per 32-group (the low one rounded for Q8: 2e-6). */
 typedef enum cybq_prefill_mode { CYBQ_PREFILL_FAST = 0, CYBQ_PREFILL_EXACT = 1 } cybq_prefill_mode;
 
 /* How the decode kernels form their weight operands.  Every form accumulates in fp32, applies the

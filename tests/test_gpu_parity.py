@@ -1463,6 +1463,38 @@ def test_prefill_rows_staged_eight_to_a_workgroup(backend, oracle, N, K, M):
     qw.free()
 
 
+@pytest.mark.parametrize("mode,bits,N,K,M", [("exact", 4, 592, 352, 83), ("exact", 8, 592, 352, 83), ("exact", 4, 1024, 4096, 256), ("exact", 8, 96, 4096, 519),
+                                             ("fast", 4, 512, 8224, 48), ("fast", 4, 6160, 512, 40)])
+def test_prefill_exact_rows_of_any_magnitude(backend, mode, bits, N, K, M):
+    """bf16 rows up to the type's largest against scales that bring them back, groups of scale zero and groups past the end of K among
+    them: the sums of a group stay in range wherever its contribution to y does, in EXACT mode and where FAST mode takes exact operands
+    (33 .. 64 rows of Q4, K over 4096, or short on a wide output)."""
+    rng = np.random.default_rng(181)
+    q = rng.integers(-(1 << (bits - 1)), 1 << (bits - 1), (N, K)).astype(np.int8)
+    s = (rng.random((N, K // 32)) * 0.004 + 0.0005).astype(np.float16)
+    s[:, 1::7] = 0
+    qw = backend.upload_quantized(q, s.view(np.uint16), bits)
+    wd = torch.from_numpy(np.repeat(s.astype(np.float64), 32, axis=1) * q).cuda()
+    powers = (0, 30, 33, 34, 35, 36, -30, -34, -36)
+    x = synth.activations(182, M, K).astype(np.float64) * (10.0 ** np.array([powers[m % len(powers)] for m in range(M)]))[:, None]
+    x[0, 5] = 3.3e38                                           # one element
+    x[9, :256] = 2e36 * np.sign(q[0, :256] + 0.5)              # eight groups of one sign against column 0
+    x[18] = 0.0
+    x = torch.from_numpy(x.astype(np.float32)).cuda().bfloat16()
+    backend.set_prefill_mode(mode)
+    try:
+        y = _run(backend, qw, x).double()
+    finally:
+        backend.set_prefill_mode("fast")
+    ref = x.double() @ wd.T
+    assert torch.isfinite(y).all() and not y[18].any()
+    norm = ref.norm(dim=1)
+    norm[18] = 1.0
+    # fp32 sums (1e-7): a row of 1e-36 has products down to 2^-149 of a sum of 2^-120
+    assert ((y - ref).norm(dim=1) / norm).max().item() < 1e-6
+    qw.free()
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("xdt", ["bf16", "f16"])
 def test_prefill_exact_operands_over_all_scales(backend, bits, xdt):
