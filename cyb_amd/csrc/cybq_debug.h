@@ -24,9 +24,8 @@ int cybq_debug_set_gemv_tuning(int waves_per_group, int rows_kernel, int unroll)
  * split K where its workgroups of up to 64 rows fit one round of CUs and fill a quarter of it; else the quicker of the tiled kernels
  * and the kernel whose waves stand side by side, by estimates), 1 the first of these for up to 64 rows whatever the width, 2 in FAST mode
  * the tiled kernels alone (on small weights at up to 64 rows two passes of the batched-rows decode kernel take the call as they do for
- * other shapes), 3 in both modes; 4: automatic, but no kernel
- * reads rows where the caller has them, all are staged; 5: automatic, but the staging launch asks for no weights ahead of the multiply; 6: automatic, it
- * asks only ahead of the kernel whose waves split K. */
+ * other shapes), 3 in both modes; 4: automatic, but no kernel reads rows where the caller has them, all are staged; 5: automatic, but the
+ * staging launch asks for no weights ahead of the multiply; 6: automatic, it asks only ahead of the kernel whose waves split K. */
 int cybq_debug_set_gemm_tuning(int rows_kernel);
 
 /* Ceiling probes for the one-row decode kernel: a kernel that issues exactly that kernel's

@@ -1177,8 +1177,8 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
 
 }  // namespace
 
-bool g_raw = true;            // (4 = gemm_cols.hip reads staged rows only)
-int g_touch = 2;              // (5 = the staging launch asks for no weights ahead of the multiply, 6 = only ahead of the few-rows kernel)
+static bool g_raw = true;     // (4 = gemm_cols.hip reads staged rows only)
+static int g_touch = 2;       // (5 = the staging launch asks for no weights ahead of the multiply, 6 = only ahead of the few-rows kernel)
 void set_gemm_tuning(int rows_kernel)
 {
     g_rows_kernel = rows_kernel >= 4 ? 0 : rows_kernel;
@@ -1315,9 +1315,10 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
             // 11.2 / 10.9 / 11.3, fp32 at 24 rows 10.5 / 10.1 / 10.4; 4096 -> 14336 at 45 / 64 rows 17.2 / 17.2 / 17.6, 18.8 / 19.0 / 19.4.
             // (A folded norm: always four, one order of its sums.)
             // Eight where that makes one workgroup per CU of a second round of four-row ones: all rows go at once then, and out in whole 128-byte
-            // lines.  bf16 of K up to 4096 at more than 6 and up to 8 rows per CU, us per call, 4 / 8 rows: 4096 -> 4096 at 1900 / 2048 rows 74.1 /
-            // 69.8, 73.8 / 67.8, Q8 78.2 / 74.4, 4096 -> 1024 at 1560 / 2048 rows 31.8 / 29.8, 35.2 / 30.8 (the pass alone 15.1 / 9.7), 2048 ->
-            // 1024 21.3 / 20.5, 22.7 / 21.4, 4096 -> 14336 at 2048 rows 205 / 204.  Outside: 4096 -> 1024 at 1400 / 1500 / 2100 / 2700 rows
+            // lines.  bf16 of K up to 4096 at more than 6 and up to 8 rows per CU, us per call, 4 / 8 rows: 4096 -> 4096 at 1900 / 2048 rows 70.4 /
+            // 68.8, 70.5 / 69.1, 4096 -> 1024 at 1560 / 2048 rows 31.8 / 29.8, 35.6 / 31.5 (the pass alone 15.1 / 9.7), 2048 -> 4096 44.4 / 42.9,
+            // 2048 -> 1024 21.3 / 20.5, 22.7 / 21.4, 4096 -> 14336 at 2048 rows 211.6 / 211.0; 30 calls of the range on N of 256 .. 8192: 5 % in the
+            // mean, none slower.  Outside: 4096 -> 1024 at 1400 / 1500 / 2100 / 2700 rows
             // 29.7 / 31.5, 30.5 / 32.6, 38.1 / 40.8, 44.2 / 45.3, 14336 -> 1024 at 3000 rows 135 / 155, fp32 4096 -> 1024 at 2048 rows 33.3 / 34.1.
             const bool eight = !epi.gamma && xdt == kBF16 && w.K <= 4096 && mc > 6 * num_cus && mc <= 8 * num_cus;
             const int stage_rows = eight ? 8 : epi.gamma ? 4 : w.K > 8192 ? (mc <= 128 ? 1 : mc <= (xdt == kF32 ? 512 : 384) ? 2 : 4) : (mc <= 48 ? 2 : 4);

@@ -121,8 +121,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     };
 
     // ---- copies into LDS.  X: block e = row block e / 4, group e % 4 of the K tile.  RAW: block e = rows 8 * (e / 2) .. + 8, half e % 2 of
-    // the K tile: whole 128-byte lines, eight lanes to a row, with piece p of row r in slot p ^ r of the row: the sixteen lanes that read
-    // one piece of sixteen rows then meet sixteen different slots.
+    // the K tile: whole 128-byte lines, eight lanes to a row, with piece p of row r in slot p ^ (r & 7) of the row: eight lanes in a row that
+    // read one piece of their rows then meet eight different slots, all 128 bytes that LDS gives in a cycle.  (Rows r and r + 8 meet the same
+    // banks, a cycle apart: 0.24 M conflict cycles over the chip at 256 rows of 4096 -> 14336, as many as with staged operands.)
     const int raw_row = lane >> 3, raw_piece = (lane & 7) ^ raw_row;
     uint32_t xrow[XC];
     int xblk[XC];
@@ -477,8 +478,11 @@ constexpr int kColsSplits = 8;               // the slab-adding pass takes as ma
 }  // namespace
 
 // Row blocks, strips per wave and splits with the shortest estimate.  A round of workgroups costs a fixed part and so much per K
-// tile (below, us; fits to 9000 forced calls of 33 .. 600 rows, N of 512 .. 32768, K of 512 .. 14336, Q4 and Q8: 3 - 5 % rms), a split
-// its slabs' way through memory.  Choosing by it costs 0.5 % against the best of all forms on these calls.
+// tile (below, us; fits to 9000 forced calls of 33 .. 600 rows, N of 512 .. 32768, K of 512 .. 14336, Q4 and Q8), a split its slabs' way
+// through memory.  FAST: 3 - 5 % rms, choosing by it costs 0.5 % against the best of all forms on these calls.  EXACT: the fits are those of
+// two operands per weight, which had twice the MFMAs.  Calls of 65 .. 2048 rows on the integer operands take 0.9 - 2.3 times the estimate (143
+// calls; in the mean 1.36 / 1.23 times with one / two strips and f16 rows, 1.23 / 1.06 with bf16 rows), so it ranks these forms no more than
+// roughly; against the kernels before (same choice, staged rows) none of 210 EXACT calls is slower, in the mean they are 1.2 times as fast.
 ColsPlan plan_gemm_cols(const WeightView& w, int mode, int M, int num_cus, size_t part_bytes)
 {
     struct Form {
