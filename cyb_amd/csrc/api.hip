@@ -519,14 +519,17 @@ int matmul_fused(cybq_ctx* ctx, const cybq_weight* w, const void* x, cybq_dtype 
     if (way == kDecode) {
         e = cybq::launch_gemv(v, x, xdt, (int)M, y, ydt, ctx->num_cus, ctx->decode_exact, epi, dscr, dscr_bytes, st);
     } else if (way == kTwoPasses) {
-        // 33..64 rows on a small weight (up to 4096 -> 6144) that the few-rows MFMA kernel does not take (exact
-        // mode, wide scales, K outside 2048 .. 8192): two passes of the batched-rows decode kernel (32 rows, then the rest) are
-        // quicker than a staging launch and a multiply although they stream the weights twice - and exact.  us per call, two passes
-        // / gemm_cols.hip with bf16 rows on Q4, at 33, 48, 64 rows: 4096 -> 4096 11.4, 12.6, 14.8 / 14.4, 14.9, 16.1, 2048 -> 6144 9.5, 9.6,
-        // 10.9 / 13.6, 14.1, 14.8.  Not with a longer K (8192 -> 512 15.0, 17.1, 20.6 / 12.7, 12.9, 13.3; 14336 -> 1024 25.9, 30.9, 38.0 /
-        // 16.9, 17.0, 17.9) nor with the shortest on a wide output (512 -> 14336 11.7, 15.8, 17.9 / 8.6, 8.8, 9.1): in FAST mode bf16 rows on Q4
-        // go through the prefill path there, with exact operands (kPrefillExact; relative L2 against float64 7.6e-7 -> 2.2e-7; f16 rows
-        // 1.5e-7 -> 2.6e-7 and Q8 1.5e-7 -> 1.7e-6 stay), unless K is so long (251 936 and more) that the scratch does not hold 256 staged rows.
+        // 33..64 rows on a small weight (up to 4096 -> 6144) that the few-rows MFMA kernel does not take (exact mode, wide scales, K outside 2048 ..
+        // 8192): two passes of the batched-rows decode kernel (32 rows, then the rest), which stream the weights twice.  The line was drawn when
+        // the prefill path had a staging launch and two MFMAs per group in EXACT mode.  With integer operands and rows read in place two passes
+        // are the quicker way on the first of the shapes below alone (on Q8 they are even).  us per call, two passes / prefill path with
+        // exact operands, at 33, 48, 64 rows.  bf16 on Q4: 2048 -> 6144 9.5, 9.5, 11.3 / 10.7, 11.2, 12.0; 4096 -> 4096 11.6, 12.5, 14.6 / 11.3, 12.0,
+        // 13.1; 1024 -> 4096 7.9, 8.7, 10.4 / 7.1, 7.1, 7.5; 4096 -> 1024 10.2, 11.0, 12.7 / 8.0, 8.3, 8.7; 768 -> 9167 11.8, 14.4, 17.4 / 7.2, 7.4, 7.8.
+        // f16 on Q4: 12576 -> 281 25.1, 29.8, 37.1 / 11.4, 11.8, 12.7; 512 -> 14336 12.5, 16.0, 18.0 / 5.8, 5.9, 6.3.  Q8 (bf16): 2048 -> 6144 11.3, 11.4, 12.9 /
+        // 11.3, 12.0, 12.6; 14336 -> 1024 31.6, 36.9, 44.2 / 13.2, 13.8, 14.8.  Relative L2 against float64, same calls: f16 6e-8 - 1.5e-7 / 6e-8 - 1.2e-7,
+        // bf16 on Q4 2.6e-7 - 5.1e-7 / 6e-8 - 1.1e-7, on Q8 7e-8 - 1.5e-7 / 6e-8 - 1.2e-7.  Moved so far: in FAST mode bf16 rows on Q4 with K over 4096 or of
+        // up to 512 on 6144 columns and more (kPrefillExact: 8192 -> 512 15.9, 17.9, 21.6 / 9.6, 9.8, 10.2; 14336 -> 1024 26.6, 31.4, 38.9 / 12.6, 13.2, 14.2;
+        // 512 -> 14336 12.3, 16.0, 18.0 / 6.4, 6.6, 6.9), unless K is so long (251 936 and more) that the scratch does not hold 256 staged rows.
         // (a context in CYBQ_PREFILL_EXACT mode asked for exact operands at this row count)
         const bool exact_ops = ctx->decode_exact || ctx->prefill_exact;
         const int64_t n_out = epi.kind == cybq::kEpiSwiglu ? w->N / 2 : w->N;
