@@ -175,12 +175,13 @@ int cybq_weight_info(const cybq_weight* w, int* quant, int64_t* N, int64_t* K,
  * (decide/pipeline.md:28,51):   y[m,n] = sum_k x[m,k] * (scale[n,k/32] * q[n,k])
  * with fp32 accumulation.
  *   x  [M,K] row-major, xdt in {F16,BF16,F32}, 16-byte aligned
- *   y  [M,N] row-major, ydt in {F32,F16,BF16} (fp32 accumulator rounded once)
+ *   y  [M,N] row-major, ydt in {F32,F16,BF16} (fp32 accumulator rounded once); must not overlap x: workgroups
+ *      that are done write y while others still read rows of x
  *   M >= 1.  M <= 32 runs the HBM-streaming decode kernels (17..32 rows of 16-bit
  *   activations: one pass with two row blocks; with a folded norm that holds for f16
  *   on outputs of 6144 or more with K of 928..1536 and 1952..3072, elsewhere it is two
  *   passes of 16 rows or, in FAST mode, a prefill kernel; 33..64 rows of 16-bit activations on a weight of up to 6144 x 4096
- *   elements: two passes, 32 rows and the rest), larger M the LDS-tiled MFMA prefill kernel (fp32
+ *   elements that the FAST prefill kernels do not take: two passes, 32 rows and the rest), larger M the LDS-tiled MFMA prefill kernel (fp32
  *   activations in CYBQ_PREFILL_EXACT mode: the decode kernel, 16 rows at a
  *   time; in FAST mode they are rounded once to f16 on the way in and take
  *   the prefill kernel from 17 rows on); there is no other path. */
