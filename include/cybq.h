@@ -104,7 +104,9 @@ typedef enum cybq_prefill_mode { CYBQ_PREFILL_FAST = 0, CYBQ_PREFILL_EXACT = 1 }
  *                     inside the tolerance; the kernel goes with N, K and the epilogue).
  *   bf16 activations  any row count, either mode: the bf16 numbers 128 + (q + bias) with the bias
  *                     removed inside the accumulation (bf16 has no packed add to take it off
- *                     beforehand); the mode only chooses the kernel for 1 - 2 rows.
+ *                     beforehand); the mode only chooses the kernel for 1 - 2 rows.  A group's sums carry the
+ *                     bias before the scale is on them: |x| up to 4e34 keeps them in fp32's range (the prefill
+ *                     kernels take any finite row).
  *   fp32 activations  exact integers in either mode (activations split into two f16 halves).
  * A 16-bit row keeps its bits in any batch of 3 .. 32 rows on weights of N = 6144 .. 28656 and K = 928 .. 4096
  * without a folded norm; elsewhere the kernel, and with it the last bits of a row, may change with the batch.  An
