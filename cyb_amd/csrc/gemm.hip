@@ -229,6 +229,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     Frag16 xa[4][MF];          // one K tile (four scale groups) of X in flight
 #pragma unroll
     for (int j = 0; j < 4; j++) load_x(xa[j], 0, j);
+    RowStats stats = {};                            // (512-row tiles have no registers for them: 4096 -> 14336 at 2048 rows 240 -> 250 us)
+    if constexpr (MF <= 2) stats = load_row_stats(ns, epi.gamma != nullptr, min(m0 + min(lane, MF * 16 - 1), M - 1), wbase);
     // Packed weights wait in registers: K tile t sits in wreg[t % SETS], requested SETS - 1
     // iterations before it is dequantised.  Loads retire in order and every iteration
     // also requests X, so two sets leave a weight tile one iteration (about 2 us) to
@@ -315,11 +317,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         return;
     }
     if (epi.gamma || ns.unscale) {     // folded RMSNorm: rstd of the row; widened activations: the row's power of two
+        float mine = 0.f;
+        if constexpr (MF <= 2) mine = row_factor(stats, ns, epi.gamma != nullptr, min(m0 + min(lane, MF * 16 - 1), M - 1), K, epi.eps);
 #pragma unroll
         for (int i = 0; i < MF; i++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const float rs = row_factor(ns, epi.gamma != nullptr, min(m0 + i * 16 + oct * 4 + r, M - 1), K, epi.eps);
+                const float rs = MF <= 2 ? __shfl(mine, i * 16 + oct * 4 + r, 64)
+                                         : row_factor(ns, epi.gamma != nullptr, min(m0 + i * 16 + oct * 4 + r, M - 1), K, epi.eps);
 #pragma unroll
                 for (int f = 0; f < NF; f++) acc[i][f][r] *= rs;
             }
@@ -501,6 +506,7 @@ __global__ __launch_bounds__((MW + 4) * 64) __attribute__((amdgpu_waves_per_eu((
     for (int d = 0; d < XD; d++)
 #pragma unroll
         for (int j = 0; j < 4; j++) load_x(xa[d][j], d, j);
+    const RowStats stats = load_row_stats(ns, epi.gamma != nullptr, min(m0 + min(lane, MF * 16 - 1), M - 1), wbase);
     __syncthreads();
     auto k_tile = [&](int kt, auto residue) {
         constexpr int D = decltype(residue)::value;                 // = kt % XD
@@ -550,11 +556,12 @@ __global__ __launch_bounds__((MW + 4) * 64) __attribute__((amdgpu_waves_per_eu((
         }
     }
     if (epi.gamma || ns.unscale) {
+        const float mine = row_factor(stats, ns, epi.gamma != nullptr, min(m0 + min(lane, MF * 16 - 1), M - 1), K, epi.eps);
 #pragma unroll
         for (int i = 0; i < MF; i++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const float rs = row_factor(ns, epi.gamma != nullptr, min(m0 + i * 16 + (lane >> 4) * 4 + r, M - 1), K, epi.eps);
+                const float rs = __shfl(mine, i * 16 + (lane >> 4) * 4 + r, 64);
 #pragma unroll
                 for (int f = 0; f < NF; f++) acc[i][f][r] *= rs;
             }

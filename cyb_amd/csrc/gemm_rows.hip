@@ -71,15 +71,17 @@ __device__ __forceinline__ void dequant_group(const WRegs<BITS>& r, int j, uint3
     for (int p = 0; p < 4; p++) b.u[p] = as_u32(as_h2(bw[p]) * s2);
 }
 
-// the finished sums of one row block (first row m0) on their way to y: row factors, SwiGLU, residual
+// the finished sums of one row block (first row m0) on their way to y: row factors, SwiGLU, residual.  stats: row m0 + lane % 16's, res: the
+// block's residual, both asked for before the waves' sums meet
 template <int NF>
 __device__ __forceinline__ void finish_row_block(float4_t (&tot)[1][NF], float* stg, int m0, int nt0, int M, const WeightView& w, void* y, int ydt, int K,
-                                                 const Epilogue& epi, const NormStats& ns, int lane)
+                                                 const Epilogue& epi, const NormStats& ns, const RowStats& stats, const Residual<1, NF>& res, int lane)
 {
     if (epi.gamma || ns.unscale) {
+        const float mine = row_factor(stats, ns, epi.gamma != nullptr, min(m0 + (lane & 15), M - 1), K, epi.eps);
 #pragma unroll
         for (int r4 = 0; r4 < 4; r4++) {
-            const float rs = row_factor(ns, epi.gamma != nullptr, min(m0 + (lane >> 4) * 4 + r4, M - 1), K, epi.eps);
+            const float rs = __shfl(mine, (lane >> 4) * 4 + r4, 64);
 #pragma unroll
             for (int f = 0; f < NF; f++) tot[0][f][r4] *= rs;
         }
@@ -96,7 +98,7 @@ __device__ __forceinline__ void finish_row_block(float4_t (&tot)[1][NF], float* 
             return;
         }
     }
-    write_rows<1, NF>(tot, stg, m0, nt0, M, w.N, y, ydt, 1.0f, epi, lane);
+    write_rows<1, NF>(tot, res, stg, m0, nt0, M, w.N, y, ydt, 1.0f, epi, lane);
 }
 
 // MF row blocks of 16 per workgroup (blockIdx.y-th MF * 16 rows of the call), NF column blocks per workgroup, WAVES
@@ -207,6 +209,11 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC 
         }
     }
     // ---- the partial sums meet: every wave leaves all of its blocks, waves 0 .. MF-1 finish a row block each
+    // (what that takes from memory is asked for first; ahead of the K loop it cost registers: 4096 -> 14336 at 64 rows 16.9 -> 17.2 us)
+    const int mb = (rb0 + min(wv, MF - 1)) * 16;               // first row of the block I finish
+    const RowStats stats = load_row_stats(ns, epi.gamma != nullptr, min(mb + (lane & 15), M - 1), wbase);
+    Residual<1, NF> res;
+    if (wv < MF) load_residual(res, mb, nt0, M, w.N, y, ydt, epi, lane);
 #pragma unroll
     for (int i = 0; i < MF; i++)
 #pragma unroll
@@ -228,7 +235,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC 
             return;
         }
     }
-    finish_row_block<NF>(tot, stg + wv * (16 * NF * 16), (rb0 + wv) * 16, nt0, M, w, y, ydt, K, epi, ns, lane);
+    finish_row_block<NF>(tot, stg + wv * (16 * NF * 16), mb, nt0, M, w, y, ydt, K, epi, ns, stats, res, lane);
 }
 
 // The same sums for outputs of more than a round of workgroups (up to 64 rows, four column blocks each): one workgroup of eight
@@ -344,6 +351,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");       // (copies past the last step)
     float4_t* const part = reinterpret_cast<float4_t*>(smem) + half * (4 * FR * 64);
     float* const stg = reinterpret_cast<float*>(smem + 8 * FR * 1024) + half * (MF * 16 * NF * 16);
+    const int mb = min(wv, MF - 1) * 16;
+    const RowStats stats = load_row_stats(ns, epi.gamma != nullptr, min(mb + (lane & 15), M - 1), wbase);
+    Residual<1, NF> res;
+    if (wv < MF) load_residual(res, mb, nt0, M, w.N, y, ydt, epi, lane);
 #pragma unroll
     for (int i = 0; i < MF; i++)
 #pragma unroll
@@ -359,7 +370,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int p = 1; p < 4; p++) s += part[(p * FR + blk) * 64 + lane];
         tot[0][f] = s;
     }
-    finish_row_block<NF>(tot, stg + wv * (16 * NF * 16), wv * 16, nt0, M, w, y, ydt, K, epi, ns, lane);
+    finish_row_block<NF>(tot, stg + wv * (16 * NF * 16), wv * 16, nt0, M, w, y, ydt, K, epi, ns, stats, res, lane);
 }
 
 template <int BITS, int MF, int DEPTH, int RING>
