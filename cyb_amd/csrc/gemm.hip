@@ -134,11 +134,13 @@ __device__ __forceinline__ void dequant_group_to_lds(const WRegs<BITS>& r, int j
 // Wave wv of eight owns MF row blocks of 16 against all NF column blocks.
 template <int BITS, int XBF, int NF, bool EXACT, int MF>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_kernel(const uint8_t* __restrict__ wbase, const u32x4_t* __restrict__ x, int KT_, int NT_, int x_row_blocks, int M,
-                                                   int n_tiles, int m_tiles, int splits, int kt_per_split, int groups, int N_,
-                                                   void* __restrict__ y, int ydt, int K_, float out_scale,
+                                                   int n_tiles, int m_tiles, int splits, int kt_per_split, int groups, int K_,
+                                                   int N_, void* __restrict__ y, int ydt, float out_scale,
                                                    float* __restrict__ part, Epilogue epi, NormStats ns)
 {
-    // (leading scalar arguments in the order of their first use: they arrive in registers at wave start)
+    // (leading scalar arguments in the order of their first use: they arrive in registers at wave start.  K among them, and the staging pass's
+    // first_group: with those the first requests wait for no argument.  us per call: 4096 -> 14336 at 64 fp32-out rows 16.9 / 16.4, 4096 -> 28672 at 64
+    // rows 28.4 / 27.2, 32-layer list at 45 rows 2555 / 2495.)
     const WeightView w = {wbase, N_, K_, NT_, KT_, BITS};
     // Workgroups are handed to the 8 XCDs round-robin (id % 8) and every XCD has
     // its own L2.  Give each XCD a contiguous run of tiles in row-block-major
@@ -370,7 +372,7 @@ __device__ __forceinline__ void static_for(F&& f)
 template <int BITS, int NF, int MF, int MW, int XD>
 __global__ __launch_bounds__((MW + 4) * 64) __attribute__((amdgpu_waves_per_eu((MW + 7) / 4, (MW + 7) / 4))) void gemm_roles_kernel(
     const uint8_t* __restrict__ wbase, const u32x4_t* __restrict__ x, int KT_, int NT_, int x_row_blocks, int M, int n_tiles,
-    int m_tiles, int groups, int N_, void* __restrict__ y, int ydt, int K_, float out_scale, Epilogue epi, NormStats ns)
+    int m_tiles, int groups, int K_, int N_, void* __restrict__ y, int ydt, float out_scale, Epilogue epi, NormStats ns)
 {
     const WeightView w = {wbase, N_, K_, NT_, KT_, BITS};
     constexpr int SW = 4;                             // staging waves
@@ -593,7 +595,7 @@ hipError_t launch_roles(const WeightView& w, const void* x, int M, void* y, int 
     const int n_tiles = (w.NT + NF - 1) / NF, m_tiles = (M + BM - 1) / BM;
     const unsigned groups = (unsigned)(((int64_t)n_tiles * m_tiles + 7) / 8 * 8);
     hipLaunchKernelGGL((gemm_roles_kernel<BITS, NF, MF, MW, XD>), dim3(groups), dim3((MW + 4) * 64), lds, st, w.base,
-                       reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT, (M + 15) / 16, M, n_tiles, m_tiles, (int)groups, w.N, y, ydt, w.K,
+                       reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT, (M + 15) / 16, M, n_tiles, m_tiles, (int)groups, w.K, w.N, y, ydt,
                        out_scale, epi, ns);
     return hipGetLastError();
 }
@@ -765,7 +767,7 @@ hipError_t launch_m(const WeightView& w, const void* x, int M, void* y, int ydt,
     const int kt_per_split = (w.KT + splits - 1) / splits;
     const unsigned groups = (unsigned)(((int64_t)n_tiles * m_tiles * splits + 7) / 8 * 8);
     hipLaunchKernelGGL(kern, dim3(groups), dim3(512), lds, st, w.base, reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT,
-                       (M + 15) / 16, M, n_tiles, m_tiles, splits, kt_per_split, (int)groups, w.N, y, ydt, w.K, out_scale, part, epi, ns);
+                       (M + 15) / 16, M, n_tiles, m_tiles, splits, kt_per_split, (int)groups, w.K, w.N, y, ydt, out_scale, part, epi, ns);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || splits == 1) return e;
     return launch_reduce(part, splits, M, w.N, y, ydt, out_scale, epi, ns, w.K, st);
@@ -1059,12 +1061,13 @@ __device__ __forceinline__ void row_chunk_values(const RowChunk<XT>& c, float v[
 // of a row meet once through LDS for the row's largest magnitude (and sum of squares).  One wave per row took 5 - 7 us for
 // 512 rows of 4096 and 10 - 12 us for rows of 14336, most of it the latency of one wave walking its row.
 template <int XT, bool NORM, int CH, int ROWS>
-__global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict__ src, u32x4_t* __restrict__ dst, int M, int K,
-                                                          Epilogue epi, float* __restrict__ ssq, float* __restrict__ unscale, Touch touch)
+__global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict__ src, u32x4_t* __restrict__ dst, int M, int K, int first_group,
+                                                          int gamma_dt, const void* __restrict__ gamma, float* __restrict__ unscale,
+                                                          float* __restrict__ ssq, Touch touch)
 {
     static_assert(XT == 1 || XT == 2, "bf16 or fp32 activations");
-    if ((int)blockIdx.x >= touch.first_group) {
-        touch_weights(touch, (int)blockIdx.x - touch.first_group, (int)threadIdx.x, 1024);
+    if ((int)blockIdx.x >= first_group) {
+        touch_weights(touch, (int)blockIdx.x - first_group, (int)threadIdx.x, 1024);
         return;
     }
     if ((int)blockIdx.x * ROWS >= M) return;                   // (rows past M; padding up to first_group)
@@ -1100,7 +1103,7 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
                 row_chunk_values<XT>(keep[i], v);
                 if (NORM) {
                     float g[8];
-                    load_gamma8_g(epi.gamma, epi.gamma_dt, c * 8, g);
+                    load_gamma8_g(gamma, gamma_dt, c * 8, g);
 #pragma unroll
                     for (int e = 0; e < 8; e++) {
                         sq = fmaf(v[e], v[e], sq);
@@ -1144,7 +1147,7 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
         row_chunk_values<XT>(ch, v);
         if (NORM) {
             float g[8];
-            load_gamma8_g(epi.gamma, epi.gamma_dt, min(c, K8 - 1) * 8, g);
+            load_gamma8_g(gamma, gamma_dt, min(c, K8 - 1) * 8, g);
 #pragma unroll
             for (int e = 0; e < 8; e++) v[e] *= g[e];
         }
@@ -1335,7 +1338,7 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
             // elements, 16384 with two rows per workgroup, 32768 with one
             const int per_row = 16 / stage_rows, batches = ((K8 + 63) / 64 + per_row - 1) / per_row;
 #define CYBQ_STAGE_ROWS(XT, NORM, CH, ROWS) \
-    hipLaunchKernelGGL((stage_rows_kernel<XT, NORM, CH, ROWS>), rgrid, dim3(1024), 0, st, xs, xst, mc, w.K, epi, ssq_part, unscale, touch)
+    hipLaunchKernelGGL((stage_rows_kernel<XT, NORM, CH, ROWS>), rgrid, dim3(1024), 0, st, xs, xst, mc, w.K, touch.first_group, epi.gamma_dt, epi.gamma, unscale, ssq_part, touch)
 #define CYBQ_STAGE_ROWS_CH(XT, NORM, ROWS, C1, C2, C3)              \
     do {                                                            \
         if (batches <= C1) CYBQ_STAGE_ROWS(XT, NORM, C1, ROWS);     \

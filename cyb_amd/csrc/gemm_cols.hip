@@ -94,7 +94,7 @@ struct ColsShape {
 template <int BITS, int MODE, int RB, int CS, int KH, bool RAW>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_cols_kernel(
     const uint8_t* __restrict__ wbase, const uint8_t* __restrict__ x, int KT_, int NT, int x_row_blocks, int M, int n_tiles, int m_tiles,
-    int splits, int kt_per_split, int groups, int N, void* __restrict__ y, int ydt, int K, float* __restrict__ part, Epilogue epi, NormStats ns)
+    int splits, int kt_per_split, int groups, int K, int N, void* __restrict__ y, int ydt, float* __restrict__ part, Epilogue epi, NormStats ns)
 {
     using S = ColsShape<BITS, MODE, RB, CS, KH>;
     constexpr int NX = S::NX, NW = S::NW, XC = S::XCOPIES, WC = S::WCOPIES, GROUPS = S::GROUPS, WORDS = S::WORDS;
@@ -469,7 +469,7 @@ hipError_t launch_cols_t(const WeightView& w, const void* x, int M, void* y, int
     const int kt_per_split = (w.KT + splits - 1) / splits;
     const unsigned groups = (unsigned)(((int64_t)n_tiles * m_tiles * splits + 7) / 8 * 8);
     hipLaunchKernelGGL((gemm_cols_kernel<BITS, MODE, RB, CS, KH, RAW>), dim3(groups), dim3(512), S::LDS, st, w.base, static_cast<const uint8_t*>(x),
-                       w.KT, w.NT, (M + 15) / 16, M, n_tiles, m_tiles, splits, kt_per_split, (int)groups, w.N, y, ydt, w.K, part, epi, ns);
+                       w.KT, w.NT, (M + 15) / 16, M, n_tiles, m_tiles, splits, kt_per_split, (int)groups, w.K, w.N, y, ydt, part, epi, ns);
     return hipGetLastError();
 }
 
