@@ -55,28 +55,33 @@ namespace {
 
 #include "gemm_parts.h"
 
-// gamma[k0 .. k0+8) as fp32 (k0 a multiple of 8, gamma 16-byte aligned)
-__device__ __forceinline__ void load_gamma8_g(const void* g, int gdt, int k0, float out[8])
+// gamma[k0 .. k0+8) (k0 a multiple of 8, gamma 16-byte aligned) as loaded: two loads whatever its type, so that a kernel can ask for it next
+// to its rows without a branch around the loads (16-bit types: the second repeats the first), and as fp32
+struct Gamma8 {
+    u32x4_t v[2];
+};
+
+__device__ __forceinline__ Gamma8 load_gamma8(const void* g, int gdt, int k0)
+{
+    const char* const p = static_cast<const char*>(g) + (int64_t)k0 * (gdt == kF32 ? 4 : 2);
+    return {{*reinterpret_cast<const u32x4_t*>(p), *reinterpret_cast<const u32x4_t*>(p + (gdt == kF32 ? 16 : 0))}};
+}
+
+__device__ __forceinline__ void gamma8_values(const Gamma8& c, int gdt, float out[8])
 {
     if (gdt == kF32) {
-        const float4_t* p = reinterpret_cast<const float4_t*>(reinterpret_cast<const float*>(g) + k0);
-        const float4_t a = p[0], b = p[1];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            out[i] = a[i];
-            out[4 + i] = b[i];
-        }
+        for (int i = 0; i < 8; i++) out[i] = __builtin_bit_cast(float, (uint32_t)c.v[i >> 2][i & 3]);
     } else {
-        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint16_t*>(g) + k0);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             if (gdt == kF16) {
-                const half2_t h = as_h2(v[i]);
+                const half2_t h = as_h2(c.v[0][i]);
                 out[2 * i] = (float)h.x;
                 out[2 * i + 1] = (float)h.y;
             } else {
-                out[2 * i] = __builtin_bit_cast(float, v[i] << 16);
-                out[2 * i + 1] = __builtin_bit_cast(float, v[i] & 0xffff0000u);
+                out[2 * i] = __builtin_bit_cast(float, c.v[0][i] << 16);
+                out[2 * i + 1] = __builtin_bit_cast(float, c.v[0][i] & 0xffff0000u);
             }
         }
     }
@@ -961,6 +966,8 @@ __global__ __launch_bounds__(256) void stage_x_kernel(const u32x4_t* __restrict_
     const int rb = blockIdx.x;
     const int c0 = blockIdx.y * (kStageGroups * 4);     // first 16 B chunk of the row handled here
     const int t = threadIdx.x;
+    Gamma8 graw = {};
+    if (NORM) graw = load_gamma8(epi.gamma, epi.gamma_dt, min(c0 + (t & 63), K8 - 1) * 8);
 #pragma unroll
     for (int it = 0; it < 4; it++) {
         const int r = it * 4 + (t >> 6), c = c0 + (t & 63);
@@ -972,7 +979,7 @@ __global__ __launch_bounds__(256) void stage_x_kernel(const u32x4_t* __restrict_
             float sq = 0.f;
             if (c < K8) {
                 float g[8];
-                load_gamma8_g(epi.gamma, epi.gamma_dt, c * 8, g);
+                gamma8_values(graw, epi.gamma_dt, g);
 #pragma unroll
                 for (int p = 0; p < 4; p++) {
                     float v0, v1;
@@ -1076,7 +1083,7 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
     __shared__ float amax_part[ROWS][PW];
     __shared__ float sq_part[ROWS][PW];
     const int rb = (int)blockIdx.x * ROWS >> 4, r0 = (int)blockIdx.x * ROWS & 15;      // row block, first of this workgroup's rows in it
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
     const int r = wv % ROWS, part = wv / ROWS;                           // my row of the workgroup's, my part of the row
     const int64_t row = min(rb * 16 + r0 + r, M - 1);      // (rows past M repeat the last one and are never read back)
     const int K8 = K >> 3, G = K8 >> 2;
@@ -1084,35 +1091,50 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
     const bool resident = pieces <= PW * CH;
 
     // ---- the row's largest magnitude (and sum of squares)
+    // What the pass waits for is latency: rows and gamma are asked for together and without branches, two pieces share a barrier on their way out.  us per
+    // call with its multiply, before / after, bf16: 4096 -> 1024 with a norm at 512 rows 20.5 / 20.4, 14336 -> 1024 at 512 rows 35.7 / 35.4 (other boxes 34.3), Q8
+    // 14336 -> 4096 at 2048 rows 209.7 / 204.9, 8192 -> 1024 with a norm at 300 rows 26.2 / 25.6, 4096 -> 28672 norm + SwiGLU at 45 rows 24.2 / 23.1.
+    // Pieces past the end of the row are its last chunk again (no branches around the loads); gamma stays with a piece where there are registers
+    // for it - elsewhere it is loaded again for the conversion - and is asked for next to it.
     RowChunk<XT> keep[CH];
+    constexpr bool GKEEP = CH * XT <= 4;
+    Gamma8 gk[NORM && GKEEP ? CH : 1];
+    auto chunk_at = [&](int p0, int i) { return (p0 + i * PW + part) * 64 + lane; };
+    auto load = [&](int p0) {
+#pragma unroll
+        for (int i = 0; i < CH; i++) keep[i] = load_row_chunk<XT>(src, row, K, min(chunk_at(p0, i), K8 - 1));
+        if constexpr (NORM && GKEEP) {
+#pragma unroll
+            for (int i = 0; i < CH; i++) gk[i] = load_gamma8(gamma, gamma_dt, min(chunk_at(p0, i), K8 - 1) * 8);
+        }
+    };
+    auto scaled = [&](int i, int c, float v[8]) {
+        float g[8];
+        gamma8_values(GKEEP ? gk[GKEEP ? i : 0] : load_gamma8(gamma, gamma_dt, min(c, K8 - 1) * 8), gamma_dt, g);
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] *= g[e];
+    };
     // (a folded norm's sum of squares is formed in an order that goes with PW = 4: the launcher keeps to it)
     static_assert(!NORM || ROWS == 4, "one order for the sums of squares");
     float amax = 0.f, sq = 0.f;
     for (int p0 = 0; p0 < pieces; p0 += PW * CH) {
+        load(p0);
 #pragma unroll
         for (int i = 0; i < CH; i++) {
-            const int piece = p0 + i * PW + part;
-            if (piece < pieces) keep[i] = load_row_chunk<XT>(src, row, K, min(piece * 64 + lane, K8 - 1));
-        }
-#pragma unroll
-        for (int i = 0; i < CH; i++) {
-            const int piece = p0 + i * PW + part;
-            const int c = piece * 64 + lane;
+            const int c = chunk_at(p0, i);
+            if (p0 + i * PW + part >= pieces) break;
             float v[8];
-            if (piece < pieces && c < K8) {
-                row_chunk_values<XT>(keep[i], v);
-                if (NORM) {
-                    float g[8];
-                    load_gamma8_g(gamma, gamma_dt, c * 8, g);
+            row_chunk_values<XT>(keep[i], v);
+            if (NORM) {
 #pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        sq = fmaf(v[e], v[e], sq);
-                        v[e] *= g[e];
-                    }
+                for (int e = 0; e < 8; e++) {
+                    const float x = c < K8 ? v[e] : 0.f;
+                    sq = fmaf(x, x, sq);
                 }
-#pragma unroll
-                for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
+                scaled(i, c, v);
             }
+#pragma unroll
+            for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
         }
     }
 #pragma unroll
@@ -1141,45 +1163,35 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
         if (NORM) ssq[row] = sq;
     }
 
-    // ---- scale, round to f16, through LDS into operand order (two tiles per part: one barrier per piece)
-    auto convert = [&](const RowChunk<XT>& ch, int c) {
-        float v[8];
-        row_chunk_values<XT>(ch, v);
-        if (NORM) {
-            float g[8];
-            load_gamma8_g(gamma, gamma_dt, min(c, K8 - 1) * 8, g);
-#pragma unroll
-            for (int e = 0; e < 8; e++) v[e] *= g[e];
-        }
-        Frag16 a;
-#pragma unroll
-        for (int p = 0; p < 4; p++) {
-            const half2_t h = {(_Float16)(v[2 * p] * s), (_Float16)(v[2 * p + 1] * s)};
-            a.u[p] = as_u32(h);
-        }
-        return a.u;
-    };
+    // ---- scale, round to f16, through LDS into operand order, two pieces at a time (one to each of a part's tiles)
     const int tp = r * 64 + lane;                           // my place among the threads of my part
     const int gl = tp / (4 * ROWS), oct = tp / ROWS & 3, rr = tp % ROWS;  // when writing out: group within the piece, k octet, row
-    int round = 0;
     for (int p0 = 0; p0 < pieces; p0 += PW * CH) {
-        if (!resident) {
+        if (!resident) load(p0);
 #pragma unroll
-            for (int i = 0; i < CH; i++) {
-                const int piece = p0 + i * PW + part;
-                if (piece < pieces) keep[i] = load_row_chunk<XT>(src, row, K, min(piece * 64 + lane, K8 - 1));
-            }
-        }
+        for (int i0 = 0; i0 < CH; i0 += 2) {
+            if (p0 + i0 * PW < pieces) {                     // (uniform over the workgroup: some part has this piece)
+                if (p0 + i0 > 0) __syncthreads();            // (the tiles have been read)
 #pragma unroll
-        for (int i = 0; i < CH; i++) {
-            if (p0 + i * PW < pieces) {                      // (uniform over the workgroup: some part has this piece)
-                const int piece = p0 + i * PW + part;
-                u32x4_t* tl = tile[part][round & 1];
-                if (piece < pieces) tl[r * kStagePitch + lane] = convert(keep[i], piece * 64 + lane);
+                for (int i = i0; i < i0 + 2 && i < CH; i++) {
+                    if (p0 + i * PW + part >= pieces) break;
+                    float v[8];
+                    row_chunk_values<XT>(keep[i], v);
+                    if (NORM) scaled(i, chunk_at(p0, i), v);
+                    Frag16 a;
+#pragma unroll
+                    for (int p = 0; p < 4; p++) {
+                        const half2_t h = {(_Float16)(v[2 * p] * s), (_Float16)(v[2 * p + 1] * s)};
+                        a.u[p] = as_u32(h);
+                    }
+                    tile[part][i - i0][r * kStagePitch + lane] = a.u;
+                }
                 __syncthreads();
-                const int g = piece * 16 + gl;
-                if (piece < pieces && g < G) dst[((int64_t)rb * G + g) * 64 + oct * 16 + r0 + rr] = tl[rr * kStagePitch + gl * 4 + oct];
-                round++;
+#pragma unroll
+                for (int i = i0; i < i0 + 2 && i < CH; i++) {
+                    const int g = (p0 + i * PW + part) * 16 + gl;
+                    if (g < G) dst[((int64_t)rb * G + g) * 64 + oct * 16 + r0 + rr] = tile[part][i - i0][rr * kStagePitch + gl * 4 + oct];
+                }
             }
         }
     }

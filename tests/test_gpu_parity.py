@@ -2006,6 +2006,28 @@ def test_folded_rmsnorm_very_long_k(backend, oracle, M, xdt, gdt):
     assert oracle.rel_l2(y.cpu().numpy(), _norm_ref(oracle, q, s, x, gamma, 1e-6, xdt)) < TIGHT
 
 
+@pytest.mark.parametrize("xdt,gdt", [("bf16", "f16"), ("bf16", "f32"), ("f32", "bf16")])
+@pytest.mark.parametrize("K", [32, 512, 544, 2048, 2080, 4128, 8224, 16416])
+def test_row_scaling_pass_at_the_edges_of_its_pieces(backend, oracle, K, xdt, gdt):
+    # pieces of 512 k, shared out to a row's waves: fewer pieces than waves, a last piece of one group, one more than all
+    # waves hold in a round, rows that do not stay in registers; with a folded norm and without (other rows per workgroup)
+    M, N, eps = 37, 48, 1e-5
+    q, s = _quant(oracle, 4, N, K, cfg=48)
+    qw = backend.upload_quantized(q, s, 4)
+    x = _x(M, K, xdt)
+    x[1] *= 1e-6                                       # another power of two, another rstd
+    gamma = (1.0 + 0.25 * torch.from_numpy(synth.activations(55, 1, K)[0])).cuda().to(TDT[gdt])
+    y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    backend.matmul_norm(qw, x, gamma, eps, y)
+    plain = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    backend.matmul(qw, x, plain)
+    torch.cuda.synchronize()
+    assert oracle.rel_l2(y.cpu().numpy(), _norm_ref(oracle, q, s, x, gamma, eps, "f32")) < 2 * FAST     # x * gamma and scale * q rounded
+    ref = oracle.matmul_f64(q, s, x.double().cpu().numpy())
+    got = plain.cpu().numpy()
+    assert oracle.rel_l2(got, ref) < FAST and oracle.rel_l2(got[1:2], ref[1:2]) < FAST
+
+
 @pytest.mark.parametrize("M", [1, 2, 4, 16])
 def test_folded_rmsnorm_counts_subnormal_inputs(backend, oracle, M):
     # a row of f16 subnormals (|x| < 6.1e-5) with an eps far below its mean square: its squares must
