@@ -364,7 +364,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // for every weight tile requested before them, and a first touch in HBM holds the matrix pipe
 // up; here the multiplying waves never wait for HBM.  Waves are dealt to the four SIMDs in turn,
 // so every SIMD carries one staging wave: the dequantisation runs in the issue slots the MFMAs
-// leave free.  MW*MF*16 x NF*16 outputs per workgroup, one barrier per K tile, no K split.
+// leave free.  MW*MF*16 x NF*16 outputs per workgroup, one barrier per K tile.  SPLIT: K over workgroups, partial sums as in gemm_kernel.
 template <int I, int N, class F>
 __device__ __forceinline__ void static_for(F&& f)
 {
@@ -374,10 +374,11 @@ __device__ __forceinline__ void static_for(F&& f)
     }
 }
 
-template <int BITS, int NF, int MF, int MW, int XD>
+template <int BITS, int NF, int MF, int MW, int XD, bool SPLIT>
 __global__ __launch_bounds__((MW + 4) * 64) __attribute__((amdgpu_waves_per_eu((MW + 7) / 4, (MW + 7) / 4))) void gemm_roles_kernel(
     const uint8_t* __restrict__ wbase, const u32x4_t* __restrict__ x, int KT_, int NT_, int x_row_blocks, int M, int n_tiles,
-    int m_tiles, int groups, int K_, int N_, void* __restrict__ y, int ydt, float out_scale, Epilogue epi, NormStats ns)
+    int m_tiles, int groups, int K_, int splits, int kt_per_split, int N_, void* __restrict__ y, int ydt, float out_scale, float* __restrict__ part,
+    Epilogue epi, NormStats ns)
 {
     const WeightView w = {wbase, N_, K_, NT_, KT_, BITS};
     constexpr int SW = 4;                             // staging waves
@@ -393,16 +394,19 @@ __global__ __launch_bounds__((MW + 4) * 64) __attribute__((amdgpu_waves_per_eu((
 
     const int per_xcd = groups >> 3;                  // (same tile order as gemm_kernel)
     const int item = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
-    if (item >= n_tiles * m_tiles) return;
-    const int tile_m = item / n_tiles, tile_n = item - tile_m * n_tiles;
+    if (item >= n_tiles * m_tiles * (SPLIT ? splits : 1)) return;
+    const int row = item / n_tiles, tile_n = item - row * n_tiles;
+    const int split = SPLIT ? row / m_tiles : 0, tile_m = row - split * m_tiles;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nt0 = tile_n * NF;
-    const int KT = w.KT, K = w.K;
+    const int K = w.K;
+    const int kt_lo = SPLIT ? split * kt_per_split : 0;              // my K tiles: [kt_lo, kt_lo + KT)
+    const int KT = SPLIT ? min(kt_per_split, w.KT - kt_lo) : w.KT;
     const int kt0 = tile_n % KT;
     auto rot = [&](int kt) {
         const int r = min(kt, KT - 1) + kt0;
-        return r >= KT ? r - KT : r;
+        return kt_lo + (r >= KT ? r - KT : r);
     };
 
     if (wave >= MW) {
@@ -562,6 +566,12 @@ __global__ __launch_bounds__((MW + 4) * 64) __attribute__((amdgpu_waves_per_eu((
             if (kt + 3 < KT) k_tile(kt + 3, std::integral_constant<int, 3>{});
         }
     }
+    if constexpr (SPLIT) {
+        const Epilogue plain = {kEpiNone, nullptr, nullptr, 0, 0.f};
+        write_rows<MF, NF>(acc, reinterpret_cast<float*>(smem) + wave * (16 * NF * 16), m0, nt0, M, w.N, part + (int64_t)split * M * w.N, kF32, 1.0f, plain,
+                           lane);
+        return;
+    }
     if (epi.gamma || ns.unscale) {
         const float mine = row_factor(stats, ns, epi.gamma != nullptr, min(m0 + min(lane, MF * 16 - 1), M - 1), K, epi.eps);
 #pragma unroll
@@ -588,21 +598,6 @@ __global__ __launch_bounds__((MW + 4) * 64) __attribute__((amdgpu_waves_per_eu((
         }
     }
     write_rows<MF, NF>(acc, reinterpret_cast<float*>(smem) + wave * (16 * NF * 16), m0, nt0, M, w.N, y, ydt, out_scale, epi, lane);
-}
-
-template <int BITS, int NF, int MF, int MW, int XD>
-hipError_t launch_roles(const WeightView& w, const void* x, int M, void* y, int ydt, float out_scale, const Epilogue& epi,
-                        const NormStats& ns, hipStream_t st)
-{
-    constexpr int lds = 2 * NF * (4 * 64) * 16;
-    constexpr int BM = MW * MF * 16;
-    (void)LdsRequest<&gemm_roles_kernel<BITS, NF, MF, MW, XD>, lds>::registered;
-    const int n_tiles = (w.NT + NF - 1) / NF, m_tiles = (M + BM - 1) / BM;
-    const unsigned groups = (unsigned)(((int64_t)n_tiles * m_tiles + 7) / 8 * 8);
-    hipLaunchKernelGGL((gemm_roles_kernel<BITS, NF, MF, MW, XD>), dim3(groups), dim3((MW + 4) * 64), lds, st, w.base,
-                       reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT, (M + 15) / 16, M, n_tiles, m_tiles, (int)groups, w.K, w.N, y, ydt,
-                       out_scale, epi, ns);
-    return hipGetLastError();
 }
 
 constexpr int kMaxSplits = 8;
@@ -760,6 +755,23 @@ hipError_t launch_reduce(const float* part, int splits, int M, int N, void* y, i
     return hipGetLastError();
 }
 
+template <int BITS, int NF, int MF, int MW, int XD, bool SPLIT = false>
+hipError_t launch_roles(const WeightView& w, const void* x, int M, void* y, int ydt, float out_scale, const Epilogue& epi,
+                        const NormStats& ns, hipStream_t st, float* part = nullptr, int splits = 1)
+{
+    constexpr int lds = 2 * NF * (4 * 64) * 16;
+    constexpr int BM = MW * MF * 16;
+    (void)LdsRequest<&gemm_roles_kernel<BITS, NF, MF, MW, XD, SPLIT>, lds>::registered;
+    const int n_tiles = (w.NT + NF - 1) / NF, m_tiles = (M + BM - 1) / BM;
+    const unsigned groups = (unsigned)(((int64_t)n_tiles * m_tiles * splits + 7) / 8 * 8);
+    hipLaunchKernelGGL((gemm_roles_kernel<BITS, NF, MF, MW, XD, SPLIT>), dim3(groups), dim3((MW + 4) * 64), lds, st, w.base,
+                       reinterpret_cast<const u32x4_t*>(x), w.KT, w.NT, (M + 15) / 16, M, n_tiles, m_tiles, (int)groups, w.K, splits,
+                       (w.KT + splits - 1) / splits, w.N, y, ydt, out_scale, part, epi, ns);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || !SPLIT) return e;
+    return launch_reduce(part, splits, M, w.N, y, ydt, out_scale, epi, ns, w.K, st);
+}
+
 template <int BITS, int XBF, int NF, bool EXACT, int MF>
 hipError_t launch_m(const WeightView& w, const void* x, int M, void* y, int ydt, float out_scale, float* part, int splits, const Epilogue& epi,
                     const NormStats& ns, hipStream_t st)
@@ -779,7 +791,7 @@ hipError_t launch_m(const WeightView& w, const void* x, int M, void* y, int ydt,
 }
 
 // What multiplies a staged chunk of M rows.
-//   kRoles   gemm_roles_kernel, mw multiplying waves (32 rows each), nf column blocks, no K split
+//   kRoles   gemm_roles_kernel, mw multiplying waves (32 rows each), nf column blocks, with eight of them K split over `splits` workgroups
 //   kTiles   gemm_kernel, mf row blocks per wave (256 or 512 rows), nf column blocks, K split over `splits` workgroups
 //   kCols    gemm_cols_kernel (gemm_cols.hip)
 struct TilePlan {
@@ -861,6 +873,11 @@ static float tiled_plan(const WeightView& w, int M, bool exact, int num_cus, siz
     const int per = (w.KT + splits - 1) / splits;
     splits = (w.KT + per - 1) / per;                             // no empty split
     plan = {TilePlan::kTiles, nf, 8, 2, splits, {}};
+    // Their K ranges go to the role-split kernel where they are long and there are three of them or up to three row tiles; the bits are the same.  us per
+    // call, gemm_kernel / role-split: 14336 -> 4096 at 512 rows 68.5 / 66.3, Q8 70.6 / 68.8, 10240 -> 3136 at 512 rows 46.3 / 44.9, 12288 -> 8192 at 256 rows
+    // 59.4 / 57.9, Q8 11168 -> 2145 at 1020 rows 69.3 / 65.2.  Two ranges of more row tiles: 14336 -> 4096 at 1000 rows 121.3 / 123.0, 5760 -> 1959 at 1551 rows
+    // 54.2 / 54.9; short ranges: Q8 14336 -> 1024 at 700 rows (14 K tiles) 39.4 / 40.0.
+    if (!exact && splits > 1 && per >= 16 && (splits >= 3 || M <= 768)) plan.kind = TilePlan::kRoles;
     const float rounds = (float)((tiles * splits + cus - 1) / cus);
     // (EXACT: fits to 254 calls of 33 .. 2048 rows on N of 256 .. 32768, 10 - 12 % rms, taken when gemm_cols.hip went over to integer operands; with
     // the lines from before, 0.9 + 2.75 per K tile, wide outputs of a short K and the odd large call stayed here that are quicker there.  us per
@@ -901,6 +918,10 @@ hipError_t launch_tiles(const TilePlan& p, const WeightView& w, const void* x, b
     }
     if constexpr (XBF == 0) {       // FAST multiplies in f16: bf16 activations were widened by the staging pass
         if (p.kind == TilePlan::kRoles) {
+            if (p.splits > 1) {
+                if (p.nf == 7) return launch_roles<BITS, 7, 2, 8, 2, true>(w, x, M, y, ydt, out_scale, epi, ns, st, part, p.splits);
+                return launch_roles<BITS, 8, 2, 8, 2, true>(w, x, M, y, ydt, out_scale, epi, ns, st, part, p.splits);
+            }
             if (p.mw == 8 && p.nf == 7) return launch_roles<BITS, 7, 2, 8, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
             if (p.mw == 8) return launch_roles<BITS, 8, 2, 8, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);
             if (p.mw == 4 && p.nf == 8) return launch_roles<BITS, 8, 2, 4, 2>(w, x, M, y, ydt, out_scale, epi, ns, st);

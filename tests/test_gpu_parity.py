@@ -2006,6 +2006,30 @@ def test_folded_rmsnorm_very_long_k(backend, oracle, M, xdt, gdt):
     assert oracle.rel_l2(y.cpu().numpy(), _norm_ref(oracle, q, s, x, gamma, 1e-6, xdt)) < TIGHT
 
 
+@pytest.mark.parametrize("bits,N,K,M,ydt", [(4, 100, 16416, 257, "f32"), (4, 112, 16384, 300, "bf16"), (8, 130, 17000 // 32 * 32, 513, "f16"),
+                                            (8, 224, 18432, 256, "f32"), (4, 2050, 6176, 200, "f32")])
+def test_role_split_kernel_over_ranges_of_k(backend, oracle, bits, N, K, M, ydt):
+    # K ranges of 16 tiles and more, a shorter last one, a padded last tile, row and column tiles that are not full, tiles of seven and
+    # eight column blocks; with a residual, and the same twice over
+    q, s = _quant(oracle, bits, N, K, cfg=49)
+    qw = backend.upload_quantized(q, s, bits)
+    x = _x(M, K, "bf16")
+    r = torch.from_numpy(synth.activations(56, M, N)).cuda().to(TDT[ydt])
+    y = torch.full((M, N), float("nan"), dtype=TDT[ydt], device="cuda")
+    y2 = torch.empty_like(y)
+    backend.set_gemm_tuning(2)          # (the tiled kernels alone: small outputs are other kernels' otherwise)
+    try:
+        backend.matmul_ex(qw, x, y, "add", r)
+        backend.matmul_ex(qw, x, y2, "add", r)
+        torch.cuda.synchronize()
+    finally:
+        backend.set_gemm_tuning(0)
+    ref = oracle.matmul_f64(q, s, x.double().cpu().numpy()) + r.double().cpu().numpy()
+    rounding = {"f32": 0.0, "f16": 5e-4, "bf16": 4e-3}[ydt]      # of the result
+    assert oracle.rel_l2(y.double().cpu().numpy(), ref) < FAST + rounding
+    assert torch.equal(y, y2)
+
+
 @pytest.mark.parametrize("xdt,gdt", [("bf16", "f16"), ("bf16", "f32"), ("f32", "bf16")])
 @pytest.mark.parametrize("K", [32, 512, 544, 2048, 2080, 4128, 8224, 16416])
 def test_row_scaling_pass_at_the_edges_of_its_pieces(backend, oracle, K, xdt, gdt):
