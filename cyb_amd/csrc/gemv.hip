@@ -800,6 +800,31 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
     // (slot = strip * MB + row block)
     float* red = reinterpret_cast<float*>(smem);
     const int sums = SUMS * nwaves;
+    // wave v finishes outputs v, v + waves, ...: number p is register p % 4 of row block p / 4 % MB of strip p / 4 / MB
+    // Their residuals are asked for before the waves' sums meet, and the outputs a wave finishes are walked without a loop, so that their reads go out
+    // together.  us per call, before / after: 14336 -> 4096 at 16 f16 rows 11.8 / 11.4, with a residual 11.9 / 11.7, at 30 rows 16.1 / 15.4, a list of
+    // 16 layers at 16 rows 741 / 733; at 8 rows the same.
+    constexpr int OUTS = NS * MB * 4, AHEAD_OUTS = (OUTS + 7) / 8;
+    auto place = [&](int p, int64_t& at) __attribute__((always_inline)) {
+        const int r = p & 3, b = (p >> 2) % MB, nt = strip0 + (p >> 2) / MB;
+        const int n = nt * 16 + (lane & 15), m = 16 * b + 4 * oct + r;
+        at = (int64_t)m * w.N + n;
+        return p < OUTS && nt < w.NT && m < M && n < w.N;
+    };
+    uint32_t residual[AHEAD_OUTS] = {};
+    if (epi.kind == kEpiAdd) {
+#pragma unroll
+        for (int k = 0; k < AHEAD_OUTS; k++) {
+            int64_t at;
+            if (place(wv + k * nwaves, at)) residual[k] = load_out_bits(epi.residual, ydt, at);
+        }
+    }
+    auto finish = [&](int p, float v, uint32_t bits) __attribute__((always_inline)) {
+        int64_t at;
+        if (!place(p, at)) return;
+        if (epi.kind == kEpiAdd) v += out_value(bits, ydt);
+        store_out(y, ydt, at, v);
+    };
 #pragma unroll
     for (int s = 0; s < NS; s++)
 #pragma unroll
@@ -874,7 +899,6 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
         return;
     }
     if constexpr (KS) {
-        constexpr int OUTS = NS * MB * 4;                 // output registers of a workgroup, 64 lanes each
         const int groups = (int)gridDim.x / splits;
         float* mine = slabs + ((size_t)split * groups + group) * (OUTS * 64);
         for (int p = wv; p < OUTS; p += nwaves) {
@@ -895,8 +919,7 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
         if (*flag == 0u) return;
         const size_t slab_stride = (size_t)groups * (OUTS * 64);
         const float* first = slabs + (size_t)group * (OUTS * 64);
-        for (int p = wv; p < OUTS; p += nwaves) {
-            const int r = p & 3, b = (p >> 2) % MB, s = (p >> 2) / MB;
+        auto whole = [&](int p) __attribute__((always_inline)) {
             float part[4];                                 // (at most four splits: rows_split_plan)
 #pragma unroll
             for (int k = 0; k < 4; k++)
@@ -905,20 +928,29 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
             float v = part[0];
 #pragma unroll
             for (int k = 1; k < 4; k++) v += k < splits ? part[k] : 0.f;
-            const int nt = strip0 + s;
-            const int n = nt * 16 + (lane & 15);
-            const int m = 16 * b + 4 * oct + r;
-            if (nt < w.NT && m < M && n < w.N) emit(y, ydt, epi, (int64_t)m * w.N + n, v);
+            return v;
+        };
+#pragma unroll
+        for (int k = 0; k < AHEAD_OUTS; k++)
+            if (wv + k * nwaves < OUTS) finish(wv + k * nwaves, whole(wv + k * nwaves), residual[k]);
+        for (int p = wv + AHEAD_OUTS * nwaves; p < OUTS; p += nwaves) {
+            int64_t at;
+            const bool mine = place(p, at) && epi.kind == kEpiAdd;
+            finish(p, whole(p), mine ? load_out_bits(epi.residual, ydt, at) : 0u);
         }
         return;
     }
-    for (int p = wv; p < NS * MB * 4; p += nwaves) {
+    auto whole = [&](int p) __attribute__((always_inline)) {
         const int r = p & 3, b = (p >> 2) % MB, s = (p >> 2) / MB;
-        const int nt = strip0 + s;
-        const int n = nt * 16 + (lane & 15);
-        const float v = sum_partials(red + ((s * MB + b) * sums * 4 + r) * 64 + lane, sums, 4 * 64) * rstd[r];
-        const int m = 16 * b + 4 * oct + r;
-        if (nt < w.NT && m < M && n < w.N) emit(y, ydt, epi, (int64_t)m * w.N + n, v);
+        return sum_partials(red + ((s * MB + b) * sums * 4 + r) * 64 + lane, sums, 4 * 64) * rstd[r];
+    };
+#pragma unroll
+    for (int k = 0; k < AHEAD_OUTS; k++)
+        if (wv + k * nwaves < OUTS) finish(wv + k * nwaves, whole(wv + k * nwaves), residual[k]);
+    for (int p = wv + AHEAD_OUTS * nwaves; p < OUTS; p += nwaves) {            // (fewer than eight waves)
+        int64_t at;
+        const bool mine = place(p, at) && epi.kind == kEpiAdd;
+        finish(p, whole(p), mine ? load_out_bits(epi.residual, ydt, at) : 0u);
     }
 }
 

@@ -41,6 +41,18 @@ __device__ __forceinline__ float load_out(const void* p, int dt, int64_t idx)
     return __builtin_bit_cast(float, (uint32_t)reinterpret_cast<const uint16_t*>(p)[idx] << 16);
 }
 
+// the same in two steps, to ask for an element ahead of its use: its bits, and their value
+__device__ __forceinline__ uint32_t load_out_bits(const void* p, int dt, int64_t idx)
+{
+    if (dt == kF32) return reinterpret_cast<const uint32_t*>(p)[idx];
+    return reinterpret_cast<const uint16_t*>(p)[idx];
+}
+
+__device__ __forceinline__ float out_value(uint32_t bits, int dt)
+{
+    return dt == kF32 ? __builtin_bit_cast(float, bits) : dt == kF16 ? f16_bits_to_f32(bits) : __builtin_bit_cast(float, bits << 16);
+}
+
 // one finished output element: residual add (fp32, before the single rounding to ydt), store
 __device__ __forceinline__ void emit(void* y, int ydt, const Epilogue& epi, int64_t idx, float v)
 {
