@@ -98,6 +98,7 @@ def load_library() -> ctypes.CDLL:
     lib.cybq_quantize.argtypes = [vp, ci, vp, i64, i64, vp, vp, vp]
     # diagnostics (cyb_amd/csrc/cybq_debug.h), not part of the operator interface
     lib.cybq_debug_set_gemm_tuning.argtypes = [ci]
+    lib.cybq_debug_prefill_plan.argtypes = [vp, vp, ci, i64, ci, ci, ctypes.POINTER(ci)]
     lib.cybq_debug_set_gemv_tuning.argtypes = [ci, ci, ci]
     lib.cybq_debug_read_weight.argtypes = [vp, i64, vp, ci, vp, vp, vp]
     lib.cybq_debug_read_pattern.argtypes = [vp, i64, vp, ci, vp]
@@ -524,8 +525,15 @@ class Backend:
 
     def set_gemm_tuning(self, rows_kernel: int = 0) -> None:
         """Experiments only: 2 leaves FAST-mode prefill calls to the tiled kernels, 3 those of both modes, 1 sends calls of
-        up to 64 rows to the K-splitting kernel whatever the output width, 4 has all rows staged before the multiply, 0 restores the automatic choice."""
+        up to 64 rows to the K-splitting kernel whatever the output width, 4 has all rows staged before the multiply, 7 is 2 with K ranges in the
+        first tiled kernel whatever their length, 0 restores the automatic choice."""
         self._lib.cybq_debug_set_gemm_tuning(rows_kernel)
+
+    def debug_prefill_plan(self, w: QWeight, xdt: int, M: int, norm: bool = False, epilogue: str = "none") -> dict:
+        """Diagnostics: what the prefill path does with such a call (cybq_debug.h)."""
+        plan = (ctypes.c_int * 4)()
+        self._check(self._lib.cybq_debug_prefill_plan(self._ctx, w.handle, xdt, M, 1 if norm else 0, EPILOGUES[epilogue], plan))
+        return {"kernel": {1: "rows", 2: "tiles", 3: "roles", 4: "cols"}.get(plan[0]), "nf": plan[1], "splits": plan[2], "stage_rows": plan[3]}
 
     def set_gemv_tuning(self, waves: int = 0, rows_kernel: int = 0, unroll: int = 0) -> None:
         """Diagnostics: waves per workgroup; decode kernel choice (0 auto, 1 always the

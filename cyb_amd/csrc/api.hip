@@ -738,6 +738,23 @@ int cybq_debug_set_gemm_tuning(int rows_kernel)
     return CYBQ_OK;
 }
 
+int cybq_debug_prefill_plan(cybq_ctx* ctx, const cybq_weight* w, cybq_dtype xdt, int64_t M, int norm, cybq_epilogue epilogue, int plan[4])
+{
+    if (!ctx) return CYBQ_ERR_INVALID;
+    if (!w || !plan || !dtype_ok(xdt)) return fail(ctx, CYBQ_ERR_INVALID, "w / plan is NULL or unknown dtype");
+    if (M < 1 || M > (1 << 24)) return fail(ctx, CYBQ_ERR_SHAPE, "M must be in 1..2^24");
+    cybq::Epilogue epi = {cybq::kEpiNone, nullptr, nullptr, 0, 0.f};
+    epi.kind = epilogue == CYBQ_EPI_ADD ? cybq::kEpiAdd : epilogue == CYBQ_EPI_SWIGLU ? cybq::kEpiSwiglu : cybq::kEpiNone;
+    if (norm) epi.gamma = ctx;                      // (asked for, never read)
+    const size_t bytes = ctx->workspace_bytes > 2 * cybq::kDecodeScratchBytes ? ctx->workspace_bytes - cybq::kDecodeScratchBytes : ctx->workspace_bytes;
+    const cybq::PrefillRoute r = cybq::prefill_route(view_of(w), (int)xdt, (int)M, ctx->num_cus, ctx->prefill_exact, bytes, epi);
+    plan[0] = r.kernel;
+    plan[1] = r.nf;
+    plan[2] = r.splits;
+    plan[3] = r.stage_rows;
+    return CYBQ_OK;
+}
+
 int cybq_debug_set_gemv_tuning(int waves_per_group, int rows_kernel, int unroll)
 {
     cybq::set_gemv_tuning(waves_per_group, rows_kernel, unroll);

@@ -25,8 +25,17 @@ int cybq_debug_set_gemv_tuning(int waves_per_group, int rows_kernel, int unroll)
  * and the kernel whose waves stand side by side, by estimates), 1 the first of these for up to 64 rows whatever the width, 2 in FAST mode
  * the tiled kernels alone (on small weights at up to 64 rows two passes of the batched-rows decode kernel take the call as they do for
  * other shapes), 3 in both modes; 4: automatic, but no kernel reads rows where the caller has them, all are staged; 5: automatic, but the
- * staging launch asks for no weights ahead of the multiply; 6: automatic, it asks only ahead of the kernel whose waves split K. */
+ * staging launch asks for no weights ahead of the multiply; 6: automatic, it asks only ahead of the kernel whose waves split K; 7: as 2, and
+ * where K is split over workgroups every wave fetches, dequantises and multiplies, however long the ranges are. */
 int cybq_debug_set_gemm_tuning(int rows_kernel);
+
+/* What the prefill path does with a call of M rows (the first that fit its scratch), the tuning above included:
+ *   plan[0]  what multiplies: 1 the kernel whose waves split K, 2 the tiled kernel whose waves all do everything, 3 the one whose waves have roles, 4 the
+ *            kernel whose waves stand side by side; 0: the path does not take such calls
+ *   plan[1]  column blocks of 16 per workgroup (1 .. 3), plan[2]  workgroups that share out K
+ *   plan[3]  rows per workgroup of the pass that finds the rows' powers of two, 0: the rows do not go through it
+ * Whether a call of up to 64 rows gets to the prefill path is decided before that. */
+int cybq_debug_prefill_plan(cybq_ctx* ctx, const cybq_weight* w, cybq_dtype xdt, int64_t M, int norm, cybq_epilogue epilogue, int plan[4]);
 
 /* Ceiling probes for the one-row decode kernel: a kernel that issues exactly that kernel's
  * memory requests for tensor `w` (one workgroup per 16-row strip, whole strip requested up

@@ -80,8 +80,15 @@ ColsPlan plan_gemm_cols(const WeightView& w, int mode, int M, int num_cus, size_
 hipError_t launch_gemm_cols(const WeightView& w, const void* x, bool raw, int mode, int M, void* y, int ydt, const ColsPlan& plan, const Epilogue& epi,
                             const float* ssq_part, int ssq_blocks, const float* unscale, float* part, hipStream_t st);
 // test/bench hook: 2 = in FAST mode the tiled kernels alone (neither the few-rows kernel nor gemm_cols.hip), 3 = in both modes,
-// 1 = the few-rows kernel whatever the width, 0 = automatic
+// 1 = the few-rows kernel whatever the width, 7 = as 2 with ranges of K in gemm_kernel, 0 = automatic
 void set_gemm_tuning(int rows_kernel);
+// what launch_gemm does with the first rows of a call that fit its scratch (tests)
+struct PrefillRoute {
+    int kernel;              // what multiplies: 1 gemm_rows.hip, 2 gemm_kernel, 3 gemm_roles_kernel, 4 gemm_cols.hip; 0: launch_gemm refuses the call
+    int nf, splits;          // column blocks of 16 per workgroup (kernels 1 .. 3), workgroups that share out K (1: gemm_rows.hip's shares are not counted)
+    int stage_rows;          // rows per workgroup of the row-scaling pass, 0: the rows do not go through it
+};
+PrefillRoute prefill_route(const WeightView& w, int xdt, int M, int num_cus, bool exact, size_t workspace_bytes, const Epilogue& epi);
 // whether launch_gemm hands a FAST-mode call of M rows with this epilogue to the few-rows kernel (the hook included)
 bool gemm_rows_takes(const WeightView& w, int M, int num_cus, const Epilogue& epi);
 

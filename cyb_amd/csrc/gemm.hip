@@ -50,6 +50,7 @@
 namespace cybq {
 
 int g_rows_kernel = 0;        // (set_gemm_tuning: 2 = the tiled kernels of this file alone in FAST mode, 3 = in both modes, 1 = the few-rows kernel whatever the width)
+static bool g_role_ranges = true;     // (7 = as 2, and ranges of K stay with gemm_kernel)
 
 namespace {
 
@@ -877,7 +878,7 @@ static float tiled_plan(const WeightView& w, int M, bool exact, int num_cus, siz
     // call, gemm_kernel / role-split: 14336 -> 4096 at 512 rows 68.5 / 66.3, Q8 70.6 / 68.8, 10240 -> 3136 at 512 rows 46.3 / 44.9, 12288 -> 8192 at 256 rows
     // 59.4 / 57.9, Q8 11168 -> 2145 at 1020 rows 69.3 / 65.2.  Two ranges of more row tiles: 14336 -> 4096 at 1000 rows 121.3 / 123.0, 5760 -> 1959 at 1551 rows
     // 54.2 / 54.9; short ranges: Q8 14336 -> 1024 at 700 rows (14 K tiles) 39.4 / 40.0.
-    if (!exact && splits > 1 && per >= 16 && (splits >= 3 || M <= 768)) plan.kind = TilePlan::kRoles;
+    if (!exact && splits > 1 && per >= 16 && (splits >= 3 || M <= 768) && g_role_ranges) plan.kind = TilePlan::kRoles;
     const float rounds = (float)((tiles * splits + cus - 1) / cus);
     // (EXACT: fits to 254 calls of 33 .. 2048 rows on N of 256 .. 32768, 10 - 12 % rms, taken when gemm_cols.hip went over to integer operands; with
     // the lines from before, 0.9 + 2.75 per K tile, wide outputs of a short K and the odd large call stayed here that are quicker there.  us per
@@ -1239,7 +1240,8 @@ static bool g_raw = true;     // (4 = gemm_cols.hip reads staged rows only)
 static int g_touch = 2;       // (5 = the staging launch asks for no weights ahead of the multiply, 6 = only ahead of the few-rows kernel)
 void set_gemm_tuning(int rows_kernel)
 {
-    g_rows_kernel = rows_kernel >= 4 ? 0 : rows_kernel;
+    g_rows_kernel = rows_kernel == 7 ? 2 : rows_kernel >= 4 ? 0 : rows_kernel;
+    g_role_ranges = rows_kernel != 7;
     g_raw = rows_kernel != 4;
     g_touch = rows_kernel == 5 ? 0 : rows_kernel == 6 ? 1 : 2;
 }
@@ -1314,6 +1316,46 @@ static int64_t staged_rows(const WeightView& w, size_t workspace_bytes)
 
 bool gemm_stages(const WeightView& w, size_t workspace_bytes) { return staged_rows(w, workspace_bytes) >= 256; }
 
+// Rows per workgroup of sixteen waves: with few of them one workgroup per four rows leaves the chip idle and a
+// row's waves walk it piece after piece; with many, the shorter runs in which the operands leave cost more (64, 32, 16
+// bytes).  us per call, 4 / 2 / 1 rows, bf16 unless noted.  K over 8192: 14336 -> 4096 at 45 rows 28.0 / 26.5 / 25.8, 128 rows
+// 39.6 / 37.1 / 35.8, 160 rows 49.3 / 47.9 / 47.4, 256 rows 47.3 / 45.9 / 47.5, 300 rows 66.5 / 64.7 / 67.3, 384 rows 68.3 / 67.8 /
+// 70.9, 448 rows 69.5 / 69.6 / 73.9, 512 rows 72.6 / 73.4 / 78.6; 9216 -> 4096 at 300 / 384 rows 48.9 / 47.5 / 48.8, 49.9 / 49.4 / 51.2;
+// 10240 -> 4096 at 384 rows 53.4 / 52.9 / 54.9; 14336 -> 1024 at 384 / 512 rows 39.6 / 40.4 / 42.0, 38.0 / 39.5 / 44.6; fp32 (twice the bytes to a row), 4 / 2 rows, 14336 -> 4096 at
+// 512 / 640 rows 76.0 / 74.4, 106.9 / 107.4, 10240 -> 14336 and 9216 -> 4096 at 512 rows 134.0 / 132.8, 54.6 / 54.3.  Shorter K:
+// 8192 -> 4096 at 45 rows 18.7 / 17.2 / 17.1, at 64 rows 21.4 / 20.0 / 19.8, at 100 rows 21.8 / 21.6 / 21.6; 4096 -> 4096 at 45 rows
+// 11.2 / 10.9 / 11.3, fp32 at 24 rows 10.5 / 10.1 / 10.4; 4096 -> 14336 at 45 / 64 rows 17.2 / 17.2 / 17.6, 18.8 / 19.0 / 19.4.
+// (A folded norm: always four, one order of its sums.)
+// Eight where that makes one workgroup per CU of a second round of four-row ones: all rows go at once then, and out in whole 128-byte
+// lines.  bf16 of K up to 4096 at more than 6 and up to 8 rows per CU, us per call, 4 / 8 rows: 4096 -> 4096 at 1900 / 2048 rows 70.4 /
+// 68.8, 70.5 / 69.1, 4096 -> 1024 at 1560 / 2048 rows 31.8 / 29.8, 35.6 / 31.5 (the pass alone 15.1 / 9.7), 2048 -> 4096 44.4 / 42.9,
+// 2048 -> 1024 21.3 / 20.5, 22.7 / 21.4, 4096 -> 14336 at 2048 rows 211.6 / 211.0; 30 calls of the range on N of 256 .. 8192: 5 % in the
+// mean, none slower.  Outside: 4096 -> 1024 at 1400 / 1500 / 2100 / 2700 rows
+// 29.7 / 31.5, 30.5 / 32.6, 38.1 / 40.8, 44.2 / 45.3, 14336 -> 1024 at 3000 rows 135 / 155, fp32 4096 -> 1024 at 2048 rows 33.3 / 34.1.
+static int rows_per_staging_workgroup(const WeightView& w, int xdt, int mc, int num_cus, bool norm)
+{
+    if (!norm && xdt == kBF16 && w.K <= 4096 && mc > 6 * num_cus && mc <= 8 * num_cus) return 8;
+    if (norm) return 4;
+    if (w.K <= 8192) return mc <= 48 ? 2 : 4;
+    return mc <= 128 ? 1 : mc <= (xdt == kF32 ? 512 : 384) ? 2 : 4;
+}
+
+// What multiplies a chunk of mc rows that fits the scratch (part_bytes: its second half): the kernel of gemm_rows.hip where rows.nf is not 0, else tiles
+struct ChunkPlan {
+    RowsPlan rows;
+    TilePlan tiles;
+};
+
+static ChunkPlan plan_chunk(const WeightView& w, int xdt, int mc, int num_cus, bool exact, size_t part_bytes, const Epilogue& epi)
+{
+    ChunkPlan p = {};
+    // few rows on a wide output, FAST mode: the kernel of gemm_rows.hip (waves split K, no LDS on the way)
+    if (!exact) p.rows = rows_plan(w, mc, num_cus, epi);
+    if (!p.rows.nf && !exact && g_rows_kernel < 2) p.rows = gemm_rows_plan_long_k(w, mc, num_cus, epi);
+    if (!p.rows.nf) p.tiles = plan_tiles(w, mc, exact, exact && xdt == kBF16, num_cus, part_bytes, epi);
+    return p;
+}
+
 hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void* y, int ydt,
                        int num_cus, bool exact, void* workspace, size_t workspace_bytes, const Epilogue& epi,
                        hipStream_t st)
@@ -1342,10 +1384,9 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
         void* yc = static_cast<char*>(y) + (size_t)m_lo * n_out * ysize;
         Epilogue ec = epi;                 // this row chunk's slice of the residual
         if (epi.kind == kEpiAdd) ec.residual = static_cast<const char*>(epi.residual) + (size_t)m_lo * n_out * ysize;
-        // few rows on a wide output, FAST mode: the kernel of gemm_rows.hip (waves split K, no LDS on the way)
-        RowsPlan plan = !exact && kdt == kF16 ? rows_plan(w, mc, num_cus, ec) : RowsPlan{0};
-        if (!plan.nf && !exact && kdt == kF16 && g_rows_kernel < 2) plan = gemm_rows_plan_long_k(w, mc, num_cus, ec);
-        const TilePlan tp = plan.nf ? TilePlan{} : plan_tiles(w, mc, exact, kdt == kBF16, num_cus, half, ec);
+        const ChunkPlan chunk = plan_chunk(w, xdt, mc, num_cus, exact, half, ec);
+        const RowsPlan& plan = chunk.rows;
+        const TilePlan& tp = chunk.tiles;
         // gemm_cols.hip takes rows that are operands as they stand from where the caller has them: no staging launch (not where y is
         // written over them).  us per call with / without it, EXACT: bf16 4096 -> 14336 at 64 / 256 rows 26.8 / 23.5, 57.7 / 53.9, 512 -> 1000
         // at 100 rows 9.9 / 7.6, 7008 -> 800 at 200 rows 17.8 / 14.0, f16 4096 -> 6144 at 512 rows 51.9 / 45.6; FAST f16 14336 -> 4096 at 45 / 128
@@ -1362,24 +1403,7 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
         } else if (widen) {
             // per-row scaled f16 operands; one sum of squares per row
             ns = NormStats{ssq_part, 1, unscale};
-            // Rows per workgroup of sixteen waves: with few of them one workgroup per four rows leaves the chip idle and a
-            // row's waves walk it piece after piece; with many, the shorter runs in which the operands leave cost more (64, 32, 16
-            // bytes).  us per call, 4 / 2 / 1 rows, bf16 unless noted.  K over 8192: 14336 -> 4096 at 45 rows 28.0 / 26.5 / 25.8, 128 rows
-            // 39.6 / 37.1 / 35.8, 160 rows 49.3 / 47.9 / 47.4, 256 rows 47.3 / 45.9 / 47.5, 300 rows 66.5 / 64.7 / 67.3, 384 rows 68.3 / 67.8 /
-            // 70.9, 448 rows 69.5 / 69.6 / 73.9, 512 rows 72.6 / 73.4 / 78.6; 9216 -> 4096 at 300 / 384 rows 48.9 / 47.5 / 48.8, 49.9 / 49.4 / 51.2;
-            // 10240 -> 4096 at 384 rows 53.4 / 52.9 / 54.9; 14336 -> 1024 at 384 / 512 rows 39.6 / 40.4 / 42.0, 38.0 / 39.5 / 44.6; fp32 (twice the bytes to a row), 4 / 2 rows, 14336 -> 4096 at
-            // 512 / 640 rows 76.0 / 74.4, 106.9 / 107.4, 10240 -> 14336 and 9216 -> 4096 at 512 rows 134.0 / 132.8, 54.6 / 54.3.  Shorter K:
-            // 8192 -> 4096 at 45 rows 18.7 / 17.2 / 17.1, at 64 rows 21.4 / 20.0 / 19.8, at 100 rows 21.8 / 21.6 / 21.6; 4096 -> 4096 at 45 rows
-            // 11.2 / 10.9 / 11.3, fp32 at 24 rows 10.5 / 10.1 / 10.4; 4096 -> 14336 at 45 / 64 rows 17.2 / 17.2 / 17.6, 18.8 / 19.0 / 19.4.
-            // (A folded norm: always four, one order of its sums.)
-            // Eight where that makes one workgroup per CU of a second round of four-row ones: all rows go at once then, and out in whole 128-byte
-            // lines.  bf16 of K up to 4096 at more than 6 and up to 8 rows per CU, us per call, 4 / 8 rows: 4096 -> 4096 at 1900 / 2048 rows 70.4 /
-            // 68.8, 70.5 / 69.1, 4096 -> 1024 at 1560 / 2048 rows 31.8 / 29.8, 35.6 / 31.5 (the pass alone 15.1 / 9.7), 2048 -> 4096 44.4 / 42.9,
-            // 2048 -> 1024 21.3 / 20.5, 22.7 / 21.4, 4096 -> 14336 at 2048 rows 211.6 / 211.0; 30 calls of the range on N of 256 .. 8192: 5 % in the
-            // mean, none slower.  Outside: 4096 -> 1024 at 1400 / 1500 / 2100 / 2700 rows
-            // 29.7 / 31.5, 30.5 / 32.6, 38.1 / 40.8, 44.2 / 45.3, 14336 -> 1024 at 3000 rows 135 / 155, fp32 4096 -> 1024 at 2048 rows 33.3 / 34.1.
-            const bool eight = !epi.gamma && xdt == kBF16 && w.K <= 4096 && mc > 6 * num_cus && mc <= 8 * num_cus;
-            const int stage_rows = eight ? 8 : epi.gamma ? 4 : w.K > 8192 ? (mc <= 128 ? 1 : mc <= (xdt == kF32 ? 512 : 384) ? 2 : 4) : (mc <= 48 ? 2 : 4);
+            const int stage_rows = rows_per_staging_workgroup(w, xdt, mc, num_cus, epi.gamma != nullptr);
             dim3 rgrid((unsigned)((mc + 15) / 16) * (16 / stage_rows));
             const Touch touch = plan_touch(w, mc, num_cus, ec, exact, rgrid.x);
             // pieces of 512 k a lane keeps in registers: the whole row when it has at most 16384 (bf16) or 8192 (fp32)
@@ -1399,7 +1423,7 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
         else if (stage_rows == 2) CYBQ_STAGE_ROWS_CH(XT, false, 2, 1, 2, 4);               \
         else CYBQ_STAGE_ROWS_CH(XT, NORM, 4, (XT == 2 ? 1 : 2), (XT == 2 ? 2 : 4), (XT == 2 ? 4 : 8)); \
     } while (0)
-            if (eight) {
+            if (stage_rows == 8) {
                 if (batches <= 2) CYBQ_STAGE_ROWS(1, false, 2, 8);
                 else CYBQ_STAGE_ROWS(1, false, 4, 8);
             } else if (xdt == kF32 && epi.gamma) CYBQ_STAGE_ROWS_N(2, true);
@@ -1434,6 +1458,26 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
+}
+
+PrefillRoute prefill_route(const WeightView& w, int xdt, int M, int num_cus, bool exact, size_t workspace_bytes, const Epilogue& epi)
+{
+    const int64_t max_rows = staged_rows(w, workspace_bytes);
+    if (max_rows < 256 || (xdt == kF32 && exact)) return {};
+    const int mc = (int)std::min<int64_t>(M, max_rows);
+    const ChunkPlan p = plan_chunk(w, xdt, mc, num_cus, exact, workspace_bytes / 2, epi);
+    PrefillRoute r = {};
+    if (!exact && xdt != kF16) r.stage_rows = rows_per_staging_workgroup(w, xdt, mc, num_cus, epi.gamma != nullptr);
+    if (p.rows.nf) {
+        r.kernel = 1;
+        r.nf = p.rows.nf;
+        r.splits = 1;
+    } else {
+        r.kernel = p.tiles.kind == TilePlan::kTiles ? 2 : p.tiles.kind == TilePlan::kRoles ? 3 : 4;
+        r.nf = p.tiles.nf;
+        r.splits = p.tiles.splits;
+    }
+    return r;
 }
 
 }  // namespace cybq

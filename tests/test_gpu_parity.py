@@ -2030,6 +2030,60 @@ def test_role_split_kernel_over_ranges_of_k(backend, oracle, bits, N, K, M, ydt)
     assert torch.equal(y, y2)
 
 
+# (the calls above are many ranges of small outputs, the last of them short ranges, which are gemm_kernel's.)  Two, three, four ranges and
+# more, one to five row tiles, seven and eight column blocks, a last range that is shorter
+@pytest.mark.parametrize("bits,N,K,M,nf,splits", [(4, 2050, 16416, 200, 8, 8), (4, 4000, 6176, 700, 8, 2), (8, 3584, 6176, 700, 7, 2), (4, 3100, 6176, 520, 8, 3),
+                                                  (4, 3600, 8224, 300, 8, 4), (8, 1568, 12320, 513, 7, 6), (4, 1000, 12320, 1030, 7, 5)])
+def test_ranges_of_k_have_the_same_bits_in_both_tiled_kernels(backend, oracle, bits, N, K, M, nf, splits):
+    """With roles or with waves that do everything (tuning 2 and 7) a K range is walked and left in its slab alike: plain, with a
+    residual, with a folded norm of bf16 and of f16 rows, as a pair."""
+    qw, wd = _random_weight(backend, bits, N, K, seed=71)
+    r = torch.from_numpy(synth.activations(72, M, N)).cuda()
+    gamma = (1.0 + 0.1 * torch.from_numpy(synth.activations(73, 1, K))[0]).cuda()
+    half = N // 32 * 16
+    qh, hd = _random_weight(backend, bits, half, K, seed=74)
+    pair = backend.fuse_pairs(qh, qh)
+    codes = {"f32": 0, "f16": 1, "bf16": 2}
+
+    def both(w, n, xdt, ydt, call, norm=False, epilogue="none"):
+        out = []
+        for tuning, kernel in ((2, "roles"), (7, "tiles")):
+            backend.set_gemm_tuning(tuning)
+            plan = backend.debug_prefill_plan(w, codes[xdt], M, norm, epilogue)
+            assert plan["kernel"] == kernel and plan["splits"] >= 2, plan
+            if w is qw:
+                assert (plan["nf"], plan["splits"]) == (nf, splits), plan
+            y = torch.full((M, n), float("nan"), dtype=TDT[ydt], device="cuda")
+            call(y)
+            out.append(y)
+        torch.cuda.synchronize()
+        assert torch.equal(*out), (xdt, ydt, norm, epilogue)
+        return out[0].double()
+
+    def rel(y, ref):
+        return ((y - ref).norm() / ref.norm()).item()
+
+    try:
+        x = _x(M, K, "bf16", cfg=75)
+        ref = x.double() @ wd.T
+        assert rel(both(qw, N, "bf16", "f32", lambda y: backend.matmul(qw, x, y)), ref) < FAST
+        rb = r.bfloat16()
+        assert rel(both(qw, N, "bf16", "bf16", lambda y: backend.matmul_ex(qw, x, y, "add", rb), epilogue="add"), ref + rb.double()) < 4e-3
+        for xdt in ("bf16", "f16"):
+            x = _x(M, K, xdt, cfg=75)
+            xd = x.double()
+            ref = (xd * torch.rsqrt((xd * xd).mean(dim=1, keepdim=True) + 1e-5) * gamma.double()) @ wd.T + r.double()
+            y = both(qw, N, xdt, "f32", lambda y: backend.matmul_norm(qw, x, gamma, 1e-5, y, "add", r), norm=True, epilogue="add")
+            assert rel(y, ref) < 2 * FAST, xdt
+        z = xd @ hd.T
+        y = both(pair, half, "f16", "f16", lambda y: backend.matmul_ex(pair, x, y, "swiglu"), epilogue="swiglu")
+        assert rel(y, torch.nn.functional.silu(z) * z) < 4e-3
+    finally:
+        backend.set_gemm_tuning(0)
+    for w in (qw, qh, pair):
+        w.free()
+
+
 @pytest.mark.parametrize("xdt,gdt", [("bf16", "f16"), ("bf16", "f32"), ("f32", "bf16")])
 @pytest.mark.parametrize("K", [32, 512, 544, 2048, 2080, 4128, 8224, 16416])
 def test_row_scaling_pass_at_the_edges_of_its_pieces(backend, oracle, K, xdt, gdt):
