@@ -2106,6 +2106,39 @@ def test_row_scaling_pass_at_the_edges_of_its_pieces(backend, oracle, K, xdt, gd
     assert oracle.rel_l2(got, ref) < FAST and oracle.rel_l2(got[1:2], ref[1:2]) < FAST
 
 
+# (plain bf16 rows of the calls above go to other kernels, and many of the fp32 ones have one way of sharing out.)  A workgroup's sixteen waves share out its
+# rows' pieces of 512 k: sixteen, eight, four to a row with one, two, four rows to the workgroup.  One piece and fewer than waves, a last piece of one group, as many
+# as stay in registers, one more; rows that are no multiple of the workgroup's
+@pytest.mark.parametrize("xdt,rows,M,K", [
+    ("bf16", 1, 37, 8224), ("bf16", 1, 37, 16384), ("bf16", 1, 37, 16416), ("bf16", 1, 33, 32768), ("bf16", 1, 33, 32800),
+    ("bf16", 2, 37, 32), ("bf16", 2, 37, 512), ("bf16", 2, 37, 544), ("bf16", 2, 37, 4096), ("bf16", 2, 37, 4128), ("bf16", 2, 37, 8192),
+    ("bf16", 2, 133, 8224), ("bf16", 2, 133, 16384), ("bf16", 2, 133, 16416),
+    ("bf16", 4, 53, 32), ("bf16", 4, 53, 2080), ("bf16", 4, 53, 4096), ("bf16", 4, 53, 4128), ("bf16", 4, 53, 8192),
+    ("bf16", 4, 389, 8224), ("bf16", 4, 389, 16384), ("bf16", 4, 389, 16416),
+    ("f32", 1, 33, 16416), ("f32", 1, 33, 32800), ("f32", 2, 37, 4128), ("f32", 2, 133, 16416), ("f32", 4, 53, 2048), ("f32", 4, 53, 2080),
+    ("f32", 4, 53, 4128), ("f32", 4, 517, 8224)])
+def test_row_scaling_pass_with_one_two_and_four_rows_to_a_workgroup(backend, oracle, xdt, rows, M, K):
+    N = 48
+    q, s = _quant(oracle, 4, N, K, cfg=76)
+    qw = backend.upload_quantized(q, s, 4)
+    x = _x(M, K, xdt, cfg=77)
+    x[1] *= 1e-6                                       # another power of two
+    y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    backend.set_gemm_tuning(2)                         # the tiled kernels, and no decode passes in their place
+    backend.set_gemv_tuning(0, 2, 0)
+    try:
+        plan = backend.debug_prefill_plan(qw, {"f32": 0, "bf16": 2}[xdt], M)
+        assert plan["stage_rows"] == rows and plan["kernel"] in ("tiles", "roles"), plan
+        backend.matmul(qw, x, y)
+        torch.cuda.synchronize()
+    finally:
+        backend.set_gemm_tuning(0)
+        backend.set_gemv_tuning(0, 0, 0)
+    ref = x.double() @ torch.from_numpy(oracle.dequant(q, s)).cuda().double().T
+    errs = ((y.double() - ref).norm(dim=1) / ref.norm(dim=1)).cpu()
+    assert errs.max().item() < 2 * FAST, int(errs.argmax())     # (a row's 48 outputs; FAST is for all of a call's)
+
+
 @pytest.mark.parametrize("M", [1, 2, 4, 16])
 def test_folded_rmsnorm_counts_subnormal_inputs(backend, oracle, M):
     # a row of f16 subnormals (|x| < 6.1e-5) with an eps far below its mean square: its squares must
