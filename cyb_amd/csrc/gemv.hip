@@ -803,7 +803,14 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
     // wave v finishes outputs v, v + waves, ...: number p is register p % 4 of row block p / 4 % MB of strip p / 4 / MB
     // Their residuals are asked for before the waves' sums meet, and the outputs a wave finishes are walked without a loop, so that their reads go out
     // together.  us per call, before / after: 14336 -> 4096 at 16 f16 rows 11.8 / 11.4, with a residual 11.9 / 11.7, at 30 rows 16.1 / 15.4, a list of
-    // 16 layers at 16 rows 741 / 733; at 8 rows the same.
+    // 16 layers at 16 rows 741 / 733; at 8 rows the same.  (KS: by every workgroup, though only the last to arrive needs them.  By that one alone, next
+    // to the slabs: f16 14336 -> 4096 with a residual at 12 / 20 / 32 rows 12.6, 16.1, 17.2 / 12.6, 16.3, 17.4, bf16 12800 -> 3584 12.1, 15.3, 16.6 /
+    // 12.0, 15.4, 16.6.)
+    // Not with a norm where a workgroup has several strips, but for nine rows and more of Q4 on up to four: the registers are full (Q4 f16 on seven and eight
+    // strips, Q8 f16 on two spill) or there is little to gain.  us per call, one after the other / ahead, f16 with a norm: 5120 -> 28672 at 9 rows
+    // 26.9 / 28.2, as pairs 29.3 / 30.2, 8192 -> 28672 pairs at 16 rows 32.0 / 32.9, Q8 8192 -> 6144 at 9 / 16 rows 19.75 / 19.99, 20.19 / 20.35, bf16 6144 ->
+    // 16384 with a residual at 8 rows 18.5 / 18.7; nine rows, up to four strips: 6144 -> 16384 18.4 / 18.0, 8192 -> 6144 with a residual 11.69 / 11.61.
+    constexpr bool AHEAD = !NORM || NS == 1 || (XR == 16 && BITS == 4 && NS <= 4);
     constexpr int OUTS = NS * MB * 4, AHEAD_OUTS = (OUTS + 7) / 8;
     auto place = [&](int p, int64_t& at) __attribute__((always_inline)) {
         const int r = p & 3, b = (p >> 2) % MB, nt = strip0 + (p >> 2) / MB;
@@ -812,7 +819,7 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
         return p < OUTS && nt < w.NT && m < M && n < w.N;
     };
     uint32_t residual[AHEAD_OUTS] = {};
-    if (epi.kind == kEpiAdd) {
+    if (AHEAD && epi.kind == kEpiAdd) {
 #pragma unroll
         for (int k = 0; k < AHEAD_OUTS; k++) {
             int64_t at;
@@ -937,6 +944,17 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
             int64_t at;
             const bool mine = place(p, at) && epi.kind == kEpiAdd;
             finish(p, whole(p), mine ? load_out_bits(epi.residual, ydt, at) : 0u);
+        }
+        return;
+    }
+    if constexpr (!AHEAD) {
+        for (int p = wv; p < OUTS; p += nwaves) {
+            const int r = p & 3, b = (p >> 2) % MB, s = (p >> 2) / MB;
+            const int nt = strip0 + s;
+            const int n = nt * 16 + (lane & 15);
+            const float v = sum_partials(red + ((s * MB + b) * sums * 4 + r) * 64 + lane, sums, 4 * 64) * rstd[r];
+            const int m = 16 * b + 4 * oct + r;
+            if (nt < w.NT && m < M && n < w.N) emit(y, ydt, epi, (int64_t)m * w.N + n, v);
         }
         return;
     }

@@ -2139,6 +2139,31 @@ def test_row_scaling_pass_with_one_two_and_four_rows_to_a_workgroup(backend, ora
     assert errs.max().item() < 2 * FAST, int(errs.argmax())     # (a row's 48 outputs; FAST is for all of a call's)
 
 
+# (residuals asked for ahead of the sums, and not: Q8, eight rows and fewer, seven strips and more)
+@pytest.mark.parametrize("bits,N,K,M,xdt", [(4, 28672, 4128, 9, "f16"), (4, 28672, 4128, 16, "bf16"), (4, 28670, 4128, 5, "f16"), (8, 6144, 4128, 9, "f16"),
+                                            (8, 6150, 4128, 16, "bf16"), (4, 9212, 4128, 13, "f16"), (4, 9212, 4128, 7, "bf16"), (4, 6142, 4128, 12, "bf16"),
+                                            (4, 6142, 4128, 3, "f16"), (4, 4096, 4128, 11, "f16"), (4, 6142, 1056, 16, "f32"), (4, 6142, 1056, 6, "f32")])
+def test_folded_rmsnorm_with_a_residual_on_several_strips(backend, bits, N, K, M, xdt):
+    qw, wd = _random_weight(backend, bits, N, K, seed=78)
+    x = _x(M, K, xdt, cfg=79)
+    gamma = (1.0 + 0.25 * torch.from_numpy(synth.activations(80, 1, K)[0])).cuda().to(TDT[xdt])
+    r = torch.from_numpy(synth.activations(81, M, N)).cuda()
+    xd = x.double()
+    # x * gamma is an operand of 16 bits where the rows are
+    v = (xd * gamma.double()).to(TDT[xdt]).double() if xdt != "f32" else xd * gamma.double()
+    ref = (v * torch.rsqrt((xd * xd).mean(dim=1, keepdim=True) + 1e-5)) @ wd.T
+    y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    for epilogue, res, want in (("none", None, ref), ("add", r, ref + r.double())):
+        backend.matmul_norm(qw, x, gamma, 1e-5, y, epilogue, res)
+        torch.cuda.synchronize()
+        assert ((y.double() - want).norm() / want.norm()).item() < TIGHT, epilogue
+    y.copy_(r)                                          # the output over the residual
+    backend.matmul_norm(qw, x, gamma, 1e-5, y, "add", y)
+    torch.cuda.synchronize()
+    assert ((y.double() - want).norm() / want.norm()).item() < TIGHT
+    qw.free()
+
+
 @pytest.mark.parametrize("M", [1, 2, 4, 16])
 def test_folded_rmsnorm_counts_subnormal_inputs(backend, oracle, M):
     # a row of f16 subnormals (|x| < 6.1e-5) with an eps far below its mean square: its squares must
