@@ -1107,7 +1107,7 @@ __device__ __forceinline__ void row_chunk_values(const RowChunk<XT>& c, float v[
 // pieces of 512 k numbered p, p + PW, ... of row r (CH of them at most stay in registers between the two steps), the parts
 // of a row meet once through LDS for the row's largest magnitude (and sum of squares).  One wave per row took 5 - 7 us for
 // 512 rows of 4096 and 10 - 12 us for rows of 14336, most of it the latency of one wave walking its row.
-template <int XT, bool NORM, int CH, int ROWS>
+template <int XT, bool NORM, int CH, int ROWS, bool GKEEP = (CH * XT <= 4)>
 __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict__ src, u32x4_t* __restrict__ dst, int M, int K, int first_group,
                                                           int gamma_dt, const void* __restrict__ gamma, float* __restrict__ unscale,
                                                           float* __restrict__ ssq, Touch touch)
@@ -1135,9 +1135,8 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
     // call with its multiply, before / after, bf16: 4096 -> 1024 with a norm at 512 rows 20.5 / 20.4, 14336 -> 1024 at 512 rows 35.7 / 35.4 (other boxes 34.3), Q8
     // 14336 -> 4096 at 2048 rows 209.7 / 204.9, 8192 -> 1024 with a norm at 300 rows 26.2 / 25.6, 4096 -> 28672 norm + SwiGLU at 45 rows 24.2 / 23.1.
     // Pieces past the end of the row are its last chunk again (no branches around the loads); gamma stays with a piece where there are registers
-    // for it - elsewhere it is loaded again for the conversion - and is asked for next to it.
+    // for it (GKEEP) - elsewhere it is loaded again for the conversion - and is asked for next to it.
     RowChunk<XT> keep[CH];
-    constexpr bool GKEEP = CH * XT <= 4;
     Gamma8 gk[NORM && GKEEP ? CH : 1];
     auto chunk_at = [&](int p0, int i) { return (p0 + i * PW + part) * 64 + lane; };
     auto load = [&](int p0) {
@@ -1409,8 +1408,8 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
             // pieces of 512 k a lane keeps in registers: the whole row when it has at most 16384 (bf16) or 8192 (fp32)
             // elements, 16384 with two rows per workgroup, 32768 with one
             const int per_row = 16 / stage_rows, batches = ((K8 + 63) / 64 + per_row - 1) / per_row;
-#define CYBQ_STAGE_ROWS(XT, NORM, CH, ROWS) \
-    hipLaunchKernelGGL((stage_rows_kernel<XT, NORM, CH, ROWS>), rgrid, dim3(1024), 0, st, xs, xst, mc, w.K, touch.first_group, epi.gamma_dt, epi.gamma, unscale, ssq_part, touch)
+#define CYBQ_STAGE_ROWS(XT, NORM, CH, ...) \
+    hipLaunchKernelGGL((stage_rows_kernel<XT, NORM, CH, __VA_ARGS__>), rgrid, dim3(1024), 0, st, xs, xst, mc, w.K, touch.first_group, epi.gamma_dt, epi.gamma, unscale, ssq_part, touch)
 #define CYBQ_STAGE_ROWS_CH(XT, NORM, ROWS, C1, C2, C3)              \
     do {                                                            \
         if (batches <= C1) CYBQ_STAGE_ROWS(XT, NORM, C1, ROWS);     \
@@ -1428,6 +1427,10 @@ hipError_t launch_gemm(const WeightView& w, const void* x, int xdt, int M, void*
                 else CYBQ_STAGE_ROWS(1, false, 4, 8);
             } else if (xdt == kF32 && epi.gamma) CYBQ_STAGE_ROWS_N(2, true);
             else if (xdt == kF32) CYBQ_STAGE_ROWS_N(2, false);
+            // bf16 rows of K over 4096 with a norm: with gamma kept (79 registers, not 47) a CU has room for one workgroup, which is all there is for it
+            // up to four rows per CU, and not beyond.  us per call, kept / loaded twice: 6144 -> 1024 at 768 / 1024 rows 30.3 / 30.9, 33.3 / 34.2, at 1040 /
+            // 1100 / 2048 / 4096 rows 36.6 / 35.7, 38.4 / 36.0, 45.4 / 42.1, 88.0 / 83.6; 8192 -> 4096 at 2048 rows 128.4 / 125.6.
+            else if (epi.gamma && batches > 2 && batches <= 4 && mc > 4 * num_cus) CYBQ_STAGE_ROWS(1, true, 4, 4, false);
             else if (epi.gamma) CYBQ_STAGE_ROWS_N(1, true);
             else CYBQ_STAGE_ROWS_N(1, false);
 #undef CYBQ_STAGE_ROWS_N

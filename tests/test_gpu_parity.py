@@ -2164,6 +2164,26 @@ def test_folded_rmsnorm_with_a_residual_on_several_strips(backend, bits, N, K, M
     qw.free()
 
 
+# (more than four rows per CU: the row-scaling pass loads gamma twice and two of its workgroups share a CU)
+@pytest.mark.parametrize("M", [1024, 1030])
+@pytest.mark.parametrize("K,gdt", [(4128, "f32"), (6144, "f16"), (8192, "bf16")])
+def test_folded_rmsnorm_of_many_rows(backend, oracle, M, K, gdt):
+    N, eps = 48, 1e-5
+    q, s = _quant(oracle, 4, N, K, cfg=82)
+    qw = backend.upload_quantized(q, s, 4)
+    x = _x(M, K, "bf16", cfg=83)
+    x[1] *= 1e-6
+    gamma = (1.0 + 0.25 * torch.from_numpy(synth.activations(84, 1, K)[0])).cuda().to(TDT[gdt])
+    y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    assert backend.debug_prefill_plan(qw, 2, M, norm=True)["stage_rows"] == 4
+    backend.matmul_norm(qw, x, gamma, eps, y)
+    torch.cuda.synchronize()
+    xd = x.double()
+    ref = (xd * torch.rsqrt((xd * xd).mean(dim=1, keepdim=True) + eps) * gamma.double()) @ torch.from_numpy(oracle.dequant(q, s)).cuda().double().T
+    errs = ((y.double() - ref).norm(dim=1) / ref.norm(dim=1)).cpu()
+    assert ((y.double() - ref).norm() / ref.norm()).item() < 2 * FAST and errs.max().item() < 4 * FAST, int(errs.argmax())
+
+
 @pytest.mark.parametrize("M", [1, 2, 4, 16])
 def test_folded_rmsnorm_counts_subnormal_inputs(backend, oracle, M):
     # a row of f16 subnormals (|x| < 6.1e-5) with an eps far below its mean square: its squares must
