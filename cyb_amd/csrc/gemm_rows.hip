@@ -211,9 +211,13 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC 
     // ---- the partial sums meet: every wave leaves all of its blocks, waves 0 .. MF-1 finish a row block each
     // (what that takes from memory is asked for first; ahead of the K loop it cost registers: 4096 -> 14336 at 64 rows 16.9 -> 17.2 us)
     const int mb = (rb0 + min(wv, MF - 1)) * 16;               // first row of the block I finish
-    const RowStats stats = load_row_stats(ns, epi.gamma != nullptr, min(mb + (lane & 15), M - 1), wbase);
+    const bool finishes = !SHARES || shares <= WAVES;          // (else the pass that adds the slabs does, and asks for it)
+    RowStats stats = {};
     Residual<1, NF> res;
-    if (wv < MF) load_residual(res, mb, nt0, M, w.N, y, ydt, epi, lane);
+    if (finishes) {
+        stats = load_row_stats(ns, epi.gamma != nullptr, min(mb + (lane & 15), M - 1), wbase);
+        if (wv < MF) load_residual(res, mb, nt0, M, w.N, y, ydt, epi, lane);
+    }
 #pragma unroll
     for (int i = 0; i < MF; i++)
 #pragma unroll
@@ -230,7 +234,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC 
         tot[0][f] = s;
     }
     if constexpr (SHARES) {
-        if (shares > WAVES) {
+        if (!finishes) {
             write_rows<1, NF>(tot, stg + wv * (16 * NF * 16), (rb0 + wv) * 16, nt0, M, w.N, slabs, kF32, 1.0f, plain, lane);
             return;
         }
