@@ -810,6 +810,9 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
     // strips, Q8 f16 on two spill) or there is little to gain.  us per call, one after the other / ahead, f16 with a norm: 5120 -> 28672 at 9 rows
     // 26.9 / 28.2, as pairs 29.3 / 30.2, 8192 -> 28672 pairs at 16 rows 32.0 / 32.9, Q8 8192 -> 6144 at 9 / 16 rows 19.75 / 19.99, 20.19 / 20.35, bf16 6144 ->
     // 16384 with a residual at 8 rows 18.5 / 18.7; nine rows, up to four strips: 6144 -> 16384 18.4 / 18.0, 8192 -> 6144 with a residual 11.69 / 11.61.
+    // Nor with fewer than eight waves (K under 2048; a K split over workgroups, six waves and more, excepted), which have up to thirty-two outputs each:
+    // one after the other / two or four ahead and the rest behind them, f16: 384 -> 24922 at 11 rows 8.5 / 10.4, 256 -> 32768 at 3 rows 7.1 / 8.8, 512 -> 32768 at
+    // 32 rows 10.3 / 12.0, 640 -> 28672 at 8 rows with a residual 11.4 / 12.7.
     constexpr bool AHEAD = !NORM || NS == 1 || (XR == 16 && BITS == 4 && NS <= 4);
     constexpr int OUTS = NS * MB * 4, AHEAD_OUTS = (OUTS + 7) / 8;
     auto place = [&](int p, int64_t& at) __attribute__((always_inline)) {
@@ -819,7 +822,7 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
         return p < OUTS && nt < w.NT && m < M && n < w.N;
     };
     uint32_t residual[AHEAD_OUTS] = {};
-    if (AHEAD && epi.kind == kEpiAdd) {
+    if (AHEAD && (KS || nwaves == 8) && epi.kind == kEpiAdd) {
 #pragma unroll
         for (int k = 0; k < AHEAD_OUTS; k++) {
             int64_t at;
@@ -947,7 +950,7 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
         }
         return;
     }
-    if constexpr (!AHEAD) {
+    if (!AHEAD || nwaves < 8) {
         for (int p = wv; p < OUTS; p += nwaves) {
             const int r = p & 3, b = (p >> 2) % MB, s = (p >> 2) / MB;
             const int nt = strip0 + s;
@@ -964,12 +967,7 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
     };
 #pragma unroll
     for (int k = 0; k < AHEAD_OUTS; k++)
-        if (wv + k * nwaves < OUTS) finish(wv + k * nwaves, whole(wv + k * nwaves), residual[k]);
-    for (int p = wv + AHEAD_OUTS * nwaves; p < OUTS; p += nwaves) {            // (fewer than eight waves)
-        int64_t at;
-        const bool mine = place(p, at) && epi.kind == kEpiAdd;
-        finish(p, whole(p), mine ? load_out_bits(epi.residual, ydt, at) : 0u);
-    }
+        if (wv + k * 8 < OUTS) finish(wv + k * 8, whole(wv + k * 8), residual[k]);
 }
 
 template <int BITS, int XMODE, int TS, int NS, int XR, int MB = 1, bool STRIPS = false, int SUMS = 1>

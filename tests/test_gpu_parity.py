@@ -2184,6 +2184,23 @@ def test_folded_rmsnorm_of_many_rows(backend, oracle, M, K, gdt):
     assert ((y.double() - ref).norm() / ref.norm()).item() < 2 * FAST and errs.max().item() < 4 * FAST, int(errs.argmax())
 
 
+# (fewer than eight waves finish a workgroup's outputs)
+@pytest.mark.parametrize("bits,N,K,M,xdt", [(4, 24922, 384, 11, "f16"), (4, 9000, 256, 3, "f16"), (8, 8533, 320, 5, "f16"), (4, 5790, 1120, 32, "bf16"), (4, 4099, 1920, 16, "f16"),
+                                            (4, 12290, 896, 16, "f32"), (8, 12290, 1056, 23, "bf16"), (4, 28672, 640, 8, "bf16")])
+def test_batched_rows_of_a_short_k_with_a_residual(backend, bits, N, K, M, xdt):
+    qw, wd = _random_weight(backend, bits, N, K, seed=85)
+    x = _x(M, K, xdt, cfg=86)
+    r = torch.from_numpy(synth.activations(87, M, N)).cuda()
+    ref = x.double() @ wd.T
+    assert ((_run(backend, qw, x).double() - ref).norm() / ref.norm()).item() < TIGHT
+    y = r.clone()                                       # the output over the residual
+    backend.matmul_ex(qw, x, y, "add", y)
+    torch.cuda.synchronize()
+    want = ref + r.double()
+    assert ((y.double() - want).norm() / want.norm()).item() < TIGHT
+    qw.free()
+
+
 @pytest.mark.parametrize("M", [1, 2, 4, 16])
 def test_folded_rmsnorm_counts_subnormal_inputs(backend, oracle, M):
     # a row of f16 subnormals (|x| < 6.1e-5) with an eps far below its mean square: its squares must
