@@ -801,19 +801,17 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
     float* red = reinterpret_cast<float*>(smem);
     const int sums = SUMS * nwaves;
     // wave v finishes outputs v, v + waves, ...: number p is register p % 4 of row block p / 4 % MB of strip p / 4 / MB
-    // Their residuals are asked for before the waves' sums meet, and the outputs a wave finishes are walked without a loop, so that their reads go out
-    // together.  us per call, before / after: 14336 -> 4096 at 16 f16 rows 11.8 / 11.4, with a residual 11.9 / 11.7, at 30 rows 16.1 / 15.4, a list of
-    // 16 layers at 16 rows 741 / 733; at 8 rows the same.  (KS: by every workgroup, though only the last to arrive needs them.  By that one alone, next
-    // to the slabs: f16 14336 -> 4096 with a residual at 12 / 20 / 32 rows 12.6, 16.1, 17.2 / 12.6, 16.3, 17.4, bf16 12800 -> 3584 12.1, 15.3, 16.6 /
-    // 12.0, 15.4, 16.6.)
-    // Not with a norm where a workgroup has several strips, but for nine rows and more of Q4 on up to four: the registers are full (Q4 f16 on seven and eight
-    // strips, Q8 f16 on two spill) or there is little to gain.  us per call, one after the other / ahead, f16 with a norm: 5120 -> 28672 at 9 rows
-    // 26.9 / 28.2, as pairs 29.3 / 30.2, 8192 -> 28672 pairs at 16 rows 32.0 / 32.9, Q8 8192 -> 6144 at 9 / 16 rows 19.75 / 19.99, 20.19 / 20.35, bf16 6144 ->
-    // 16384 with a residual at 8 rows 18.5 / 18.7; nine rows, up to four strips: 6144 -> 16384 18.4 / 18.0, 8192 -> 6144 with a residual 11.69 / 11.61.
-    // Nor with fewer than eight waves (K under 2048; a K split over workgroups, six waves and more, excepted), which have up to thirty-two outputs each:
-    // one after the other / two or four ahead and the rest behind them, f16: 384 -> 24922 at 11 rows 8.5 / 10.4, 256 -> 32768 at 3 rows 7.1 / 8.8, 512 -> 32768 at
-    // 32 rows 10.3 / 12.0, 640 -> 28672 at 8 rows with a residual 11.4 / 12.7.
-    constexpr bool AHEAD = !NORM || NS == 1 || (XR == 16 && BITS == 4 && NS <= 4);
+    // With one strip to a workgroup of eight waves, an output to a wave at most, and where K is split over workgroups, residuals are asked for before the
+    // waves' sums meet and the outputs are not walked in a loop.  us per call, loop / ahead, f16: 4096 -> 4096 at 16 rows 5.34 / 5.21, at 8 rows with a
+    // residual 4.93 / 4.78, with a norm at 16 rows 6.30 / 6.10, bf16 at 32 rows 7.30 / 7.08, Q8 at 16 rows with a residual 6.22 / 6.06; K split: 14336 ->
+    // 4096 at 16 rows 12.9 / 12.4, at 30 rows with a residual 18.4 / 17.6.
+    // (K split: by every workgroup, though only the last to arrive needs them.  By that one alone, next to the slabs: f16 14336 -> 4096 with a residual at
+    // 12 / 20 / 32 rows 12.6, 16.1, 17.2 / 12.6, 16.3, 17.4, bf16 12800 -> 3584 12.1, 15.3, 16.6 / 12.0, 15.4, 16.6.)
+    // Not with more strips, which have little to gain and whose registers are full: pairs 8192 -> 3584 at 6 f16 rows 8.1 / 8.4, Q8 5120 -> 6144 at 32 bf16 rows
+    // 15.9 / 16.3, 2048 -> 4096 5.6 / 5.7, 5120 -> 28672 with a norm at 9 f16 rows 26.9 / 28.2 (spills); no pairs, 5120 -> 6144 at 32 rows f16 0.7 % less, bf16
+    // 1 % more.  Nor with fewer than eight waves (K under 2048): 256 -> 4096 Q8 at 32 rows 5.3 / 5.5, 256 -> 469 at 42 rows 9.3 / 10.1, four strips 384 -> 24922
+    // at 11 rows 9.4 / 10.4.
+    constexpr bool AHEAD = KS || NS == 1;
     constexpr int OUTS = NS * MB * 4, AHEAD_OUTS = (OUTS + 7) / 8;
     auto place = [&](int p, int64_t& at) __attribute__((always_inline)) {
         const int r = p & 3, b = (p >> 2) % MB, nt = strip0 + (p >> 2) / MB;
@@ -950,24 +948,21 @@ void gemv_rows_kernel(const uint8_t* __restrict__ wbase, const uint16_t* __restr
         }
         return;
     }
-    if (!AHEAD || nwaves < 8) {
-        for (int p = wv; p < OUTS; p += nwaves) {
-            const int r = p & 3, b = (p >> 2) % MB, s = (p >> 2) / MB;
-            const int nt = strip0 + s;
-            const int n = nt * 16 + (lane & 15);
-            const float v = sum_partials(red + ((s * MB + b) * sums * 4 + r) * 64 + lane, sums, 4 * 64) * rstd[r];
-            const int m = 16 * b + 4 * oct + r;
-            if (nt < w.NT && m < M && n < w.N) emit(y, ydt, epi, (int64_t)m * w.N + n, v);
+    if constexpr (AHEAD) {
+        if (nwaves == 8) {
+            const int r = wv & 3, b = (wv >> 2) % MB;
+            if (wv < OUTS) finish(wv, sum_partials(red + (b * sums * 4 + r) * 64 + lane, sums, 4 * 64) * rstd[r], residual[0]);
+            return;
         }
-        return;
     }
-    auto whole = [&](int p) __attribute__((always_inline)) {
+    for (int p = wv; p < OUTS; p += nwaves) {
         const int r = p & 3, b = (p >> 2) % MB, s = (p >> 2) / MB;
-        return sum_partials(red + ((s * MB + b) * sums * 4 + r) * 64 + lane, sums, 4 * 64) * rstd[r];
-    };
-#pragma unroll
-    for (int k = 0; k < AHEAD_OUTS; k++)
-        if (wv + k * 8 < OUTS) finish(wv + k * 8, whole(wv + k * 8), residual[k]);
+        const int nt = strip0 + s;
+        const int n = nt * 16 + (lane & 15);
+        const float v = sum_partials(red + ((s * MB + b) * sums * 4 + r) * 64 + lane, sums, 4 * 64) * rstd[r];
+        const int m = 16 * b + 4 * oct + r;
+        if (nt < w.NT && m < M && n < w.N) emit(y, ydt, epi, (int64_t)m * w.N + n, v);
+    }
 }
 
 template <int BITS, int XMODE, int TS, int NS, int XR, int MB = 1, bool STRIPS = false, int SUMS = 1>
