@@ -144,9 +144,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                                                    int N_, void* __restrict__ y, int ydt, float out_scale,
                                                    float* __restrict__ part, Epilogue epi, NormStats ns)
 {
-    // (leading scalar arguments in the order of their first use: they arrive in registers at wave start.  K among them, and the staging pass's
-    // first_group: with those the first requests wait for no argument.  us per call: 4096 -> 14336 at 64 fp32-out rows 16.9 / 16.4, 4096 -> 28672 at 64
-    // rows 28.4 / 27.2, 32-layer list at 45 rows 2555 / 2495.)
+    // (leading scalar arguments in the order of their first use: they arrive in registers at wave start.  With K behind the output's address, us per call: here no
+    // difference, 14336 -> 4096 at 1000 rows 119.8 / 119.8; in gemm_roles_kernel 14336 -> 4096 at 512 rows 67.2 / 66.8, 10240 -> 3136 46.2 / 45.8, 4096 -> 6144 with
+    // a norm 37.3 / 37.1.)
     const WeightView w = {wbase, N_, K_, NT_, KT_, BITS};
     // Workgroups are handed to the 8 XCDs round-robin (id % 8) and every XCD has
     // its own L2.  Give each XCD a contiguous run of tiles in row-block-major
@@ -804,6 +804,10 @@ struct TilePlan {
 // The tiled kernels' way with a call, and an estimate of its time behind the staging pass in us (< 0: whatever the others take).
 // The estimates are fits to 1900 calls of 33 .. 600 rows on N of 512 .. 32768, K of 512 .. 14336 (Q4 and Q8, bf16; 4 - 8 % rms): a
 // round of workgroups costs a fixed part and so much per K tile, whatever the number of workgroups in it.
+// For the K ranges of the role-split kernel it is gemm_kernel's line, 7 % too long (52 calls: 0.81 - 0.99 of gemm_kernel's time, about 1.12 per K tile instead of
+// 1.29).  It stays for what it decides, against gemm_cols.hip, whose line is off by as much: of 36 calls drawn from those that 1.12 would move from there,
+// 18 take 4.7 % less in the mean (Q8 8480 -> 7056 at 182 bf16 rows 47.9 / 42.2) and 18 up to 19 % more (f16 rows, which have no staging launch there: Q8 12032 -> 1007
+// at 1298 rows 46.1 / 54.9, Q4 7744 -> 1663 at 1502 49.4 / 56.6).
 static float tiled_plan(const WeightView& w, int M, bool exact, int num_cus, size_t part_bytes, const Epilogue& epi, TilePlan& plan)
 {
     const int64_t cus = num_cus;
@@ -874,7 +878,8 @@ static float tiled_plan(const WeightView& w, int M, bool exact, int num_cus, siz
     const int per = (w.KT + splits - 1) / splits;
     splits = (w.KT + per - 1) / per;                             // no empty split
     plan = {TilePlan::kTiles, nf, 8, 2, splits, {}};
-    // Their K ranges go to the role-split kernel where they are long and there are three of them or up to three row tiles; the bits are the same.  us per
+    // Their K ranges go to the role-split kernel where they are long and there are three of them or up to three row tiles; the bits are the same (a tuning
+    // value keeps them in gemm_kernel, and a test compares).  us per
     // call, gemm_kernel / role-split: 14336 -> 4096 at 512 rows 68.5 / 66.3, Q8 70.6 / 68.8, 10240 -> 3136 at 512 rows 46.3 / 44.9, 12288 -> 8192 at 256 rows
     // 59.4 / 57.9, Q8 11168 -> 2145 at 1020 rows 69.3 / 65.2.  Two ranges of more row tiles: 14336 -> 4096 at 1000 rows 121.3 / 123.0, 5760 -> 1959 at 1551 rows
     // 54.2 / 54.9; short ranges: Q8 14336 -> 1024 at 700 rows (14 K tiles) 39.4 / 40.0.
@@ -1132,8 +1137,11 @@ __global__ __launch_bounds__(1024) void stage_rows_kernel(const void* __restrict
 
     // ---- the row's largest magnitude (and sum of squares)
     // What the pass waits for is latency: rows and gamma are asked for together and without branches, two pieces share a barrier on their way out.  us per
-    // call with its multiply, before / after, bf16: 4096 -> 1024 with a norm at 512 rows 20.5 / 20.4, 14336 -> 1024 at 512 rows 35.7 / 35.4 (other boxes 34.3), Q8
-    // 14336 -> 4096 at 2048 rows 209.7 / 204.9, 8192 -> 1024 with a norm at 300 rows 26.2 / 25.6, 4096 -> 28672 norm + SwiGLU at 45 rows 24.2 / 23.1.
+    // call with its multiply, without the three / with them, bf16: 14336 -> 1024 at 512 rows 35.0 / 33.9, 14336 -> 4096 at 45 rows 22.6 / 22.2, Q8 at 2048 rows
+    // 214.2 / 209.6, 4096 -> 1024 with a norm at 512 rows 20.2 / 20.0, 8192 -> 1024 with a norm at 300 rows 26.2 / 25.5, 4096 -> 28672 norm + SwiGLU at 45 rows 27.7 /
+    // 26.9.  One of them taken out of the three: gamma kept 25.9 / 25.5, 27.7 / 26.8 in the last two (19.7 / 19.9 at 512 rows of 4096); the shared barrier 34.6 /
+    // 34.4, 22.6 / 22.4, 209.5 / 208.8 in the first three; what is left there is the loads'.  (The first touching workgroup's number comes in a register too, ahead
+    // of what only that one reads: 4096 -> 14336 at 64 rows 16.9 / 16.4, 4096 -> 28672 SwiGLU at 64 rows 28.4 / 27.2.)
     // Pieces past the end of the row are its last chunk again (no branches around the loads); gamma stays with a piece where there are registers
     // for it (GKEEP) - elsewhere it is loaded again for the conversion - and is asked for next to it.
     RowChunk<XT> keep[CH];
